@@ -86,7 +86,8 @@ struct AttnMinWaves { static constexpr int N = (HS == 32 && MODE == ATTN_BIAS) ?
 
 // OUT_FP8: write e4m3 (value*out_scale) instead of the input element type.
 // COOP: the workgroup's outputs leave through an LDS tile as whole row segments (see s_out below; the launcher says when).
-template <int HS, int MODE, int OUT_FP8, int IN_DT, int COOP = 0>
+// LAST (ATTN_CAUSAL): only token 63's output is wanted: the query tile of tokens 32..63 alone runs and that one row is stored, at row b.
+template <int HS, int MODE, int OUT_FP8, int IN_DT, int COOP = 0, int LAST = 0>
 __global__ void __launch_bounds__(64 * AttnWaves<MODE>::N, (AttnMinWaves<HS, MODE>::N)) attention_kernel(const AttnArgs a) {
   typedef Half16<IN_DT> H16;
   typedef typename H16::vec hvec;
@@ -99,6 +100,8 @@ __global__ void __launch_bounds__(64 * AttnWaves<MODE>::N, (AttnMinWaves<HS, MOD
   // per row. A wave's own output is 64 row pieces of 32 (e4m3) or 64 bytes, which it would have to store 16 bytes per
   // lane and row, a quarter or an eighth of a line at a time; gathered here, the workgroup stores whole lines (measured
   // on 4096 positions x 32 heads in e4m3: the stores were 9 % of the kernel's bytes and 21 % of its time).
+  static_assert(!LAST || (MODE == ATTN_CAUSAL && !COOP), "one-row form");
+  constexpr int IT0 = LAST ? 1 : 0;   // first query tile
   static_assert(!COOP || (HS == 32 && (NW == 4 || NW == 8 || NW == 16)), "the output tile is laid out for head size 32");
   constexpr int OSZ = OUT_FP8 ? 1 : 2;
   constexpr int OROW = NW * HS * OSZ, OSTRIDE = OROW + 16;
@@ -185,7 +188,9 @@ __global__ void __launch_bounds__(64 * AttnWaves<MODE>::N, (AttnMinWaves<HS, MOD
     for (int ks = 0; ks < KS; ++ks) {
       const uint16_t* qa = qp + (long)(32 * t + lr) * a.ldq + 16 * ks + 8 * g;
       const uint16_t* ka = kp + (long)(32 * t + lr) * a.ldk + 16 * ks + 8 * g;
-      if (qk_once) {
+      if (LAST && t < IT0) {
+        kf[t][ks] = *reinterpret_cast<const hvec*>(ka);
+      } else if (qk_once) {
         qf[t][ks] = __builtin_bit_cast(hvec, attn_load_once(qa));
         kf[t][ks] = __builtin_bit_cast(hvec, attn_load_once(ka));
       } else {
@@ -209,7 +214,7 @@ __global__ void __launch_bounds__(64 * AttnWaves<MODE>::N, (AttnMinWaves<HS, MOD
       bp += (long)unit * 4096 + (lane << 3);
     }
 #pragma unroll
-    for (int it = 0; it < 2; ++it)
+    for (int it = IT0; it < 2; ++it)
 #pragma unroll
       for (int jt = 0; jt < 2; ++jt)
 #pragma unroll
@@ -222,7 +227,7 @@ __global__ void __launch_bounds__(64 * AttnWaves<MODE>::N, (AttnMinWaves<HS, MOD
 #pragma unroll
   for (int jt = 0; jt < 2; ++jt)
 #pragma unroll
-    for (int it = 0; it < 2; ++it)
+    for (int it = IT0; it < 2; ++it)
 #pragma unroll
       for (int r = 0; r < 16; ++r) s[jt][it][r] = 0.f;
 
@@ -234,7 +239,7 @@ __global__ void __launch_bounds__(64 * AttnWaves<MODE>::N, (AttnMinWaves<HS, MOD
 #pragma unroll
     for (int jt = 0; jt < 2; ++jt)
 #pragma unroll
-      for (int it = 0; it < 2; ++it)
+      for (int it = IT0; it < 2; ++it)
 #pragma unroll
         for (int r = 0; r < 16; ++r) sp[jt][it][r] = 0.f;
 #pragma unroll
@@ -249,7 +254,7 @@ __global__ void __launch_bounds__(64 * AttnWaves<MODE>::N, (AttnMinWaves<HS, MOD
 #pragma unroll
       for (int t = 0; t < 2; ++t) pf[t] = *reinterpret_cast<const hvec*>(pp + (long)(32 * t + lr) * ldp + 16 * ks + 8 * g);
 #pragma unroll
-      for (int it = 0; it < 2; ++it) {
+      for (int it = IT0; it < 2; ++it) {
         const hvec qu = add_bias_h<H16>(qf[it][ks], ub);
         const hvec qv = add_bias_h<H16>(qf[it][ks], vb);
 #pragma unroll
@@ -265,7 +270,7 @@ __global__ void __launch_bounds__(64 * AttnWaves<MODE>::N, (AttnMinWaves<HS, MOD
 #pragma unroll
     for (int jt = 0; jt < 2; ++jt)
 #pragma unroll
-      for (int it = 0; it < 2; ++it)
+      for (int it = IT0; it < 2; ++it)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const int m = 32 * jt + 8 * (r >> 2) + 4 * g + (r & 3);
@@ -277,7 +282,7 @@ __global__ void __launch_bounds__(64 * AttnWaves<MODE>::N, (AttnMinWaves<HS, MOD
 #pragma unroll
     for (int jt = 0; jt < 2; ++jt)
 #pragma unroll
-      for (int it = 0; it < 2; ++it)
+      for (int it = IT0; it < 2; ++it)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const int j = 32 * jt + 8 * (r >> 2) + 4 * g + (r & 3);
@@ -294,12 +299,12 @@ __global__ void __launch_bounds__(64 * AttnWaves<MODE>::N, (AttnMinWaves<HS, MOD
 #pragma unroll
       for (int jt = 0; jt < 2; ++jt)
 #pragma unroll
-        for (int it = 0; it < 2; ++it)
+        for (int it = IT0; it < 2; ++it)
           s[jt][it] = H16::mfma(kf[jt][ks], qf[it][ks], s[jt][it]);
 
     if constexpr (MODE == ATTN_BIAS) {
 #pragma unroll
-      for (int it = 0; it < 2; ++it)
+      for (int it = IT0; it < 2; ++it)
 #pragma unroll
         for (int jt = 0; jt < 2; ++jt)
 #pragma unroll
@@ -316,7 +321,7 @@ __global__ void __launch_bounds__(64 * AttnWaves<MODE>::N, (AttnMinWaves<HS, MOD
 #pragma unroll
       for (int jt = 0; jt < 2; ++jt)
 #pragma unroll
-        for (int it = 0; it < 2; ++it)
+        for (int it = IT0; it < 2; ++it)
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
             float x = s[jt][it][r] * a.scale;
@@ -333,7 +338,7 @@ __global__ void __launch_bounds__(64 * AttnWaves<MODE>::N, (AttnMinWaves<HS, MOD
   // ---- softmax over keys (registers + lane^32) ------------------------------------------
   float inv_l[2];
 #pragma unroll
-  for (int it = 0; it < 2; ++it) {
+  for (int it = IT0; it < 2; ++it) {
     float mx = -INFINITY;
 #pragma unroll
     for (int jt = 0; jt < 2; ++jt)
@@ -365,7 +370,7 @@ __global__ void __launch_bounds__(64 * AttnWaves<MODE>::N, (AttnMinWaves<HS, MOD
 #pragma unroll
   for (int dt = 0; dt < DT_TILES; ++dt)
 #pragma unroll
-    for (int it = 0; it < 2; ++it)
+    for (int it = IT0; it < 2; ++it)
 #pragma unroll
       for (int r = 0; r < 16; ++r) o[dt][it][r] = 0.f;
 
@@ -374,7 +379,7 @@ __global__ void __launch_bounds__(64 * AttnWaves<MODE>::N, (AttnMinWaves<HS, MOD
     const int jt = kb >> 1, kh = kb & 1;
     hvec pf[2];
 #pragma unroll
-    for (int it = 0; it < 2; ++it)
+    for (int it = IT0; it < 2; ++it)
 #pragma unroll
       for (int e = 0; e < 8; ++e) pf[it][e] = (typename H16::elem)s[jt][it][8 * kh + e];
 #pragma unroll
@@ -385,15 +390,16 @@ __global__ void __launch_bounds__(64 * AttnWaves<MODE>::N, (AttnMinWaves<HS, MOD
       const uint4 packed = make_uint4(lo.x, lo.y, hi.x, hi.y);
       const hvec vf = __builtin_bit_cast(hvec, packed);
 #pragma unroll
-      for (int it = 0; it < 2; ++it) o[dt][it] = H16::mfma(vf, pf[it], o[dt][it]);
+      for (int it = IT0; it < 2; ++it) o[dt][it] = H16::mfma(vf, pf[it], o[dt][it]);
     }
   }
 
   // ---- normalise and store ----------------------------------------------------------------
   float am = 0.f;
 #pragma unroll
-  for (int it = 0; it < 2; ++it) {
-    const long row = (long)b * 64 + 32 * it + lr;
+  for (int it = IT0; it < 2; ++it) {
+    const long row = LAST ? (long)b : (long)b * 64 + 32 * it + lr;
+    const bool keep_row = !LAST || lr == 31;
 #pragma unroll
     for (int dt = 0; dt < DT_TILES; ++dt)
 #pragma unroll
@@ -427,12 +433,12 @@ __global__ void __launch_bounds__(64 * AttnWaves<MODE>::N, (AttnMinWaves<HS, MOD
         if constexpr (OUT_FP8) {
           const uint2 w = g ? make_uint2(r0, pk[keep][0]) : make_uint2(pk[keep][0], r0);
           if constexpr (coop) *reinterpret_cast<uint2*>(s_out + (32 * it + lr) * OSTRIDE + (wave * HS + d) * OSZ) = w;
-          else *reinterpret_cast<uint2*>(reinterpret_cast<uint8_t*>(a.out) + off) = w;
+          else if (keep_row) *reinterpret_cast<uint2*>(reinterpret_cast<uint8_t*>(a.out) + off) = w;
         } else {
           const uint32_t r1 = __shfl_xor(pk[give][1], 32, 64);
           const uint4 w = g ? make_uint4(r0, r1, pk[keep][0], pk[keep][1]) : make_uint4(pk[keep][0], pk[keep][1], r0, r1);
           if constexpr (coop) *reinterpret_cast<uint4*>(s_out + (32 * it + lr) * OSTRIDE + (wave * HS + d) * OSZ) = w;
-          else *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(a.out) + off) = w;
+          else if (keep_row) *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(a.out) + off) = w;
         }
       }
   }
@@ -476,7 +482,7 @@ __global__ void __launch_bounds__(256) causal_long_kernel(const AttnArgs a) {
   const int lr = lane & 31, g = lane >> 5;
   const int T = a.T, nqb = (T + 63) >> 6;
   const int unit = blockIdx.x * 4 + wave;
-  if (unit >= a.B * a.H * nqb) return;
+  if (unit >= a.B * a.H * (a.last_row ? 1 : nqb)) return;
   // Longest units (last query block) first: they walk the most key blocks.
   const int qb = nqb - 1 - unit / (a.B * a.H);
   const int bh = unit % (a.B * a.H);
@@ -614,9 +620,9 @@ __global__ void __launch_bounds__(256) causal_long_kernel(const AttnArgs a) {
 #pragma unroll
   for (int it = 0; it < 2; ++it) {
     const int i = 64 * qb + 32 * it + lr;
-    if (i >= T) continue;
+    if (i >= T || (a.last_row && i != T - 1)) continue;
     const float inv_l = 1.0f / run_l[it];
-    const long row = row0 + i;
+    const long row = a.last_row ? (long)b : row0 + i;
 #pragma unroll
     for (int dt = 0; dt < DT_TILES; ++dt)
 #pragma unroll
@@ -645,7 +651,7 @@ __global__ void __launch_bounds__(256) causal_long_kernel(const AttnArgs a) {
 
 template <int HS, int IN_DT>
 static hipError_t launch_causal_long_dt(const AttnArgs& a, hipStream_t st) {
-  const long units = (long)a.B * a.H * ((a.T + 63) / 64);
+  const long units = (long)a.B * a.H * (a.last_row ? 1 : (a.T + 63) / 64);   // (the last token sits in the block that is walked first)
   const dim3 grid((unsigned)((units + 3) / 4)), block(256);
   if (a.out_dtype == DT_FP8) hipLaunchKernelGGL((causal_long_kernel<HS, 1, IN_DT>), grid, block, 0, st, a);
   else if (a.out_dtype == IN_DT) hipLaunchKernelGGL((causal_long_kernel<HS, 0, IN_DT>), grid, block, 0, st, a);
@@ -667,9 +673,17 @@ static hipError_t launch_attn_dt(const AttnArgs& a, hipStream_t st) {
     // Whole workgroups only: H a multiple of 4 puts four heads of one position in every workgroup and leaves none partly
     // filled; 16-byte stores need rows and base aligned to that.
     const int osz = a.out_dtype == DT_FP8 ? 1 : 2;
-    if (a.H % NW == 0 && (a.ldo * osz) % 16 == 0 && (reinterpret_cast<uintptr_t>(a.out) & 15) == 0) {
+    if (!a.last_row && a.H % NW == 0 && (a.ldo * osz) % 16 == 0 && (reinterpret_cast<uintptr_t>(a.out) & 15) == 0) {
       if (a.out_dtype == DT_FP8) hipLaunchKernelGGL((attention_kernel<HS, MODE, 1, IN_DT, 1>), grid, block, 0, st, a);
       else if (a.out_dtype == IN_DT) hipLaunchKernelGGL((attention_kernel<HS, MODE, 0, IN_DT, 1>), grid, block, 0, st, a);
+      else return hipErrorInvalidValue;
+      return hipGetLastError();
+    }
+  }
+  if constexpr (MODE == ATTN_CAUSAL) {
+    if (a.last_row) {
+      if (a.out_dtype == DT_FP8) hipLaunchKernelGGL((attention_kernel<HS, MODE, 1, IN_DT, 0, 1>), grid, block, 0, st, a);
+      else if (a.out_dtype == IN_DT) hipLaunchKernelGGL((attention_kernel<HS, MODE, 0, IN_DT, 0, 1>), grid, block, 0, st, a);
       else return hipErrorInvalidValue;
       return hipGetLastError();
     }
@@ -704,6 +718,7 @@ hipError_t launch_attention(const AttnArgs& a, int head_dim, hipStream_t st) {
   if (a.ldq % 8 || a.ldk % 8 || a.ldv % 8 || a.ldo % 4 || a.qk_hstride % 8 || (a.qk_hstride && (a.qk_hstride < head_dim || (a.T != 0 && a.T != 64))) ||
       (reinterpret_cast<uintptr_t>(a.q) & 15) || (reinterpret_cast<uintptr_t>(a.k) & 15) || (reinterpret_cast<uintptr_t>(a.v) & 15))
     return hipErrorInvalidValue;
+  if (a.last_row && (a.mode != ATTN_CAUSAL || a.amax)) return hipErrorInvalidValue;
   if (a.mode == ATTN_BIAS && !a.bias) return hipErrorInvalidValue;
   if (a.mode == ATTN_BIAS && a.bias_blocked && ((long)a.B * a.H) % 256 != 0) return hipErrorInvalidValue;
   if (a.mode == ATTN_RELSHIFT && (!a.pos || !a.u_bias || !a.v_bias)) return hipErrorInvalidValue;

@@ -222,6 +222,7 @@ struct AttnArgs {
   long ldo;
   float* amax;
   int B, H, mode, out_dtype;
+  int last_row;         // ATTN_CAUSAL: only the last token's row of each position is wanted, written at row b of `out`
   int T;                // tokens per position; 0 or 64 for the single-tile kernel, more only with ATTN_CAUSAL
   int in_dtype;         // DT_BF16 or DT_F16: element type of q, k, v, bias and pos
   float scale, out_scale;

@@ -597,9 +597,14 @@ int Model::forward_chunk(const float* planes, const uint8_t* ids, const uint8_t*
   const float attn_scale = cfg.arch == CRL_ARCH_BT4 ? 1.0f / std::sqrt((float)C) : 1.0f / std::sqrt((float)hs);
   const float alpha = cfg.arch == CRL_ARCH_BT4CLASS ? std::pow(2.0f * (float)L, -0.25f) : 1.0f;
 
+  // GPT64 asked for the last token's logits alone: behind its keys and values, the last layer runs on that token's row of
+  // every position only (queries, output projection, MLP: 10/12 of the layer's products; bit-equal, a row's result does
+  // not depend on the other rows). The rows are compact from the attention on: ao [mb, C], the stream in ws.t [mb, C].
+  const bool one_row = gpt && policy && !all_logits && !calibrate && L > 0;
   for (int l = l0; l < l1; ++l) {
     const Layer& ly = layers[l];
     const bool last = l + 1 == l1;
+    const bool tail = one_row && last;
     const void* a_in; int a_dt; float a_sc = 1.f;
     if (gpt) {
       // h = LN1(x)
@@ -612,7 +617,15 @@ int Model::forward_chunk(const float* planes, const uint8_t* ids, const uint8_t*
     {
       GOpt o; o.a_scale = a_sc;
       if (cfg.arch == CRL_ARCH_BT4CLASS) { o.C2 = ws.comp; o.ldc2 = cfg.smolgen_compress; o.nsplit = 3 * C; }
-      RUN(gemm(ly.qkv, a_in, C, a_dt, ws.qkv, 3 * C, ad, M, o, st));
+      // (the third of the product that makes unread queries costs more than a second launch from about 16384 rows on)
+      if (tail && M >= 16384) {
+        char* const qkv_last = reinterpret_cast<char*>(ws.qkv) + (size_t)(T - 1) * 3 * C * dtype_size(ad);
+        const char* const a_last = reinterpret_cast<const char*>(a_in) + (size_t)(T - 1) * C * dtype_size(a_dt);
+        RUN(gemm(ly.qkv.rows(C, 2 * C), a_in, C, a_dt, reinterpret_cast<char*>(ws.qkv) + (size_t)C * dtype_size(ad), 3 * C, ad, M, o, st));
+        RUN(gemm(ly.qkv.rows(0, C), a_last, (long)T * C, a_dt, qkv_last, (long)T * 3 * C, ad, mb, o, st));
+      } else {
+        RUN(gemm(ly.qkv, a_in, C, a_dt, ws.qkv, 3 * C, ad, M, o, st));
+      }
     }
     if (kv_capture) HIPCHK(launch_kv_store(ws.qkv, kv_layers[l], mb, T, kv_Tmax, C, st));
     const void* bias_tile = nullptr;
@@ -644,7 +657,7 @@ int Model::forward_chunk(const float* planes, const uint8_t* ids, const uint8_t*
       a.bias = bias_tile; a.bias_blocked = bias_blocked ? 1 : 0; a.pos = ly.pos; a.u_bias = ly.u_bias; a.v_bias = ly.v_bias;
       a.out = f8 ? (void*)ws.ao8 : (void*)ws.ao; a.ldo = C; a.out_dtype = f8 ? DT_FP8 : ad;
       a.out_scale = f8 ? act_scale(l, 1) : 1.f; a.amax = am(l, 1);
-      a.B = mb; a.H = H; a.scale = attn_scale; a.in_dtype = ad; a.T = T;
+      a.B = mb; a.H = H; a.scale = attn_scale; a.in_dtype = ad; a.T = T; a.last_row = tail ? 1 : 0;
       a.mode = gpt ? ATTN_CAUSAL : cfg.arch == CRL_ARCH_BT4 ? ATTN_RELSHIFT : ATTN_BIAS;
       prof_begin(1, st);
       hipError_t he = launch_attention(a, hs, st);
@@ -655,13 +668,16 @@ int Model::forward_chunk(const float* planes, const uint8_t* ids, const uint8_t*
     const int ao_dt = f8 ? DT_FP8 : ad;
     if (gpt) {
       // x += proj(ao);  h = LN2(x);  x += proj2(gelu(fc(h)))
-      { GOpt o; o.res = ws.x; o.ldr = C; o.res_dt = xdt; o.a_scale = f8 ? act_scale(l, 1) : 1.f;
-        RUN(gemm(ly.proj, ao_in, C, ao_dt, ws.x, C, xdt, M, o, st)); }
-      RUN(lnorm(ws.x, C, xdt, ly.ln2_g, ly.ln2_b, f8 ? nullptr : ws.h, ad, f8 ? ws.h8 : nullptr, f8 ? act_scale(l, 2) : 1.f, C, M, C, am(l, 2), st));
+      const int rows = tail ? mb : M;
+      void* const x = tail ? ws.t : ws.x;
+      const char* const x_res = reinterpret_cast<const char*>(ws.x) + (tail ? (size_t)(T - 1) * C * dtype_size(xdt) : 0);
+      { GOpt o; o.res = x_res; o.ldr = tail ? (long)T * C : C; o.res_dt = xdt; o.a_scale = f8 ? act_scale(l, 1) : 1.f;
+        RUN(gemm(ly.proj, ao_in, C, ao_dt, x, C, xdt, rows, o, st)); }
+      RUN(lnorm(x, C, xdt, ly.ln2_g, ly.ln2_b, f8 ? nullptr : ws.h, ad, f8 ? ws.h8 : nullptr, f8 ? act_scale(l, 2) : 1.f, C, rows, C, am(l, 2), st));
       { GOpt o; o.act = ACT_GELU; o.a_scale = f8 ? act_scale(l, 2) : 1.f; o.out_scale = f8 ? act_scale(l, 3) : 1.f; o.amax = am(l, 3);
-        RUN(gemm(ly.ff1, f8 ? (const void*)ws.h8 : (const void*)ws.h, C, ao_dt, f8 ? (void*)ws.f8 : (void*)ws.f, F, ao_dt, M, o, st)); }
-      { GOpt o; o.res = ws.x; o.ldr = C; o.res_dt = xdt; o.a_scale = f8 ? act_scale(l, 3) : 1.f;
-        RUN(gemm(ly.ff2, f8 ? (const void*)ws.f8 : (const void*)ws.f, F, ao_dt, ws.x, C, xdt, M, o, st)); }
+        RUN(gemm(ly.ff1, f8 ? (const void*)ws.h8 : (const void*)ws.h, C, ao_dt, f8 ? (void*)ws.f8 : (void*)ws.f, F, ao_dt, rows, o, st)); }
+      { GOpt o; o.res = x; o.ldr = C; o.res_dt = xdt; o.a_scale = f8 ? act_scale(l, 3) : 1.f;
+        RUN(gemm(ly.ff2, f8 ? (const void*)ws.f8 : (const void*)ws.f, F, ao_dt, x, C, xdt, rows, o, st)); }
     } else {
       // t = x + alpha*proj(ao);  h = LN1(t). With `fold` the normalised tensors x and h exist only as e4m3 copies
       // (the products' operands): the LayerNorm launches leave their row statistics behind, and the product that
@@ -718,8 +734,8 @@ int Model::forward_chunk(const float* planes, const uint8_t* ids, const uint8_t*
     }
     if (policy) {
       // ln_f and lm_head on the last token only (model_bis.py:195-196, 369-370).
-      const char* last_tok = reinterpret_cast<const char*>(ws.x) + (size_t)(T - 1) * C * dtype_size(xdt);
-      RUN(lnorm(last_tok, (long)T * C, xdt, lnf_g, lnf_b, f8h ? nullptr : ws.hl, hd, f8h ? ws.hl8 : nullptr, hsc, C, mb, C, nullptr, st));
+      const char* last_tok = one_row ? reinterpret_cast<const char*>(ws.t) : reinterpret_cast<const char*>(ws.x) + (size_t)(T - 1) * C * dtype_size(xdt);
+      RUN(lnorm(last_tok, one_row ? C : (long)T * C, xdt, lnf_g, lnf_b, f8h ? nullptr : ws.hl, hd, f8h ? ws.hl8 : nullptr, hsc, C, mb, C, nullptr, st));
       GOpt o; o.a_scale = hsc;
       RUN(gemm(lm_head, f8h ? (const void*)ws.hl8 : (const void*)ws.hl, C, f8h ? DT_FP8 : hd, policy, VOCAB_RL, DT_F32, mb, o, st));
     }

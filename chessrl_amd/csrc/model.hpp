@@ -22,6 +22,15 @@ struct Lin {
   float* b = nullptr;
   int N = 0, K = 0, dt = DT_BF16;
   float wscale = 1.f;
+  // Output rows [first, first + count) of this layer, as a layer of its own on the same memory.
+  Lin rows(int first, int count) const {
+    Lin r = *this;
+    if (w) r.w = static_cast<char*>(w) + (size_t)first * K * dtype_size(dt);
+    if (w8) r.w8 = static_cast<char*>(w8) + (size_t)first * K;
+    if (b) r.b = b + first;
+    r.N = count;
+    return r;
+  }
 };
 
 struct Layer {

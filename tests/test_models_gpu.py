@@ -738,6 +738,21 @@ def test_generate_forced_tokens(cuda):
     assert row[1:i].count(1926) == 5 and row[i + 2] == 1927
 
 
+@pytest.mark.parametrize("kw", [{}, {"act_dtype": "f16"}, {"fp8": True}, {"stream_f32": False}])
+@pytest.mark.parametrize("B,t", [(1, 0), (3, 1), (255, 0), (256, 0), (250, 3), (130, 66)])
+def test_gpt_last_token_row(cuda, kw, B, t):
+    """The logits of the last token alone, whose last layer runs on one row per position (with its queries in a product of
+    their own from 16384 rows on), are bit-equal to that token's row of the all-token logits."""
+    m = models.GPT(models.GPTConfig(block_size=256, vocab_size=1929, n_layer=2, n_head=4, n_embd=256), **kw)
+    planes = positions(B, seed=9)[0].to(cuda)
+    idx = torch.randint(0, 1924, (B, t), generator=torch.Generator().manual_seed(3)).to(cuda)
+    if kw.get("fp8"):
+        m.calibrate(planes)
+    last = m._engine.forward_tokens(planes, idx, last=True)[0]
+    every = m._engine.forward_tokens(planes, idx, last=False, every=True)[1]
+    assert torch.equal(last, every[:, -1])
+
+
 def test_empty_batch(cuda):
     """B = 0 gives empty outputs (what the reference's torch modules do), for the board forward and the token forward."""
     m = models.BT4Class(2, 256, 384, 8)
