@@ -509,13 +509,13 @@ int crl_model_set_amax(crl_model* m, const float* in, int n) {
 }
 int crl_model_forward(crl_model* m, const float* planes, int B, float* policy_logits, float* wdl_logits, void* stream) {
   if (m && B == 0) return CRL_OK;  // an empty batch writes nothing (its buffers may be null)
-  if (!m || !planes) return arg_fail("crl_model_forward: bad arguments");
+  if (!m || !planes || !policy_logits) return arg_fail("crl_model_forward: bad arguments");
   return m->impl.forward(planes, nullptr, nullptr, B, policy_logits, wdl_logits, false, (hipStream_t)stream);
 }
 int crl_model_forward_compact(crl_model* m, const uint8_t* ids, const uint8_t* flags, int B, float* policy_logits,
                               float* wdl_logits, void* stream) {
   if (m && B == 0) return CRL_OK;
-  if (!m || !ids || !flags) return arg_fail("crl_model_forward_compact: bad arguments");
+  if (!m || !ids || !flags || !policy_logits) return arg_fail("crl_model_forward_compact: bad arguments");
   return m->impl.forward(nullptr, ids, flags, B, policy_logits, wdl_logits, false, (hipStream_t)stream);
 }
 int crl_model_forward_tokens(crl_model* m, const float* planes, const int64_t* idx, int B, int t, float* last_logits,
@@ -588,7 +588,7 @@ static int evaluate_boards(crl_model* m, int n, int chunk, float temperature, fl
     if (rc == CRL_OK) PIPE_HIP(hipEventRecord(s.uploaded, P.copy_st));
     if (rc == CRL_OK) PIPE_HIP(hipStreamWaitEvent(P.comp_st, s.uploaded, 0));
     if (rc) break;
-    rc = m->impl.forward(nullptr, s.d_ids, s.d_flags, cnt, s.d_logits, has_wdl ? s.d_wdl : nullptr, false, P.comp_st);
+    rc = m->impl.forward(nullptr, s.d_ids, s.d_flags, cnt, need_policy || !has_wdl ? s.d_logits : nullptr, has_wdl && (wdl || !need_policy) ? s.d_wdl : nullptr, false, P.comp_st);
     if (rc) break;
     if (need_policy) {
       SoftmaxArgs a;

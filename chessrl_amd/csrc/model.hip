@@ -499,14 +499,14 @@ float Model::act_scale(int layer, int slot) const {
 
 int Model::forward(const float* planes, const uint8_t* ids, const uint8_t* flags, int B, float* policy, float* wdl,
                    bool calibrate, hipStream_t st) {
-  if (!policy) { set_error("forward: bad arguments"); return CRL_ERR_ARG; }
+  if (!policy && !wdl) { set_error("forward: bad arguments"); return CRL_ERR_ARG; }
   return forward_tokens(planes, ids, flags, nullptr, 0, B, policy, nullptr, wdl, calibrate, st);
 }
 
 int Model::forward_tokens(const float* planes, const uint8_t* ids, const uint8_t* flags, const int64_t* idx, int t, int B,
                           float* policy, float* all_logits, float* wdl, bool calibrate, hipStream_t st) {
   if (!finalized) { set_error("forward: call crl_model_finalize first"); return CRL_ERR_STATE; }
-  if (B < 0 || t < 0 || (!planes && !(ids && flags)) || (!policy && !all_logits)) { set_error("forward: bad arguments"); return CRL_ERR_ARG; }
+  if (B < 0 || t < 0 || (!planes && !(ids && flags)) || (!policy && !all_logits && !wdl)) { set_error("forward: bad arguments"); return CRL_ERR_ARG; }
   if ((t > 0 || all_logits) && cfg.arch != CRL_ARCH_GPT64) { set_error("forward: move tokens and per-token logits exist only for CRL_ARCH_GPT64"); return CRL_ERR_ARG; }
   if (t > 0 && !idx) { set_error("forward: move tokens missing"); return CRL_ERR_ARG; }
   const int T = 64 + t;
@@ -750,6 +750,7 @@ int Model::forward_chunk(const float* planes, const uint8_t* ids, const uint8_t*
     { GOpt o; o.act = hact; RUN(gemm(val2, ws.v1, 8192, hd, ws.v2, 128, hd, mb, o, st)); }
     { GOpt o; RUN(gemm(val3, ws.v2, 128, hd, wdl, 3, DT_F32, mb, o, st)); }
   }
+  if (!policy) return CRL_OK;   // value only (the 1-ply search)
   {
     GOpt o; o.act = hact;
     if (cfg.arch == CRL_ARCH_BT4) { o.res = pe_head; o.ldr = C; o.res_dt = hd; o.res_rows = 64; }

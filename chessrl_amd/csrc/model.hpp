@@ -114,6 +114,7 @@ struct Model {
   ~Model();
   int set_weight(const char* key, const float* data, long numel);
   int finalize();
+  // policy or wdl may be null (not both): that head is then left out.
   int forward(const float* planes, const uint8_t* ids, const uint8_t* flags, int B, float* policy, float* wdl, bool calibrate, hipStream_t st);
   // CRL_ARCH_GPT64 with t move tokens after the 64 board tokens; policy = logits of the last token [B,V],
   // all_logits = logits of every token [B, 64+t, V]; either may be null.
