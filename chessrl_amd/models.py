@@ -566,7 +566,10 @@ class GPT(_ModelBase):
         t = idx.shape[1]
         if 64 + t > self.config.block_size:
             raise ValueError("Cannot forward sequence of length %d, block size is %d" % (64 + t, self.config.block_size))
-        targets = torch.cat((torch.full((B, 64), 1928, device=dev, dtype=torch.int64), idx), dim=1).roll(-1, dims=1)
+        # 64 board tokens (ignored), then the move tokens, shifted left by one (the wrapped-round first one is ignored too)
+        targets = torch.full((B, 64 + t), 1928, device=dev, dtype=torch.int64)
+        if t:
+            targets[:, 63:63 + t] = idx
         if not compute_loss:
             return self._engine.forward_tokens(planes, idx, last=True)[0].unsqueeze(1), None, targets
         logits = self._engine.forward_tokens(planes, idx, last=False, every=True)[1]
