@@ -638,12 +638,12 @@ static hipError_t launch_in_out(const GemmArgs& a, int tile, hipStream_t st) {
   // CU of its own (M=4096, N=1024, bf16: 20.1 -> 16.3 us at K=1024, 27.9 -> 23.0 at K=1536) and level beyond (384 tiles: 26.6 -> 24.9 us
   // from warm caches, 768 tiles: 48.1 -> 49.2 us; no difference inside a 64-position forward pass), so tile 2 picks it for
   // at most as many tiles as there are CUs.
-  if (tile == 15 || tile == 16) return slabs && !a.res_stats && gemm_dmam_has(IN_DT, OUT_DT) ? launch_gemm_dmam(a, IN_DT, OUT_DT, st, tile == 16 ? 32 : 64) : hipErrorInvalidValue;
+  if (tile == 15 || tile == 16) return slabs && !a.res_stats && gemm_dmam_has(IN_DT, OUT_DT) ? launch_gemm_dmas(a, IN_DT, OUT_DT, st, tile == 16 ? 32 : 64) : hipErrorInvalidValue;
   if (tile == 11 && !slabs) tile = 12;
   if (tile == 2 || tile == 11) {
     const long mid_tiles = (long)((a.M + 127) / 128) * ((a.N + 127) / 128);
     const bool can = slabs && !a.res_stats && gemm_dmam_has(IN_DT, OUT_DT) && mid_tiles < 65536;
-    if (can && (tile == 11 || mid_tiles <= device_cus())) return launch_gemm_dmam(a, IN_DT, OUT_DT, st, 128);
+    if (can && (tile == 11 || mid_tiles <= device_cus())) return launch_gemm_dmam(a, IN_DT, OUT_DT, st);
     if (tile == 11) return hipErrorInvalidValue;
   }
   if (tile == 2 || tile == 12) return launch_cfg<CfgMid, IN_DT, OUT_DT>(a, st);

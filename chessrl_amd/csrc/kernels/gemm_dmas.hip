@@ -1,0 +1,26 @@
+// Instances of the 64x64 and 32x32 GEMMs of gemm_dmas_kernel.hpp, in a translation unit of their own.
+#include "gemm_dmas_kernel.hpp"
+
+namespace crl {
+
+template <typename S>
+static hipError_t launch_small(const GemmArgs& a, int in_dt, int out_dt, hipStream_t st) {
+  if (in_dt == DT_FP8) {
+    switch (out_dt) {
+      case DT_BF16: return launch_dmas<S, DT_FP8, DT_BF16>(a, st);
+      case DT_F16: return launch_dmas<S, DT_FP8, DT_F16>(a, st);
+      case DT_FP8: return launch_dmas<S, DT_FP8, DT_FP8>(a, st);
+    }
+  }
+  if (in_dt == DT_BF16 && out_dt == DT_BF16) return launch_dmas<S, DT_BF16, DT_BF16>(a, st);
+  if (in_dt == DT_F16 && out_dt == DT_F16) return launch_dmas<S, DT_F16, DT_F16>(a, st);
+  if (in_dt == DT_BF16 && out_dt == DT_F32) return launch_dmas<S, DT_BF16, DT_F32>(a, st);
+  return hipErrorInvalidValue;
+}
+
+// tile_size: 64 (eight stages) or 32 (sixteen); the operand types are those of gemm_dmam_has.
+hipError_t launch_gemm_dmas(const GemmArgs& a, int in_dt, int out_dt, hipStream_t st, int tile_size) {
+  return tile_size == 64 ? launch_small<DmasCfg<64>>(a, in_dt, out_dt, st) : launch_small<DmasCfg<32>>(a, in_dt, out_dt, st);
+}
+
+}  // namespace crl
