@@ -613,9 +613,9 @@ static hipError_t launch_in_out(const GemmArgs& a, int tile, hipStream_t st) {
       tile = (long)((a.M + 31) / 32) * ((a.N + 31) / 32) <= device_cus() ? 16 : small <= device_cus() ? 15 : 11;
   }
   if (tile == 6 || tile == 8) return hipErrorInvalidValue;   // codes of two retired kernels
-  // The 256x256 tile has three kernels. Eight waves in step (gemm_dma_kernel.hpp, tile 7): every operand type, any K. The
-  // same with its address arithmetic out of the main loop (gemm_dmaf_kernel.hpp, tile 10): K in whole 128-byte slabs;
-  // bit-equal and faster (the GEMMs of a 4096-position e4m3 forward: -4.9 %), so tile 3 means this one where it exists.
+  // The 256x256 tile has three kernels. Eight waves in step (gemm_dma_kernel.hpp, tile 7): every operand type, any K.
+  // Eight waves taking turns, persistent workgroups (gemm_dmaf_kernel.hpp, tile 10): K in whole 128-byte slabs;
+  // bit-equal and faster (M=64000, bf16: N=3104 436 -> 354 us, N=1024 with residual 160 -> 133), so tile 3 means this one where it exists.
   // Four software-pipelined waves with 16x16x128 MFMAs (gemm_sp2_kernel.hpp, tile 9): e4m3, whole slabs; the faster main
   // loop (1.63 against 1.96 us per slab on random data) and the slower prologue and epilogue (10.0 against 7.7 us per
   // tile): it takes over from K = 4096 on.
@@ -630,7 +630,7 @@ static hipError_t launch_in_out(const GemmArgs& a, int tile, hipStream_t st) {
     if constexpr (IN_DT == DT_FP8 && OUT_DT != DT_F32) return launch_gemm_sp2(a, OUT_DT, st);
     else return hipErrorInvalidValue;
   }
-  if (tile == 10) return gemm_dmaf_has(IN_DT, OUT_DT, a.res_stats != nullptr) ? launch_gemm_dmaf(a, IN_DT, OUT_DT, st) : hipErrorInvalidValue;
+  if (tile == 10) return gemm_dmaf_has(IN_DT, OUT_DT, a.res_stats != nullptr) ? launch_gemm_dmaf(a, IN_DT, OUT_DT, device_cus(), st) : hipErrorInvalidValue;
   if (tile == 3 || tile == 7) return launch_gemm_dma(a, IN_DT, OUT_DT, st);
   // The 128x128 tile has the register-staged kernel (any K, fp32 outputs, normalised residuals; two workgroups per CU;
   // tile 12 names it) and, for K in whole slabs, the direct-to-LDS kernel with three slabs in flight

@@ -1,14 +1,27 @@
-// C[M,N] = epilogue(A[M,K] · W[N,K]^T), e4m3 or 16-bit operands, K a whole number of 128-byte slabs: the eight-wave in-step
-// 256x256 kernel of gemm_dma_kernel.hpp with its address arithmetic taken out of the main loop. There a wave issues,
-// per slab of 16 MFMAs, 24 LDS reads and 8 loads, another 85 vector ALU instructions: a 64-bit add, a compare and two
-// selects per load (slab offset, K tail from a block of zeros), an add per fragment read. Here
-//  * LDS is laid out weight rows of stage 0, of stage 1 (32 KB each), then activation rows of stage 0, of stage 1, so a
-//    stage is bit 15 of an address: a fragment address is one of four lane registers per operand plus an instruction
-//    immediate, and all eight registers change stage with one XOR each per slab;
-//  * loads use buffer addressing: descriptor base = tile origin (scalar), a fixed lane offset, the slab offset in a
-//    scalar register; past the end of K they go through a descriptor of zero length (they move nothing and keep the
-//    instruction stream free of branches).
-// Same tile walk, same K order and same epilogue as gemm_dma_kernel.hpp: the outputs are bit-equal.
+// C[M,N] = epilogue(A[M,K] . W[N,K]^T), e4m3 or 16-bit operands, K a whole number of 128-byte slabs: the 256x256 workgroup tile of
+// the large products. Eight waves (two per SIMD) of 128x64 outputs, two LDS stages of 64 KB filled by direct-to-LDS loads.
+//
+// The two waves of a SIMD take turns: waves 0-3 (group 0) multiply while waves 4-7 (group 1) read fragments and request slabs,
+// and the other way round, with a workgroup barrier at every change. A load instruction of 64 x 16 bytes holds its wave for 100
+// cycles and more; with both waves of a SIMD loading first and multiplying afterwards (this kernel's earlier form) a slab took the
+// load time plus the MFMA time, 1.8-2.1 us, and the matrix pipe stood still for half of it. In turns a slab of 2048 MFMA cycles
+// takes 2360-2540 (e4m3, K = 16384: 2.67 -> 2.95 PFLOP/s; bf16, M = 64000, N = 3072, K = 1024: 1.02 -> 1.11).
+//
+// A slab is two phases. Phase 0 reads the weight fragments of the slab and the activation fragments of row blocks 0 and 1,
+// phase 1 those of row blocks 2 and 3; 16 of the slab's 24 LDS rows per 8 are free after phase 0. Requests follow: phase 1 asks
+// for six eighths of the slab after next (weights and row blocks 0, 1), the next phase 0 for the last two. No wait ever drains
+// the queue: eight loads of a wave stay in flight across every barrier.
+//
+// Workgroups are persistent (one per CU) where the epilogue below exists for the call, and the stream of requested slabs runs on
+// across tiles: the first slab and a half of the next tile is on its way while a tile's results are written, which took 3200
+// cycles of prologue and 1800 of workgroup turnover off each tile's 29000 (e4m3, K = 1024) to 49000 (bf16). The epilogue
+// therefore lives outside the ring, in 2 KB of LDS per wave: results are finished in the accumulator layout (four consecutive
+// columns of one row), converted, and turned through LDS in their output type, so that a store writes 64-byte row segments
+// (32-byte ones cost three times as much: 5200 against 1550 cycles per tile). A 16-bit residual takes the same way in reverse.
+// Stores and residual loads go through buffer descriptors that end with the tile, so ragged M and N need no branches, and every
+// wave issues the same number of them, which the counted waits rely on.
+//
+// Same K order and same arithmetic per element as the other tiled kernels: the outputs are bit-equal.
 #pragma once
 #include "gemm_dma_kernel.hpp"
 
@@ -17,17 +30,12 @@ namespace crl {
 struct DmafCfg {
   static constexpr int BM = 256, BN = 256, WGM = 2, WGN = 4, NW = 8, NT = 512;
   static constexpr int WM = 128, WN = 64, TM = 4, TN = 2;
-  static constexpr int ROWB = 128, LOADS = 8;
-  static constexpr int RING_BYTES = 2 * (BM + BN) * ROWB;   // 128 KB
-  static constexpr int EPI_BYTES = NW * 32 * WN * 4;        // 64 KB: the two weight stages
-  static constexpr int STATS_OFF = RING_BYTES + 256;        // behind the landing strip of the L2 touches
-  static constexpr int COLS_OFF = STATS_OFF + NW * 2 * WM * 4;   // per-column epilogue constants: [wave][bias, gain, offset][WN]
+  static constexpr int ROWB = 128, LOADS = 8, FIRST = 6;    // load instructions of a wave per slab; those of phase 1
+  static constexpr int RING_BYTES = 2 * (BM + BN) * ROWB;   // 128 KB: weight rows of both stages, then activation rows
+  static constexpr int PATCH_OFF = RING_BYTES, PATCH = 2048;           // a wave's patch: 32 rows of 64 bytes
+  static constexpr int COLS_OFF = PATCH_OFF + NW * PATCH;              // per-column constants: [wave][bias, gain, offset][WN]
   static constexpr int LDS_BYTES = COLS_OFF + NW * 3 * WN * 4;
-  // XTRA instances: up to 32 weight rows beyond the last tile column, two stages of 4 KB on an 8 KB boundary (a stage is
-  // bit 12 of an address there).
-  static constexpr int XTRA_OFF = (LDS_BYTES + 8191) / 8192 * 8192;
-  static constexpr int LDS_BYTES_XTRA = XTRA_OFF + 8192;
-  static_assert(LDS_BYTES_XTRA <= 160 * 1024, "LDS of a CU");
+  static_assert(LDS_BYTES <= 160 * 1024, "LDS of a CU");
 };
 
 // The tile walk's constants, worked out once on the host: the walk divides a workgroup index by six launch constants,
@@ -55,158 +63,156 @@ inline DmafWalk dmaf_walk(int M, int N, bool fp8) {
   return w;
 }
 
-// LEAN: the epilogue without its edge and type guards (gemm_epilogue's LEAN; dmaf_lean_ok says when).
-// XTRA: the tile columns cover the first nsplit columns only (nsplit a multiple of 256), and the workgroups of the last
-// tile column also compute the up to 32 columns behind them (the second output of a column split): every wave one more
-// 32x32 MFMA tile per K step, rows [32 wn, +32) of its 128, on weight rows that four more loads per slab bring in. Same
-// operands in the same K order as a tile column of their own would use (bit-equal), without that column's second pass
-// over the activations.
-template <int IN_DT, int OUT_DT, int RES_NORM = 0, int LEAN = 0, int XTRA = 0>
-__global__ void __launch_bounds__(DmafCfg::NT, 2) gemm_dmaf_kernel(const GemmArgs a, const int pf, const DmafWalk wk) {
+
+// What happens to the sums of a tile (all but DMAF_GENERAL persistent):
+enum {
+  DMAF_GENERAL = 0,       // anything: gemm_epilogue through the ring, one tile per workgroup
+  DMAF_GENERAL_NORM = 1,  // the same with a residual normalised on the fly
+  DMAF_PLAIN = 2,         // no residual, alpha = 1
+  DMAF_RES16 = 3,         // 16-bit residual
+  DMAF_RESNORM = 4,       // 16-bit residual normalised on the fly
+  DMAF_RES32 = 5          // fp32 residual, fp32 output
+};
+
+template <int N>
+__device__ __forceinline__ void wait_vmcnt_lgkm0() { __builtin_amdgcn_s_waitcnt((N & 0xF) | ((N >> 4) << 14) | (0x7 << 4)); }
+__device__ __forceinline__ void dmaf_barrier() { asm volatile("s_barrier" ::: "memory"); }
+// (functions of their own, like dmam_load16: inside a kernel template these builtins can make the host pass drop the kernel's stub)
+__device__ __forceinline__ void dmaf_load16(__amdgpu_buffer_rsrc_t r, uint8_t* dst, int voff, int soff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, voff, soff, 0, 0);
+}
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t dmaf_rsrc(const void* base, long span) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)(span < 0x7fffffffL ? span : 0x7fffffffL), 0x00020000);
+}
+// The value, in a register the compiler cannot trace back: address arithmetic built on it stays where it is written instead of
+// being hoisted out of the tile loop into registers of its own.
+__device__ __forceinline__ int dmaf_here(int x) {
+  asm volatile("" : "+v"(x));
+  return x;
+}
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ u32x2_t dmaf_get8(__amdgpu_buffer_rsrc_t r, int off) { return __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0); }
+__device__ __forceinline__ u32x4_t dmaf_get16_nt(__amdgpu_buffer_rsrc_t r, int off) { return __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 2); }
+__device__ __forceinline__ void dmaf_put16_nt(u32x4_t v, __amdgpu_buffer_rsrc_t r, int off) { __builtin_amdgcn_raw_buffer_store_b128(v, r, off, 0, 2); }
+__device__ __forceinline__ void dmaf_put16(u32x4_t v, __amdgpu_buffer_rsrc_t r, int off) { __builtin_amdgcn_raw_buffer_store_b128(v, r, off, 0, 0); }
+
+template <int IN_DT, int OUT_DT, int EPI, int ACT = ACT_NONE>
+__global__ void __launch_bounds__(DmafCfg::NT, 2) gemm_dmaf_kernel(const GemmArgs a, const DmafWalk wk, const int tiles) {
   typedef DmafCfg Cfg;
+  constexpr bool PERSIST = EPI >= DMAF_PLAIN;
   constexpr int ESZ = IN_DT == DT_FP8 ? 1 : 2;                      // bytes per operand element
+  constexpr int OSZ = OUT_DT == DT_F32 ? 4 : OUT_DT == DT_FP8 ? 1 : 2;
   constexpr int KSTEPS = Cfg::ROWB / (IN_DT == DT_FP8 ? 64 : 32);   // MFMA K steps per slab
-  constexpr int BM = Cfg::BM, BN = Cfg::BN, TM = Cfg::TM, TN = Cfg::TN, LOADS = Cfg::LOADS;
+  constexpr int BM = Cfg::BM, BN = Cfg::BN, TM = Cfg::TM, TN = Cfg::TN, LOADS = Cfg::LOADS, FIRST = Cfg::FIRST;
   extern __shared__ __align__(16) uint8_t smem[];
 
   // (the wave index as a scalar: everything derived from it, LDS destinations and descriptors, stays in scalar registers)
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave % Cfg::WGM, wn = wave / Cfg::WGM;
+  const int wm = wave % Cfg::WGM, wn = wave / Cfg::WGM, grp = wave >> 2;
   const int lr = lane & 31, g = lane >> 5;
+  const int nslab = a.K * ESZ / Cfg::ROWB;  // the launcher sends only whole slabs of K here
 
-  const int tiles_n = wk.tiles_n;
-  const int nblk = gridDim.x;
+  // Workgroup b runs on XCD b & 7, which owns a contiguous range of the tile order. With fewer workgroups than tiles (a
+  // multiple of eight then) an XCD's workgroups take its tiles in turn.
+  int tile = blockIdx.x, hi = tiles, step = tiles;
+  if ((int)gridDim.x < tiles) {
+    const int xcd = blockIdx.x & 7;
+    tile = (int)((long)tiles * xcd >> 3) + ((int)blockIdx.x >> 3);
+    hi = (int)((long)tiles * (xcd + 1) >> 3);
+    step = (int)gridDim.x >> 3;
+    if (tile >= hi) return;
+  } else {
+    const int per = tiles >> 3;
+    if (tile < (per << 3)) tile = (tile & 7) * per + (tile >> 3);
+  }
+
   // Tiles are walked from the last row of tiles to the first. The kernels around a product (norms, attention) walk their
   // rows upwards, so this product starts on the rows its producer wrote last and ends on the rows its consumer reads first,
   // which are the ones the memory-side cache still holds (measured on a 4096-position pass: -0.4 ms over its 60 launches).
-  int pid = nblk - 1 - (int)blockIdx.x;
-  {
-    const int per = nblk >> 3;
-    if (pid < (per << 3)) pid = (pid & 7) * per + (pid >> 3);
-  }
-  // Tile order inside an XCD's range: groups of 8 x w tiles (M x N), w = 3 or 4, as in gemm_dma_kernel.hpp.
-  int tile_m = dmaf_div(pid, wk.m_tn), tile_n = pid - tile_m * tiles_n;
-  int grp_w = 4, grp_q = tile_n & 3;
-  if (wk.grouped) {
-    constexpr int GM = 8;
-    const int wb = wk.wb, extra = wk.extra, big = wk.big;
-    const int sr = dmaf_div(pid, wk.m_8tn), rem = pid - sr * (GM * tiles_n);
-    int gi, r2, rq;
-    if (rem < big) { grp_w = wb + 1; gi = dmaf_div(rem, wk.m_8w1); r2 = rem - gi * GM * grp_w; rq = dmaf_div(r2, wk.m_w1); }
-    else { grp_w = wb; const int rem2 = rem - big; gi = dmaf_div(rem2, wk.m_8w0); r2 = rem2 - gi * GM * wb; rq = dmaf_div(r2, wk.m_w0); gi += extra; }
-    grp_q = r2 - rq * grp_w;
-    tile_m = sr * GM + rq;
-    tile_n = gi * wb + (gi < extra ? gi : extra) + grp_q;
-  }
-  const int m0 = tile_m * BM, n0 = tile_n * BN;
-  const int nslab = a.K * ESZ / Cfg::ROWB;  // the launcher sends only whole slabs of K here
+  // Inside an XCD's range: groups of 8 x w tiles (M x N), w = 3 or 4, as in gemm_dma_kernel.hpp.
+  auto tile_pos = [&](int t, int& tm, int& tn) {
+    const int pid = tiles - 1 - t;
+    if (wk.grouped) {
+      constexpr int GM = 8;
+      const int sr = dmaf_div(pid, wk.m_8tn), rem = pid - sr * (GM * wk.tiles_n);
+      int gi, r2, rq, gw;
+      if (rem < wk.big) { gw = wk.wb + 1; gi = dmaf_div(rem, wk.m_8w1); r2 = rem - gi * GM * gw; rq = dmaf_div(r2, wk.m_w1); tn = gi * gw; }
+      else { gw = wk.wb; const int rem2 = rem - wk.big; gi = dmaf_div(rem2, wk.m_8w0); r2 = rem2 - gi * GM * gw; rq = dmaf_div(r2, wk.m_w0); tn = (gi + wk.extra) * gw + wk.extra; }
+      tm = sr * GM + rq;
+      tn += r2 - rq * gw;
+    } else {
+      tm = dmaf_div(pid, wk.m_tn);
+      tn = pid - tm * wk.tiles_n;
+    }
+  };
 
-  // Loader role: waves 0-3 fill weight rows [64w, +64) of a stage, waves 4-7 activation rows [64(w-4), +64): 8 rows per
-  // wave-instruction, eight 16-byte chunks per row, the swizzle applied on the global side (row 8 i + lane / 8 of the
-  // wave's 64 has swizzle (lane / 8) ^ i).
-  const bool loads_a = wave >= 4;
-  const int rbase = (wave & 3) * 64;
-  const int ld = (loads_a ? a.lda : a.ldw) * ESZ;   // row stride in bytes
-  const int rows_left = loads_a ? a.M - m0 : a.N - n0;
+  // ---- the stream of requested slabs (l_*: where it stands; it runs up to two slabs ahead, across tiles)
+  // Load i of a wave, 8 rows of 128 bytes: weight rows 32 wave + 8 i (i < 4); activation rows 16 (wave & 3) + 8 (i & 1) of
+  // the 64 that row blocks 0, 1 (i = 4, 5) or 2, 3 (i = 6, 7) of wave row wave / 4 have. The swizzle is applied on the global side.
   uint32_t voff[LOADS];
+  __amdgpu_buffer_rsrc_t rsrc_w, rsrc_x;
+  const int ldab = (int)a.lda * ESZ, ldwb = (int)a.ldw * ESZ;
+  int l_tile = tile, l_slab = 0;
+  uint32_t l_stage = 0;
+  auto stream_tile = [&]() {
+    int tm, tn;
+    tile_pos(l_tile, tm, tn);
+    const int ln = dmaf_here(lane);
+    const int m0 = tm * BM, n0 = tn * BN, leftx = a.M - m0, leftw = a.N - n0, l8 = ln >> 3;
 #pragma unroll
-  for (int i = 0; i < LOADS; ++i) {
-    int r = rbase + 8 * i + (lane >> 3);
-    r = r < rows_left ? r : rows_left - 1;
-    voff[i] = (uint32_t)r * (uint32_t)ld + (((lane & 7) ^ (lane >> 3) ^ i) << 4);
-  }
-  auto make_rsrc = [&](const void* base, long rows, long ldb) {
-    const long span = (rows < 256 ? rows : 256) * ldb;
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)(span < 0x7fffffffL ? span : 0x7fffffffL), 0x00020000);
+    for (int i = 0; i < LOADS; ++i) {
+      int r = i >= 4 ? (wave >> 2) * 128 + (wave & 3) * 16 + ((i & 2) ? 64 : 0) + 8 * (i & 1) + l8 : wave * 32 + 8 * i + l8;
+      const int sw = l8 ^ ((i >= 4 ? 2 * (wave & 3) + (i & 1) : 4 * (wave & 1) + i) & 7);
+      const int left = i >= 4 ? leftx : leftw;
+      r = r < left ? r : left - 1;
+      voff[i] = (uint32_t)r * (uint32_t)(i >= 4 ? ldab : ldwb) + (((ln & 7) ^ sw) << 4);
+    }
+    rsrc_w = dmaf_rsrc(reinterpret_cast<const uint8_t*>(a.W) + (long)n0 * ldwb, (long)(leftw < 256 ? leftw : 256) * ldwb);
+    rsrc_x = dmaf_rsrc(reinterpret_cast<const uint8_t*>(a.A) + (long)m0 * ldab, (long)(leftx < 256 ? leftx : 256) * ldab);
   };
-  const __amdgpu_buffer_rsrc_t rsrc_w = make_rsrc(reinterpret_cast<const uint8_t*>(a.W) + (long)n0 * a.ldw * ESZ, a.N - n0, (long)a.ldw * ESZ);
-  const __amdgpu_buffer_rsrc_t rsrc_x = make_rsrc(reinterpret_cast<const uint8_t*>(a.A) + (long)m0 * a.lda * ESZ, a.M - m0, (long)a.lda * ESZ);
-  const __amdgpu_buffer_rsrc_t rsrc_none = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.A), 0, 0, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rsrc_mine = loads_a ? rsrc_x : rsrc_w;
-  const uint32_t lds_load0 = (loads_a ? 65536u : 0u) + rbase * Cfg::ROWB;   // stage 0
-  auto issue_one = [&](int slab, const __amdgpu_buffer_rsrc_t& r, auto ic) {
+  auto issue = [&](auto ic) {
     constexpr int i = decltype(ic)::value;
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)(smem + (lds_load0 ^ ((slab & 1) << 15)) + i * 1024), 16,
-                                             (int)voff[i], slab * Cfg::ROWB, 0, 0);
+    const uint32_t d = i >= 4 ? 65536u + ((wave >> 2) * 128 + (wave & 3) * 16 + ((i & 2) ? 64 : 0) + 8 * (i & 1)) * 128u : (wave * 32 + 8 * i) * 128u;
+    dmaf_load16(i >= 4 ? rsrc_x : rsrc_w, smem + (d ^ l_stage), (int)voff[i], l_slab * Cfg::ROWB);
   };
-  // XTRA: waves 0-3 bring in eight of the extra weight rows each.
-  const bool extra = XTRA != 0 && tile_n == tiles_n - 1;
-  const int n_x = n0 + BN;   // first extra column
-  uint32_t voff_x = 0;
-  __amdgpu_buffer_rsrc_t rsrc_xw = rsrc_none;
-  if constexpr (XTRA != 0) {
-    if (extra && !loads_a) {
-      const int rows_x = a.N - n_x < 32 ? a.N - n_x : 32;
-      int r = 8 * wave + (lane >> 3);
-      r = r < rows_x ? r : rows_x - 1;
-      voff_x = (uint32_t)r * (uint32_t)ld + (((lane & 7) ^ (lane >> 3) ^ wave) << 4);
-      rsrc_xw = make_rsrc(reinterpret_cast<const uint8_t*>(a.W) + (long)n_x * a.ldw * ESZ, rows_x, (long)a.ldw * ESZ);
+  auto request_first = [&]() {   // weights and row blocks 0, 1 of the stream's next slab
+    if (l_slab == nslab) {
+      l_slab = 0;
+      l_tile += step;
+      if (PERSIST && l_tile < hi) stream_tile();
+      else rsrc_w = rsrc_x = dmaf_rsrc(a.A, 0);   // past the end: loads that move nothing keep the counts
     }
-  }
-  auto issue_extra = [&](int slab, bool live) {
-    if constexpr (XTRA != 0) {
-      if (extra && !loads_a)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(live ? rsrc_xw : rsrc_none,
-                                                 (__attribute__((address_space(3))) void*)(smem + Cfg::XTRA_OFF + ((slab & 1) << 12) + wave * 1024), 16,
-                                                 (int)voff_x, slab * Cfg::ROWB, 0, 0);
-    }
+    static_for<0, FIRST>(issue);
   };
-  // The first slab is requested as early as its addresses exist; everything else the prologue sets up follows.
-  static_for<0, LOADS>([&](auto ic) { issue_one(0, rsrc_mine, ic); });
-  issue_extra(0, true);
+  auto request_rest = [&]() {    // its row blocks 2, 3
+    static_for<FIRST, LOADS>(issue);
+    ++l_slab;
+    l_stage ^= 32768u;
+  };
+  stream_tile();
+  request_first();
+  request_rest();
+  request_first();
   __builtin_amdgcn_sched_barrier(0);
 
+  int tm0, tn0;
+  tile_pos(tile, tm0, tn0);
+  int m0 = tm0 * BM, n0 = tn0 * BN;
   // The per-column constants of the epilogue (bias; gain and offset of a residual normalised on the fly) for this wave's
-  // 64 columns, one column per lane, landed outside the ring: requested first, in LDS long before the epilogue asks.
-  // Columns past N repeat the last one; nothing of theirs is stored.
-  {
+  // 64 columns, one column per lane. Columns past N repeat the last one; nothing of theirs is stored.
+  auto load_cols = [&]() {
     int n = n0 + wn * Cfg::WN + lane;
     n = n < a.N ? n : a.N - 1;
     uint8_t* cols = smem + Cfg::COLS_OFF + wave * (3 * Cfg::WN * 4);
     if (a.bias)
       __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(a.bias + n), (__attribute__((address_space(3))) void*)cols, 4, 0, 0);
-    if constexpr (RES_NORM != 0) {
+    if constexpr (EPI == DMAF_RESNORM || EPI == DMAF_GENERAL_NORM) {
       __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(a.res_gamma + n),
                                        (__attribute__((address_space(3))) void*)(cols + Cfg::WN * 4), 4, 0, 0);
       if (a.res_beta)
         __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(a.res_beta + n),
                                          (__attribute__((address_space(3))) void*)(cols + 2 * Cfg::WN * 4), 4, 0, 0);
-    }
-  }
-  if constexpr (RES_NORM != 0) {
-    // Statistics of this wave's 128 rows (two rows = 16 bytes per lane), requested before anything else and landed
-    // outside the ring.
-    int m = m0 + wm * Cfg::WM + 2 * lane;
-    m = m + 1 < a.M ? m : 0;
-    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(a.res_stats + 2 * (long)m),
-                                     (__attribute__((address_space(3))) void*)(smem + Cfg::STATS_OFF + wave * (2 * Cfg::WM * 4)), 16, 0, 0);
-  }
-
-
-  // L2 touches, as in gemm_dma_kernel.hpp: wave 0 touches its share of the activation lines of a slab `pf` slabs before
-  // anybody loads it, wave 1 its share of the weight lines; one dword per 128-byte line into an LDS strip nobody reads.
-  uint32_t pf_off = 0;
-  int pf_n = 0, pf_step = 0;
-  if (pf > 0 && wave < 2) {
-    if (wave == 0) {
-      pf_n = grp_w >= 4 ? 1 : grp_w >= 2 ? 2 : 4;   // ceil(4 / grp_w)
-      int r = ((grp_q * pf_n) & 3) * 64 + lane;
-      r = r < a.M - m0 ? r : a.M - m0 - 1;
-      pf_off = (uint32_t)r * (uint32_t)(a.lda * ESZ);
-      pf_step = (m0 + 256 <= a.M) ? 64 * a.lda * ESZ : 0;
-    } else {
-      pf_n = 1;
-      int r = (tile_m & 7) * 32 + (lane & 31);
-      r = r < a.N - n0 ? r : a.N - n0 - 1;
-      pf_off = (uint32_t)r * (uint32_t)(a.ldw * ESZ) + (lane >> 5) * 64;
-    }
-  }
-  const __amdgpu_buffer_rsrc_t rsrc_pf = wave == 0 ? rsrc_x : rsrc_w;
-  auto prefetch = [&](int slab) {
-    if (pf_n > 0 && slab < nslab) {
-      for (int i = 0; i < pf_n; ++i)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_pf, (__attribute__((address_space(3))) void*)(smem + Cfg::RING_BYTES), 4,
-                                                 (int)pf_off, slab * Cfg::ROWB + i * pf_step, 0, 0);
     }
   };
 
@@ -222,7 +228,7 @@ __global__ void __launch_bounds__(DmafCfg::NT, 2) gemm_dmaf_kernel(const GemmArg
   // c = 4 ks + half + 2g for e4m3 (two pieces per K step of 64 bytes) and c = 2 ks + g for 16-bit operands (one piece
   // per K step of 32 bytes), and swizzle(row) = swizzle(lr) ^ 4 (t & 1). With L = (2g or g) ^ swizzle(lr) the chunk is
   // Kc ^ L for a compile-time Kc that takes four values (0, 1, 4, 5 or 0, 2, 4, 6): four lane addresses per operand
-  // plus the immediate 4096 t cover every read of a stage.
+  // plus the immediate 4096 t cover every read of a stage. A stage is bit 15 of an address.
   const int L0 = (IN_DT == DT_FP8 ? 2 * g : g) ^ lds_swizzle(lr);
   const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t*)smem);
   uint32_t wb[4], xb[4];
@@ -232,136 +238,342 @@ __global__ void __launch_bounds__(DmafCfg::NT, 2) gemm_dmaf_kernel(const GemmArg
     wb[k] = lds0 + (wn * Cfg::WN + lr) * Cfg::ROWB + ((kc ^ L0) << 4);
     xb[k] = lds0 + 65536 + (wm * Cfg::WM + lr) * Cfg::ROWB + ((kc ^ L0) << 4);
   }
-  auto read_piece = [&](bool is_w, int t, int ks, int half) -> i32x4_t {
+  auto lds_piece = [](uint32_t addr) -> i32x4_t { return *reinterpret_cast<const __attribute__((address_space(3))) i32x4_t*>(addr); };
+  auto read_piece = [&](const uint32_t (&b)[4], int t, int ks, int half) -> i32x4_t {
     const int kc = (IN_DT == DT_FP8 ? 4 * ks + half : 2 * ks) ^ (4 * (t & 1));
     const int k = IN_DT == DT_FP8 ? ((kc & 1) | ((kc >> 2) << 1)) : kc >> 1;
-    return *reinterpret_cast<const __attribute__((address_space(3))) i32x4_t*>((is_w ? wb[k] : xb[k]) + t * 32 * Cfg::ROWB);
+    return lds_piece(b[k] + t * 32 * Cfg::ROWB);
   };
-
-  // XTRA: fragment addresses of the extra weight rows (row lr of 32) and of this wave's rows [32 wn, +32) of its activation block.
-  uint32_t eb[4] = {0, 0, 0, 0};
-  f32x16_t accx;
-#pragma unroll
-  for (int r = 0; r < 16; ++r) accx[r] = 0.f;
-  const uint32_t xrow_off = (uint32_t)wn * 32 * Cfg::ROWB;
-  if constexpr (XTRA != 0) {
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const int kc = (k & 1) | ((k >> 1) << 2);
-      eb[k] = lds0 + Cfg::XTRA_OFF + lr * Cfg::ROWB + ((kc ^ L0) << 4);
-    }
-  }
+  auto read_frag = [&](const uint32_t (&b)[4], int t, auto ksc) {
+    constexpr int ks = decltype(ksc)::value;
+    Frag<IN_DT> f;
+    f.lo = read_piece(b, t, ks, 0);
+    if constexpr (IN_DT == DT_FP8) f.hi = read_piece(b, t, ks, 1);
+    return f;
+  };
+  Frag<IN_DT> wf[KSTEPS][TN], xf[KSTEPS][2];
 
   // A wave whose 128x64 part lies wholly outside C still takes its share of the loads and every barrier.
-  const bool wave_active = (m0 + wm * Cfg::WM < a.M) && (n0 + wn * Cfg::WN < a.N);
+  bool wave_active = (m0 + wm * Cfg::WM < a.M) && (n0 + wn * Cfg::WN < a.N);
 
-
-  for (int s0 = 1; s0 < 1 + pf; ++s0) prefetch(s0);
-
-  for (int slab = 0; slab < nslab; ++slab) {
-    wait_vmcnt<0>();
-    __syncthreads();
-    const __amdgpu_buffer_rsrc_t rnext = slab + 1 < nslab ? rsrc_mine : rsrc_none;
-    prefetch(slab + 1 + pf);
-    if (!wave_active) {
-      static_for<0, LOADS>([&](auto ic) { issue_one(slab + 1, rnext, ic); });
-      issue_extra(slab + 1, slab + 1 < nslab);
-      continue;
-    }
+  auto read_phase = [&](auto pc) {
+    constexpr int p = decltype(pc)::value;
     static_for<0, KSTEPS>([&](auto ksc) {
       constexpr int ks = decltype(ksc)::value;
-      Frag<IN_DT> wf[TN], xf[TM];
+      if constexpr (p == 0) {
 #pragma unroll
-      for (int tn = 0; tn < TN; ++tn) {
-        wf[tn].lo = read_piece(true, tn, ks, 0);
-        if constexpr (IN_DT == DT_FP8) wf[tn].hi = read_piece(true, tn, ks, 1);
+        for (int tn = 0; tn < TN; ++tn) wf[ks][tn] = read_frag(wb, tn, ksc);
       }
 #pragma unroll
-      for (int tm = 0; tm < TM; ++tm) {
-        xf[tm].lo = read_piece(false, tm, ks, 0);
-        if constexpr (IN_DT == DT_FP8) xf[tm].hi = read_piece(false, tm, ks, 1);
-      }
-      static_for<0, TN * TM>([&](auto ic) {
-        constexpr int i = decltype(ic)::value;
-        constexpr int tn = i / TM, tm = i % TM;
-        acc[tn][tm] = mfma_frag<IN_DT>(wf[tn], xf[tm], acc[tn][tm]);
-        // The next slab's loads go out one at a time, one behind each of the slab's first eight MFMAs, held in place by
-        // scheduling barriers: the last of them then has the rest of the slab's MFMAs in which to land before the wave
-        // waits for it. Measured on the products of a large pass, e4m3: spread over all sixteen MFMAs (one behind every
-        // second) +3.8 %, starting one MFMA earlier or two later, or two loads behind each of four MFMAs, +1 %; 16-bit
-        // operands (32 MFMAs per slab): all eight at the head of the slab +2.6 %, behind every second of the first sixteen +2.6 %.
-        if constexpr (ks == 0) {
-          __builtin_amdgcn_sched_barrier(0);
-          issue_one(slab + 1, rnext, std::integral_constant<int, i>{});
-          if constexpr (i == TN * TM - 1) issue_extra(slab + 1, slab + 1 < nslab);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-      });
-      if constexpr (XTRA != 0 && IN_DT == DT_FP8) {
-        if (extra) {
-          constexpr int k0 = (4 * ks) & 1 | (((4 * ks) >> 2) << 1), k1 = ((4 * ks + 1) & 1) | (((4 * ks + 1) >> 2) << 1);
-          Frag<IN_DT> wfx, xfx;
-          wfx.lo = *reinterpret_cast<const __attribute__((address_space(3))) i32x4_t*>(eb[k0]);
-          wfx.hi = *reinterpret_cast<const __attribute__((address_space(3))) i32x4_t*>(eb[k1]);
-          // (rows 32 t + lr of a block carry the swizzle of lr with bit 2 flipped for odd t: the other pair of lane addresses)
-          const uint32_t xa0 = ((wn & 1) ? xb[k0 ^ 2] : xb[k0]) + xrow_off, xa1 = ((wn & 1) ? xb[k1 ^ 2] : xb[k1]) + xrow_off;
-          xfx.lo = *reinterpret_cast<const __attribute__((address_space(3))) i32x4_t*>(xa0);
-          xfx.hi = *reinterpret_cast<const __attribute__((address_space(3))) i32x4_t*>(xa1);
-          accx = mfma_frag<IN_DT>(wfx, xfx, accx);
-        }
-      }
+      for (int t = 0; t < 2; ++t) xf[ks][t] = read_frag(xb, 2 * p + t, ksc);
     });
-    if constexpr (XTRA != 0) {
+  };
+  auto multiply_phase = [&](auto pc) {
+    constexpr int p = decltype(pc)::value;
+    __builtin_amdgcn_sched_barrier(0);
+    dmaf_barrier();
+    __builtin_amdgcn_s_setprio(1);
+    if (wave_active) {
+      static_for<0, KSTEPS>([&](auto ksc) {
+        constexpr int ks = decltype(ksc)::value;
 #pragma unroll
-      for (int k = 0; k < 4; ++k) eb[k] ^= 4096u;
+        for (int tn = 0; tn < TN; ++tn)
+#pragma unroll
+          for (int t = 0; t < 2; ++t) acc[tn][2 * p + t] = mfma_frag<IN_DT>(wf[ks][tn], xf[ks][t], acc[tn][2 * p + t]);
+      });
     }
-    // The address registers follow the ring to the other stage.
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_setprio(0);
+  };
+  typedef std::integral_constant<int, 0> P0;
+  typedef std::integral_constant<int, 1> P1;
+
+  // ---- epilogue of the persistent instances
+  // Accumulator layout: acc[tn][tm][4 q + e] is row 32 tm + lr, column 32 tn + 8 q + 4 g + e of the wave's 128x64 part.
+  // Store layout (16 bytes per lane): rows er + 8 it of a row block, 16-byte chunk ec of a 128-byte row segment (e4m3: rows
+  // er + 16 it, chunk ec of a 64-byte one). A wave's patch is two halves of 32 rows of 64 bytes, column blocks 0 and 1: its own
+  // 2 KB and 2 KB of the ring, row blocks 2 and 3 of the last slab's stage, which nothing is requested into until every wave is
+  // through with its epilogue. 16-byte chunks are swizzled over groups of four rows (256 bytes are one pass of all banks).
+  constexpr int EPR = OUT_DT == DT_FP8 ? 4 : 8, ITS = 32 * EPR / 64;   // lanes per row, store instructions per row block
+  constexpr bool HAS_RES = EPI == DMAF_RES16 || EPI == DMAF_RESNORM || EPI == DMAF_RES32;
+  constexpr int RSZ = EPI == DMAF_RES32 ? 4 : 2;
+  // A step of the epilogue: a row block (its 64 columns), with fp32 outputs the half of one, 32 columns.
+  constexpr int NSTEP = OUT_DT == DT_F32 ? 2 * TM : TM;
+  uint8_t* const patch0 = smem + Cfg::PATCH_OFF + wave * Cfg::PATCH;
+  const float* const cols = reinterpret_cast<const float*>(smem + Cfg::COLS_OFF) + wave * (3 * Cfg::WN);
+  u32x4_t res[HAS_RES ? 2 : 1][ITS];        // residual of the next two steps
+  u32x2_t row_st[EPI == DMAF_RESNORM ? 2 : 1];   // 1/std and -mean/std of the lane's row in them
+  __amdgpu_buffer_rsrc_t rsrc_r = dmaf_rsrc(a.A, 0);
+  int vres = 0, res_step = 0;
+  auto res_begin = [&]() {
+    const int ln = dmaf_here(lane);
+    const int rows = a.M - m0 < BM ? a.M - m0 : BM, left = a.N - n0 < BN ? a.N - n0 : BN;
+    res_step = (int)a.ldr * RSZ;
+    rsrc_r = dmaf_rsrc(reinterpret_cast<const char*>(a.res) + (long)m0 * res_step + (long)n0 * RSZ, (long)(rows - 1) * res_step + (long)left * RSZ);
+    vres = (wm * Cfg::WM + ln / EPR) * res_step + wn * Cfg::WN * RSZ + (ln % EPR) * 16;
+  };
+  auto res_load = [&](auto sc) {
+    constexpr int st = decltype(sc)::value, tm = st % TM, half = st / TM;
+    if constexpr (HAS_RES && st < NSTEP) {
 #pragma unroll
-    for (int k = 0; k < 4; ++k) { wb[k] ^= 32768u; xb[k] ^= 32768u; }
+      for (int it = 0; it < ITS; ++it) res[st & 1][it] = dmaf_get16_nt(rsrc_r, vres + half * 128 + (tm * 32 + it * (64 / EPR)) * res_step);
+      if constexpr (EPI == DMAF_RESNORM)
+        row_st[st & 1] = dmaf_get8(dmaf_rsrc(a.res_stats + 2 * (long)m0, (long)(a.M - m0) * 8), (wm * Cfg::WM + tm * 32 + (dmaf_here(lane) & 31)) * 8);
+    }
+  };
+  auto activate = [&](float v) -> float {
+    if constexpr (ACT == ACT_GELU) return act_gelu(v);
+    else if constexpr (ACT == ACT_MISH) return act_mish(v);
+    else return v;
+  };
+  // e4m3(out_scale * mish(x)) in the fused form of gemm_epilogue
+  auto mish8 = [&](float accv, float bias, float v) -> float {
+    constexpr float L2E = 1.4426950408889634f;
+    const float nexp = __builtin_amdgcn_exp2f(fmaf(accv, a.descale * L2E, bias * L2E));
+    return v * fmaf(fast_rcp(fmaf(nexp, nexp + 2.f, 2.f)), -2.f * a.out_scale, a.out_scale);
+  };
+  auto epilogue = [&](uint32_t last_stage) {
+    const int ln = dmaf_here(lane), er = ln / EPR, ec = ln % EPR, lr = ln & 31, g = ln >> 5;
+    const bool first = n0 < a.nsplit;      // (a tile lies on one side of the split: the launcher checks)
+    const int ldob = (int)(first ? a.ldc : a.ldc2) * OSZ, rows = a.M - m0 < BM ? a.M - m0 : BM;
+    int left = (first ? a.nsplit : a.N) - n0;
+    left = left < BN ? left : BN;
+    const __amdgpu_buffer_rsrc_t rsrc_o = dmaf_rsrc(reinterpret_cast<char*>(first ? a.C : a.C2) + (long)m0 * ldob + (long)(first ? n0 : n0 - a.nsplit) * OSZ,
+                                                    (long)(rows - 1) * ldob + (long)left * OSZ);
+    const int vout = (wm * Cfg::WM + er) * ldob + wn * Cfg::WN * OSZ + ec * 16;
+    constexpr int NOWHERE = (int)0x80000000u;
+    const bool nt = a.stream_out != 0;
+    auto put = [&](u32x4_t v, int off) {
+      if (nt) dmaf_put16_nt(v, rsrc_o, off);
+      else dmaf_put16(v, rsrc_o, off);
+    };
+    uint8_t* const patch1 = smem + 65536 + last_stage + (wave >> 2) * 16384 + 8192 + (wave & 3) * 2048;
+    auto at = [&](uint8_t* half, int r, int c) -> uint8_t* { return half + r * 64 + ((c ^ ((r >> 2) & 3)) << 4); };
+    // this lane's chunk of row er + 8 it in the store layout
+    uint8_t* const mine = ec < 4 ? patch0 : patch1;
+    auto turned = [&](int it) -> u32x4_t { return *reinterpret_cast<const u32x4_t*>(at(mine, er + it * (64 / EPR), ec & 3)); };
+    auto col_const = [&](const float* c, int base, bool have, float (&o)[16]) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const f32x4_t v = have ? *reinterpret_cast<const f32x4_t*>(c + base + 8 * q + 4 * g) : f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[4 * q + e] = v[e];
+      }
+    };
+    if constexpr (OUT_DT == DT_FP8) {
+      const int v0 = wn * Cfg::WN + ec * 16 < left ? vout : NOWHERE;
+      float bias16[2][16];
+#pragma unroll
+      for (int tn = 0; tn < TN; ++tn) col_const(cols, tn * 32, a.bias != nullptr, bias16[tn]);
+      static_for<0, TM>([&](auto tmc) {
+        constexpr int tm = decltype(tmc)::value;
+#pragma unroll
+        for (int tn = 0; tn < TN; ++tn)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            float v[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const float s = acc[tn][tm][4 * q + e];
+              v[e] = fmaf(s, a.descale, bias16[tn][4 * q + e]);
+              if constexpr (ACT == ACT_MISH) v[e] = mish8(s, bias16[tn][4 * q + e], v[e]);
+              else v[e] = activate(v[e]) * a.out_scale;
+            }
+            *reinterpret_cast<uint32_t*>(at(patch0, lr, 2 * tn + (q >> 1)) + 8 * (q & 1) + 4 * g) = pack_fp8x4(v[0], v[1], v[2], v[3]);
+          }
+        wave_lds_fence();
+#pragma unroll
+        for (int it = 0; it < ITS; ++it) put(turned(it), v0 + (tm * 32 + it * 16) * ldob);
+        wave_lds_fence();
+      });
+    } else if constexpr (OUT_DT == DT_F32) {
+      // Raw sums through the patch, 32 columns at a time; bias, activation and residual in the store layout (4 columns per lane).
+      static_for<0, NSTEP>([&](auto sc) {
+        constexpr int st = decltype(sc)::value, tn = st / TM, tm = st % TM;
+        const int v0 = wn * Cfg::WN + tn * 32 + ec * 4 < left ? vout + tn * 128 : NOWHERE;
+        const f32x4_t bv = a.bias ? *reinterpret_cast<const f32x4_t*>(cols + tn * 32 + ec * 4) : f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          *reinterpret_cast<f32x4_t*>(at(q < 2 ? patch0 : patch1, lr, 2 * (q & 1) + g)) = f32x4_t{acc[tn][tm][4 * q], acc[tn][tm][4 * q + 1], acc[tn][tm][4 * q + 2], acc[tn][tm][4 * q + 3]};
+        wave_lds_fence();
+#pragma unroll
+        for (int it = 0; it < ITS; ++it) {
+          const u32x4_t s = turned(it);
+          u32x4_t o;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            float v = activate(fmaf(__uint_as_float(s[e]), a.descale, bv[e]));
+            if constexpr (HAS_RES) v = fmaf(v, a.alpha, __uint_as_float(res[st & 1][it][e]));
+            o[e] = __float_as_uint(v);
+          }
+          put(o, v0 + (tm * 32 + it * 8) * ldob);
+        }
+        wave_lds_fence();
+        res_load(std::integral_constant<int, st + 2>{});
+      });
+    } else {
+      const int v0 = wn * Cfg::WN + ec * 8 < left ? vout : NOWHERE;
+      static_for<0, NSTEP>([&](auto sc) {
+        constexpr int tm = decltype(sc)::value;
+        if constexpr (HAS_RES) {   // the residual from the store layout to the accumulator layout
+#pragma unroll
+          for (int it = 0; it < ITS; ++it) *reinterpret_cast<u32x4_t*>(at(mine, er + it * 8, ec & 3)) = res[tm & 1][it];
+          wave_lds_fence();
+        }
+        float st0 = 0.f, st1 = 0.f;
+        if constexpr (EPI == DMAF_RESNORM) { st0 = __uint_as_float(row_st[tm & 1][0]); st1 = __uint_as_float(row_st[tm & 1][1]); }
+        res_load(std::integral_constant<int, tm + 2>{});
+        static_for<0, TN>([&](auto tc) {
+          constexpr int tn = decltype(tc)::value;
+          uint8_t* const half = tn ? patch1 : patch0;
+          uint32_t resw[8];
+          if constexpr (HAS_RES) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+              const u32x2_t x = *reinterpret_cast<const u32x2_t*>(at(half, lr, q) + 8 * g);
+              resw[2 * q] = x[0]; resw[2 * q + 1] = x[1];
+            }
+          }
+          float bias16[16], gain16[16];
+          col_const(cols, tn * 32, a.bias != nullptr, bias16);
+          if constexpr (EPI == DMAF_RESNORM) {
+            col_const(cols + Cfg::WN, tn * 32, true, gain16);
+            if (a.res_beta) {   // the offset joins the bias (which is multiplied by alpha)
+              const float inv_alpha = 1.0f / a.alpha;
+#pragma unroll
+              for (int q = 0; q < 4; ++q) {
+                const f32x4_t v = *reinterpret_cast<const f32x4_t*>(cols + 2 * Cfg::WN + tn * 32 + 8 * q + 4 * g);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) bias16[4 * q + e] += v[e] * inv_alpha;
+              }
+            }
+          }
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            float v[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const int i = 4 * q + e;
+              v[e] = activate(fmaf(acc[tn][tm][i], a.descale, bias16[i]));
+              if constexpr (HAS_RES) {
+                const uint32_t rw = resw[i >> 1];
+                const float r = OUT_DT == DT_F16 ? f16_bits_to_f32((uint16_t)((e & 1) ? (rw >> 16) : (rw & 0xffff)))
+                                                 : __uint_as_float((e & 1) ? (rw & 0xffff0000u) : (rw << 16));
+                if constexpr (EPI == DMAF_RESNORM)
+                  v[e] = fmaf(v[e], a.alpha, fmaf(r, st0, st1) * gain16[i]);
+                else
+                  v[e] = fmaf(v[e], a.alpha, r);
+              }
+              // (a multiply-add that rounds straight to f16 would skip the rounding to fp32 that the other tiles' epilogues make)
+              if constexpr (OUT_DT == DT_F16) asm volatile("" : "+v"(v[e]));
+            }
+            u32x2_t w;
+            if constexpr (OUT_DT == DT_F16) {
+              w[0] = (uint32_t)f32_to_f16_bits(v[0]) | ((uint32_t)f32_to_f16_bits(v[1]) << 16);
+              w[1] = (uint32_t)f32_to_f16_bits(v[2]) | ((uint32_t)f32_to_f16_bits(v[3]) << 16);
+            } else {
+              w[0] = pack_bf16x2(v[0], v[1]);
+              w[1] = pack_bf16x2(v[2], v[3]);
+            }
+            *reinterpret_cast<u32x2_t*>(at(half, lr, q) + 8 * g) = w;
+          }
+        });
+        wave_lds_fence();
+#pragma unroll
+        for (int it = 0; it < ITS; ++it) put(turned(it), v0 + (tm * 32 + it * 8) * ldob);
+        wave_lds_fence();
+      });
+    }
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+      for (int j = 0; j < TM; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+  };
+  // Stores an epilogue issues behind its last load (a wave waits past them for the slabs requested before).
+  constexpr int ESTORES = PERSIST ? NSTEP * ITS : 0;
+  constexpr int INFLIGHT = LOADS;   // FIRST of the slab after next and LOADS - FIRST of the next one
+
+  wait_vmcnt<INFLIGHT>();
+  dmaf_barrier();
+  uint32_t r_stage = 0;   // stage of the slab being read
+  bool later = false;   // a tile before this one has left stores in flight
+  for (;;) {
+    if (grp) dmaf_barrier();   // group 1 runs one phase behind
+    for (int slab = 0; slab < nslab; ++slab) {
+      const bool last = slab + 1 == nslab;
+      read_phase(P0{});
+      __builtin_amdgcn_sched_barrier(0);
+      request_rest();
+      if (slab == 0) load_cols();
+      __builtin_amdgcn_sched_barrier(0);
+      // Row blocks 2, 3 of this slab: requested before the last INFLIGHT loads (and before the previous tile's stores).
+      if (slab == 0 && later) wait_vmcnt_lgkm0<INFLIGHT + ESTORES>();
+      else wait_vmcnt_lgkm0<INFLIGHT>();
+      multiply_phase(P0{});
+      dmaf_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+      read_phase(P1{});
+      __builtin_amdgcn_sched_barrier(0);
+      request_first();
+      r_stage ^= 32768u;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) { wb[k] ^= 32768u; xb[k] ^= 32768u; }
+      if constexpr (HAS_RES) {
+        if (last) { res_begin(); res_load(P0{}); }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if (!PERSIST && last) wait_vmcnt_lgkm0<0>();   // (the ring becomes epilogue scratch)
+      else if (slab == 0 && later) wait_vmcnt_lgkm0<INFLIGHT + ESTORES>();
+      else if (HAS_RES && last) wait_vmcnt_lgkm0<INFLIGHT + ITS + (EPI == DMAF_RESNORM ? 1 : 0)>();
+      else wait_vmcnt_lgkm0<INFLIGHT>();
+      multiply_phase(P1{});
+      if (!(last && grp)) dmaf_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (!PERSIST) break;
+    res_load(P1{});
+    epilogue(r_stage ^ 32768u);
+    tile += step;
+    if (tile >= hi) break;
+    tile_pos(tile, tm0, tn0);
+    m0 = tm0 * BM; n0 = tn0 * BN;
+    wave_active = (m0 + wm * Cfg::WM < a.M) && (n0 + wn * Cfg::WN < a.N);
+    later = true;
+    dmaf_barrier();
   }
-
-  wait_vmcnt<0>();
-  __syncthreads();  // every wave is done with the ring (and the empty loads past the end have retired) before it becomes epilogue scratch
-
-  gemm_epilogue<Cfg::WM, Cfg::WN, OUT_DT, RES_NORM, LEAN>(a, acc, reinterpret_cast<float*>(smem) + wave * (32 * Cfg::WN),
+  if constexpr (!PERSIST) {
+    // (every wave's ring reads and loads are behind the last barrier of group 0 and the last but one of group 1)
+    gemm_epilogue<Cfg::WM, Cfg::WN, OUT_DT, EPI == DMAF_GENERAL_NORM ? 1 : 0, 0>(a, acc, reinterpret_cast<float*>(smem) + wave * (32 * Cfg::WN),
                                                      m0 + wm * Cfg::WM, n0 + wn * Cfg::WN, lane,
-                                                     reinterpret_cast<float*>(smem + Cfg::STATS_OFF) + wave * (2 * Cfg::WM),
-                                                     reinterpret_cast<const float*>(smem + Cfg::COLS_OFF) + wave * (3 * Cfg::WN));
-  if constexpr (XTRA != 0) {
-    if (extra) {
-      // The extra columns' 32x32 tile of this wave, through the same patch (its bias comes from global memory).
-      f32x16_t ax[1][1];
-      ax[0][0] = accx;
-      wave_lds_fence();
-      gemm_epilogue<32, 32, OUT_DT, 0, LEAN>(a, ax, reinterpret_cast<float*>(smem) + wave * (32 * Cfg::WN),
-                                             m0 + wm * Cfg::WM + wn * 32, n_x, lane);
-    }
+                                                     reinterpret_cast<float*>(smem + 65536) + wave * (2 * Cfg::WM), cols);
+  } else {
+    wait_vmcnt<0>();   // no load to LDS outlives its workgroup
   }
 }
 
-// 0: the general epilogue; 1: without edge, alignment and type guards; 2: with the call's shape fixed at compile time as well
-// (see gemm_epilogue), which is what the products of a large forward pass are.
-inline int dmaf_lean_level(const GemmArgs& a, int out_dt, bool res_norm);
-inline bool dmaf_lean_ok(const GemmArgs& a) {
-  return a.M % DmafCfg::BM == 0 && a.vec_ok && a.N % 8 == 0 && a.nsplit % 8 == 0 && !a.amax && a.res_rows == 0 && !a.ln_out &&
-         (!a.res || a.res_dtype == DT_BF16);
+// Which instance serves a call. 0 / 1: the general ones.
+inline int dmaf_epilogue(const GemmArgs& a, int in_dt, int out_dt) {
+  const int general = a.res_stats ? DMAF_GENERAL_NORM : DMAF_GENERAL, osz = out_dt == DT_F32 ? 4 : out_dt == DT_FP8 ? 1 : 2;
+  // 16-byte stores of whole column groups inside one tile, offsets inside a tile that fit 31 bits, two slabs at least (the
+  // constants of a tile land during its second slab)
+  if (!a.vec_ok || a.N % (out_dt == DT_FP8 ? 16 : 8) || (a.nsplit < a.N && a.nsplit % DmafCfg::BN) || a.amax || a.res_rows > 0 || a.ln_out) return general;
+  if ((long)a.K * (in_dt == DT_FP8 ? 1 : 2) < 2 * DmafCfg::ROWB) return general;
+  if (a.ldc * osz * 256 >= (1L << 31) || a.ldc2 * osz * 256 >= (1L << 31) || (a.res && a.ldr * 4 * 256 >= (1L << 31)) || a.ldc < a.nsplit) return general;
+  if (a.res_stats) return a.act == ACT_NONE && out_dt == DT_BF16 ? DMAF_RESNORM : general;
+  if (!a.res) {
+    if (a.alpha != 1.f || out_dt == DT_F32) return general;
+    if (out_dt == DT_FP8) return a.act == ACT_MISH || a.act == ACT_GELU ? DMAF_PLAIN : general;
+    return a.act == ACT_NONE || a.act == ACT_MISH || (a.act == ACT_GELU && out_dt == DT_BF16 && in_dt == DT_BF16) ? DMAF_PLAIN : general;
+  }
+  if (out_dt == DT_F32) return a.res_dtype == DT_F32 && a.act == ACT_NONE ? DMAF_RES32 : general;
+  if (out_dt == DT_FP8 || a.res_dtype != out_dt) return general;
+  return a.act == ACT_NONE || (a.act == ACT_GELU && out_dt == DT_BF16 && in_dt == DT_BF16) ? DMAF_RES16 : general;
 }
 
-inline int dmaf_lean_level(const GemmArgs& a, int out_dt, bool res_norm) {
-  if (!dmaf_lean_ok(a)) return 0;
-  if (!a.stream_out) return 1;
-  if (res_norm) return a.act == ACT_NONE ? 2 : 1;
-  if (a.res || a.alpha != 1.f) return 1;
-  return a.act == (out_dt == DT_FP8 ? ACT_MISH : ACT_NONE) ? 2 : 1;
-}
-
-// Whether the XTRA instance serves this call: a column split at a multiple of 256 with at most 32 columns behind it.
-inline bool dmaf_xtra_ok(const GemmArgs& a) {
-  return a.C2 != nullptr && a.nsplit >= 256 && a.nsplit % 256 == 0 && a.N > a.nsplit && a.N - a.nsplit <= 32;
-}
-
-template <int IN_DT, int OUT_DT, int RES_NORM = 0, int LEAN = 0, int XTRA = 0>
-static hipError_t launch_dmaf(const GemmArgs& a, hipStream_t st) {
+template <int IN_DT, int OUT_DT, int EPI, int ACT = ACT_NONE>
+static hipError_t launch_dmaf(const GemmArgs& a, int cus, hipStream_t st) {
   static std::atomic<bool> attr_set[16] = {};
   hipError_t e = hipSuccess;
   // Whole slabs of K only, and lane offsets inside a tile's 256 rows that fit 31 bits.
@@ -369,20 +581,20 @@ static hipError_t launch_dmaf(const GemmArgs& a, hipStream_t st) {
   if ((a.K * ESZ) % DmafCfg::ROWB != 0 || a.K <= 0 || (long)a.lda * ESZ * 256 >= (1L << 31) || (long)a.ldw * ESZ * 256 >= (1L << 31)) return hipErrorInvalidValue;
   int dev = 0;
   (void)hipGetDevice(&dev);
-  auto kern = gemm_dmaf_kernel<IN_DT, OUT_DT, RES_NORM, LEAN, XTRA>;
-  constexpr int LDS = XTRA ? DmafCfg::LDS_BYTES_XTRA : DmafCfg::LDS_BYTES;
-  if (!attr_set[dev]) {
+  auto kern = gemm_dmaf_kernel<IN_DT, OUT_DT, EPI, ACT>;
+  constexpr int LDS = DmafCfg::LDS_BYTES;
+  if (dev < 0 || dev >= 16 || !attr_set[dev]) {
     e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
     if (e != hipSuccess) return e;
-    attr_set[dev] = true;
+    if (dev >= 0 && dev < 16) attr_set[dev] = true;
   }
-  const int Nt = XTRA ? a.nsplit : a.N;   // columns the tile columns cover
-  const int tiles_n = (Nt + DmafCfg::BN - 1) / DmafCfg::BN;
+  const int tiles_n = (a.N + DmafCfg::BN - 1) / DmafCfg::BN;
   const int tiles = ((a.M + DmafCfg::BM - 1) / DmafCfg::BM) * tiles_n;
-  // (the L2 touches pay for e4m3 operands only: the 16-bit instances lose 2-6 % with them)
-  const int pf = (IN_DT == DT_FP8 && tiles_n % 4 == 0 && (long)a.K >= 8 * DmafCfg::ROWB) ? 2 : 0;
   if (tiles >= 65536) return hipErrorInvalidValue;   // (the walk's divisions are exact below that; the caller has another kernel)
-  hipLaunchKernelGGL(kern, dim3(tiles), dim3(DmafCfg::NT), LDS, st, a, pf, dmaf_walk(a.M, Nt, IN_DT == DT_FP8));
+  // One workgroup per CU walks the tiles (a multiple of eight, so that every XCD has its share), or one per tile.
+  const int slots = cus >= 8 ? cus & ~7 : 256;
+  const int grid = EPI >= DMAF_PLAIN && tiles > slots ? slots : tiles;
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(DmafCfg::NT), LDS, st, a, dmaf_walk(a.M, a.N, IN_DT == DT_FP8), tiles);
   return hipGetLastError();
 }
 

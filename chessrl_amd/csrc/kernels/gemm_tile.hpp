@@ -519,9 +519,9 @@ hipError_t launch_gemm_dma(const GemmArgs& a, int in_dt, int out_dt, hipStream_t
 // One 256-byte block of zeros per device (gemm.hip): the source of K-tail chunks for the direct-to-LDS loads.
 const uint8_t* device_zeros(hipError_t* err);
 hipError_t launch_gemm_dma_resnorm(const GemmArgs& a, hipStream_t st);   // gemm_dma_resnorm.hip
-// gemm_dmaf.hip: the eight-wave in-step tile with address arithmetic kept out of the main loop (K in whole 128-byte slabs).
+// gemm_dmaf.hip: the 256x256 tile whose waves take turns at multiplying and loading (K in whole 128-byte slabs), on `cus` compute units.
 bool gemm_dmaf_has(int in_dt, int out_dt, bool res_norm);
-hipError_t launch_gemm_dmaf(const GemmArgs& a, int in_dt, int out_dt, hipStream_t st);
+hipError_t launch_gemm_dmaf(const GemmArgs& a, int in_dt, int out_dt, int cus, hipStream_t st);
 // gemm_dmam.hip: the 128x128 tile fed by direct-to-LDS loads through a four-stage ring (K in whole 128-byte slabs, no normalised residual).
 bool gemm_dmam_has(int in_dt, int out_dt);
 hipError_t launch_gemm_dmam(const GemmArgs& a, int in_dt, int out_dt, hipStream_t st);
