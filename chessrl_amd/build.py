@@ -23,6 +23,7 @@ SOURCES = [
     "kernels/gemm_dmam.hip",
     "kernels/gemm_dmas.hip",
     "kernels/gemm_shortk.hip",
+    "kernels/gemm_norm.hip",
     "kernels/norm_embed.hip",
     "kernels/attention.hip",
     "kernels/heads.hip",

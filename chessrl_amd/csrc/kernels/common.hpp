@@ -160,6 +160,22 @@ struct GemmArgs {
   int c_blocked;
 };
 
+// LayerNorm (or RMSNorm) of X's rows and the product with W behind it, one launch (gemm_norm_kernel.hpp).
+struct NormGemmArgs {
+  const float* x; long ldx;                    // [M, K] rows to normalise
+  const float* gamma; const float* beta;       // [K]; beta may be null
+  float eps; int rms;
+  float x_scale;                               // e4m3 operands: the normalised values are multiplied by this before the conversion
+  const void* W; long ldw;                     // [N, K]
+  const float* bias;                           // [N] or null
+  void* out; void* out2; long ldo, ldo2;       // [M, nsplit] and [M, N - nsplit]
+  int M, N, K, nsplit, act, out_dtype, vec_ok;
+  float descale, out_scale;
+};
+int device_cus();   // compute units of the current device (gemm.hip)
+int gemm_norm_width(int M, int N, int K, int in_dt, int cus);
+hipError_t launch_gemm_norm(NormGemmArgs a, int in_dt, int width, bool k_parallel, hipStream_t st);
+
 struct LayerNormArgs {
   const void* x;        // [rows, C]
   const float* gamma;   // [C]
@@ -277,6 +293,8 @@ struct SampleArgs {
   long end_think, end_tok, end_variation;
   float temperature;
   uint64_t seed;
+  const float* wte; const float* pe; // optional (with emb_out): token [V, emb_C] and position embeddings;
+  void* emb_out; int emb_C, emb_dtype;   // [B, emb_C] receives wte[token] + pe[64 + k]
   const int* dyn_k;                  // optional device counter: k and step are read from it (graph replays), step_out advances with it
 };
 
@@ -324,8 +342,6 @@ hipError_t launch_widen(const void* src, int dt, float* dst, long n, hipStream_t
 hipError_t launch_kv_store(const void* qkv, void* cache, int B, int T, int Tmax, int C, hipStream_t st);
 // dyn_k (optional, device): the kernels take the token index k from it instead of from their arguments, so one captured
 // graph serves every step: position = 64 + k, keys = 65 + k.
-hipError_t launch_decode_embed(const int64_t* tok, const float* wte, const float* pe, int pos, const int* dyn_k, void* out, int B, int C, int V,
-                               int out_dtype, hipStream_t st);
 hipError_t launch_decode_attention(const void* q, long ldq, const void* cache, int Tmax, int C, int n, const int* dyn_k, void* out, long ldo,
                                    int B, int H, int head_dim, int in_dtype, float scale, hipStream_t st);
 // staging [B, 2C] -> row (pos or 64 + *dyn_k) of every sequence's [Tmax, 2C] cache

@@ -18,9 +18,10 @@ static hipError_t launch_small(const GemmArgs& a, int in_dt, int out_dt, hipStre
   return hipErrorInvalidValue;
 }
 
-// tile_size: 64 (eight stages) or 32 (sixteen); the operand types are those of gemm_dmam_has.
+// tile_size: 64 (eight stages) or 32 (sixteen); the operand types are those of gemm_dmam_has. With k_parallel set the 32x32 tile spreads K over four waves.
 hipError_t launch_gemm_dmas(const GemmArgs& a, int in_dt, int out_dt, hipStream_t st, int tile_size) {
-  return tile_size == 64 ? launch_small<DmasCfg<64>>(a, in_dt, out_dt, st) : launch_small<DmasCfg<32>>(a, in_dt, out_dt, st);
+  if (tile_size == 64) return launch_small<DmasCfg<64>>(a, in_dt, out_dt, st);
+  return a.k_parallel ? launch_small<DmasCfg<32, 4>>(a, in_dt, out_dt, st) : launch_small<DmasCfg<32>>(a, in_dt, out_dt, st);
 }
 
 }  // namespace crl

@@ -21,13 +21,15 @@
 namespace crl {
 
 // BT = 64: eight stages of 16 KB, four computing waves of 32x32; BT = 32: sixteen stages of 8 KB, one. Eight loading waves either
-// way, which keep AHEAD slabs requested (at the CU's load rate a slab of 8 KB takes 128 cycles, and memory some 1000), and one
+// way, which keep AHEAD slabs requested (at the CU's load rate a slab of 8 KB takes 128 cycles, and memory some 1000; twelve of them delay the first: GPT one position 217 -> 228 us), and one
 // wave that fetches what the epilogue needs.
-template <int BT>
+// KP > 1 (token steps, whose sums may be added in another order): KP computing waves per 32x32 take the slabs in turn.
+template <int BT, int KP_ = 1>
 struct DmasCfg {
   static_assert(BT == 64 || BT == 32, "two tile sizes");
+  static_assert(KP_ == 1 || (BT == 32 && KP_ <= 4), "patches of the K groups lie in stages nothing is loaded into any more");
   static constexpr int BM = BT, BN = BT, WGM = BT / 32, WGN = BT / 32;
-  static constexpr int NCOMP = WGM * WGN, NLOAD = 8, NT = 64 * (NCOMP + NLOAD + 1);
+  static constexpr int KP = KP_, NCOMP = WGM * WGN * KP, NLOAD = 8, NT = 64 * (NCOMP + NLOAD + 1);
   static constexpr int ROWB = 128, NSTAGE = 512 / BT, AHEAD = 6;
   static constexpr int LOADS = 2 * BT / (8 * NLOAD);           // load instructions (8 rows each) of a wave per stage
   static constexpr int STAGE = BN * ROWB;                      // bytes of one operand's rows in one stage
@@ -290,17 +292,23 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_dmas_kernel(const SmallArgs s) {
     // This thread's part of the epilogue: row er, columns ec .. ec + EV - 1 of the tile.
     constexpr int TPR = BN / EV;   // threads per row
     const int et = tid - 64 * Cfg::NCOMP, er = et / TPR, ec = (et % TPR) * EV;
-    const float* patch = reinterpret_cast<const float*>(smem + Cfg::patch_off(nslab, (er >> 5) + (ec >> 5) * Cfg::WGM));
     const int pr = er & 31, pc = ec & 31;
     float acc[EV];
-    if constexpr (EV == 8) {
-      const f32x4_t lo = *reinterpret_cast<const f32x4_t*>(patch + pr * 32 + (((pc >> 2) ^ (pr & 7)) << 2));
-      const f32x4_t hi = *reinterpret_cast<const f32x4_t*>(patch + pr * 32 + ((((pc >> 2) + 1) ^ (pr & 7)) << 2));
 #pragma unroll
-      for (int e = 0; e < 4; ++e) { acc[e] = lo[e]; acc[4 + e] = hi[e]; }
-    } else {
-      const float2 p2 = *reinterpret_cast<const float2*>(patch + pr * 32 + (((pc >> 2) ^ (pr & 7)) << 2) + (pc & 3));
-      acc[0] = p2.x; acc[1] = p2.y;
+    for (int p = 0; p < Cfg::KP; ++p) {
+      const float* patch = reinterpret_cast<const float*>(smem + Cfg::patch_off(nslab, (er >> 5) + (ec >> 5) * Cfg::WGM + p * Cfg::WGM * Cfg::WGN));
+      float part[EV];
+      if constexpr (EV == 8) {
+        const f32x4_t lo = *reinterpret_cast<const f32x4_t*>(patch + pr * 32 + (((pc >> 2) ^ (pr & 7)) << 2));
+        const f32x4_t hi = *reinterpret_cast<const f32x4_t*>(patch + pr * 32 + ((((pc >> 2) + 1) ^ (pr & 7)) << 2));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) { part[e] = lo[e]; part[4 + e] = hi[e]; }
+      } else {
+        const float2 p2 = *reinterpret_cast<const float2*>(patch + pr * 32 + (((pc >> 2) ^ (pr & 7)) << 2) + (pc & 3));
+        part[0] = p2.x; part[1] = p2.y;
+      }
+#pragma unroll
+      for (int e = 0; e < EV; ++e) acc[e] = p == 0 ? part[e] : acc[e] + part[e];
     }
     if (__builtin_expect(small_tile_full(s, n0, BN), 1))
       small_full<OUT_DT, EV>(s, acc, m0 + er, n0 + ec, n0 < s.nsplit, reinterpret_cast<const float*>(smem + Cfg::BIAS_OFF) + ec,
@@ -309,7 +317,7 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_dmas_kernel(const SmallArgs s) {
     return;
   }
 
-  const int wm = wave % Cfg::WGM, wn = wave / Cfg::WGM;
+  const int wm = wave % Cfg::WGM, wn = wave / Cfg::WGM % Cfg::WGN;
   if (m0 + wm * 32 >= s.M || n0 + wn * 32 >= s.N) {
     for (int slab = 0; slab <= nslab; ++slab) dmas_barrier();
     return;
@@ -344,33 +352,45 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_dmas_kernel(const SmallArgs s) {
     }
   };
   __builtin_amdgcn_s_setprio(2);
-  dmas_barrier();
   Frags f0, f1;
-  static_for<0, KSTEPS>([&](auto ksc) { read_step(0, f0, ksc); });
-  auto step = [&](int slab, Frags& cur, Frags& nxt) {
-    dmas_barrier();    // slab + 1 has landed
-    const uint32_t soff = ((slab + 1) & (NSTAGE - 1)) * STAGE;
-    static_for<0, KSTEPS>([&](auto ksc) {
-      constexpr int ks = decltype(ksc)::value;
-      acc = mfma_frag<IN_DT>(cur.w[ks], cur.x[ks], acc);
-      __builtin_amdgcn_sched_barrier(0);
-      read_step(soff, nxt, ksc);
-      __builtin_amdgcn_sched_barrier(0);
-    });
-  };
   auto last_step = [&](Frags& cur) {
     static_for<0, KSTEPS>([&](auto ksc) { constexpr int ks = decltype(ksc)::value; acc = mfma_frag<IN_DT>(cur.w[ks], cur.x[ks], acc); });
   };
-  int slab = 0;
-  for (; slab + 2 < nslab; slab += 2) {
-    step(slab, f0, f1);
-    step(slab + 1, f1, f0);
-  }
-  if (slab + 1 < nslab) {
-    step(slab, f0, f1);
-    last_step(f1);
+  if constexpr (Cfg::KP > 1) {
+    // This wave's slabs are kp, kp + KP, ...: read from LDS and multiplied when they have landed.
+    const int kp = wave / (Cfg::WGM * Cfg::WGN);
+#pragma unroll 1
+    for (int slab = 0; slab < nslab; ++slab) {
+      dmas_barrier();
+      if (slab % Cfg::KP != kp) continue;
+      static_for<0, KSTEPS>([&](auto ksc) { read_step((slab & (NSTAGE - 1)) * STAGE, f0, ksc); });
+      last_step(f0);
+    }
   } else {
-    last_step(f0);
+    dmas_barrier();
+    static_for<0, KSTEPS>([&](auto ksc) { read_step(0, f0, ksc); });
+    auto step = [&](int slab, Frags& cur, Frags& nxt) {
+      dmas_barrier();    // slab + 1 has landed
+      const uint32_t soff = ((slab + 1) & (NSTAGE - 1)) * STAGE;
+      static_for<0, KSTEPS>([&](auto ksc) {
+        constexpr int ks = decltype(ksc)::value;
+        acc = mfma_frag<IN_DT>(cur.w[ks], cur.x[ks], acc);
+        __builtin_amdgcn_sched_barrier(0);
+        read_step(soff, nxt, ksc);
+        __builtin_amdgcn_sched_barrier(0);
+      });
+    };
+    int slab = 0;
+    for (; slab + 2 < nslab; slab += 2) {
+      step(slab, f0, f1);
+      step(slab + 1, f1, f0);
+    }
+    if (slab + 1 < nslab) {
+      step(slab, f0, f1);
+      last_step(f1);
+    } else {
+      last_step(f0);
+    }
   }
   // The sums go to this wave's patch, rows of 32 floats in 16-byte chunks swizzled by row: acc[4 rq + e] is column 8 rq + 4 g + e of row lr.
   float* const patch = reinterpret_cast<float*>(smem + Cfg::patch_off(nslab, wave));

@@ -1,0 +1,262 @@
+// C[M,N] = act(descale * norm(X)[M,K] · W[N,K]^T + bias): a LayerNorm (or RMSNorm) of fp32 rows of K <= 1024 columns and the product that
+// reads it as one launch, for products so small that every tile of 32 x 32 or 32 x 64 has a CU of its own (GPT on one to a few
+// positions, the token steps of generation). There a norm is a launch of 4 us around a handful of rows. Here every workgroup normalises
+// its 32 rows itself: sixteen waves take two rows each, requested before anything is waited for, the workgroup's weight rows
+// follow straight to LDS, and the normalised rows go to LDS as the operand. With both operands whole in LDS (32 K + BN K elements, at most
+// 150 KB) there is no ring and no barrier until the sums are done.
+// Bound by the CU's load rate at first (200 KB at 64 bytes a clock: 3500 of 11000 cycles), then by the norm's own vector instructions, which
+// every tile column repeats. Measured in place: K = 768, N = 2304, 128 rows 8.4 us (12.4 for the norm riding on the K-sliced product before it and the
+// product), 64 rows 7.3 us (8.5 for two launches). The same for the 16-bit rows of 1024 columns of the BT4-class trunk took 9.4 us against 8.7
+// for two launches and is not here.
+// The norm's arithmetic is that of layernorm_kernel row by row and the product adds K in the order of the other tiled kernels (KP = 1): bit-equal to
+// the two launches. KP = 4 (token steps, which may add in another order): four waves share a tile's K and their sums are added in order.
+#pragma once
+#include "gemm_dmaf_kernel.hpp"
+#include "norm_rows.hpp"
+
+namespace crl {
+
+struct NormGemmKArgs {
+  NormGemmArgs a;
+  int nslab, tiles_m;
+  uint32_t m_tm;
+  int per_xcd;
+};
+
+template <int IN_DT, int BN, int KP>
+__global__ void __launch_bounds__(1024) gemm_norm_kernel(const NormGemmKArgs s) {
+  constexpr int ESZ = IN_DT == DT_FP8 ? 1 : 2, ROWB = 128, BM = 32, NB = BN / 32;
+  constexpr int KSTEPS = ROWB / (IN_DT == DT_FP8 ? 64 : 32);
+  constexpr int EV = BM * BN / 1024;                // consecutive columns of an epilogue thread: 1 or 2
+  static_assert(NB * KP <= 16, "waves that multiply");
+  extern __shared__ __align__(16) uint8_t smem[];
+  const NormGemmArgs& a = s.a;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int nslab = s.nslab;
+  // Workgroup b runs on XCD b & 7, which owns a contiguous range of the column-major tile order: the tiles that share weight rows sit together.
+  int pid = blockIdx.x;
+  if (pid < (s.per_xcd << 3)) pid = (pid & 7) * s.per_xcd + (pid >> 3);
+  const int tile_n = dmaf_div(pid, s.m_tm), tile_m = pid - tile_n * s.tiles_m;
+  const int m0 = tile_m * BM, n0 = tile_n * BN;
+  uint8_t* const lds_w = smem;                                   // [slab][BN rows][128 bytes]
+  uint8_t* const lds_a = smem + nslab * BN * ROWB;               // [slab][32 rows][128 bytes]
+
+  float* const lds_g = reinterpret_cast<float*>(lds_a + nslab * BM * ROWB);   // [K] gain, then [K] offset
+
+  // ---- rows of X: wave w takes rows 2 w and 2 w + 1. A lane's 16 columns are those of layernorm_kernel (norm_columns).
+  const int C = a.K;
+  float x[2][2][8];
+  auto has = [&](int i, int h) { return (2 * i + h) * 256 < C; };   // (whole groups of 256 columns: the same for all lanes)
+  // Gain and offset first: when a wave's rows are there, so is its share of these.
+  // 256 columns per wave-instruction, waves 0-3 and 4-7
+  if (wave < 8) {
+    const float* src = wave < 4 ? a.gamma : a.beta;
+    const int c = (wave & 3) * 256 + lane * 4;
+    if (src && (wave & 3) * 256 < C)
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src + (c < C ? c : 0)),
+                                       (__attribute__((address_space(3))) void*)(lds_g + (wave >> 2) * 1024 + (wave & 3) * 256), 16, 0, 0);
+    else if (!src) *reinterpret_cast<f32x4_t*>(lds_g + 1024 + (wave & 3) * 256 + lane * 4) = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  }
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    int m = m0 + wave * 2 + r;
+    m = m < a.M ? m : a.M - 1;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) load_norm8<DT_F32>(a.x, (long)m * a.ldx, i, lane, C, x[r][i]);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  // ---- weight rows: 8 rows of 128 bytes per instruction, the swizzle applied on the global side
+  {
+    constexpr int GR = BN / 8;                                   // row groups of a slab
+    const int grp = wave % GR, s0 = wave / GR, l8 = lane >> 3;
+    const int ldb = (int)a.ldw * ESZ, left = a.N - n0;
+    int r = grp * 8 + l8;
+    r = r < left ? r : left - 1;
+    const int voff = r * ldb + (((lane & 7) ^ l8 ^ (grp & 7)) << 4);
+    const __amdgpu_buffer_rsrc_t rs = dmaf_rsrc(reinterpret_cast<const uint8_t*>(a.W) + (long)n0 * ldb, (long)(left < BN ? left : BN) * ldb);
+    // (always the same number, those past K out of bounds and into a spare kilobyte: a wait for what was requested before can then count past them)
+    const __amdgpu_buffer_rsrc_t none = dmaf_rsrc(a.W, 0);
+#pragma unroll
+    for (int j = 0; j < GR; ++j) {
+      const int sl = s0 + j * (16 / GR);
+      dmaf_load16(sl < nslab ? rs : none, sl < nslab ? lds_w + (sl * BN + grp * 8) * ROWB : reinterpret_cast<uint8_t*>(lds_g) + 8192, voff, sl * ROWB);
+    }
+  }
+  // the bias of this thread's columns
+  const int er = tid / (BN / EV), ec = (tid % (BN / EV)) * EV;
+  float bias[EV];
+#pragma unroll
+  for (int e = 0; e < EV; ++e) {
+    const int n = n0 + ec + e;
+    bias[e] = a.bias && n < a.N ? a.bias[n] : 0.f;
+  }
+  // ---- the norm
+  const float inv_c = fast_rcp((float)C);
+  float mean[2], rstd[2];
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    float sum = 0.f;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        if (has(i, h)) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) sum += x[r][i][4 * h + e];
+        }
+    mean[r] = a.rms ? 0.f : wave_sum(sum) * inv_c;
+    float q = 0.f;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        if (has(i, h)) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) { x[r][i][4 * h + e] -= mean[r]; q += x[r][i][4 * h + e] * x[r][i][4 * h + e]; }   // (from here on x - mean)
+        }
+    rstd[r] = rsqrtf(wave_sum(q) * inv_c + a.eps);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  dmaf_barrier();      // every wave has its rows, and so gain and offset are there
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    const int row = wave * 2 + r;
+    // A lane's place in the operand: 16-byte chunk of the column's 128-byte slab row; further groups of columns lie whole slabs behind.
+    constexpr int GB = 4 * ESZ;       // bytes of the lane's consecutive columns
+    const int lb = lane * GB;
+    uint8_t* const dst = lds_a + ((lb >> 7) * BM + row) * ROWB + ((((lb & 127) >> 4) ^ lds_swizzle(row)) << 4) + (lb & 15);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        if (has(i, h)) {
+          const int col = norm_column(true, i, h, lane);
+          const f32x4_t gv = *reinterpret_cast<const f32x4_t*>(lds_g + col), bv = *reinterpret_cast<const f32x4_t*>(lds_g + 1024 + col);
+          float y[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) y[e] = x[r][i][4 * h + e] * rstd[r] * gv[e] + bv[e];
+          uint8_t* const d = dst + (2 * i + h) * 64 * GB / 128 * (BM * ROWB);
+          if constexpr (IN_DT == DT_FP8) *reinterpret_cast<uint32_t*>(d) = pack_fp8x4(y[0] * a.x_scale, y[1] * a.x_scale, y[2] * a.x_scale, y[3] * a.x_scale);
+          else if constexpr (IN_DT == DT_BF16) *reinterpret_cast<uint2*>(d) = make_uint2(pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3]));
+          else
+            *reinterpret_cast<uint2*>(d) = make_uint2((uint32_t)f32_to_f16_bits(y[0]) | ((uint32_t)f32_to_f16_bits(y[1]) << 16),
+                                                      (uint32_t)f32_to_f16_bits(y[2]) | ((uint32_t)f32_to_f16_bits(y[3]) << 16));
+        }
+  }
+  wait_vmcnt_lgkm0<0>();
+  dmaf_barrier();      // the operands are there
+
+
+  // ---- the product
+  const int nb = wave % NB, kp = wave / NB;
+  f32x16_t acc;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+  const bool multiplies = wave < NB * KP && n0 + nb * 32 < a.N;
+  const int lr = lane & 31, g = lane >> 5;
+  if (multiplies) {
+    const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t*)smem);
+    const int LW = (IN_DT == DT_FP8 ? 2 * g : g) ^ lds_swizzle(nb * 32 + lr), LX = (IN_DT == DT_FP8 ? 2 * g : g) ^ lds_swizzle(lr);
+    uint32_t wb[4], xb[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int kc = IN_DT == DT_FP8 ? ((k & 1) | ((k >> 1) << 2)) : 2 * k;
+      wb[k] = lds0 + (nb * 32 + lr) * ROWB + ((kc ^ LW) << 4);
+      xb[k] = lds0 + nslab * BN * ROWB + lr * ROWB + ((kc ^ LX) << 4);
+    }
+    struct Frags { Frag<IN_DT> w[KSTEPS], x[KSTEPS]; };
+    auto piece = [](uint32_t at) -> i32x4_t { return *reinterpret_cast<const __attribute__((address_space(3))) i32x4_t*>(at); };
+    auto read_step = [&](int slab, Frags& f, auto ksc) {
+      constexpr int ks = decltype(ksc)::value;
+      const uint32_t wo = slab * BN * ROWB, xo = slab * BM * ROWB;
+      if constexpr (IN_DT == DT_FP8) {
+        f.w[ks].lo = piece(wb[2 * ks] + wo); f.w[ks].hi = piece(wb[2 * ks + 1] + wo);
+        f.x[ks].lo = piece(xb[2 * ks] + xo); f.x[ks].hi = piece(xb[2 * ks + 1] + xo);
+      } else {
+        f.w[ks].lo = piece(wb[ks] + wo);
+        f.x[ks].lo = piece(xb[ks] + xo);
+      }
+    };
+    int slab = nslab * kp / KP;
+    const int end = nslab * (kp + 1) / KP;
+    Frags f0, f1;
+    static_for<0, KSTEPS>([&](auto ksc) { read_step(slab < end ? slab : 0, f0, ksc); });
+    auto step = [&](int next, Frags& cur, Frags& nxt) {
+      static_for<0, KSTEPS>([&](auto ksc) {
+        constexpr int ks = decltype(ksc)::value;
+        acc = mfma_frag<IN_DT>(cur.w[ks], cur.x[ks], acc);
+        __builtin_amdgcn_sched_barrier(0);
+        read_step(next, nxt, ksc);
+        __builtin_amdgcn_sched_barrier(0);
+      });
+    };
+    auto last_step = [&](Frags& cur) {
+      static_for<0, KSTEPS>([&](auto ksc) { constexpr int ks = decltype(ksc)::value; acc = mfma_frag<IN_DT>(cur.w[ks], cur.x[ks], acc); });
+    };
+    for (; slab + 2 < end; slab += 2) { step(slab + 1, f0, f1); step(slab + 2, f1, f0); }
+    if (slab + 1 < end) { step(slab + 1, f0, f1); last_step(f1); }
+    else if (slab < end) last_step(f0);
+  }
+  dmaf_barrier();   // both operands are read: their space becomes the patches of the sums
+  if (multiplies) {
+    float* const patch = reinterpret_cast<float*>(smem) + wave * 1024;
+#pragma unroll
+    for (int rq = 0; rq < 4; ++rq)
+      *reinterpret_cast<f32x4_t*>(patch + lr * 32 + (((2 * rq + g) ^ (lr & 7)) << 2)) = f32x4_t{acc[4 * rq], acc[4 * rq + 1], acc[4 * rq + 2], acc[4 * rq + 3]};
+  }
+  __syncthreads();
+  // ---- epilogue: row er, columns ec .. ec + EV - 1
+  const int m = m0 + er, n = n0 + ec;
+  if (m >= a.M || n >= a.N) return;
+  float v[EV];
+#pragma unroll
+  for (int e = 0; e < EV; ++e) v[e] = 0.f;
+#pragma unroll
+  for (int p = 0; p < KP; ++p) {
+    const float* patch = reinterpret_cast<const float*>(smem) + (p * NB + (ec >> 5)) * 1024 + er * 32 + ((((ec & 31) >> 2) ^ (er & 7)) << 2) + (ec & 3);
+#pragma unroll
+    for (int e = 0; e < EV; ++e) v[e] = p == 0 ? patch[e] : v[e] + patch[e];
+  }
+  const bool fused_mish = a.out_dtype == DT_FP8 && a.act == ACT_MISH;   // as in gemm_epilogue
+#pragma unroll
+  for (int e = 0; e < EV; ++e) {
+    const float sum = v[e];
+    v[e] = fmaf(sum, a.descale, bias[e]);
+    if (fused_mish) {
+      constexpr float L2E = 1.4426950408889634f;
+      const float nexp = __builtin_amdgcn_exp2f(fmaf(sum, a.descale * L2E, bias[e] * L2E));
+      v[e] *= fmaf(fast_rcp(fmaf(nexp, nexp + 2.f, 2.f)), -2.f * a.out_scale, a.out_scale);
+    } else {
+      v[e] = apply_act(v[e], a.act);
+      if (a.out_dtype == DT_FP8) v[e] *= a.out_scale;
+    }
+    if (a.out_dtype == DT_F16) asm volatile("" : "+v"(v[e]));   // (rounded to fp32 first, as everywhere else)
+  }
+  const bool first = n < a.nsplit;
+  void* const out = first ? a.out : a.out2;
+  const long o = first ? (long)m * a.ldo + n : (long)m * a.ldo2 + (n - a.nsplit);
+  if constexpr (EV == 2) {
+    if (a.vec_ok && n + EV <= a.N) {
+      if (a.out_dtype == DT_F32) *reinterpret_cast<float2*>(reinterpret_cast<float*>(out) + o) = make_float2(v[0], v[1]);
+      else if (a.out_dtype == DT_FP8) *reinterpret_cast<uint16_t*>(reinterpret_cast<uint8_t*>(out) + o) = (uint16_t)pack_fp8x4(v[0], v[1], v[0], v[1]);
+      else *reinterpret_cast<uint32_t*>(reinterpret_cast<uint16_t*>(out) + o) = a.out_dtype == DT_BF16 ? pack_bf16x2(v[0], v[1]) : (uint32_t)f32_to_f16_bits(v[0]) | ((uint32_t)f32_to_f16_bits(v[1]) << 16);
+      return;
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < EV; ++e) {
+    const int c = n + e;
+    if (c >= a.N) break;
+    void* const d = c < a.nsplit ? a.out : a.out2;
+    const long at = c < a.nsplit ? (long)m * a.ldo + c : (long)m * a.ldo2 + (c - a.nsplit);
+    switch (a.out_dtype) {
+      case DT_F32: reinterpret_cast<float*>(d)[at] = v[e]; break;
+      case DT_BF16: reinterpret_cast<uint16_t*>(d)[at] = f32_to_bf16_bits(v[e]); break;
+      case DT_F16: reinterpret_cast<uint16_t*>(d)[at] = f32_to_f16_bits(v[e]); break;
+      default: reinterpret_cast<uint8_t*>(d)[at] = f32_to_fp8(v[e]); break;
+    }
+  }
+}
+
+}  // namespace crl

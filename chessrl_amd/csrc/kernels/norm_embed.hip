@@ -13,53 +13,9 @@
 //
 // One 64-lane wave owns one row; a lane keeps VPL vectors of 8 consecutive columns in
 // registers, so a row is read once and the statistics are two wave reductions.
-#include "common.hpp"
+#include "norm_rows.hpp"
 
 namespace crl {
-
-template <int DT>
-__device__ __forceinline__ void load8(const void* base, long off, float v[8]) {
-  if constexpr (DT == DT_F32) {
-    const float4* p = reinterpret_cast<const float4*>(reinterpret_cast<const float*>(base) + off);
-    float4 a = p[0], b = p[1];
-    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
-  } else {
-    uint4 u = *reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(base) + off);
-    const uint32_t w[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      if constexpr (DT == DT_BF16) {
-        v[2 * i] = bf16_bits_to_f32((uint16_t)(w[i] & 0xffff));
-        v[2 * i + 1] = bf16_bits_to_f32((uint16_t)(w[i] >> 16));
-      } else {
-        v[2 * i] = f16_bits_to_f32((uint16_t)(w[i] & 0xffff));
-        v[2 * i + 1] = f16_bits_to_f32((uint16_t)(w[i] >> 16));
-      }
-    }
-  }
-}
-
-__device__ __forceinline__ void store8(void* base, long off, const float v[8], int dt) {
-  if (dt == DT_F32) {
-    float4* p = reinterpret_cast<float4*>(reinterpret_cast<float*>(base) + off);
-    p[0] = make_float4(v[0], v[1], v[2], v[3]);
-    p[1] = make_float4(v[4], v[5], v[6], v[7]);
-  } else if (dt == DT_BF16) {
-    uint4 u = make_uint4(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7]));
-    *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(base) + off) = u;
-  } else {
-    uint32_t w[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) w[i] = (uint32_t)f32_to_f16_bits(v[2 * i]) | ((uint32_t)f32_to_f16_bits(v[2 * i + 1]) << 16);
-    *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(base) + off) = make_uint4(w[0], w[1], w[2], w[3]);
-  }
-}
-
-__device__ __forceinline__ void store8_fp8(uint8_t* base, long off, const float v[8], float scale) {
-  uint2 u = make_uint2(pack_fp8x4(v[0] * scale, v[1] * scale, v[2] * scale, v[3] * scale),
-                       pack_fp8x4(v[4] * scale, v[5] * scale, v[6] * scale, v[7] * scale));
-  *reinterpret_cast<uint2*>(base + off) = u;
-}
 
 // Normalise the VPL*8 values a lane holds (columns col0(i) = (i*64+lane)*8) and write them.
 // rms: RMSNorm (mean taken as zero, no offset): y = x * rsqrt(mean(x^2) + eps) * gamma.
@@ -103,29 +59,78 @@ __device__ __forceinline__ void ln_finish(float (&x)[VPL][8], int lane, int C, c
   }
 }
 
+// (fp32 rows: a lane's columns are two groups of four per vector, see norm_column; 16-bit rows: eight consecutive ones)
 template <int IN_DT, int VPL, bool FULL = false>
 __global__ void __launch_bounds__(256) layernorm_kernel(const LayerNormArgs a) {
+  constexpr bool F32 = IN_DT == DT_F32;
   const int lane = threadIdx.x & 63;
   const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (row >= a.rows) return;
-  float x[VPL][8], y[VPL][8];
+  const int C = FULL ? VPL * 512 : a.C;
+  auto has = [&](int i, int h) { return FULL || norm_column(F32, i, h, lane) < C; };
+  float x[VPL][8];
 #pragma unroll
-  for (int i = 0; i < VPL; ++i) {
-    const int col = (i * 64 + lane) * 8;
-    if (FULL || col < a.C) load8<IN_DT>(a.x, (long)row * a.ldx + col, x[i]);
-  }
-  ln_finish<VPL, FULL>(x, lane, a.C, a.gamma, a.beta, a.eps, y, a.stats ? a.stats + 2 * (long)row : nullptr, a.rms != 0);
+  for (int i = 0; i < VPL; ++i) load_norm8<IN_DT>(a.x, (long)row * a.ldx, i, lane, C, x[i]);
+  float s = 0.f;
+#pragma unroll
+  for (int i = 0; i < VPL; ++i)
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      if (has(i, h)) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s += x[i][4 * h + e];
+      }
+  // (1 / C by the hardware reciprocal, exact for the power-of-two widths and within one unit in the last place otherwise:
+  // two IEEE divisions are 22 of a row's ~400 instructions)
+  const float inv_c = fast_rcp((float)C);
+  const bool rms = a.rms != 0;
+  const float mean = rms ? 0.f : wave_sum(s) * inv_c;
+  const float* const beta = rms ? nullptr : a.beta;
+  float q = 0.f;
+#pragma unroll
+  for (int i = 0; i < VPL; ++i)
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      if (has(i, h)) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) { const float d = x[i][4 * h + e] - mean; q += d * d; }
+      }
+  const float rstd = rsqrtf(wave_sum(q) * inv_c + a.eps);
+  if (a.stats && lane == 0) *reinterpret_cast<float2*>(a.stats + 2 * (long)row) = make_float2(rstd, -mean * rstd);   // (x - mean) * rstd = x * s0 + s1
   float am = 0.f;
 #pragma unroll
   for (int i = 0; i < VPL; ++i) {
-    const int col = (i * 64 + lane) * 8;
-    if (FULL || col < a.C) {
-      if (a.out) store8(a.out, (long)row * a.ldo + col, y[i], a.out_dtype);
-      if (a.out_b) store8(a.out_b, (long)row * a.ldo + col, y[i], a.out_b_dtype);
-      if (a.out_fp8) store8_fp8(a.out_fp8, (long)row * a.ldo + col, y[i], a.fp8_scale);
-      if (a.amax) {
+    float y[8];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) am = fmaxf(am, fabsf(y[i][e]));
+    for (int h = 0; h < 2; ++h)
+      if (has(i, h)) {
+        const int col = norm_column(F32, i, h, lane);
+        const float4 gv = *reinterpret_cast<const float4*>(a.gamma + col);
+        const float g[4] = {gv.x, gv.y, gv.z, gv.w};
+        float bo[4] = {0.f, 0.f, 0.f, 0.f};
+        if (beta) {
+          const float4 bv = *reinterpret_cast<const float4*>(beta + col);
+          bo[0] = bv.x; bo[1] = bv.y; bo[2] = bv.z; bo[3] = bv.w;
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y[4 * h + e] = (x[i][4 * h + e] - mean) * rstd * g[e] + bo[e];
+        if (a.amax) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) am = fmaxf(am, fabsf(y[4 * h + e]));
+        }
+        if constexpr (F32) {
+          const long off = (long)row * a.ldo + col;
+          if (a.out) store4(a.out, off, y + 4 * h, a.out_dtype);
+          if (a.out_b) store4(a.out_b, off, y + 4 * h, a.out_b_dtype);
+          if (a.out_fp8) store4_fp8(a.out_fp8, off, y + 4 * h, a.fp8_scale);
+        }
+      }
+    if constexpr (!F32) {
+      if (has(i, 0)) {
+        const long off = (long)row * a.ldo + norm_column(false, i, 0, lane);
+        if (a.out) store8(a.out, off, y, a.out_dtype);
+        if (a.out_b) store8(a.out_b, off, y, a.out_b_dtype);
+        if (a.out_fp8) store8_fp8(a.out_fp8, off, y, a.fp8_scale);
       }
     }
   }

@@ -492,6 +492,25 @@ int Model::lnorm(const void* x, long ldx, int in_dt, const float* g, const float
   return CRL_OK;
 }
 
+// (fp32 rows only; the profiling mode times norms and products apart)
+bool Model::norm_gemm_can(int M, const Lin& L, int in_dt, int x_dt) const {
+  return !profiling && x_dt == DT_F32 && gemm_norm_width(M, L.N, L.K, in_dt, device_cus()) != 0;
+}
+
+int Model::norm_gemm(const void* x, long ldx, const float* g, const float* b, const Lin& L, int in_dt, void* C, long ldc, int out_dt, int M, const GOpt& o,
+                     hipStream_t st) {
+  NormGemmArgs a;
+  std::memset(&a, 0, sizeof(a));
+  a.x = reinterpret_cast<const float*>(x); a.ldx = ldx; a.gamma = g; a.beta = b; a.eps = cfg.eps; a.rms = cfg.norm_rms; a.x_scale = o.a_scale;
+  a.W = in_dt == DT_FP8 ? L.w8 : L.w; a.ldw = L.K; a.bias = L.b;
+  if (!a.W) { set_error("norm_gemm: weight copy for the requested element type is missing"); return CRL_ERR_STATE; }
+  a.out = C; a.ldo = ldc; a.out2 = o.C2; a.ldo2 = o.ldc2; a.nsplit = o.nsplit;
+  a.M = M; a.N = L.N; a.K = L.K; a.act = o.act; a.out_dtype = out_dt;
+  a.descale = in_dt == DT_FP8 ? 1.f / (o.a_scale * L.wscale) : 1.f; a.out_scale = o.out_scale;
+  HIPCHK(launch_gemm_norm(a, in_dt, gemm_norm_width(M, L.N, L.K, in_dt, device_cus()), o.k_parallel, st));
+  return CRL_OK;
+}
+
 float Model::act_scale(int layer, int slot) const {
   const float am = amax_host[(size_t)layer * AMAX_SLOTS + slot];
   return am > 0.f ? 448.f / am : 1.f;
@@ -601,14 +620,19 @@ int Model::forward_chunk(const float* planes, const uint8_t* ids, const uint8_t*
   // every position only (queries, output projection, MLP: 10/12 of the layer's products; bit-equal, a row's result does
   // not depend on the other rows). The rows are compact from the attention on: ao [mb, C], the stream in ws.t [mb, C].
   const bool one_row = gpt && policy && !all_logits && !calibrate && L > 0;
+  // GPT64, few rows: a norm runs inside the product behind it (norm_gemm; bit-equal to the two launches). Not while maxima are collected.
+  auto fuses = [&](int rows, const Lin& lin, int dt) { return gpt && !calibrate && norm_gemm_can(rows, lin, dt, xdt); };
   for (int l = l0; l < l1; ++l) {
     const Layer& ly = layers[l];
     const bool last = l + 1 == l1;
     const bool tail = one_row && last;
     const void* a_in; int a_dt; float a_sc = 1.f;
-    if (gpt) {
+    const bool fused_qkv = fuses(M, ly.qkv, f8 ? DT_FP8 : ad);
+    if (gpt && !fused_qkv) {
       // h = LN1(x)
       RUN(lnorm(ws.x, C, xdt, ly.ln1_g, ly.ln1_b, f8 ? nullptr : ws.h, ad, f8 ? ws.h8 : nullptr, f8 ? act_scale(l, 0) : 1.f, C, M, C, am(l, 0), st));
+    }
+    if (gpt) {
       a_in = f8 ? (const void*)ws.h8 : (const void*)ws.h; a_dt = f8 ? DT_FP8 : ad; a_sc = f8 ? act_scale(l, 0) : 1.f;
     } else {
       a_in = f8 ? (const void*)ws.x8 : (const void*)x_op; a_dt = f8 ? DT_FP8 : ad; a_sc = f8 ? act_scale(l, 0) : 1.f;
@@ -618,7 +642,9 @@ int Model::forward_chunk(const float* planes, const uint8_t* ids, const uint8_t*
       GOpt o; o.a_scale = a_sc;
       if (cfg.arch == CRL_ARCH_BT4CLASS) { o.C2 = ws.comp; o.ldc2 = cfg.smolgen_compress; o.nsplit = 3 * C; }
       // (the third of the product that makes unread queries costs more than a second launch from about 16384 rows on)
-      if (tail && M >= 16384) {
+      if (fused_qkv) {
+        RUN(norm_gemm(ws.x, C, ly.ln1_g, ly.ln1_b, ly.qkv, a_dt, ws.qkv, 3 * C, ad, M, o, st));
+      } else if (tail && M >= 16384) {
         char* const qkv_last = reinterpret_cast<char*>(ws.qkv) + (size_t)(T - 1) * 3 * C * dtype_size(ad);
         const char* const a_last = reinterpret_cast<const char*>(a_in) + (size_t)(T - 1) * C * dtype_size(a_dt);
         RUN(gemm(ly.qkv.rows(C, 2 * C), a_in, C, a_dt, reinterpret_cast<char*>(ws.qkv) + (size_t)C * dtype_size(ad), 3 * C, ad, M, o, st));
@@ -673,9 +699,14 @@ int Model::forward_chunk(const float* planes, const uint8_t* ids, const uint8_t*
       const char* const x_res = reinterpret_cast<const char*>(ws.x) + (tail ? (size_t)(T - 1) * C * dtype_size(xdt) : 0);
       { GOpt o; o.res = x_res; o.ldr = tail ? (long)T * C : C; o.res_dt = xdt; o.a_scale = f8 ? act_scale(l, 1) : 1.f;
         RUN(gemm(ly.proj, ao_in, C, ao_dt, x, C, xdt, rows, o, st)); }
-      RUN(lnorm(x, C, xdt, ly.ln2_g, ly.ln2_b, f8 ? nullptr : ws.h, ad, f8 ? ws.h8 : nullptr, f8 ? act_scale(l, 2) : 1.f, C, rows, C, am(l, 2), st));
       { GOpt o; o.act = ACT_GELU; o.a_scale = f8 ? act_scale(l, 2) : 1.f; o.out_scale = f8 ? act_scale(l, 3) : 1.f; o.amax = am(l, 3);
-        RUN(gemm(ly.ff1, f8 ? (const void*)ws.h8 : (const void*)ws.h, C, ao_dt, f8 ? (void*)ws.f8 : (void*)ws.f, F, ao_dt, rows, o, st)); }
+        void* const f = f8 ? (void*)ws.f8 : (void*)ws.f;
+        if (fuses(rows, ly.ff1, ao_dt)) {
+          RUN(norm_gemm(x, C, ly.ln2_g, ly.ln2_b, ly.ff1, ao_dt, f, F, ao_dt, rows, o, st));
+        } else {
+          RUN(lnorm(x, C, xdt, ly.ln2_g, ly.ln2_b, f8 ? nullptr : ws.h, ad, f8 ? ws.h8 : nullptr, f8 ? act_scale(l, 2) : 1.f, C, rows, C, am(l, 2), st));
+          RUN(gemm(ly.ff1, f8 ? (const void*)ws.h8 : (const void*)ws.h, C, ao_dt, f, F, ao_dt, rows, o, st));
+        } }
       { GOpt o; o.res = x; o.ldr = C; o.res_dt = xdt; o.a_scale = f8 ? act_scale(l, 3) : 1.f;
         RUN(gemm(ly.ff2, f8 ? (const void*)ws.f8 : (const void*)ws.f, F, ao_dt, x, C, xdt, rows, o, st)); }
     } else {
@@ -735,8 +766,12 @@ int Model::forward_chunk(const float* planes, const uint8_t* ids, const uint8_t*
     if (policy) {
       // ln_f and lm_head on the last token only (model_bis.py:195-196, 369-370).
       const char* last_tok = one_row ? reinterpret_cast<const char*>(ws.t) : reinterpret_cast<const char*>(ws.x) + (size_t)(T - 1) * C * dtype_size(xdt);
-      RUN(lnorm(last_tok, one_row ? C : (long)T * C, xdt, lnf_g, lnf_b, f8h ? nullptr : ws.hl, hd, f8h ? ws.hl8 : nullptr, hsc, C, mb, C, nullptr, st));
       GOpt o; o.a_scale = hsc;
+      if (fuses(mb, lm_head, f8h ? DT_FP8 : hd)) {
+        RUN(norm_gemm(last_tok, one_row ? C : (long)T * C, lnf_g, lnf_b, lm_head, f8h ? DT_FP8 : hd, policy, VOCAB_RL, DT_F32, mb, o, st));
+        return CRL_OK;
+      }
+      RUN(lnorm(last_tok, one_row ? C : (long)T * C, xdt, lnf_g, lnf_b, f8h ? nullptr : ws.hl, hd, f8h ? ws.hl8 : nullptr, hsc, C, mb, C, nullptr, st));
       RUN(gemm(lm_head, f8h ? (const void*)ws.hl8 : (const void*)ws.hl, C, f8h ? DT_FP8 : hd, policy, VOCAB_RL, DT_F32, mb, o, st));
     }
     return CRL_OK;
@@ -887,39 +922,58 @@ int Model::generate(const float* planes, int B, int steps, float temperature, ui
     sa.ld_out = (long)steps * VOCAB_RL;
     sa.B = B; sa.V = VOCAB_RL; sa.k = k; sa.step = k; sa.rules = rules; sa.out_logits = out_logits; sa.dyn_k = dyn;
     sa.end_think = END_THINK; sa.end_tok = END; sa.end_variation = END_VARIATION; sa.temperature = temperature; sa.seed = seed;
+    if (!sample_only) { sa.wte = wte_f32; sa.pe = pe_f32; sa.emb_out = ws.x; sa.emb_C = C; sa.emb_dtype = xdt; }
     STEP_HIP(launch_sample(sa, s));
     if (sample_only) return CRL_OK;
     const int pos = 64 + k;    // sequence position of token k
-    STEP_HIP(launch_decode_embed(gen_tok, wte_f32, pe_f32, pos, dyn, ws.x, B, C, VOCAB_RL, xdt, s));
-    bool normed = false;   // ws.h (or, after the last layer, ws.hl) already holds the next LayerNorm's output
+    // Few sequences: every norm runs inside the product behind it. Otherwise the norms behind the two residual products ride on
+    // those products' second pass where they are K-sliced (normed: ws.h, or after the last layer ws.hl, holds the next norm's output).
+    const bool fused = norm_gemm_can(B, layers[0].qkv, ad, xdt) && norm_gemm_can(B, layers[0].ff1, ad, xdt);
+    const bool fused_head = fused && norm_gemm_can(B, lm_head, hd, xdt);
+    bool normed = false;
     for (int l = 0; l < L; ++l) {
       const Layer& ly = layers[l];
-      if (!normed) STEP_RUN(lnorm(ws.x, C, xdt, ly.ln1_g, ly.ln1_b, ws.h, ad, nullptr, 1.f, C, B, C, nullptr, s));
-      if (dyn) {
-        // q -> ws.qkv [B,C]; k|v -> staging, then to the row the counter names
-        GOpt o; o.k_parallel = true; o.C2 = gen_kv_stage; o.ldc2 = 2 * C; o.nsplit = C;
-        STEP_RUN(gemm(ly.qkv, ws.h, C, ad, ws.qkv, C, ad, B, o, s));
-        STEP_HIP(launch_kv_append(gen_kv_stage, kv_layers[l], B, kv_Tmax, C, 0, dyn, s));
-      } else {
-        // q -> ws.qkv [B,C]; k|v -> row `pos` of every sequence's cache
-        GOpt o; o.k_parallel = true; o.C2 = reinterpret_cast<uint16_t*>(kv_layers[l]) + (size_t)pos * 2 * C; o.ldc2 = (long)kv_Tmax * 2 * C; o.nsplit = C;
-        STEP_RUN(gemm(ly.qkv, ws.h, C, ad, ws.qkv, C, ad, B, o, s));
+      {
+        // q -> ws.qkv [B,C]; k|v -> row `pos` of every sequence's cache, in a replayed step by way of a staging area (the row is the counter's)
+        GOpt o; o.k_parallel = true; o.nsplit = C;
+        if (dyn) { o.C2 = gen_kv_stage; o.ldc2 = 2 * C; }
+        else { o.C2 = reinterpret_cast<uint16_t*>(kv_layers[l]) + (size_t)pos * 2 * C; o.ldc2 = (long)kv_Tmax * 2 * C; }
+        if (fused) {
+          STEP_RUN(norm_gemm(ws.x, C, ly.ln1_g, ly.ln1_b, ly.qkv, ad, ws.qkv, C, ad, B, o, s));
+        } else {
+          if (!normed) STEP_RUN(lnorm(ws.x, C, xdt, ly.ln1_g, ly.ln1_b, ws.h, ad, nullptr, 1.f, C, B, C, nullptr, s));
+          STEP_RUN(gemm(ly.qkv, ws.h, C, ad, ws.qkv, C, ad, B, o, s));
+        }
+        if (dyn) STEP_HIP(launch_kv_append(gen_kv_stage, kv_layers[l], B, kv_Tmax, C, 0, dyn, s));
       }
       STEP_HIP(launch_decode_attention(ws.qkv, C, kv_layers[l], kv_Tmax, C, pos + 1, dyn, ws.ao, C, B, H, hs, ad, attn_scale, s));
       bool normed2 = false;
       { GOpt o; o.k_parallel = true; o.res = ws.x; o.ldr = C; o.res_dt = xdt;
-        o.ln_g = ly.ln2_g; o.ln_b = ly.ln2_b; o.ln_out = ws.h; o.ln_dt = ad; o.ln_folded = &normed2;
+        if (!fused) { o.ln_g = ly.ln2_g; o.ln_b = ly.ln2_b; o.ln_out = ws.h; o.ln_dt = ad; o.ln_folded = &normed2; }
         STEP_RUN(gemm(ly.proj, ws.ao, C, ad, ws.x, C, xdt, B, o, s)); }
-      if (!normed2) STEP_RUN(lnorm(ws.x, C, xdt, ly.ln2_g, ly.ln2_b, ws.h, ad, nullptr, 1.f, C, B, C, nullptr, s));
-      { GOpt o; o.k_parallel = true; o.act = ACT_GELU; STEP_RUN(gemm(ly.ff1, ws.h, C, ad, ws.f, F, ad, B, o, s)); }
-      { // the norm that reads this GEMM's result (the next layer's ln_1, or ln_f) rides on its second pass where it is K-sliced
-        GOpt o; o.k_parallel = true; o.res = ws.x; o.ldr = C; o.res_dt = xdt; o.ln_folded = &normed;
-        if (l + 1 < L) { o.ln_g = layers[l + 1].ln1_g; o.ln_b = layers[l + 1].ln1_b; o.ln_out = ws.h; o.ln_dt = ad; }
-        else { o.ln_g = lnf_g; o.ln_b = lnf_b; o.ln_out = ws.hl; o.ln_dt = hd; }
+      { GOpt o; o.k_parallel = true; o.act = ACT_GELU;
+        if (fused) {
+          STEP_RUN(norm_gemm(ws.x, C, ly.ln2_g, ly.ln2_b, ly.ff1, ad, ws.f, F, ad, B, o, s));
+        } else {
+          if (!normed2) STEP_RUN(lnorm(ws.x, C, xdt, ly.ln2_g, ly.ln2_b, ws.h, ad, nullptr, 1.f, C, B, C, nullptr, s));
+          STEP_RUN(gemm(ly.ff1, ws.h, C, ad, ws.f, F, ad, B, o, s));
+        } }
+      { GOpt o; o.k_parallel = true; o.res = ws.x; o.ldr = C; o.res_dt = xdt;
+        normed = false;
+        if (!fused) {
+          o.ln_folded = &normed;
+          if (l + 1 < L) { o.ln_g = layers[l + 1].ln1_g; o.ln_b = layers[l + 1].ln1_b; o.ln_out = ws.h; o.ln_dt = ad; }
+          else { o.ln_g = lnf_g; o.ln_b = lnf_b; o.ln_out = ws.hl; o.ln_dt = hd; }
+        }
         STEP_RUN(gemm(ly.ff2, ws.f, F, ad, ws.x, C, xdt, B, o, s)); }
     }
-    if (!normed) STEP_RUN(lnorm(ws.x, C, xdt, lnf_g, lnf_b, ws.hl, hd, nullptr, 1.f, C, B, C, nullptr, s));
-    { GOpt o; o.k_parallel = true; STEP_RUN(gemm(lm_head, ws.hl, C, hd, gen_logits, VOCAB_RL, DT_F32, B, o, s)); }
+    { GOpt o; o.k_parallel = true;
+      if (fused_head) {
+        STEP_RUN(norm_gemm(ws.x, C, lnf_g, lnf_b, lm_head, hd, gen_logits, VOCAB_RL, DT_F32, B, o, s));
+      } else {
+        if (!normed) STEP_RUN(lnorm(ws.x, C, xdt, lnf_g, lnf_b, ws.hl, hd, nullptr, 1.f, C, B, C, nullptr, s));
+        STEP_RUN(gemm(lm_head, ws.hl, C, hd, gen_logits, VOCAB_RL, DT_F32, B, o, s));
+      } }
     if (dyn) STEP_HIP(launch_add_int(gen_k, 1, s));
     return CRL_OK;
 #undef STEP_HIP

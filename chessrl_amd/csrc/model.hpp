@@ -146,6 +146,9 @@ struct Model {
   int lnorm(const void* x, long ldx, int in_dt, const float* g, const float* b, void* out, int out_dt, uint8_t* out8, float scale8,
             long ldo, int rows, int C, float* amax, hipStream_t st, float* stats = nullptr, void* out_b = nullptr, int out_b_dt = DT_BF16,
             bool trunk = true);
+  // Norm of x's rows (fp32) and the product behind it in one launch; in_dt is the product's operand type. norm_gemm_can: the call is small enough.
+  bool norm_gemm_can(int M, const Lin& L, int in_dt, int x_dt) const;
+  int norm_gemm(const void* x, long ldx, const float* g, const float* b, const Lin& L, int in_dt, void* C, long ldc, int out_dt, int M, const GOpt& o, hipStream_t st);
   float act_scale(int layer, int slot) const;
   void prof_begin(int fam, hipStream_t st);
   void prof_end(hipStream_t st);

@@ -738,6 +738,37 @@ def test_generate_forced_tokens(cuda):
     assert row[1:i].count(1926) == 5 and row[i + 2] == 1927
 
 
+@pytest.mark.parametrize("kw", [{}, {"act_dtype": "f16"}, {"fp8": True}, {"norm_rms": True}, {"fp8": True, "stream_f32": False}])
+@pytest.mark.parametrize("n_head,n_embd", [(12, 768), (8, 256), (10, 320)])
+def test_gpt_norm_inside_the_product_is_bit_equal(cuda, kw, n_head, n_embd):
+    """Calls of few rows run their norms inside the products (32 columns per workgroup, then 64, then two launches as the batch
+    grows; never with a 16-bit stream or a width that is not whole groups of 256 columns): a position's logits have the same bits in every batch."""
+    planes, _ = positions(40, seed=3)
+    m = models.GPT(models.GPTConfig(block_size=128, vocab_size=1929, n_layer=2, n_head=n_head, n_embd=n_embd), **kw)
+    x = planes.to(cuda)
+    if kw.get("fp8"):
+        m.calibrate(x)
+    base = m.forward((x, None))[0]
+    idx = torch.randint(0, 1924, (40, 3), generator=torch.Generator().manual_seed(1)).to(cuda)
+    tokens = m.forward((x, idx))[0]
+    for B in (1, 2, 3, 5, 7, 11, 33):
+        assert torch.equal(m.forward((x[:B].contiguous(), None))[0], base[:B]), B
+        assert torch.equal(m.forward((x[:B].contiguous(), idx[:B].contiguous()))[0], tokens[:B]), B
+
+
+@pytest.mark.parametrize("kw", [{}, {"norm_rms": True}])
+def test_generate_rows_do_not_depend_on_the_batch(cuda, kw):
+    """Token steps of 1 to 160 sequences: norms inside the products, K of the residual products over four waves. Same sums for
+    every tile width, so a sequence's tokens and logits have the same bits in every such batch."""
+    planes, _ = positions(160, seed=8)
+    m = models.GPT(models.GPTConfig(block_size=256, vocab_size=1929, n_layer=2, n_head=12, n_embd=768), **kw)
+    x = planes.to(cuda)
+    seq, out = m._engine.generate(x, 6, T=0.0, rules=False, want_step_out=True, out_logits=True)
+    for B in (1, 31, 33, 64, 129):
+        s, o = m._engine.generate(x[:B].contiguous(), 6, T=0.0, rules=False, want_step_out=True, out_logits=True)
+        assert torch.equal(s, seq[:B]) and torch.equal(o, out[:B]), B
+
+
 @pytest.mark.parametrize("kw", [{}, {"act_dtype": "f16"}, {"fp8": True}, {"stream_f32": False}])
 @pytest.mark.parametrize("B,t", [(1, 0), (3, 1), (255, 0), (256, 0), (250, 3), (130, 66)])
 def test_gpt_last_token_row(cuda, kw, B, t):
