@@ -571,7 +571,7 @@ static hipError_t launch_splitk(const GemmArgs& a, int ks, int per, hipStream_t 
 template <int IN_DT, int OUT_DT>
 static hipError_t launch_in_out(const GemmArgs& a, int tile, hipStream_t st) {
   if (a.ln_out && !gemm_folds_layernorm(a, IN_DT)) return hipErrorInvalidValue;   // only the K-sliced path has a whole row in one place
-  if (a.res_stats && (a.k_parallel || (tile >= 4 && tile != 7 && tile != 9 && tile != 10 && tile != 12))) return hipErrorInvalidValue;   // the tiled kernels only
+  if (a.res_stats && (a.k_parallel || (tile >= 4 && tile != 7 && (tile < 9 || tile > 12)))) return hipErrorInvalidValue;   // the tiled kernels only
   // K = 256 e4m3 elements into a large 16-bit output (the attention-bias generator): the kernel whose workgroups keep
   // their rows of A and walk N (gemm_shortk_kernel.hpp; tile 13). It is the only one that writes the blocked layout, and
   // that is what it is for: M = 131072, N = 4096 takes 280 us through the 256x256 tile, 310 us here row-major and 191 us
@@ -589,9 +589,7 @@ static hipError_t launch_in_out(const GemmArgs& a, int tile, hipStream_t st) {
     if (tile == 4) tile = 1;
   }
   if (tile == 0) {
-    // Largest tile that still gives (nearly) every CU a workgroup. One round of 256x256 tiles takes about as long
-    // whether 160 or 256 CUs have one (33-37 us at K=1024 in bf16), and from about 160 tiles on that is less than the
-    // 128x128 tiles need (M=4096, N=3104: 47 -> 37 us; M=8192, N=1536: 39 -> 35 us; 128 tiles or fewer: slower).
+    // Largest tile that still gives (nearly) every CU a workgroup; which of the pipelined kernels takes it is decided below.
     const long big = (long)((a.M + 255) / 256) * ((a.N + 255) / 256);
     const long mid = (long)((a.M + 127) / 128) * ((a.N + 127) / 128);
     tile = big >= 160 ? 3 : mid >= 256 ? 2 : 1;
@@ -609,13 +607,25 @@ static hipError_t launch_in_out(const GemmArgs& a, int tile, hipStream_t st) {
       const int ks = splitk_plan_fixed(a, IN_DT == DT_FP8 ? 1 : 2, &per);
       if (ks > 1) return launch_splitk<CfgSmallK4, IN_DT, OUT_DT>(a, ks, per, st);
     }
-    // Fewer than 256 tiles of 128x128 and K in whole slabs: the ring kernels of gemm_dmam_kernel.hpp (bit-equal). On 32x32
-    // tiles while every such tile has a CU of its own (tile 16; one position), else on 64x64 tiles while every one of
-    // those has (tile 15; M=64, N=1024, K=1024 bf16 with weights from HBM: 13.6 us register-staged, 8.4 us on 15; from
-    // warm caches 9.1, 7.6 and, on 16, 6.9 us), on 128x128 tiles beyond (tile 11; M=1024, N=3104: 20.7 -> 14.9 us;
-    // M=2048, N=1536: 18.0 -> 14.1 us; M=512, N=3104: 13.9 -> 12.5 us; level at M=1024, N=1536 and M=2048, N=1024).
-    if (tile == 1 && ring_ok)
+    // K in whole slabs: the kernels with direct-to-LDS rings (bit-equal). 32x32 tiles while every such tile has a CU of its own
+    // (tile 16; one position), else 64x64 tiles while every one of those has (tile 15; M=1024, N=1024, K=1024 bf16: 6.0 us, 9.8 on 128x128).
+    // Beyond, 128x128 (tile 11) or 256x256 (tile 3), both persistent: a round of 256x256 tiles over the CUs takes as long as 2.55 rounds
+    // of 128x128 ones with 16-bit operands (K=1024: 27 against 10.5 us) and as 3.3 with e4m3, whose larger tile spends more of its time in prologue and
+    // epilogue (16.5 against 5 us); K=256 (the bias generator) is mostly epilogue: 4.2, on many rounds 3.3. Measured over M = 256 .. 16384 at N = 1024, 1536, 2304, 3104, 4096,
+    // the rule is within 5 % of the better tile but for partly filled rounds (at most 11 %).
+    if (!a.k_parallel && tile != 5) {
+      const bool slabs = ((long)a.K * (IN_DT == DT_FP8 ? 1 : 2)) % 128 == 0;
+      const long cus = device_cus() > 0 ? device_cus() : 256;
+      if (ring_ok && small <= cus) {
+        tile = (long)((a.M + 31) / 32) * ((a.N + 31) / 32) <= cus ? 16 : 15;
+      } else if (slabs && gemm_dmam_has(IN_DT, OUT_DT) && mid < 65536) {
+        const long kb = (long)a.K * (IN_DT == DT_FP8 ? 1 : 2);
+        const double ratio = kb <= 512 ? (big <= 2 * cus ? 4.2 : 3.3) : IN_DT == DT_FP8 ? 3.3 : 2.55;
+        tile = ratio * (double)((big + cus - 1) / cus) <= (double)((mid + cus - 1) / cus) ? 3 : 11;
+      }
+    } else if (tile == 1 && ring_ok) {
       tile = (long)((a.M + 31) / 32) * ((a.N + 31) / 32) <= device_cus() ? 16 : small <= device_cus() ? 15 : 11;
+    }
   }
   if (tile == 6 || tile == 8) return hipErrorInvalidValue;   // codes of two retired kernels
   // The 256x256 tile has three kernels. Eight waves in step (gemm_dma_kernel.hpp, tile 7): every operand type, any K.
@@ -637,18 +647,15 @@ static hipError_t launch_in_out(const GemmArgs& a, int tile, hipStream_t st) {
   }
   if (tile == 10) return gemm_dmaf_has(IN_DT, OUT_DT, a.res_stats != nullptr) ? launch_gemm_dmaf(a, IN_DT, OUT_DT, device_cus(), st) : hipErrorInvalidValue;
   if (tile == 3 || tile == 7) return launch_gemm_dma(a, IN_DT, OUT_DT, st);
-  // The 128x128 tile has the register-staged kernel (any K, fp32 outputs, normalised residuals; two workgroups per CU;
-  // tile 12 names it) and, for K in whole slabs, the direct-to-LDS kernel with three slabs in flight
-  // (gemm_dmam_kernel.hpp, tile 11; bit-equal; one workgroup per CU). The second is 15 to 20 % faster while every tile has a
-  // CU of its own (M=4096, N=1024, bf16: 20.1 -> 16.3 us at K=1024, 27.9 -> 23.0 at K=1536) and level beyond (384 tiles: 26.6 -> 24.9 us
-  // from warm caches, 768 tiles: 48.1 -> 49.2 us; no difference inside a 64-position forward pass), so tile 2 picks it for
-  // at most as many tiles as there are CUs.
+  // The 128x128 tile has the register-staged kernel (any K, every type; two workgroups per CU; tile 12 names it) and, for K in whole slabs, the one
+  // with loading and multiplying waves (gemm_dmam_kernel.hpp, tile 11; bit-equal; M=4096, bf16: N=1024, K=1024 16.5 -> 13.9 us,
+  // N=1536 27.9 -> 20.9).
   if (tile == 15 || tile == 16) return slabs && !a.res_stats && gemm_dmam_has(IN_DT, OUT_DT) ? launch_gemm_dmas(a, IN_DT, OUT_DT, st, tile == 16 ? 32 : 64) : hipErrorInvalidValue;
   if (tile == 11 && !slabs) tile = 12;
   if (tile == 2 || tile == 11) {
     const long mid_tiles = (long)((a.M + 127) / 128) * ((a.N + 127) / 128);
-    const bool can = slabs && !a.res_stats && gemm_dmam_has(IN_DT, OUT_DT) && mid_tiles < 65536;
-    if (can && (tile == 11 || mid_tiles <= device_cus())) return launch_gemm_dmam(a, IN_DT, OUT_DT, st);
+    const bool can = slabs && gemm_dmam_has(IN_DT, OUT_DT) && mid_tiles < 65536;
+    if (can) return launch_gemm_dmam(a, IN_DT, OUT_DT, device_cus(), st);
     if (tile == 11) return hipErrorInvalidValue;
   }
   if (tile == 2 || tile == 12) return launch_cfg<CfgMid, IN_DT, OUT_DT>(a, st);

@@ -77,7 +77,8 @@ enum {
 template <int N>
 __device__ __forceinline__ void wait_vmcnt_lgkm0() { __builtin_amdgcn_s_waitcnt((N & 0xF) | ((N >> 4) << 14) | (0x7 << 4)); }
 __device__ __forceinline__ void dmaf_barrier() { asm volatile("s_barrier" ::: "memory"); }
-// (functions of their own, like dmam_load16: inside a kernel template these builtins can make the host pass drop the kernel's stub)
+// (functions of their own, not lambdas: inside a kernel template, where an argument depends on a template parameter, the load builtin makes the host pass drop the
+// kernel's stub without a diagnostic; the library then fails to load over the unresolved name, which the build checks for)
 __device__ __forceinline__ void dmaf_load16(__amdgpu_buffer_rsrc_t r, uint8_t* dst, int voff, int soff) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, voff, soff, 0, 0);
 }
@@ -93,6 +94,7 @@ __device__ __forceinline__ int dmaf_here(int x) {
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ u32x2_t dmaf_get8(__amdgpu_buffer_rsrc_t r, int off) { return __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0); }
+__device__ __forceinline__ u32x4_t dmaf_get16(__amdgpu_buffer_rsrc_t r, int off) { return __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0); }
 __device__ __forceinline__ u32x4_t dmaf_get16_nt(__amdgpu_buffer_rsrc_t r, int off) { return __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 2); }
 __device__ __forceinline__ void dmaf_put16_nt(u32x4_t v, __amdgpu_buffer_rsrc_t r, int off) { __builtin_amdgcn_raw_buffer_store_b128(v, r, off, 0, 2); }
 __device__ __forceinline__ void dmaf_put16(u32x4_t v, __amdgpu_buffer_rsrc_t r, int off) { __builtin_amdgcn_raw_buffer_store_b128(v, r, off, 0, 0); }
@@ -554,11 +556,11 @@ __global__ void __launch_bounds__(DmafCfg::NT, 2) gemm_dmaf_kernel(const GemmArg
 }
 
 // Which instance serves a call. 0 / 1: the general ones.
-inline int dmaf_epilogue(const GemmArgs& a, int in_dt, int out_dt) {
+inline int dmaf_epilogue(const GemmArgs& a, int in_dt, int out_dt, int tile_cols = DmafCfg::BN) {
   const int general = a.res_stats ? DMAF_GENERAL_NORM : DMAF_GENERAL, osz = out_dt == DT_F32 ? 4 : out_dt == DT_FP8 ? 1 : 2;
   // 16-byte stores of whole column groups inside one tile, offsets inside a tile that fit 31 bits, two slabs at least (the
   // constants of a tile land during its second slab)
-  if (!a.vec_ok || a.N % (out_dt == DT_FP8 ? 16 : 8) || (a.nsplit < a.N && a.nsplit % DmafCfg::BN) || a.amax || a.res_rows > 0 || a.ln_out) return general;
+  if (!a.vec_ok || a.N % (out_dt == DT_FP8 ? 16 : 8) || (a.nsplit < a.N && a.nsplit % tile_cols) || a.amax || a.res_rows > 0 || a.ln_out) return general;
   if ((long)a.K * (in_dt == DT_FP8 ? 1 : 2) < 2 * DmafCfg::ROWB) return general;
   if (a.ldc * osz * 256 >= (1L << 31) || a.ldc2 * osz * 256 >= (1L << 31) || (a.res && a.ldr * 4 * 256 >= (1L << 31)) || a.ldc < a.nsplit) return general;
   if (a.res_stats) return a.act == ACT_NONE && out_dt == DT_BF16 ? DMAF_RESNORM : general;

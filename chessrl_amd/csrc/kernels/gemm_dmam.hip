@@ -1,5 +1,4 @@
-// Instances of the 128x128 GEMM fed by direct-to-LDS loads through a ring of stages (gemm_dmam_kernel.hpp), in a translation
-// unit of their own.
+// Instances of the 128x128 GEMM with loading and multiplying waves (gemm_dmam_kernel.hpp), in a translation unit of their own.
 #include "gemm_dmam_kernel.hpp"
 
 namespace crl {
@@ -11,23 +10,37 @@ bool gemm_dmam_has(int in_dt, int out_dt) {
   return in_dt == out_dt && (in_dt == DT_BF16 || in_dt == DT_F16);
 }
 
-hipError_t launch_gemm_dmam(const GemmArgs& a, int in_dt, int out_dt, hipStream_t st) {
-  // (whole tiles in M, aligned rows, a bf16 residual or none, no maximum: the instances without the epilogue's guards)
-  const bool lean = a.M % DmamCfg::BM == 0 && a.vec_ok && a.N % 8 == 0 && a.nsplit % 8 == 0 && !a.amax && a.res_rows == 0 && !a.ln_out &&
-                    (!a.res || a.res_dtype == DT_BF16);
-  if (lean && in_dt == DT_FP8 && out_dt == DT_BF16) return launch_dmam<DT_FP8, DT_BF16, 1>(a, st);
-  if (lean && in_dt == DT_FP8 && out_dt == DT_FP8) return launch_dmam<DT_FP8, DT_FP8, 1>(a, st);
-  if (lean && in_dt == DT_BF16 && out_dt == DT_BF16) return launch_dmam<DT_BF16, DT_BF16, 1>(a, st);
+hipError_t launch_gemm_dmam(const GemmArgs& a, int in_dt, int out_dt, int cus, hipStream_t st) {
+  // (the conditions of the 256x256 tile, and a column split on this tile's boundary)
+  const int epi = dmaf_epilogue(a, in_dt, out_dt, DmamCfg::BN);
+#define DMAM(IN, OUT, EPI, ACT) launch_dmam<IN, OUT, EPI, ACT>(a, cus, st)
+  if (a.res_stats) {
+    if (in_dt != DT_FP8 || out_dt != DT_BF16 || !a.res || a.res_dtype != DT_BF16 || !a.res_gamma || a.res_rows > 0 || a.alpha == 0.f) return hipErrorInvalidValue;
+    return epi == DMAF_RESNORM ? DMAM(DT_FP8, DT_BF16, DMAF_RESNORM, ACT_NONE) : DMAM(DT_FP8, DT_BF16, DMAF_GENERAL_NORM, ACT_NONE);
+  }
   if (in_dt == DT_FP8) {
     switch (out_dt) {
-      case DT_BF16: return launch_dmam<DT_FP8, DT_BF16>(a, st);
-      case DT_F16: return launch_dmam<DT_FP8, DT_F16>(a, st);
-      case DT_FP8: return launch_dmam<DT_FP8, DT_FP8>(a, st);
+      case DT_BF16:
+        if (epi == DMAF_PLAIN && a.act == ACT_NONE) return DMAM(DT_FP8, DT_BF16, DMAF_PLAIN, ACT_NONE);
+        return epi == DMAF_RES16 ? DMAM(DT_FP8, DT_BF16, DMAF_RES16, ACT_NONE) : DMAM(DT_FP8, DT_BF16, DMAF_GENERAL, ACT_NONE);
+      case DT_F16: return DMAM(DT_FP8, DT_F16, DMAF_GENERAL, ACT_NONE);
+      case DT_FP8:
+        if (epi == DMAF_PLAIN) return a.act == ACT_MISH ? DMAM(DT_FP8, DT_FP8, DMAF_PLAIN, ACT_MISH) : DMAM(DT_FP8, DT_FP8, DMAF_PLAIN, ACT_GELU);
+        return DMAM(DT_FP8, DT_FP8, DMAF_GENERAL, ACT_NONE);
     }
   }
-  if (in_dt == DT_BF16 && out_dt == DT_BF16) return launch_dmam<DT_BF16, DT_BF16>(a, st);
-  if (in_dt == DT_F16 && out_dt == DT_F16) return launch_dmam<DT_F16, DT_F16>(a, st);
-  if (in_dt == DT_BF16 && out_dt == DT_F32) return launch_dmam<DT_BF16, DT_F32>(a, st);
+  if (in_dt == DT_BF16 && out_dt == DT_BF16) {
+    if (epi == DMAF_PLAIN)
+      return a.act == ACT_GELU ? DMAM(DT_BF16, DT_BF16, DMAF_PLAIN, ACT_GELU) : a.act == ACT_MISH ? DMAM(DT_BF16, DT_BF16, DMAF_PLAIN, ACT_MISH) : DMAM(DT_BF16, DT_BF16, DMAF_PLAIN, ACT_NONE);
+    if (epi == DMAF_RES16) return a.act == ACT_GELU ? DMAM(DT_BF16, DT_BF16, DMAF_RES16, ACT_GELU) : DMAM(DT_BF16, DT_BF16, DMAF_RES16, ACT_NONE);
+    return DMAM(DT_BF16, DT_BF16, DMAF_GENERAL, ACT_NONE);
+  }
+  if (in_dt == DT_F16 && out_dt == DT_F16) {
+    if (epi == DMAF_PLAIN) return a.act == ACT_MISH ? DMAM(DT_F16, DT_F16, DMAF_PLAIN, ACT_MISH) : DMAM(DT_F16, DT_F16, DMAF_PLAIN, ACT_NONE);
+    return epi == DMAF_RES16 ? DMAM(DT_F16, DT_F16, DMAF_RES16, ACT_NONE) : DMAM(DT_F16, DT_F16, DMAF_GENERAL, ACT_NONE);
+  }
+  if (in_dt == DT_BF16 && out_dt == DT_F32) return epi == DMAF_RES32 ? DMAM(DT_BF16, DT_F32, DMAF_RES32, ACT_NONE) : DMAM(DT_BF16, DT_F32, DMAF_GENERAL, ACT_NONE);
+#undef DMAM
   return hipErrorInvalidValue;
 }
 

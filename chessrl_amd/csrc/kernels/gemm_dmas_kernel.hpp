@@ -59,7 +59,7 @@ struct SmallArgs {
 };
 
 __device__ __forceinline__ void dmas_barrier() { asm volatile("s_barrier" ::: "memory"); }
-// (a function of its own, like dmam_load16: inside a kernel template this builtin makes the host pass drop the kernel's stub)
+// (a function of its own, like dmaf_load16: inside a kernel template this builtin makes the host pass drop the kernel's stub)
 __device__ __forceinline__ void dmas_load16(__amdgpu_buffer_rsrc_t r, uint8_t* dst, int voff, int soff) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, voff, soff, 0, 0);
 }

@@ -522,9 +522,9 @@ hipError_t launch_gemm_dma_resnorm(const GemmArgs& a, hipStream_t st);   // gemm
 // gemm_dmaf.hip: the 256x256 tile whose waves take turns at multiplying and loading (K in whole 128-byte slabs), on `cus` compute units.
 bool gemm_dmaf_has(int in_dt, int out_dt, bool res_norm);
 hipError_t launch_gemm_dmaf(const GemmArgs& a, int in_dt, int out_dt, int cus, hipStream_t st);
-// gemm_dmam.hip: the 128x128 tile fed by direct-to-LDS loads through a four-stage ring (K in whole 128-byte slabs, no normalised residual).
+// gemm_dmam.hip: the 128x128 tile with loading and multiplying waves (K in whole 128-byte slabs), on `cus` compute units.
 bool gemm_dmam_has(int in_dt, int out_dt);
-hipError_t launch_gemm_dmam(const GemmArgs& a, int in_dt, int out_dt, hipStream_t st);
+hipError_t launch_gemm_dmam(const GemmArgs& a, int in_dt, int out_dt, int cus, hipStream_t st);
 // gemm_dmas.hip: the 64x64 and 32x32 tiles of products that leave every tile a CU (the operand types of gemm_dmam_has).
 hipError_t launch_gemm_dmas(const GemmArgs& a, int in_dt, int out_dt, hipStream_t st, int tile_size);
 // gemm_shortk.hip: K = 256 e4m3 operands, bare scaled product: a workgroup keeps 256 rows of A in registers and walks N.
