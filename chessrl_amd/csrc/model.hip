@@ -177,13 +177,29 @@ static std::vector<float> cat(std::initializer_list<const std::vector<float>*> p
   return r;
 }
 
+// W [N, K] with `rows` rows and `cols` columns, the new ones zero.
+static std::vector<float> pad_to(const std::vector<float>& W, int N, int K, int rows, int cols) {
+  std::vector<float> r((size_t)rows * cols, 0.f);
+  for (int n = 0; n < N; ++n) std::copy(W.begin() + (size_t)n * K, W.begin() + (size_t)(n + 1) * K, r.begin() + (size_t)n * cols);
+  return r;
+}
+
+int Model::make_ffn(Layer& ly, const std::vector<float>& w1, const std::vector<float>& b1, const std::vector<float>& w2, const std::vector<float>& b2) {
+  const int C = cfg.d_model, F = cfg.d_ff, FP = ff_cols(), ad = cfg.act_dtype;
+  const std::vector<float> b1p = pad_to(b1, 1, F, 1, FP);
+  int rc = make_lin(ly.ff1, pad_to(w1, F, C, FP, C), &b1p, FP, C, ad, cfg.fp8 != 0);
+  if (rc) return rc;
+  ly.ff1.pad_N = ly.ff2.pad_K = FP - F;
+  return make_lin(ly.ff2, pad_to(w2, C, F, C, FP), &b2, C, FP, ad, cfg.fp8 != 0);
+}
+
 int Model::finalize() {
   for (auto& e : expected)
     if (!host.count(e.first)) { set_error("finalize: missing weight " + e.first); return CRL_ERR_STATE; }
   for (void* p : allocs) (void)hipFree(p);
   allocs.clear();
   layers.assign(cfg.n_layer, Layer());
-  const int C = cfg.d_model, F = cfg.d_ff, H = cfg.n_head;
+  const int C = cfg.d_model, H = cfg.n_head;
   const bool f8 = cfg.fp8 != 0;
   const int hd = cfg.head_dtype, ad = cfg.act_dtype;
   int rc;
@@ -220,8 +236,7 @@ int Model::finalize() {
       UP(w(p + "ln_2.weight"), DT_F32, ly.ln2_g); UP(w(p + "ln_2.bias"), DT_F32, ly.ln2_b);
       LIN(ly.qkv, w(p + "attn.c_attn.weight"), &w(p + "attn.c_attn.bias"), 3 * C, C, ad, f8);
       LIN(ly.proj, w(p + "attn.c_proj.weight"), &w(p + "attn.c_proj.bias"), C, C, ad, f8);
-      LIN(ly.ff1, w(p + "mlp.c_fc.weight"), &w(p + "mlp.c_fc.bias"), F, C, ad, f8);
-      LIN(ly.ff2, w(p + "mlp.c_proj.weight"), &w(p + "mlp.c_proj.bias"), C, F, ad, f8);
+      rc = make_ffn(ly, w(p + "mlp.c_fc.weight"), w(p + "mlp.c_fc.bias"), w(p + "mlp.c_proj.weight"), w(p + "mlp.c_proj.bias")); if (rc) return rc;
     }
     UP(w("transformer.ln_f.weight"), DT_F32, lnf_g); UP(w("transformer.ln_f.bias"), DT_F32, lnf_b);
     rc = make_lin(lm_head, head_w, nullptr, VOCAB_RL, C, hd, f8 && cfg.fp8_lm_head > 0, head_amax); if (rc) return rc;
@@ -262,8 +277,7 @@ int Model::finalize() {
       }
       LIN(ly.qkv, wq, &bq, nq, C, ad, f8);
       LIN(ly.proj, w(p + "attention.out_proj.weight"), &w(p + "attention.out_proj.bias"), C, C, ad, f8);
-      LIN(ly.ff1, w(p + "ff1.weight"), &w(p + "ff1.bias"), F, C, ad, f8);
-      LIN(ly.ff2, w(p + "ff2.weight"), &w(p + "ff2.bias"), C, F, ad, f8);
+      rc = make_ffn(ly, w(p + "ff1.weight"), w(p + "ff1.bias"), w(p + "ff2.weight"), w(p + "ff2.bias")); if (rc) return rc;
       UP(w(p + "norm1.weight"), DT_F32, ly.ln1_g); UP(w(p + "norm1.bias"), DT_F32, ly.ln1_b);
       UP(w(p + "norm2.weight"), DT_F32, ly.ln2_g); UP(w(p + "norm2.bias"), DT_F32, ly.ln2_b);
       if (cfg.arch == CRL_ARCH_BT4) {
@@ -348,7 +362,7 @@ int Model::ensure_ws(int mb) {
   for (void* p : ws_allocs) (void)hipFree(p);
   ws_allocs.clear();
   ws_mb = 0;
-  const size_t M = (size_t)mb * 64, C = cfg.d_model, F = cfg.d_ff, H = cfg.n_head;
+  const size_t M = (size_t)mb * 64, C = cfg.d_model, F = ff_cols(), H = cfg.n_head;
   int rc;
 #define WS(ptr, bytes) do { rc = dev_alloc((void**)&(ptr), (bytes), true); if (rc) return rc; } while (0)
   const bool sf32_post = cfg.arch != CRL_ARCH_GPT64 && cfg.stream_f32 > 0;   // post-LN trunks keep x, t and h in the stream's type
@@ -469,7 +483,7 @@ int Model::gemm(const Lin& L, const void* A, long lda, int in_dt, void* C, long 
     *o.c_blocked = g.c_blocked != 0;
   }
   const int fam = in_dt == DT_FP8 ? 0 : 5;
-  if (profiling) prof_flops[fam] += 2.0 * M * (double)L.N * L.K;
+  if (profiling) prof_flops[fam] += 2.0 * M * (double)(L.N - L.pad_N) * (L.K - L.pad_K);
   prof_begin(fam, st);
   hipError_t e = launch_gemm(g, in_dt == DT_FP8 ? DT_FP8 : L.dt, out_dt, 0, st);
   prof_end(st);
@@ -549,7 +563,7 @@ int Model::forward_tokens(const float* planes, const uint8_t* ids, const uint8_t
 
 int Model::forward_chunk(const float* planes, const uint8_t* ids, const uint8_t* flags, const int64_t* idx, int t, int mb,
                          float* policy, float* all_logits, float* wdl, bool calibrate, hipStream_t st, const LayerWindow* win) {
-  const int C = cfg.d_model, F = cfg.d_ff, H = cfg.n_head, L = cfg.n_layer, hs = C / H;
+  const int C = cfg.d_model, F = ff_cols(), H = cfg.n_head, L = cfg.n_layer, hs = C / H;
   // Layers [l0, l1) of this call: the whole trunk, or the window of run_layers (its input comes from the caller instead of
   // the embedding, its first layer reads that input as a plain residual and its last one writes the 16-bit output).
   const int l0 = win ? win->first : 0, l1 = win ? win->last : L;
@@ -840,6 +854,13 @@ int Model::debug_read(const char* name, void* out, long bytes, hipStream_t st) {
   else if (n == "t") { src = ws.t; cap = M * C * ((cfg.arch != CRL_ARCH_GPT64 && cfg.stream_f32 > 0) ? 4 : 2); }
   else { set_error("debug_read: unknown tensor " + n); return CRL_ERR_ARG; }
   if ((size_t)bytes > cap) { set_error("debug_read: " + n + " holds " + std::to_string(cap) + " bytes"); return CRL_ERR_ARG; }
+  const size_t FP = (size_t)ff_cols();
+  if (n == "f8" && FP != F) {   // rows lie FP apart
+    const size_t rows = (size_t)bytes / F, rest = (size_t)bytes - rows * F;
+    if (rows) HIPCHK(hipMemcpy2DAsync(out, F, src, FP, F, rows, hipMemcpyDeviceToDevice, st));
+    if (rest) HIPCHK(hipMemcpyAsync((char*)out + rows * F, (const char*)src + rows * FP, rest, hipMemcpyDeviceToDevice, st));
+    return CRL_OK;
+  }
   HIPCHK(hipMemcpyAsync(out, src, (size_t)bytes, hipMemcpyDeviceToDevice, st));
   return CRL_OK;
 }
@@ -863,7 +884,7 @@ int Model::generate(const float* planes, int B, int steps, float temperature, ui
   if (!finalized) { set_error("generate: call crl_model_finalize first"); return CRL_ERR_STATE; }
   if (cfg.arch != CRL_ARCH_GPT64) { set_error("generate: only CRL_ARCH_GPT64 generates sequences"); return CRL_ERR_ARG; }
   if (!planes || !seq || B <= 0 || steps < 1 || temperature < 0.f) { set_error("generate: bad arguments"); return CRL_ERR_ARG; }
-  const int C = cfg.d_model, F = cfg.d_ff, H = cfg.n_head, L = cfg.n_layer, hs = C / H;
+  const int C = cfg.d_model, F = ff_cols(), H = cfg.n_head, L = cfg.n_layer, hs = C / H;
   const int Tmax = 64 + steps;   // the last sampled token is never fed back
   if (Tmax > pe_rows || Tmax > 1024) { set_error("generate: 64 + steps exceeds the positional table or 1024 tokens"); return CRL_ERR_ARG; }
   if ((long)B * 65 > (long)cfg.micro_batch * 64) { set_error("generate: batch too large for one micro-batch"); return CRL_ERR_ARG; }

@@ -106,6 +106,27 @@ def test_bt4_torch(cuda, cfg, act="bf16"):
     assert top1_agreement(pol, rpol, mask) >= 0.98
 
 
+@pytest.mark.parametrize("arch,fp8,Fm,FP", [("bt4", False, 248, 256), ("bt4", False, 1000, 1024), ("bt4class", True, 240, 256)])
+def test_padded_ffn_equals_the_model_with_the_zeros_in_its_weights(cuda, arch, fp8, Fm, FP):
+    """Hidden FFN tensors whose rows are filled up to whole slabs: bit-equal to the model that holds the zeros itself, and read back unpadded."""
+    L, Cm, H = 2, 256, 8
+    oracle = om.test_init_(om.BT4Oracle(L, Cm, Fm, H) if arch == "bt4" else om.BT4ClassOracle(policy_leela, L, Cm, Fm, H), seed=5)
+    planes = positions(70, seed=6, leela=arch == "bt4class")[0].to(cuda)
+    zeros = torch.nn.functional.pad
+    pad = lambda k, v: zeros(v, (0, 0, 0, FP - Fm)) if "ff1.weight" in k else zeros(v, (0, FP - Fm)) if "ff1.bias" in k or "ff2.weight" in k else v
+    out = []
+    for width, state in ((Fm, oracle.state_dict()), (FP, {k: pad(k, v) for k, v in oracle.state_dict().items()})):
+        m = (models.BT4 if arch == "bt4" else models.BT4Class)(L, Cm, width, H, fp8=fp8)
+        m.load_state_dict(state)
+        if fp8:
+            m.calibrate(planes)
+        rows = [m.evaluate(planes[:n].contiguous()) for n in (1, 70)]
+        hidden = m._engine.read_tensor("f8", (70 * 64, width))[:, :Fm] if fp8 else planes[0]
+        out.append([t for r in rows for t in r] + [hidden])
+    for a, b in zip(*out):
+        assert torch.equal(a, b)
+
+
 def test_bt4_fp32_stream(cuda):
     """BT4 with the residual stream kept in fp32 (16-bit GEMM operands): closer to the oracle than the 16-bit stream."""
     oracle = om.test_init_(om.BT4Oracle(10, 512, 736, 8), seed=1)
