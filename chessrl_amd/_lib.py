@@ -7,6 +7,8 @@ missing or a call fails, an exception is raised.
 import ctypes as C
 import os
 
+import numpy as np
+
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libchessrl_amd.so")
 
@@ -117,6 +119,21 @@ def check(rc, what=""):
 
 
 def str_array(strings):
-    arr = (C.c_char_p * len(strings))()
+    """char*[] of str or bytes. ASCII strings share one buffer (1500 FENs: 36 us instead of 176)."""
+    n = len(strings)
+    try:
+        text = ("\0".join(strings) + "\0").encode()
+    except TypeError:
+        text = b""
+    if n and text:
+        ends = np.cumsum(np.fromiter(map(len, strings), np.uintp, n) + np.uintp(1), dtype=np.uintp)
+        if int(ends[-1]) == len(text):
+            start = np.empty(n, np.uintp)
+            start[0], start[1:] = 0, ends[:-1]
+            start += np.uintp(C.cast(C.c_char_p(text), C.c_void_p).value)
+            arr = (C.c_char_p * n).from_buffer(start)
+            arr._text = text
+            return arr
+    arr = (C.c_char_p * n)()
     arr[:] = [s.encode() if isinstance(s, str) else s for s in strings]
     return arr

@@ -1,6 +1,10 @@
 // extern "C" surface declared in include/chessrl_amd.h.
 #include <algorithm>
+#include <atomic>
+#include <condition_variable>
 #include <cstring>
+#include <mutex>
+#include <system_error>
 #include <thread>
 
 #include "model.hpp"
@@ -18,29 +22,45 @@ int arg_fail(const char* msg) {
   return CRL_ERR_ARG;
 }
 
-// Run fn(i) for i in [0,n) on a few host threads; returns the first non-zero result.
+// Run fn(i) for i in [0,n) on this thread and a few more, one for every `grain` items; returns the result of the lowest i
+// that failed. Blocks of 16 are handed out in turn: starting a thread takes 10-20 us here, and with fixed shares the last
+// one to start was the last to end. For the same reason work of less than a microsecond an item takes a grain of 192: 1500
+// FENs to compact boards took 340 us in fixed shares on 16 threads, 236 in turn, 188 on 8.
 template <typename Fn>
-int parallel_for(int n, int threads, Fn fn) {
+int parallel_for(int n, int threads, Fn fn, int grain = 64) {
+  constexpr int BLOCK = 16;
   if (threads <= 0) threads = (int)std::min<unsigned>(16, std::max<unsigned>(1, std::thread::hardware_concurrency()));
-  threads = std::min(threads, std::max(1, n / 64));
+  threads = std::min(threads, std::max(1, n / grain));
   if (threads <= 1) {
     for (int i = 0; i < n; ++i) { int rc = fn(i); if (rc) return rc; }
     return 0;
   }
-  std::vector<int> rcs(threads, 0);
-  std::vector<std::string> errs(threads);
-  std::vector<std::thread> pool;
-  for (int t = 0; t < threads; ++t)
-    pool.emplace_back([&, t]() {
-      for (int i = t; i < n; i += threads) {
-        int rc = fn(i);
-        if (rc) { rcs[t] = rc; errs[t] = get_error(); return; }
+  std::atomic<int> next{0};
+  std::atomic<bool> failed{false};
+  std::mutex mu;
+  int bad = n, bad_rc = 0;
+  std::string bad_err;
+  // (a block below a failed one was handed out before it and is walked to its end, so the lowest failure is always found)
+  auto work = [&]() {
+    while (!failed.load(std::memory_order_relaxed)) {
+      const int b = next.fetch_add(BLOCK, std::memory_order_relaxed);
+      if (b >= n) return;
+      for (int i = b; i < std::min(n, b + BLOCK); ++i) {
+        const int rc = fn(i);
+        if (!rc) continue;
+        std::lock_guard<std::mutex> g(mu);
+        if (i < bad) { bad = i; bad_rc = rc; bad_err = get_error(); }
+        failed.store(true, std::memory_order_relaxed);
+        return;
       }
-    });
+    }
+  };
+  std::vector<std::thread> pool;
+  for (int t = 1; t < threads; ++t) pool.emplace_back(work);
+  work();
   for (auto& th : pool) th.join();
-  for (int t = 0; t < threads; ++t)
-    if (rcs[t]) { set_error(errs[t]); return rcs[t]; }
-  return 0;
+  if (bad_rc) set_error(bad_err);
+  return bad_rc;
 }
 
 int parse(const char* fen, Board& b) {
@@ -129,7 +149,7 @@ int crl_encode_fens_compact(const char* const* fens, int n, uint8_t* ids, uint8_
     if (rc) return rc;
     b.compact(ids + (size_t)i * 64, flags + (size_t)i * 4);
     return 0;
-  });
+  }, 192);
 }
 int crl_legal_masks(const char* const* fens, int n, uint8_t* masks, int32_t* counts, int threads) {
   if (n < 0 || (n && (!fens || !masks))) return arg_fail("crl_legal_masks: bad arguments");
@@ -394,13 +414,15 @@ int crl_masked_nll_mean(const float* logp, const int64_t* target, int64_t ignore
 // one copy stream, one compute stream (both default priority), events per slot.
 struct FenPipeline {
   int chunk = 0, vocab = 0;
-  hipStream_t copy_st = nullptr, comp_st = nullptr;
+  hipStream_t copy_st = nullptr, comp_st = nullptr, down_st = nullptr;   // uploads, device work, downloads
+  static constexpr int PIECES = 8;
   struct Slot {
     uint8_t *h_ids = nullptr, *h_flags = nullptr, *h_mask = nullptr;  // pinned inputs
     float *h_probs = nullptr, *h_wdl = nullptr; int32_t* h_best = nullptr;  // pinned outputs
     uint8_t *d_ids = nullptr, *d_flags = nullptr, *d_mask = nullptr;
     float *d_logits = nullptr, *d_probs = nullptr, *d_wdl = nullptr; int32_t* d_best = nullptr;
-    hipEvent_t uploaded = nullptr, done = nullptr;
+    hipEvent_t uploaded = nullptr, masked = nullptr, computed = nullptr, done = nullptr, piece[PIECES] = {};
+    int pieces = 0;            // parts the probabilities come down in, each with its event
     int first = 0, count = 0;  // positions of the chunk in flight (count 0 = idle)
   } slot[2];
   void release() {
@@ -409,13 +431,16 @@ struct FenPipeline {
       (void)hipHostFree(s.h_probs); (void)hipHostFree(s.h_wdl); (void)hipHostFree(s.h_best);
       (void)hipFree(s.d_ids); (void)hipFree(s.d_flags); (void)hipFree(s.d_mask);
       (void)hipFree(s.d_logits); (void)hipFree(s.d_probs); (void)hipFree(s.d_wdl); (void)hipFree(s.d_best);
-      if (s.uploaded) (void)hipEventDestroy(s.uploaded);
-      if (s.done) (void)hipEventDestroy(s.done);
+      for (hipEvent_t ev : {s.uploaded, s.masked, s.computed, s.done})
+        if (ev) (void)hipEventDestroy(ev);
+      for (hipEvent_t ev : s.piece)
+        if (ev) (void)hipEventDestroy(ev);
       s = Slot();
     }
     if (copy_st) (void)hipStreamDestroy(copy_st);
     if (comp_st) (void)hipStreamDestroy(comp_st);
-    copy_st = comp_st = nullptr;
+    if (down_st) (void)hipStreamDestroy(down_st);
+    copy_st = comp_st = down_st = nullptr;
     chunk = 0;
   }
   hipError_t ensure(int want_chunk, int V) {
@@ -425,6 +450,7 @@ struct FenPipeline {
 #define PIPE_TRY(call) do { e = (call); if (e != hipSuccess) { release(); return e; } } while (0)
     PIPE_TRY(hipStreamCreateWithFlags(&copy_st, hipStreamNonBlocking));
     PIPE_TRY(hipStreamCreateWithFlags(&comp_st, hipStreamNonBlocking));
+    PIPE_TRY(hipStreamCreateWithFlags(&down_st, hipStreamNonBlocking));
     const size_t c = (size_t)want_chunk;
     for (Slot& s : slot) {
       PIPE_TRY(hipHostMalloc((void**)&s.h_ids, c * 64, hipHostMallocDefault));
@@ -440,8 +466,8 @@ struct FenPipeline {
       PIPE_TRY(hipMalloc((void**)&s.d_probs, c * V * sizeof(float)));
       PIPE_TRY(hipMalloc((void**)&s.d_wdl, c * 3 * sizeof(float)));
       PIPE_TRY(hipMalloc((void**)&s.d_best, c * sizeof(int32_t)));
-      PIPE_TRY(hipEventCreateWithFlags(&s.uploaded, hipEventDisableTiming));
-      PIPE_TRY(hipEventCreateWithFlags(&s.done, hipEventDisableTiming));
+      for (hipEvent_t* ev : {&s.uploaded, &s.masked, &s.computed, &s.done}) PIPE_TRY(hipEventCreateWithFlags(ev, hipEventDisableTiming));
+      for (hipEvent_t& ev : s.piece) PIPE_TRY(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
     }
 #undef PIPE_TRY
     chunk = want_chunk; vocab = V;
@@ -533,14 +559,18 @@ int crl_model_generate(crl_model* m, const float* planes, int B, int steps, floa
 
 // The chunked host -> device -> host pipeline behind crl_model_evaluate_fens and crl_model_search_1ply: position i of
 // the job is produced by get(i, board) on the host threads. The legal-move masks and the masked softmax are skipped
-// when neither probabilities nor best moves are asked for (value-only evaluation).
-template <typename GetBoard>
+// when neither probabilities nor best moves are asked for (value-only evaluation). meanwhile() runs once on this thread,
+// while the device is busy with the last chunk.
+// A chunk's forward pass needs the boards alone, so it is queued before the legal moves are generated (1500 positions: 0.6 ms
+// on 16 threads), which the softmax waits for; the probabilities come down on a stream of their own, in parts that are
+// copied to the caller as they arrive.
+template <typename GetBoard, typename Meanwhile>
 static int evaluate_boards(crl_model* m, int n, int chunk, float temperature, float* probs, float* wdl, int32_t* best, int threads,
-                           GetBoard get) {
+                           GetBoard get, Meanwhile meanwhile) {
   const int V = m->impl.vocab;
   const bool leela = m->impl.cfg.arch == CRL_ARCH_BT4CLASS, has_wdl = m->impl.cfg.arch != CRL_ARCH_GPT64;
   const bool need_policy = probs || best;
-  if (n == 0) return CRL_OK;
+  if (n == 0) { meanwhile(); return CRL_OK; }
   if (chunk > n) chunk = n;
   FenPipeline& P = m->pipe;
   // The pipeline runs on streams of its own and shares the model's workspace with every other entry point: work a
@@ -551,12 +581,45 @@ static int evaluate_boards(crl_model* m, int n, int chunk, float temperature, fl
   if (e != hipSuccess) return hip_fail("evaluate: waiting for earlier work on the device", e);
   e = P.ensure(chunk, V);
   if (e != hipSuccess) return hip_fail("evaluate: staging buffers", e);
+  auto piece_row = [](const FenPipeline::Slot& s, int p) { return (int)((int64_t)s.count * p / s.pieces); };
   // Results of a finished slot go from pinned staging to the caller's arrays.
   auto drain = [&](FenPipeline::Slot& s) -> hipError_t {
     if (s.count == 0) return hipSuccess;
-    hipError_t de = hipEventSynchronize(s.done);
+    if (probs) {
+      // A thread for each part but the last, which this one copies (one thread took 0.45 ms for the 11.6 MB of 1500 positions
+      // behind the device's 0.2). They are started while the device is still at work.
+      auto copy = [&](int p) {
+        const int r0 = piece_row(s, p), r1 = piece_row(s, p + 1);
+        std::memcpy(probs + (size_t)(s.first + r0) * V, s.h_probs + (size_t)r0 * V, sizeof(float) * (size_t)(r1 - r0) * V);
+      };
+      std::mutex mu;
+      std::condition_variable cv;
+      int arrived = 0;          // parts that are down; -1: the wait failed
+      std::thread hands[FenPipeline::PIECES];
+      for (int p = 0; p + 1 < s.pieces; ++p) {
+        try {
+          hands[p] = std::thread([&, p]() {
+            std::unique_lock<std::mutex> l(mu);
+            cv.wait(l, [&]() { return arrived < 0 || arrived > p; });
+            if (arrived < 0) return;
+            l.unlock();
+            copy(p);
+          });
+        } catch (const std::system_error&) {}   // then this thread copies the part
+      }
+      hipError_t pe = hipSuccess;
+      for (int p = 0; p < s.pieces && pe == hipSuccess; ++p) {
+        pe = hipEventSynchronize(s.piece[p]);
+        { std::lock_guard<std::mutex> g(mu); arrived = pe == hipSuccess ? p + 1 : -1; }
+        cv.notify_all();
+        if (pe == hipSuccess && !hands[p].joinable()) copy(p);
+      }
+      for (std::thread& h : hands)
+        if (h.joinable()) h.join();
+      if (pe != hipSuccess) return pe;
+    }
+    const hipError_t de = hipEventSynchronize(s.done);
     if (de != hipSuccess) return de;
-    if (probs) std::memcpy(probs + (size_t)s.first * V, s.h_probs, sizeof(float) * (size_t)s.count * V);
     if (wdl) std::memcpy(wdl + (size_t)s.first * 3, s.h_wdl, sizeof(float) * (size_t)s.count * 3);
     if (best) std::memcpy(best + s.first, s.h_best, sizeof(int32_t) * (size_t)s.count);
     s.count = 0;
@@ -564,6 +627,7 @@ static int evaluate_boards(crl_model* m, int n, int chunk, float temperature, fl
   };
   int rc = CRL_OK;
   int k = 0;
+  std::vector<Board> boards((size_t)chunk);
   for (int first = 0; first < n && rc == CRL_OK; first += chunk, ++k) {
     FenPipeline::Slot& s = P.slot[k & 1];
     e = drain(s);  // the chunk that used this slot two steps ago
@@ -571,42 +635,57 @@ static int evaluate_boards(crl_model* m, int n, int chunk, float temperature, fl
     const int cnt = std::min(chunk, n - first);
     // Host work of this chunk overlaps the device work of the previous one.
     rc = parallel_for(cnt, threads, [&](int i) {
-      Board b;
-      int prc = get(first + i, b);
+      const int prc = get(first + i, boards[(size_t)i]);
       if (prc) return prc;
-      b.compact(s.h_ids + (size_t)i * 64, s.h_flags + (size_t)i * 4);
-      if (!need_policy) return 0;
-      if (leela) legal_mask_leela(b, s.h_mask + (size_t)i * V);
-      else legal_mask_rl(b, s.h_mask + (size_t)i * V);
+      boards[(size_t)i].compact(s.h_ids + (size_t)i * 64, s.h_flags + (size_t)i * 4);
       return 0;
-    });
+    }, 192);
     if (rc) break;
-#define PIPE_HIP(call) do { e = (call); if (e != hipSuccess) { rc = hip_fail("evaluate", e); } } while (0)
+#define PIPE_HIP(call) do { if (rc == CRL_OK) { e = (call); if (e != hipSuccess) { rc = hip_fail("evaluate", e); } } } while (0)
     PIPE_HIP(hipMemcpyAsync(s.d_ids, s.h_ids, (size_t)cnt * 64, hipMemcpyHostToDevice, P.copy_st));
-    if (rc == CRL_OK) PIPE_HIP(hipMemcpyAsync(s.d_flags, s.h_flags, (size_t)cnt * 4, hipMemcpyHostToDevice, P.copy_st));
-    if (rc == CRL_OK && need_policy) PIPE_HIP(hipMemcpyAsync(s.d_mask, s.h_mask, (size_t)cnt * V, hipMemcpyHostToDevice, P.copy_st));
-    if (rc == CRL_OK) PIPE_HIP(hipEventRecord(s.uploaded, P.copy_st));
-    if (rc == CRL_OK) PIPE_HIP(hipStreamWaitEvent(P.comp_st, s.uploaded, 0));
+    PIPE_HIP(hipMemcpyAsync(s.d_flags, s.h_flags, (size_t)cnt * 4, hipMemcpyHostToDevice, P.copy_st));
+    PIPE_HIP(hipEventRecord(s.uploaded, P.copy_st));
+    PIPE_HIP(hipStreamWaitEvent(P.comp_st, s.uploaded, 0));
     if (rc) break;
     rc = m->impl.forward(nullptr, s.d_ids, s.d_flags, cnt, need_policy || !has_wdl ? s.d_logits : nullptr, has_wdl && (wdl || !need_policy) ? s.d_wdl : nullptr, false, P.comp_st);
     if (rc) break;
     if (need_policy) {
+      rc = parallel_for(cnt, threads, [&](int i) {
+        if (leela) legal_mask_leela(boards[(size_t)i], s.h_mask + (size_t)i * V);
+        else legal_mask_rl(boards[(size_t)i], s.h_mask + (size_t)i * V);
+        return 0;
+      });
+      PIPE_HIP(hipMemcpyAsync(s.d_mask, s.h_mask, (size_t)cnt * V, hipMemcpyHostToDevice, P.copy_st));
+      PIPE_HIP(hipEventRecord(s.masked, P.copy_st));
+      PIPE_HIP(hipStreamWaitEvent(P.comp_st, s.masked, 0));
       SoftmaxArgs a;
       std::memset(&a, 0, sizeof(a));
       a.logits = s.d_logits; a.ldl = V; a.mask = s.d_mask; a.ldm = V; a.probs = probs ? s.d_probs : nullptr; a.ldp = V;
       a.argmax = s.d_best; a.B = cnt; a.V = V; a.temperature = temperature;
       PIPE_HIP(launch_masked_softmax(a, P.comp_st));
     }
-    if (rc == CRL_OK && probs) PIPE_HIP(hipMemcpyAsync(s.h_probs, s.d_probs, sizeof(float) * (size_t)cnt * V, hipMemcpyDeviceToHost, P.comp_st));
-    if (rc == CRL_OK && wdl) PIPE_HIP(hipMemcpyAsync(s.h_wdl, s.d_wdl, sizeof(float) * (size_t)cnt * 3, hipMemcpyDeviceToHost, P.comp_st));
-    if (rc == CRL_OK && best) PIPE_HIP(hipMemcpyAsync(s.h_best, s.d_best, sizeof(int32_t) * (size_t)cnt, hipMemcpyDeviceToHost, P.comp_st));
-    if (rc == CRL_OK) PIPE_HIP(hipEventRecord(s.done, P.comp_st));
+    PIPE_HIP(hipEventRecord(s.computed, P.comp_st));
+    PIPE_HIP(hipStreamWaitEvent(P.down_st, s.computed, 0));
+    if (rc == CRL_OK) {
+      s.first = first; s.count = cnt;
+      s.pieces = std::min(FenPipeline::PIECES, std::max(1, (int)((int64_t)cnt * V * 4 >> 20)));   // of a megabyte or more
+    }
+    if (probs)
+      for (int p = 0; p < s.pieces; ++p) {
+        const int r0 = piece_row(s, p), r1 = piece_row(s, p + 1);
+        PIPE_HIP(hipMemcpyAsync(s.h_probs + (size_t)r0 * V, s.d_probs + (size_t)r0 * V, sizeof(float) * (size_t)(r1 - r0) * V, hipMemcpyDeviceToHost, P.down_st));
+        PIPE_HIP(hipEventRecord(s.piece[p], P.down_st));
+      }
+    if (wdl) PIPE_HIP(hipMemcpyAsync(s.h_wdl, s.d_wdl, sizeof(float) * (size_t)cnt * 3, hipMemcpyDeviceToHost, P.down_st));
+    if (best) PIPE_HIP(hipMemcpyAsync(s.h_best, s.d_best, sizeof(int32_t) * (size_t)cnt, hipMemcpyDeviceToHost, P.down_st));
+    PIPE_HIP(hipEventRecord(s.done, P.down_st));
 #undef PIPE_HIP
-    if (rc == CRL_OK) { s.first = first; s.count = cnt; }
   }
-  // Leave nothing in flight, also on an error path (the staging buffers are reused by the next call).
+  if (rc == CRL_OK) meanwhile();
+  // Leave nothing in flight, also on an error path (the staging buffers are reused by the next call). Older chunk first.
   const std::string err = rc ? std::string(get_error()) : std::string();
-  for (FenPipeline::Slot& s : P.slot) {
+  for (int j = 0; j < 2; ++j) {
+    FenPipeline::Slot& s = P.slot[(k + j) & 1];
     if (rc == CRL_OK) {
       e = drain(s);
       if (e != hipSuccess) rc = hip_fail("evaluate: wait", e);
@@ -617,6 +696,7 @@ static int evaluate_boards(crl_model* m, int n, int chunk, float temperature, fl
   if (rc != CRL_OK) {
     (void)hipStreamSynchronize(P.copy_st);
     (void)hipStreamSynchronize(P.comp_st);
+    (void)hipStreamSynchronize(P.down_st);
     if (!err.empty()) set_error(err);
   }
   return rc;
@@ -628,7 +708,7 @@ int crl_model_evaluate_fens(crl_model* m, const char* const* fens, int n, int ch
   if (!m || n < 0 || (n && !fens) || chunk <= 0) return arg_fail("crl_model_evaluate_fens: bad arguments");
   if (!m->impl.finalized) { set_error("crl_model_evaluate_fens: call crl_model_finalize first"); return CRL_ERR_STATE; }
   if (wdl && m->impl.cfg.arch == CRL_ARCH_GPT64) return arg_fail("crl_model_evaluate_fens: this architecture has no value head");
-  return evaluate_boards(m, n, chunk, temperature, probs, wdl, best, threads, [&](int i, Board& b) { return parse(fens[i], b); });
+  return evaluate_boards(m, n, chunk, temperature, probs, wdl, best, threads, [&](int i, Board& b) { return parse(fens[i], b); }, []() {});
 }
 
 int crl_model_search_1ply(crl_model* m, const char* const* fens, int n, int chunk, float temperature, uint64_t seed, char* best_uci6,
@@ -663,15 +743,21 @@ int crl_model_search_1ply(crl_model* m, const char* const* fens, int n, int chun
     // board.push(move); board.fen() and back (value.py:336-340, 288): the en-passant square survives only where a
     // capture is legal, which is what the planes of the child position are then built from.
     const int i = root_of[(size_t)c];
-    Board child = roots[i];
-    child.make(moves[i][(size_t)(c - first[i])]);
-    return parse(child.fen(true).c_str(), b);
+    b = roots[i];
+    b.make(moves[i][(size_t)(c - first[i])]);
+    b.drop_idle_ep();
+    return 0;
+  }, [&]() {
+    for (int i = 0; i < n; ++i) {
+      if (n_moves) n_moves[i] = (int)moves[i].size();
+      if (!moves_uci6) continue;
+      for (int64_t c = first[i]; c < first[i + 1]; ++c) put_str(moves_uci6 + (size_t)c * 6, 6, move_uci(moves[i][(size_t)(c - first[i])]));
+    }
   });
   if (rc) return rc;
   // Per root: value of each child for the side to move at the root, then the pick (value.py:343-352, 372-395).
   for (int i = 0; i < n; ++i) {
     const int nm = (int)moves[i].size();
-    if (n_moves) n_moves[i] = nm;
     if (best_uci6) std::memset(best_uci6 + (size_t)i * 6, 0, 6);
     if (nm == 0) continue;
     std::vector<float> val((size_t)nm);
@@ -682,7 +768,6 @@ int crl_model_search_1ply(crl_model* m, const char* const* fens, int n, int chun
       const float inv = 1.0f / (e0 + e1 + e2);
       val[(size_t)c] = 0.5f * e1 * inv + (roots[i].white_to_move ? e2 : e0) * inv;
       if (values) values[first[i] + c] = val[(size_t)c];
-      if (moves_uci6) put_str(moves_uci6 + (size_t)(first[i] + c) * 6, 6, move_uci(moves[i][(size_t)c]));
     }
     int pick = 0;
     for (int c = 1; c < nm; ++c)

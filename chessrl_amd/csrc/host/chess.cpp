@@ -332,6 +332,15 @@ uint64_t Board::perft(int depth) const {
   return n;
 }
 
+bool Board::ep_capture_legal() const {
+  if (ep < 0) return false;
+  std::vector<Move> mv;
+  legal(mv);
+  for (const Move& m : mv)
+    if (m.flag == 2) return true;
+  return false;
+}
+
 std::string Board::fen(bool ep_legal_only) const {
   std::string s;
   for (int r = 7; r >= 0; --r) {
@@ -355,14 +364,7 @@ std::string Board::fen(bool ep_legal_only) const {
     if (cr & CR_BQ) s += "q";
   }
   s += " ";
-  bool write_ep = ep >= 0;
-  if (write_ep && ep_legal_only) {
-    write_ep = false;
-    std::vector<Move> mv;
-    legal(mv);
-    for (const Move& m : mv) if (m.flag == 2) { write_ep = true; break; }
-  }
-  if (write_ep) { s.push_back((char)('a' + file_of(ep))); s.push_back((char)('1' + rank_of(ep))); }
+  if (ep >= 0 && (!ep_legal_only || ep_capture_legal())) { s.push_back((char)('a' + file_of(ep))); s.push_back((char)('1' + rank_of(ep))); }
   else s += "-";
   s += " " + std::to_string(halfmove) + " " + std::to_string(fullmove);
   return s;

@@ -46,6 +46,9 @@ struct Board {
   // legal (what python-chess board.fen() does for the child positions built in
   // new_paradigm/value.py:337-339).
   std::string fen(bool ep_legal_only = true) const;
+  bool ep_capture_legal() const;
+  // What fen() and set_fen() leave of the en-passant square: nothing where no capture on it is legal.
+  void drop_idle_ep() { if (ep >= 0 && !ep_capture_legal()) ep = -1; }
 
   // Rights filtered the way python-chess cleans them: the right counts only if the
   // king stands on e1/e8 and the rook on its corner.

@@ -313,17 +313,16 @@ class _Engine:
         vals = torch.empty((max(cap, 1),), dtype=torch.float32) if want_values else None
         check(lib().crl_model_search_1ply(self.handle, arr, n, int(chunk), float(T), int(seed) & (2 ** 64 - 1), best, counts,
                                           mv, _ptr(vals), cap, int(threads)), "crl_model_search_1ply")
-        braw = best.raw                       # .raw copies the whole buffer: take it once
-        moves = [braw[6 * i:6 * i + 6].split(b"\0")[0].decode() for i in range(n)]
+        # (one conversion for all names: a slice, a split and a decode each took 0.25 ms for 1440 moves)
+        names = lambda buf, k: np.frombuffer(buf, dtype="S6", count=k).astype("U6").tolist()
+        moves = names(best, n)
         if not want_values:
             return moves
-        mraw = mv.raw
-        per_root, o = [], 0
-        for i in range(n):
-            k = counts[i]
-            per_root.append(([mraw[6 * (o + c):6 * (o + c) + 6].split(b"\0")[0].decode() for c in range(k)], vals[o:o + k].clone()))
-            o += k
-        return moves, per_root
+        counts = list(counts)[:n]
+        total = sum(counts)
+        uci, ends = names(mv, total), np.cumsum([0] + counts).tolist()
+        values = vals[:total].clone().split(counts)
+        return moves, [(uci[ends[i]:ends[i + 1]], values[i]) for i in range(n)]
 
     def run_layers(self, x_in, first, last):
         """Encoder layers [first, last) on a caller-supplied layer input (cuda float32 [B,64,C]) -> output of layer
