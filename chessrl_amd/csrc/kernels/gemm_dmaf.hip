@@ -25,7 +25,8 @@ hipError_t launch_gemm_dmaf(const GemmArgs& a, int in_dt, int out_dt, int cus, h
         if (epi == DMAF_PLAIN) return a.act == ACT_MISH ? DMAF(DT_FP8, DT_BF16, DMAF_PLAIN, ACT_MISH) : DMAF(DT_FP8, DT_BF16, DMAF_PLAIN, ACT_NONE);
         return epi == DMAF_RES16 ? DMAF(DT_FP8, DT_BF16, DMAF_RES16, ACT_NONE) : DMAF(DT_FP8, DT_BF16, DMAF_GENERAL, ACT_NONE);
       case DT_F16: return DMAF(DT_FP8, DT_F16, DMAF_GENERAL, ACT_NONE);
-      case DT_F32: return epi == DMAF_RES32 ? DMAF(DT_FP8, DT_F32, DMAF_RES32, ACT_NONE) : DMAF(DT_FP8, DT_F32, DMAF_GENERAL, ACT_NONE);
+      case DT_F32: if (epi == DMAF_PLAIN) return DMAF(DT_FP8, DT_F32, DMAF_PLAIN, ACT_NONE);
+        return epi == DMAF_RES32 ? DMAF(DT_FP8, DT_F32, DMAF_RES32, ACT_NONE) : DMAF(DT_FP8, DT_F32, DMAF_GENERAL, ACT_NONE);
       case DT_FP8:
         if (epi == DMAF_PLAIN) return a.act == ACT_MISH ? DMAF(DT_FP8, DT_FP8, DMAF_PLAIN, ACT_MISH) : DMAF(DT_FP8, DT_FP8, DMAF_PLAIN, ACT_GELU);
         return DMAF(DT_FP8, DT_FP8, DMAF_GENERAL, ACT_NONE);
@@ -41,6 +42,7 @@ hipError_t launch_gemm_dmaf(const GemmArgs& a, int in_dt, int out_dt, int cus, h
     if (epi == DMAF_PLAIN) return a.act == ACT_MISH ? DMAF(DT_F16, DT_F16, DMAF_PLAIN, ACT_MISH) : DMAF(DT_F16, DT_F16, DMAF_PLAIN, ACT_NONE);
     return epi == DMAF_RES16 ? DMAF(DT_F16, DT_F16, DMAF_RES16, ACT_NONE) : DMAF(DT_F16, DT_F16, DMAF_GENERAL, ACT_NONE);
   }
+  if (in_dt == DT_BF16 && out_dt == DT_F32 && epi == DMAF_PLAIN) return DMAF(DT_BF16, DT_F32, DMAF_PLAIN, ACT_NONE);
   if (in_dt == DT_BF16 && out_dt == DT_F32) return epi == DMAF_RES32 ? DMAF(DT_BF16, DT_F32, DMAF_RES32, ACT_NONE) : DMAF(DT_BF16, DT_F32, DMAF_GENERAL, ACT_NONE);
 #undef DMAF
   return hipErrorInvalidValue;

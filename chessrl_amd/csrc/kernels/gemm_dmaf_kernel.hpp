@@ -99,6 +99,12 @@ __device__ __forceinline__ u32x4_t dmaf_get16_nt(__amdgpu_buffer_rsrc_t r, int o
 __device__ __forceinline__ void dmaf_put16_nt(u32x4_t v, __amdgpu_buffer_rsrc_t r, int off) { __builtin_amdgcn_raw_buffer_store_b128(v, r, off, 0, 2); }
 __device__ __forceinline__ void dmaf_put16(u32x4_t v, __amdgpu_buffer_rsrc_t r, int off) { __builtin_amdgcn_raw_buffer_store_b128(v, r, off, 0, 0); }
 
+// The 1 to 3 columns of a 16-byte chunk that a ragged row still has (have; otherwise nothing is stored).
+__device__ __forceinline__ void dmaf_put_part(u32x4_t v, __amdgpu_buffer_rsrc_t r, int off, int have) {
+#pragma unroll
+  for (int e = 0; e < 3; ++e) __builtin_amdgcn_raw_buffer_store_b32(v[e], r, e < have && have < 4 ? off + 4 * e : (int)0x80000000u, 0, 0);
+}
+
 template <int IN_DT, int OUT_DT, int EPI, int ACT = ACT_NONE>
 __global__ void __launch_bounds__(DmafCfg::NT, 2) gemm_dmaf_kernel(const GemmArgs a, const DmafWalk wk, const int tiles) {
   typedef DmafCfg Cfg;
@@ -344,7 +350,7 @@ __global__ void __launch_bounds__(DmafCfg::NT, 2) gemm_dmaf_kernel(const GemmArg
                                                     (long)(rows - 1) * ldob + (long)left * OSZ);
     const int vout = (wm * Cfg::WM + er) * ldob + wn * Cfg::WN * OSZ + ec * 16;
     constexpr int NOWHERE = (int)0x80000000u;
-    const bool nt = a.stream_out != 0;
+    const bool nt = a.stream_out != 0 && (OUT_DT != DT_F32 || ldob % 128 == 0);   // (part of a line with the hint takes three times as long)
     auto put = [&](u32x4_t v, int off) {
       if (nt) dmaf_put16_nt(v, rsrc_o, off);
       else dmaf_put16(v, rsrc_o, off);
@@ -390,9 +396,12 @@ __global__ void __launch_bounds__(DmafCfg::NT, 2) gemm_dmaf_kernel(const GemmArg
       });
     } else if constexpr (OUT_DT == DT_F32) {
       // Raw sums through the patch, 32 columns at a time; bias, activation and residual in the store layout (4 columns per lane).
+      // Without a residual the rows may have any length (16-byte stores need 4-byte alignment only): the 1929 logits of 32768 rows,
+      // K = 768, took 260 us through the general epilogue and 128 here.
       static_for<0, NSTEP>([&](auto sc) {
         constexpr int st = decltype(sc)::value, tn = st / TM, tm = st % TM;
-        const int v0 = wn * Cfg::WN + tn * 32 + ec * 4 < left ? vout + tn * 128 : NOWHERE;
+        const int have = left - (wn * Cfg::WN + tn * 32 + ec * 4);
+        const int v0 = have >= (HAS_RES ? 1 : 4) ? vout + tn * 128 : NOWHERE;
         const f32x4_t bv = a.bias ? *reinterpret_cast<const f32x4_t*>(cols + tn * 32 + ec * 4) : f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int q = 0; q < 4; ++q)
@@ -409,6 +418,9 @@ __global__ void __launch_bounds__(DmafCfg::NT, 2) gemm_dmaf_kernel(const GemmArg
             o[e] = __float_as_uint(v);
           }
           put(o, v0 + (tm * 32 + it * 8) * ldob);
+          if constexpr (!HAS_RES) {
+            if (left & 3) dmaf_put_part(o, rsrc_o, vout + tn * 128 + (tm * 32 + it * 8) * ldob, have);
+          }
         }
         wave_lds_fence();
         res_load(std::integral_constant<int, st + 2>{});
@@ -557,6 +569,10 @@ __global__ void __launch_bounds__(DmafCfg::NT, 2) gemm_dmaf_kernel(const GemmArg
 
 // Which instance serves a call. 0 / 1: the general ones.
 inline int dmaf_epilogue(const GemmArgs& a, int in_dt, int out_dt, int tile_cols = DmafCfg::BN) {
+  // (fp32 rows without a residual: any length, see the epilogue)
+  if (out_dt == DT_F32 && !a.res && !a.res_stats && a.alpha == 1.f && a.act == ACT_NONE && a.nsplit >= a.N && !a.amax && !a.ln_out && a.res_rows == 0 &&
+      (in_dt == DT_BF16 || in_dt == DT_FP8) && (long)a.K * (in_dt == DT_FP8 ? 1 : 2) >= 2 * DmafCfg::ROWB && a.ldc * 4 * 256 < (1L << 31))
+    return DMAF_PLAIN;
   const int general = a.res_stats ? DMAF_GENERAL_NORM : DMAF_GENERAL, osz = out_dt == DT_F32 ? 4 : out_dt == DT_FP8 ? 1 : 2;
   // 16-byte stores of whole column groups inside one tile, offsets inside a tile that fit 31 bits, two slabs at least (the
   // constants of a tile land during its second slab)

@@ -39,6 +39,7 @@ hipError_t launch_gemm_dmam(const GemmArgs& a, int in_dt, int out_dt, int cus, h
     if (epi == DMAF_PLAIN) return a.act == ACT_MISH ? DMAM(DT_F16, DT_F16, DMAF_PLAIN, ACT_MISH) : DMAM(DT_F16, DT_F16, DMAF_PLAIN, ACT_NONE);
     return epi == DMAF_RES16 ? DMAM(DT_F16, DT_F16, DMAF_RES16, ACT_NONE) : DMAM(DT_F16, DT_F16, DMAF_GENERAL, ACT_NONE);
   }
+  if (in_dt == DT_BF16 && out_dt == DT_F32 && epi == DMAF_PLAIN) return DMAM(DT_BF16, DT_F32, DMAF_PLAIN, ACT_NONE);
   if (in_dt == DT_BF16 && out_dt == DT_F32) return epi == DMAF_RES32 ? DMAM(DT_BF16, DT_F32, DMAF_RES32, ACT_NONE) : DMAM(DT_BF16, DT_F32, DMAF_GENERAL, ACT_NONE);
 #undef DMAM
   return hipErrorInvalidValue;

@@ -245,9 +245,9 @@ __global__ void __launch_bounds__(DmamCfg::NT) gemm_dmam_kernel(const GemmArgs a
       const __amdgpu_buffer_rsrc_t rsrc_o = dmaf_rsrc(reinterpret_cast<char*>(first ? a.C : a.C2) + (long)m0 * ldob + (long)(first ? n0 : n0 - a.nsplit) * OSZ,
                                                       (long)(rows - 1) * ldob + (long)left * OSZ);
       constexpr int NOWHERE = (int)0x80000000u, CPL = 16 / OSZ;     // columns per lane in the store layout
-      const bool nt = a.stream_out != 0;
+      const bool nt = a.stream_out != 0 && (OUT_DT != DT_F32 || ldob % 128 == 0);
       auto put = [&](u32x4_t v, int row, int col) {
-        const int off = wn * Cfg::WN + col < left ? (wm * Cfg::WM + row) * ldob + (wn * Cfg::WN + col) * OSZ : NOWHERE;
+        const int off = wn * Cfg::WN + col + (OUT_DT == DT_F32 && !HAS_RES ? 3 : 0) < left ? (wm * Cfg::WM + row) * ldob + (wn * Cfg::WN + col) * OSZ : NOWHERE;
         if (nt) dmaf_put16_nt(v, rsrc_o, off);
         else dmaf_put16(v, rsrc_o, off);
       };
@@ -287,6 +287,10 @@ __global__ void __launch_bounds__(DmamCfg::NT) gemm_dmam_kernel(const GemmArgs a
               o[e] = __float_as_uint(v);
             }
             put(o, t * 32 + er + 16 * it, half * 16 + ec * 4);
+            if constexpr (!HAS_RES) {
+              const int col = wn * Cfg::WN + half * 16 + ec * 4;
+              if (left & 3) dmaf_put_part(o, rsrc_o, (wm * Cfg::WM + t * 32 + er + 16 * it) * ldob + col * 4, left - col);
+            }
           }
           wave_lds_fence();
         });

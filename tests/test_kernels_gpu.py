@@ -300,6 +300,23 @@ def test_gemm_split_output_last_tile_column_carries_the_columns_behind_it(cuda, 
     assert torch.allclose(got, ref, rtol=2 ** -6, atol=2 ** -6 * ref.abs().max().item())
 
 
+@pytest.mark.parametrize("M,N,gap", [(300, 1929, 0), (257, 1, 0), (130, 255, 1), (512, 258, 0), (70000, 771, 0), (128, 256, 3), (1000, 67, 0)])
+@pytest.mark.parametrize("dt,tiles", [("bf16", (10, 11)), ("fp8", (10,))])
+def test_gemm_fp32_rows_of_any_length_equal_the_small_tile(cuda, M, N, gap, dt, tiles):
+    """Bare fp32 products of the persistent tiles with rows at 4-byte alignment, one to three columns in the last 16-byte chunk
+    and columns behind a row that stay as they are."""
+    torch.manual_seed(M + N)
+    K = 256
+    A, W = torch.randn(M, K, device=cuda), torch.randn(N, K, device=cuda)
+    A, W = (A.to(torch.float8_e4m3fn), W.to(torch.float8_e4m3fn)) if dt == "fp8" else (A.bfloat16(), W.bfloat16())
+    bias = torch.randn(N, device=cuda)
+    want = run_gemm(A, W, _lib.F32, bias=bias, descale=0.5, tile=1, ldc=N + gap)
+    for tile in tiles:
+        got = run_gemm(A, W, _lib.F32, bias=bias, descale=0.5, tile=tile, ldc=N + gap)
+        assert torch.equal(got, want)
+        assert gap == 0 or (got._base[:, N:] == 0).all()
+
+
 @pytest.mark.parametrize("M,N,K", [(128, 128, 64), (128, 128, 256), (4096, 1024, 1024), (4096, 1536, 1024), (4096, 1024, 1536), (2048, 4096, 256),
                                    (300, 700, 512), (1000, 3104, 1024), (4096, 200, 192), (130, 129, 128), (640, 3104, 1088),
                                    (64, 1024, 1024), (64, 3104, 1536), (37, 3, 128), (1, 1929, 4096), (512, 1536, 640)])
