@@ -777,6 +777,28 @@ def test_gpt_norm_inside_the_product_is_bit_equal(cuda, kw, n_head, n_embd):
         assert torch.equal(m.forward((x[:B].contiguous(), idx[:B].contiguous()))[0], tokens[:B]), B
 
 
+@pytest.mark.parametrize("kw", [{}, {"norm_rms": True}, {"fp8": True}])
+@pytest.mark.parametrize("n_head,n_embd", [(8, 256), (12, 768), (16, 1024)])
+def test_gpt_norm_inside_the_product_takes_every_gain_and_offset(cuda, kw, n_head, n_embd):
+    """Gains and offsets that differ from column to column and from layer to layer, one of them large: eight waves bring them to
+    LDS for all sixteen, or write zeros where a norm has no offset. A column that came late would show against the two launches of the
+    large batch, bit for bit."""
+    planes, _ = positions(40, seed=13)
+    m = models.GPT(models.GPTConfig(block_size=128, vocab_size=1929, n_layer=2, n_head=n_head, n_embd=n_embd), **kw)
+    sd, g = m.state_dict(), torch.Generator().manual_seed(n_embd)
+    for k in sd:
+        if ".ln_" in k:
+            sd[k] = torch.randn(sd[k].shape, generator=g) + (1.0 if k.endswith("weight") else 0.0)
+            sd[k][-1] = 5.0
+    m.load_state_dict(sd)
+    x = planes.to(cuda)
+    if kw.get("fp8"):
+        m.calibrate(x)
+    base = m.forward((x, None))[0]
+    for B in (1, 2, 3, 5):
+        assert torch.equal(m.forward((x[:B].contiguous(), None))[0], base[:B]), B
+
+
 @pytest.mark.parametrize("kw", [{}, {"norm_rms": True}])
 def test_generate_rows_do_not_depend_on_the_batch(cuda, kw):
     """Token steps of 1 to 160 sequences: norms inside the products, K of the residual products over four waves. Same sums for
