@@ -141,6 +141,10 @@ __global__ void __launch_bounds__(1024) gemm_norm_kernel(const NormGemmKArgs s) 
           float y[4];
 #pragma unroll
           for (int e = 0; e < 4; ++e) y[e] = x[r][i][4 * h + e] * rstd[r] * gv[e] + bv[e];
+          if constexpr (IN_DT == DT_F16) {   // (rounded to fp32 first, as layernorm_kernel does: a multiply-add straight to f16 rounds once)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) asm volatile("" : "+v"(y[e]));
+          }
           uint8_t* const d = dst + (2 * i + h) * 64 * GB / 128 * (BM * ROWB);
           if constexpr (IN_DT == DT_FP8) *reinterpret_cast<uint32_t*>(d) = pack_fp8x4(y[0] * a.x_scale, y[1] * a.x_scale, y[2] * a.x_scale, y[3] * a.x_scale);
           else if constexpr (IN_DT == DT_BF16) *reinterpret_cast<uint2*>(d) = make_uint2(pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3]));

@@ -777,7 +777,7 @@ def test_gpt_norm_inside_the_product_is_bit_equal(cuda, kw, n_head, n_embd):
         assert torch.equal(m.forward((x[:B].contiguous(), idx[:B].contiguous()))[0], tokens[:B]), B
 
 
-@pytest.mark.parametrize("kw", [{}, {"norm_rms": True}, {"fp8": True}])
+@pytest.mark.parametrize("kw", [{}, {"norm_rms": True}, {"act_dtype": "f16"}, {"fp8": True}])
 @pytest.mark.parametrize("n_head,n_embd", [(8, 256), (12, 768), (16, 1024)])
 def test_gpt_norm_inside_the_product_takes_every_gain_and_offset(cuda, kw, n_head, n_embd):
     """Gains and offsets that differ from column to column and from layer to layer, one of them large: eight waves bring them to
