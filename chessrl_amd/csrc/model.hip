@@ -473,9 +473,10 @@ int Model::gemm(const Lin& L, const void* A, long lda, int in_dt, void* C, long 
     g.nsplit = g.N;
     g.ln_gamma = o.ln_g; g.ln_beta = o.ln_b; g.ln_out = o.ln_out; g.ln_ldo = L.N; g.ln_out_dtype = o.ln_dt; g.ln_eps = cfg.eps;
     g.ln_rms = cfg.norm_rms;
-    const bool fold = !profiling && gemm_folds_layernorm(g, in_dt == DT_FP8 ? DT_FP8 : L.dt);
+    const bool fold = gemm_folds_layernorm(g, in_dt == DT_FP8 ? DT_FP8 : L.dt);
     if (o.ln_folded) *o.ln_folded = fold;
     if (!fold) { g.ln_gamma = g.ln_beta = nullptr; g.ln_out = nullptr; }
+    else if (profiling) ++prof_n[2];
   }
   if (o.c_blocked) {
     g.c_blocked = 1;
@@ -506,9 +507,9 @@ int Model::lnorm(const void* x, long ldx, int in_dt, const float* g, const float
   return CRL_OK;
 }
 
-// (fp32 rows only; the profiling mode times norms and products apart)
+// (fp32 rows only)
 bool Model::norm_gemm_can(int M, const Lin& L, int in_dt, int x_dt) const {
-  return !profiling && x_dt == DT_F32 && gemm_norm_width(M, L.N, L.K, in_dt, device_cus()) != 0;
+  return x_dt == DT_F32 && gemm_norm_width(M, L.N, L.K, in_dt, device_cus()) != 0;
 }
 
 int Model::norm_gemm(const void* x, long ldx, const float* g, const float* b, const Lin& L, int in_dt, void* C, long ldc, int out_dt, int M, const GOpt& o,
@@ -521,7 +522,12 @@ int Model::norm_gemm(const void* x, long ldx, const float* g, const float* b, co
   a.out = C; a.ldo = ldc; a.out2 = o.C2; a.ldo2 = o.ldc2; a.nsplit = o.nsplit;
   a.M = M; a.N = L.N; a.K = L.K; a.act = o.act; a.out_dtype = out_dt;
   a.descale = in_dt == DT_FP8 ? 1.f / (o.a_scale * L.wscale) : 1.f; a.out_scale = o.out_scale;
-  HIPCHK(launch_gemm_norm(a, in_dt, gemm_norm_width(M, L.N, L.K, in_dt, device_cus()), o.k_parallel, st));
+  const int fam = in_dt == DT_FP8 ? 0 : 5;
+  if (profiling) { prof_flops[fam] += 2.0 * M * (double)(L.N - L.pad_N) * (L.K - L.pad_K); ++prof_n[2]; }
+  prof_begin(fam, st);
+  const hipError_t e = launch_gemm_norm(a, in_dt, gemm_norm_width(M, L.N, L.K, in_dt, device_cus()), o.k_parallel, st);
+  prof_end(st);
+  HIPCHK(e);
   return CRL_OK;
 }
 

@@ -311,7 +311,9 @@ double crl_model_flops_per_position(const crl_model* m);
 /* Switch: bracket every kernel launch with HIP events on the call's stream; each forward then
  * ends with a stream synchronise and accumulates, per kernel family, the elapsed milliseconds,
  * the launch count and (GEMMs) the 2*M*N*K work. Families: 0 fp8 GEMM, 1 attention,
- * 2 LayerNorm, 3 embedding, 4 policy QK^T, 5 16-bit GEMM. flops6 may be NULL. */
+ * 2 LayerNorm, 3 embedding, 4 policy QK^T, 5 16-bit GEMM. flops6 may be NULL. The switch changes neither the kernels
+ * that run nor a bit of their results (only crl_model_set_decode_graph's replay gives way to plain launches). A norm that
+ * runs inside a product's launch is counted under LayerNorm, its time is part of the product's. */
 int crl_model_set_profiling(crl_model* m, int on);
 int crl_model_get_profile(crl_model* m, double* ms6, int64_t* launches6, double* flops6);
 
