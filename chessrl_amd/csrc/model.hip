@@ -196,6 +196,7 @@ int Model::make_ffn(Layer& ly, const std::vector<float>& w1, const std::vector<f
 int Model::finalize() {
   for (auto& e : expected)
     if (!host.count(e.first)) { set_error("finalize: missing weight " + e.first); return CRL_ERR_STATE; }
+  if (tail_mb) tail_mb = -1;
   for (void* p : allocs) (void)hipFree(p);
   allocs.clear();
   layers.assign(cfg.n_layer, Layer());
@@ -585,10 +586,13 @@ int Model::forward_chunk(const float* planes, const uint8_t* ids, const uint8_t*
   const int xdt = sf32 ? DT_F32 : ad;
   auto am = [&](int l, int slot) -> float* { return calibrate ? amax_dev + (size_t)l * AMAX_SLOTS + slot : nullptr; };
   int rc;
+  tail_mb = 0;
 #define RUN(call) do { rc = (call); if (rc) return rc; } while (0)
 
   // ---- embedding
-  if (win) {
+  if (win && !win->x_in) {
+    // (the stream as the last call left it)
+  } else if (win) {
     const long n = (long)M * C;
     HIPCHK(launch_convert(win->x_in, ws.x, n, xdt, 1.f, st));
     if (f8 && !gpt) HIPCHK(launch_convert(win->x_in, ws.x8, n, DT_FP8, act_scale(l0, 0), st));
@@ -641,7 +645,7 @@ int Model::forward_chunk(const float* planes, const uint8_t* ids, const uint8_t*
   // not depend on the other rows). The rows are compact from the attention on: ao [mb, C], the stream in ws.t [mb, C].
   const bool one_row = gpt && policy && !all_logits && !calibrate && L > 0;
   // GPT64, few rows: a norm runs inside the product behind it (norm_gemm; bit-equal to the two launches). Not while maxima are collected.
-  auto fuses = [&](int rows, const Lin& lin, int dt) { return gpt && !calibrate && norm_gemm_can(rows, lin, dt, xdt); };
+  auto fuses = [&](int rows, const Lin& lin, int dt) { return gpt && !calibrate && !win && norm_gemm_can(rows, lin, dt, xdt); };
   for (int l = l0; l < l1; ++l) {
     const Layer& ly = layers[l];
     const bool last = l + 1 == l1;
@@ -721,7 +725,8 @@ int Model::forward_chunk(const float* planes, const uint8_t* ids, const uint8_t*
         RUN(gemm(ly.proj, ao_in, C, ao_dt, x, C, xdt, rows, o, st)); }
       { GOpt o; o.act = ACT_GELU; o.a_scale = f8 ? act_scale(l, 2) : 1.f; o.out_scale = f8 ? act_scale(l, 3) : 1.f; o.amax = am(l, 3);
         void* const f = f8 ? (void*)ws.f8 : (void*)ws.f;
-        if (fuses(rows, ly.ff1, ao_dt)) {
+        // (e4m3: the last layer's FFN-1 input stays behind for debug_read, unless it is one row per position)
+        if (!(f8 && last && !tail) && fuses(rows, ly.ff1, ao_dt)) {
           RUN(norm_gemm(x, C, ly.ln2_g, ly.ln2_b, ly.ff1, ao_dt, f, F, ao_dt, rows, o, st));
         } else {
           RUN(lnorm(x, C, xdt, ly.ln2_g, ly.ln2_b, f8 ? nullptr : ws.h, ad, f8 ? ws.h8 : nullptr, f8 ? act_scale(l, 2) : 1.f, C, rows, C, am(l, 2), st));
@@ -762,8 +767,12 @@ int Model::forward_chunk(const float* planes, const uint8_t* ids, const uint8_t*
   }
 
   if (win) {
-    HIPCHK(launch_widen(ws.x, gpt ? xdt : hd, win->x_out, (long)M * C, st));
+    if (win->x_out) HIPCHK(launch_widen(ws.x, gpt ? xdt : hd, win->x_out, (long)M * C, st));
     return CRL_OK;
+  }
+  if (one_row && f8) {
+    tail_mb = mb; tail_t = t;
+    std::copy_n(amax_host.begin() + (size_t)(L - 1) * AMAX_SLOTS, AMAX_SLOTS, tail_amax);
   }
 
   // ---- heads
@@ -847,6 +856,21 @@ int Model::run_layers(const float* x_in, int B, int first, int last, float* x_ou
   return forward_chunk(nullptr, nullptr, nullptr, nullptr, 0, B, &dummy_policy, nullptr, nullptr, false, st, &w);
 }
 
+// The last layer of a call that ran it on one row per position, on every token: its input is still in ws.x (the compact rows went to ws.t).
+int Model::finish_last_layer(hipStream_t st) {
+  if (tail_mb < 0) { set_error("debug_read: the weights have been replaced since the last forward"); return CRL_ERR_STATE; }
+  if (tail_mb == 0) return CRL_OK;
+  const auto row = amax_host.begin() + (size_t)(cfg.n_layer - 1) * AMAX_SLOTS;
+  const bool timed = profiling;
+  profiling = false;     // no part of a call
+  std::swap_ranges(tail_amax, tail_amax + AMAX_SLOTS, row);   // its scales, whatever has been set since
+  LayerWindow w{cfg.n_layer - 1, cfg.n_layer, nullptr, nullptr};
+  const int rc = forward_chunk(nullptr, nullptr, nullptr, nullptr, tail_t, tail_mb, nullptr, nullptr, nullptr, false, st, &w);
+  std::swap_ranges(tail_amax, tail_amax + AMAX_SLOTS, row);
+  profiling = timed;
+  return rc;
+}
+
 int Model::debug_read(const char* name, void* out, long bytes, hipStream_t st) {
   if (!name || !out || bytes < 0 || ws_mb == 0) { set_error("debug_read: bad arguments, or no forward has run yet"); return CRL_ERR_ARG; }
   const size_t M = (size_t)ws_mb * 64, C = cfg.d_model, F = cfg.d_ff;
@@ -860,6 +884,7 @@ int Model::debug_read(const char* name, void* out, long bytes, hipStream_t st) {
   else if (n == "t") { src = ws.t; cap = M * C * ((cfg.arch != CRL_ARCH_GPT64 && cfg.stream_f32 > 0) ? 4 : 2); }
   else { set_error("debug_read: unknown tensor " + n); return CRL_ERR_ARG; }
   if ((size_t)bytes > cap) { set_error("debug_read: " + n + " holds " + std::to_string(cap) + " bytes"); return CRL_ERR_ARG; }
+  if (n == "h8" || n == "ao8" || n == "f8") { const int rc = finish_last_layer(st); if (rc) return rc; }
   const size_t FP = (size_t)ff_cols();
   if (n == "f8" && FP != F) {   // rows lie FP apart
     const size_t rows = (size_t)bytes / F, rest = (size_t)bytes - rows * F;

@@ -60,8 +60,8 @@ struct GOpt;
 // A run of consecutive encoder layers on a caller-supplied input (Model::run_layers).
 struct LayerWindow {
   int first, last;
-  const float* x_in;   // device f32 [positions*64, d_model]: input of layer `first`
-  float* x_out;        // device f32, same shape: output of layer `last - 1`
+  const float* x_in;   // device f32 [positions*64, d_model]: input of layer `first`; null: ws.x as it is
+  float* x_out;        // device f32, same shape: output of layer `last - 1`; null: not wanted
 };
 
 struct Model {
@@ -96,6 +96,10 @@ struct Model {
   std::vector<float> amax_host;
   Workspace ws;
   int ws_mb = 0;
+  // An e4m3 GPT64 call for the last token's logits: positions and move tokens whose last layer ran on one row per position (0: all tokens
+  // ran; -1: the weights have been replaced since), and that layer's row of the amax table.
+  int tail_mb = 0, tail_t = 0;
+  float tail_amax[AMAX_SLOTS];
   // generation state, grown on demand: per layer [B, Tmax, 2C] 16-bit keys|values, newest tokens, counters, logits
   std::vector<void*> kv_layers;
   std::vector<void*> gen_allocs;
@@ -134,6 +138,7 @@ struct Model {
   // normalised output in the 16-bit type as the trunk's last layer does; everything between runs as in forward().
   int run_layers(const float* x_in, int B, int first, int last, float* x_out, hipStream_t st);
   // Copies a workspace tensor as the last call left it ("x8", "h8", "ao8", "f8": the e4m3 operand copies; "t") to `out`.
+  // The last layer's are those of every token also where the call ran it on one row per position.
   int debug_read(const char* name, void* out, long bytes, hipStream_t st);
   // Sequence generation with cached keys/values (model_bis.py:213-263 with rules, 266-311 without): seq [B, steps+1]
   // receives <thinking> and then `steps` sampled tokens; step_out [B, steps, V] (optional) the probabilities of
@@ -158,6 +163,7 @@ struct Model {
   // Norm of x's rows (fp32) and the product behind it in one launch; in_dt is the product's operand type. norm_gemm_can: the call is small enough.
   bool norm_gemm_can(int M, const Lin& L, int in_dt, int x_dt) const;
   int norm_gemm(const void* x, long ldx, const float* g, const float* b, const Lin& L, int in_dt, void* C, long ldc, int out_dt, int M, const GOpt& o, hipStream_t st);
+  int finish_last_layer(hipStream_t st);
   float act_scale(int layer, int slot) const;
   void prof_begin(int fam, hipStream_t st);
   void prof_end(hipStream_t st);

@@ -302,7 +302,9 @@ int crl_model_search_1ply(crl_model* m, const char* const* fens, int n, int chun
  * input and hold its output to a per-layer bar. crl_model_read_tensor copies one of the workspace tensors the last call
  * left behind to `out` (device): "x8", "h8", "ao8" (e4m3 [tokens, d_model]: the inputs of q|k|v, of FFN-1 and of the
  * out-projection), "f8" (e4m3 [tokens, d_ff]: the input of FFN-2), "t" (the un-normalised residual sum in the stream's
- * type); only the e4m3 copies an fp8 model writes are meaningful. */
+ * type); only the e4m3 copies an fp8 model writes are meaningful. They are the last layer's, for every token of the last
+ * micro-batch (a call for GPT64's last-token logits runs that layer on the last token only; the first read behind it runs the
+ * layer on all tokens, on `stream`); after per-token logits from an e4m3 lm_head "h8" holds lm_head's input instead. */
 int crl_model_run_layers(crl_model* m, const float* x_in, int B, int first, int last, float* x_out, void* stream);
 int crl_model_read_tensor(crl_model* m, const char* name, void* out, int64_t bytes, void* stream);
 int crl_model_vocab(const crl_model* m);

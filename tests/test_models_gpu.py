@@ -841,6 +841,29 @@ def test_gpt_last_token_row(cuda, kw, B, t):
     assert torch.equal(last, every[:, -1])
 
 
+@pytest.mark.parametrize("kw", [{}, {"stream_f32": False}])
+@pytest.mark.parametrize("B,t", [(1, 0), (3, 2), (40, 0), (256, 0)])
+def test_gpt_read_tensor_after_last_token_logits_holds_every_token(cuda, kw, B, t):
+    """The e4m3 operands of the last layer are there for every token after a call that needed the last token's only (norms inside
+    the products, apart, and queries in a product of their own), also when other scales are set before the first read."""
+    C, F = 256, 1024
+    m = models.GPT(models.GPTConfig(block_size=128, vocab_size=1929, n_layer=2, n_head=8, n_embd=C), fp8=True, fp8_lm_head=False, **kw)
+    planes = positions(B, seed=9)[0].to(cuda)
+    idx = torch.randint(0, 1924, (B, t), generator=torch.Generator().manual_seed(3)).to(cuda)
+    m.calibrate(planes)
+    eng, rows = m._engine, B * (64 + t)
+    read = lambda: [eng.read_tensor(n, (rows, w)) for n, w in (("ao8", C), ("h8", C), ("f8", F))]
+    eng.forward_tokens(planes, idx, last=False, every=True)
+    want = read()
+    eng.forward_tokens(planes[:1] * 0, idx[:1], last=False, every=True)
+    eng.forward_tokens(planes, idx, last=True)
+    amax = eng.get_amax()
+    eng.set_amax(2 * amax)
+    assert all(torch.equal(a, b) for a, b in zip(read(), want))
+    assert all(torch.equal(a, b) for a, b in zip(read(), want))
+    assert (eng.get_amax() == 2 * amax).all()
+
+
 def test_empty_batch(cuda):
     """B = 0 gives empty outputs (what the reference's torch modules do), for the board forward and the token forward."""
     m = models.BT4Class(2, 256, 384, 8)
