@@ -612,18 +612,21 @@ static hipError_t launch_in_out(const GemmArgs& a, int tile, hipStream_t st) {
     // Beyond, 128x128 (tile 11) or 256x256 (tile 3), both persistent: a round of 256x256 tiles over the CUs takes as long as 2.55 rounds
     // of 128x128 ones with 16-bit operands (K=1024: 27 against 10.5 us) and as 3.3 with e4m3, whose larger tile spends more of its time in prologue and
     // epilogue (16.5 against 5 us); K=256 (the bias generator) is mostly epilogue: 4.2, on many rounds 3.3. Measured over M = 256 .. 16384 at N = 1024, 1536, 2304, 3104, 4096,
-    // the rule is within 5 % of the better tile but for partly filled rounds (at most 11 %).
-    if (!a.k_parallel && tile != 5) {
+    // the rule is within 5 % of the better tile but for partly filled rounds (at most 11 %). At K=256 the 128x128 tile lives from weights that stay in an XCD's
+    // 4 MB of L2 beside the rows and results that pass through: each XCD walks all of N row of tiles by row of tiles. Up to 3 MB it keeps its 3.5-4 us a round; from
+    // 3.5 MB on a round takes 4.6 and more (bf16, N=8192, 4 MB, on the smaller and on the larger tile: M=1024 10.3 and 12.0 us, 2048 18.3 and 13.9, 3072 23.0 and 22.2,
+    // 4096 33.4 and 23.2; N=6144, 3 MB: M=4096 20.2 and 21.3): 3.0.
+    if (!a.k_parallel) {
       const bool slabs = ((long)a.K * (IN_DT == DT_FP8 ? 1 : 2)) % 128 == 0;
       const long cus = device_cus() > 0 ? device_cus() : 256;
       if (ring_ok && small <= cus) {
         tile = (long)((a.M + 31) / 32) * ((a.N + 31) / 32) <= cus ? 16 : 15;
       } else if (slabs && gemm_dmam_has(IN_DT, OUT_DT) && mid < 65536) {
         const long kb = (long)a.K * (IN_DT == DT_FP8 ? 1 : 2);
-        const double ratio = kb <= 512 ? (big <= 2 * cus ? 4.2 : 3.3) : IN_DT == DT_FP8 ? 3.3 : 2.55;
+        const double ratio = kb <= 512 ? (a.N * kb > (3L << 20) ? 3.0 : big <= 2 * cus ? 4.2 : 3.3) : IN_DT == DT_FP8 ? 3.3 : 2.55;
         tile = ratio * (double)((big + cus - 1) / cus) <= (double)((mid + cus - 1) / cus) ? 3 : 11;
       }
-    } else if (tile == 1 && ring_ok) {
+    } else if (tile == 1 && ring_ok) {   // (token steps)
       tile = (long)((a.M + 31) / 32) * ((a.N + 31) / 32) <= device_cus() ? 16 : small <= device_cus() ? 15 : 11;
     }
   }

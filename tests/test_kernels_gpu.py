@@ -365,6 +365,19 @@ def test_gemm_mid_tile_direct_to_lds_equals_register_staged(cuda, M, N, K, dt):
     assert torch.allclose(out.float(), ref, rtol=2 ** -7, atol=2 ** -7 * ref.abs().max().item()), (out.float() - ref).abs().max()
 
 
+@pytest.mark.parametrize("M,N", [(1, 8192), (250, 8192), (1279, 8192), (1281, 8192), (2048, 6144), (2048, 6160), (4100, 8192), (3000, 12301)])
+@pytest.mark.parametrize("dt", ["bf16", "f16", "fp8"])
+def test_gemm_short_k_either_side_of_the_tile_rule(cuda, M, N, dt):
+    """Rows of K of 512 bytes, where the automatic tile depends on rounds of tiles and on whether the weights stay in L2 (3 MB: 6144
+    rows of them): the same bits as the 64x64 tile on every side of both lines."""
+    torch.manual_seed(M + N)
+    t = {"bf16": torch.bfloat16, "f16": torch.float16, "fp8": torch.float8_e4m3fn}[dt]
+    K = 512 if dt == "fp8" else 256
+    A, W = torch.randn(M, K, device=cuda).to(t), torch.randn(N, K, device=cuda).to(t)
+    bias, ldc, out = torch.randn(N, device=cuda), (N + 7) // 8 * 8, _lib.F16 if dt == "f16" else _lib.BF16
+    assert torch.equal(run_gemm(A, W, out, bias=bias, descale=0.1, ldc=ldc), run_gemm(A, W, out, bias=bias, descale=0.1, ldc=ldc, tile=1))
+
+
 @pytest.mark.parametrize("M,N,out_dt", [(8448, 4096, _lib.BF16), (16384, 4096, _lib.F16), (131328, 384, _lib.BF16), (131072, 4096, _lib.BF16)])
 def test_gemm_short_k_rows_resident_equals_tiled(cuda, M, N, out_dt):
     """K = 256 e4m3 elements into a large 16-bit output (the attention-bias generator's product): the kernel whose
