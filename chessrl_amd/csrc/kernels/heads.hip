@@ -347,7 +347,8 @@ hipError_t launch_token_scores(const TokenScoreArgs& a, hipStream_t st) {
 // waves and one row at a time, 7 us so).
 constexpr int NLL_NT = 1024, NLL_INFLIGHT = 8;
 __global__ void __launch_bounds__(NLL_NT) masked_nll_mean_kernel(const float* logp, const int64_t* target, long ignore_index, int rows, float* out) {
-  __shared__ float s_sum[NLL_NT / 64], s_cnt[NLL_NT / 64];
+  __shared__ float s_sum[NLL_NT / 64];
+  __shared__ int s_cnt[NLL_NT / 64];
   float sum = 0.f;
   int cnt = 0;
   for (long r0 = threadIdx.x; r0 < rows; r0 += NLL_INFLIGHT * NLL_NT) {
@@ -364,13 +365,15 @@ __global__ void __launch_bounds__(NLL_NT) masked_nll_mean_kernel(const float* lo
       if (tg[i] != ignore_index) { sum -= lp[i]; ++cnt; }
   }
   sum = wave_sum(sum);
-  const float wcnt = wave_sum((float)cnt);   // (whole numbers: exact in any order up to 2^24 rows)
-  if ((threadIdx.x & 63) == 0) { s_sum[threadIdx.x >> 6] = sum; s_cnt[threadIdx.x >> 6] = wcnt; }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) cnt += __shfl_xor(cnt, o, 64);
+  if ((threadIdx.x & 63) == 0) { s_sum[threadIdx.x >> 6] = sum; s_cnt[threadIdx.x >> 6] = cnt; }
   __syncthreads();
   if (threadIdx.x == 0) {
-    float total = 0.f, n = 0.f;
+    float total = 0.f;
+    int n = 0;
     for (int w = 0; w < NLL_NT / 64; ++w) { total += s_sum[w]; n += s_cnt[w]; }
-    out[0] = n > 0.f ? total / n : 0.f;
+    out[0] = n > 0 ? total / (float)n : 0.f;
   }
 }
 

@@ -686,6 +686,21 @@ def test_token_scores_and_cross_entropy(cuda, V):
     assert lib().crl_token_scores(p(x), V, None, 0, None, rows, 4096, 0, None, None, None, None) != 0
 
 
+def test_masked_nll_mean_counts_rows_beyond_what_a_float_counts(cuda):
+    """2^24 rows of the first fourteen waves and one each of the last two: a count in floats would stay at 2^24."""
+    blocks, ign = 18725, -1
+    tgt = torch.zeros(blocks, 16, 64, dtype=torch.int64, device=cuda)
+    tgt[:, 14:] = ign
+    tgt[:6, 0] = ign                                  # 14 * 64 * 18725 - 6 * 64 = 2^24
+    tgt[0, 14, 0] = tgt[0, 15, 0] = 0
+    assert (tgt != ign).sum().item() == 2 ** 24 + 2
+    logp = torch.zeros(tgt.shape, device=cuda)
+    logp[100, :14] = -1.0                             # 896: exact in any order
+    out = torch.empty(1, device=cuda)
+    check(lib().crl_masked_nll_mean(p(logp), p(tgt), ign, tgt.numel(), p(out), stream()), "crl_masked_nll_mean")
+    assert out.item() == (torch.tensor(896.0) / torch.tensor(2.0 ** 24 + 2)).item()
+
+
 def test_sample_distribution_and_argmax(cuda):
     """crl_sample draws from softmax(logits/T): empirical frequencies over 200k rows, arg-max for T=0."""
     V, B = 37, 200000
