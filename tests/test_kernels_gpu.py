@@ -197,8 +197,8 @@ def test_gemm_fp8(cuda, M, N, K, tile):
                                    (20000, 1024, 1536), (2048, 200, 512), (2048, 1700, 1040), (300, 700, 736), (256, 4096, 256), (4096, 1024, 4096), (16384, 3104, 1024), (33000, 1024, 320)])
 @pytest.mark.parametrize("alt", [9, 10])
 def test_gemm_fp8_256x256_kernels_agree(cuda, M, N, K, alt):
-    """The other 256x256 e4m3 kernels against the general one (tile 7): the eight-wave one with its address arithmetic
-    out of the main loop (tile 10, what the forward pass runs) adds up K in the same order, so its outputs are bit-equal;
+    """The other 256x256 e4m3 kernels against the general one (tile 7): the eight-wave one whose waves take turns at loading
+    and multiplying (tile 10, what the forward pass runs; here with a running maximum, i.e. its general epilogue) adds up K in the same order, so its outputs are bit-equal;
     the four-wave one with 16x16x128 MFMAs (tile 9) agrees to summation-order noise. bf16 output with bias, activation and residual, and e4m3 output with a scale. K of 1 to 64 steps, K tails
     (where 9 and 10 hand over to 7), odd step counts, ragged M and N, more tiles than CUs."""
     torch.manual_seed(M + N + K)
@@ -233,11 +233,11 @@ def test_gemm_fp8_256x256_kernels_agree(cuda, M, N, K, alt):
 
 @pytest.mark.parametrize("M,N,K", [(4096, 1536, 1024), (16384, 3104, 1024), (65536, 1536, 1024), (32768, 1024, 1536), (256, 256, 128)])
 def test_gemm_guardless_epilogue_instances_equal_general_kernel(cuda, M, N, K):
-    """With M in whole 256-row tiles, aligned rows, a bf16 residual or none and no running maximum, tile 10 runs instances
-    whose epilogue has no edge, alignment or type guards, and for outputs beyond 64 MB ones whose activation, residual and
-    store kind are fixed at compile time as well (what a 4096-position forward runs: a plain scaled product into bf16, mish
-    into scaled e4m3). Same arithmetic: bit-equal to the general kernel (tile 7) in every combination, including the ones
-    that fall back to the guarded instance (activation with a residual) and a last tile column that is mostly outside N."""
+    """With aligned rows, a bf16 residual or none and no running maximum, tile 10 runs persistent instances whose epilogue has
+    no edge, alignment or type guards and whose activation and residual are fixed at compile time (what a
+    4096-position forward runs: a plain scaled product into bf16, mish into scaled e4m3); outputs beyond 64 MB are stored past
+    the caches. Same arithmetic: bit-equal to the general kernel (tile 7) in every combination, including the ones
+    that fall back to the general epilogue (activation with a residual) and a last tile column that is mostly outside N."""
     torch.manual_seed(M + N + K)
     A = (torch.randn(M, K, device=cuda) * 30).to(torch.float8_e4m3fn)
     W = (torch.randn(N, K, device=cuda) * 30).to(torch.float8_e4m3fn)
@@ -258,19 +258,18 @@ def test_gemm_guardless_epilogue_instances_equal_general_kernel(cuda, M, N, K):
             assert (a8 != b8).float().mean().item() < 1e-4 and torch.allclose(a8, b8, rtol=2 ** -3, atol=2 ** -9)
         else:
             assert torch.equal(lean, general), (M, N, K, kw["out_dt"], sorted(args))
-        # the 128x128 tile has such an instance too (tile 11, where M is whole 128-row tiles) against its register-staged
-        # twin with the general epilogue (tile 12)
+        # the 128x128 tile has such instances too (tile 11), here against the register-staged kernel with the general
+        # epilogue (tile 12)
         if M <= 16384:
             assert torch.equal(run_gemm(A, W, kw["out_dt"], tile=11, **args), run_gemm(A, W, kw["out_dt"], tile=12, **args)), (M, N, K, sorted(args))
 
 
 @pytest.mark.parametrize("M,nsplit,extra,K", [(16384, 3072, 32, 1024), (12288, 3072, 16, 1536), (1024, 512, 32, 256), (16640, 3072, 32, 1024), (16384, 3072, 40, 1024)])
 def test_gemm_split_output_last_tile_column_carries_the_columns_behind_it(cuda, M, nsplit, extra, K):
-    """crl_gemm_split: columns [0, nsplit) into C, the rest into C2. Where the 16-bit output passes 64 MB, M is whole tiles
-    and at most 32 columns lie behind a split at a multiple of 256, tile 10 computes them in the workgroups of the last
-    tile column (no tile column of their own); the general kernel (tile 7) and the cases outside those conditions (a small
-    output, 40 columns, a ragged M) give them a tile column. Same sums either way: both outputs bit-equal, and equal to the
-    unsplit product."""
+    """crl_gemm_split: columns [0, nsplit) into C, the rest into C2. The columns behind a split at a multiple of 256 are a last,
+    mostly empty tile column, which tile 10 writes to C2 through the epilogue that does without guards and stops at its end; large and
+    small outputs, whole and ragged M, with and without a bias. Both outputs bit-equal to the general kernel's (tile 7) and
+    to the automatic choice's, and equal to the unsplit product."""
     torch.manual_seed(M + nsplit + extra + K)
     N = nsplit + extra
     A = (torch.randn(M, K, device=cuda) * 30).to(torch.float8_e4m3fn)
@@ -322,9 +321,9 @@ def test_gemm_fp32_rows_of_any_length_equal_the_small_tile(cuda, M, N, gap, dt, 
                                    (64, 1024, 1024), (64, 3104, 1536), (37, 3, 128), (1, 1929, 4096), (512, 1536, 640)])
 @pytest.mark.parametrize("dt", ["bf16", "fp8", "f16"])
 def test_gemm_mid_tile_direct_to_lds_equals_register_staged(cuda, M, N, K, dt):
-    """The 128x128 tile fed by direct-to-LDS loads through a four-stage ring (tile 11, what the library picks for up to 256
-    such tiles when K is whole 128-byte slabs), the 64x64 tile on an eight-stage ring (tile 15, for up to 256 of those) and
-    the 32x32 tile on a sixteen-stage ring (tile 16, likewise) against the register-staged kernel (tile 12): same sums, bit-equal outputs; with bias, activation, residual and a
+    """The 128x128 tile fed by direct-to-LDS loads through a four-stage ring (tile 11, what the library picks between one tile of 64x64 per CU
+    and the batches of the 256x256 tile when K is whole 128-byte slabs; here with a running maximum, i.e. its general epilogue), the 64x64 tile
+    on an eight-stage ring (tile 15, while every such tile has a CU) and the 32x32 tile on a sixteen-stage ring (tile 16, likewise) against the register-staged kernel (tile 12): same sums, bit-equal outputs; with bias, activation, residual and a
     scaled e4m3 output. 1 to 32 slabs (fewer slabs than ring stages included), ragged M and N, K that is not whole slabs
     (where 11 hands over to 12 and 15 and 16 are refused)."""
     torch.manual_seed(M + N + K)
@@ -376,6 +375,29 @@ def test_gemm_short_k_either_side_of_the_tile_rule(cuda, M, N, dt):
     A, W = torch.randn(M, K, device=cuda).to(t), torch.randn(N, K, device=cuda).to(t)
     bias, ldc, out = torch.randn(N, device=cuda), (N + 7) // 8 * 8, _lib.F16 if dt == "f16" else _lib.BF16
     assert torch.equal(run_gemm(A, W, out, bias=bias, descale=0.1, ldc=ldc), run_gemm(A, W, out, bias=bias, descale=0.1, ldc=ldc, tile=1))
+
+
+@pytest.mark.parametrize("tile,M,N,K", [(11, 4225, 1024, 256), (11, 8191, 1536, 192), (11, 20000, 136, 512), (11, 127, 1024, 128), (11, 33000, 128, 1024),
+                                        (10, 33025, 1024, 256), (10, 16383, 1536, 512), (10, 70000, 264, 128), (10, 255, 256, 192)])
+@pytest.mark.parametrize("dt,out,kw", [("bf16", "bf16", dict(res=1)), ("bf16", "bf16", dict(res=1, act=1)), ("bf16", "bf16", dict(act=2)), ("f16", "f16", dict(res=1)),
+                                       ("bf16", "f32", dict(res=1)), ("fp8", "bf16", dict(res=1)), ("fp8", "fp8", dict(act=1))])
+def test_gemm_persistent_tiles_on_ragged_edges_equal_the_small_tile(cuda, tile, M, N, K, dt, out, kw):
+    """Workgroups that walk several tiles (more tiles than CUs, no whole number of rounds) or one, rows that end inside a tile, columns
+    that end inside one, 2 to 16 slabs of K: residuals of 16 bits and fp32 and the activations that have an epilogue of their own.
+    No running maximum, which would send the call to the general epilogue. Bit-equal to the 64x64 tile; nothing else is written."""
+    T = {"bf16": torch.bfloat16, "f16": torch.float16, "fp8": torch.float8_e4m3fn, "f32": torch.float32}
+    O = {"bf16": _lib.BF16, "f16": _lib.F16, "fp8": _lib.FP8, "f32": _lib.F32}
+    torch.manual_seed(M + N)
+    K = K * (2 if dt == "fp8" else 1)
+    A, W = torch.randn(M, K, device=cuda).to(T[dt]), (torch.randn(N, K, device=cuda) * K ** -0.5).to(T[dt])
+    args = dict(bias=torch.randn(N, device=cuda), descale=0.75, act=kw.get("act", 0), ldc=N + 16)
+    if kw.get("res"):
+        args.update(res=torch.randn(M, N + 8, device=cuda).to(T[out]), alpha=0.43)
+    if out == "fp8":
+        args.update(out_scale=30.0)
+    got, want = run_gemm(A, W, O[out], tile=tile, **args), run_gemm(A, W, O[out], tile=1, **args)
+    assert torch.equal(got, want)
+    assert (got._base[:, N:] == 0).all()
 
 
 @pytest.mark.parametrize("M,N,out_dt", [(8448, 4096, _lib.BF16), (16384, 4096, _lib.F16), (131328, 384, _lib.BF16), (131072, 4096, _lib.BF16)])

@@ -208,6 +208,21 @@ def test_bt4class_batch_invariance(cuda, fp8):
     assert torch.equal(p3.cpu(), pol.cpu()[perm]) and torch.equal(w3.cpu(), wdl.cpu()[perm])
 
 
+def test_bt4class_fp8_residuals_normalised_on_ragged_persistent_tiles(cuda):
+    """Full width in e4m3: 33, 65, 129 and 131 positions end inside a 128-row tile, the last two on workgroups that walk several
+    tiles; 1025 end inside a 256-row one. The residual that is normalised in the epilogue has the same bits on all of them and alone."""
+    m = models.BT4Class(2, 1024, 1536, 32, fp8=True)
+    m.load_state_dict(om.test_init_(om.BT4ClassOracle(policy_leela, 2, 1024, 1536, 32), seed=2).state_dict())
+    x = positions(1025, seed=12, leela=True)[0].to(cuda)
+    m.calibrate(x[:128].contiguous())
+    pol, wdl = m(x)
+    for B in (1, 33, 65, 129, 131):
+        p2, w2 = m(x[:B].contiguous())
+        assert torch.equal(p2, pol[:B]) and torch.equal(w2, wdl[:B]), B
+    p2, w2 = m(x[896:].contiguous())
+    assert torch.equal(p2, pol[896:]) and torch.equal(w2, wdl[896:])
+
+
 _FULL = {}
 
 
