@@ -262,7 +262,6 @@ __global__ void __launch_bounds__(DmamCfg::NT) gemm_dmam_kernel(const GemmArgs a
       auto activate = [&](float v) -> float {
         if constexpr (ACT == ACT_GELU) return act_gelu(v);
         else if constexpr (ACT == ACT_MISH) return act_mish(v);
-        else if constexpr (ACT == ACT_SWISH) return act_swish(v);
         else return v;
       };
       if constexpr (OUT_DT == DT_F32) {
