@@ -5,8 +5,8 @@
 // follow straight to LDS, and the normalised rows go to LDS as the operand. With both operands whole in LDS (32 K + BN K elements, at most
 // 150 KB) there is no ring; one barrier stands between gain and offset and their use, one between the operands and the product.
 // Bound by the CU's load rate at first (200 KB at 64 bytes a clock: 3500 of 11000 cycles), then by the norm's own vector instructions, which
-// every tile column repeats. The two add up: row loads and bias sit under lane conditions (columns past K, columns past N), so the compiler drains
-// every request, the weight rows among them, in front of the first use of a row. Measured in place: K = 768, N = 2304, 128 rows 8.4 us (12.4 for the norm riding on the K-sliced product before it and the
+// every tile column repeats. One counted wait behind the last request lets the statistics run under the weight loads; the normalised rows wait for
+// them all the same, because the compiler drains every load into LDS in front of the first write to it. Measured in place: K = 768, N = 2304, 128 rows 8.4 us (12.4 for the norm riding on the K-sliced product before it and the
 // product), 64 rows 7.3 us (8.5 for two launches). The same for the 16-bit rows of 1024 columns of the BT4-class trunk took 9.4 us against 8.7
 // for two launches and is not here.
 // The norm's arithmetic is that of layernorm_kernel row by row and the product adds K in the order of the other tiled kernels (KP = 1): bit-equal to
@@ -48,7 +48,7 @@ __global__ void __launch_bounds__(1024) gemm_norm_kernel(const NormGemmKArgs s) 
   const int C = a.K;
   float x[2][2][8];
   auto has = [&](int i, int h) { return (2 * i + h) * 256 < C; };   // (whole groups of 256 columns: the same for all lanes)
-  // Gain and offset are requested first: the wait in front of the barrier behind the norm counts past the weight rows to them.
+  // Gain and offset first.
   // 256 columns per wave-instruction, waves 0-3 and 4-7
   if (wave < 8) {
     const float* src = wave < 4 ? a.gamma : a.beta;
@@ -58,13 +58,20 @@ __global__ void __launch_bounds__(1024) gemm_norm_kernel(const NormGemmKArgs s) 
                                        (__attribute__((address_space(3))) void*)(lds_g + (wave >> 2) * 1024 + (wave & 3) * 256), 16, 0, 0);
     else if (!src) *reinterpret_cast<f32x4_t*>(lds_g + 1024 + (wave & 3) * 256 + lane * 4) = f32x4_t{0.f, 0.f, 0.f, 0.f};
   }
-  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int r = 0; r < 2; ++r) {
     int m = m0 + wave * 2 + r;
     m = m < a.M ? m : a.M - 1;
 #pragma unroll
     for (int i = 0; i < 2; ++i) load_norm8<DT_F32>(a.x, (long)m * a.ldx, i, lane, C, x[r][i]);
+  }
+  // the bias of this thread's columns
+  const int er = tid / (BN / EV), ec = (tid % (BN / EV)) * EV;
+  float bias[EV];
+#pragma unroll
+  for (int e = 0; e < EV; ++e) {
+    const int n = n0 + ec + e;
+    bias[e] = a.bias ? a.bias[n < a.N ? n : a.N - 1] : 0.f;
   }
   __builtin_amdgcn_sched_barrier(0);
   // ---- weight rows: 8 rows of 128 bytes per instruction, the swizzle applied on the global side
@@ -76,7 +83,7 @@ __global__ void __launch_bounds__(1024) gemm_norm_kernel(const NormGemmKArgs s) 
     r = r < left ? r : left - 1;
     const int voff = r * ldb + (((lane & 7) ^ l8 ^ (grp & 7)) << 4);
     const __amdgpu_buffer_rsrc_t rs = dmaf_rsrc(reinterpret_cast<const uint8_t*>(a.W) + (long)n0 * ldb, (long)(left < BN ? left : BN) * ldb);
-    // (always the same number, those past K out of bounds and into a spare kilobyte: a wait for what was requested before counts past them)
+    // (always the same number, those past K out of bounds and into a spare kilobyte: the wait for what was requested before counts past them)
     const __amdgpu_buffer_rsrc_t none = dmaf_rsrc(a.W, 0);
 #pragma unroll
     for (int j = 0; j < GR; ++j) {
@@ -84,14 +91,11 @@ __global__ void __launch_bounds__(1024) gemm_norm_kernel(const NormGemmKArgs s) 
       dmaf_load16(sl < nslab ? rs : none, sl < nslab ? lds_w + (sl * BN + grp * 8) * ROWB : reinterpret_cast<uint8_t*>(lds_g) + 8192, voff, sl * ROWB);
     }
   }
-  // the bias of this thread's columns
-  const int er = tid / (BN / EV), ec = (tid % (BN / EV)) * EV;
-  float bias[EV];
-#pragma unroll
-  for (int e = 0; e < EV; ++e) {
-    const int n = n0 + ec + e;
-    bias[e] = a.bias && n < a.N ? a.bias[n] : 0.f;
-  }
+  __builtin_amdgcn_sched_barrier(0);
+  // Everything requested before the GR weight rows is there: this wave's rows and bias, and its share of gain and offset (the zeros in the place of
+  // an offset are a write to LDS), which the barrier behind the statistics then hands to every wave; the barrier itself waits for nothing.
+  wait_vmcnt_lgkm0<GR>();
+  __builtin_amdgcn_sched_barrier(0);
   // ---- the norm
   const float inv_c = fast_rcp((float)C);
   float mean[2], rstd[2];
@@ -119,9 +123,6 @@ __global__ void __launch_bounds__(1024) gemm_norm_kernel(const NormGemmKArgs s) 
     rstd[r] = rsqrtf(wave_sum(q) * inv_c + a.eps);
   }
   __builtin_amdgcn_sched_barrier(0);
-  // Gain and offset for every wave to read: this wave's share was requested before its GR weight requests, and the zeros in the place of an offset are
-  // a write to LDS. The barrier itself waits for neither.
-  wait_vmcnt_lgkm0<GR>();
   dmaf_barrier();
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
