@@ -75,8 +75,8 @@ __device__ __forceinline__ void wave_lds_fence() {
 }
 
 // 16 bytes read once (a 16-bit residual row segment): loaded with the non-temporal hint so that it does not displace
-// the operand tiles the workgroups of an XCD share in L2 (an fp32 residual stream measured 2 % slower with the hint
-// and keeps plain loads).
+// the operand tiles the workgroups of an XCD share in L2 (in this epilogue an fp32 residual stream measured 2 % slower with
+// the hint and keeps plain loads; the persistent 256x256 tile has its own, see gemm_dmaf_kernel.hpp).
 __device__ __forceinline__ uint4 nt_load16(const char* p) {
   const i32x4_t v = __builtin_nontemporal_load(reinterpret_cast<const i32x4_t*>(p));
   return make_uint4((uint32_t)v[0], (uint32_t)v[1], (uint32_t)v[2], (uint32_t)v[3]);

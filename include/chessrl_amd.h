@@ -111,18 +111,19 @@ int crl_random_positions(uint64_t seed, int n, int max_plies, double late_fracti
  * most 256 columns whose K is 8 KB or more per row are always K-sliced the same way (a function of N and K alone), so
  * the row-count independence holds for them too. The first K-sliced launch on a stream allocates that stream's
  * workspace: issue it once outside any graph capture. 7, 9 and 10 name the 256x256 kernels explicitly: 7 = eight waves in
- * step (any K, any operand type), 10 = the same with its address arithmetic kept out of the main loop (K in whole
- * 128-byte slabs; 3 runs this one where it applies), both with the sums and result bits of 1-3; 9 = four
+ * step (any K, any operand type), 10 = eight waves that take turns at loading and multiplying, in persistent workgroups where
+ * its own epilogue serves the call (K in whole 128-byte slabs, the types of 15 and 16 and e4m3 operands with an fp32 output; 3 runs
+ * this one where it applies), both with the sums and result bits of 1-3; 9 = four
  * software-pipelined waves with 16x16x128 MFMAs (e4m3 operands, whole slabs; what 3 runs from K = 4096 on; these MFMAs
  * add 128 products per instruction instead of 64, so a sum can differ from the others' in its last fp32 bits); 6 and 8
  * are not assigned (CRL_ERR_ARG). 9 and 10 fall back to 7 where K is not whole slabs. 11 and 12 name the two
- * 128x128 kernels (same sums and bits as 2): 11 = fed by direct-to-LDS loads through a four-stage ring (whole slabs; what 2
- * runs for at most one tile per CU), 12 = register-staged (any K; 11 hands over to it where K is not whole slabs).
+ * 128x128 kernels (same sums and bits as 2): 11 = loading and multiplying waves around a four-stage ring of direct-to-LDS loads (whole
+ * slabs, the types of 15 and 16; what 2 runs where it applies), 12 = register-staged (any K; 11 hands over to it where K is not whole slabs).
  * 15 and 16 = the 64x64 tile on an eight-stage and the 32x32 tile on a sixteen-stage ring of direct-to-LDS loads (same sums
  * and bits as 1; whole slabs; e4m3 operands with a 16-bit or e4m3 output, bf16/f16 operands with an output of their own
- * type, bf16 operands with an fp32 output; else CRL_ERR_ARG). Below 256 tiles of
- * 128x128, tile 0 runs 16 while every 32x32 tile has a CU of its own, 15 while every 64x64 tile has, 11 beyond, and 1 where
- * they do not apply.
+ * type, bf16 operands with an fp32 output; else CRL_ERR_ARG). Where those apply, tile 0 runs 16 while every 32x32 tile has a CU
+ * of its own, 15 while every 64x64 tile has, and beyond that 11 or 3, whichever takes fewer rounds of its tiles over the CUs at the measured time
+ * of a round; elsewhere 3 from 160 tiles of 256x256 on, 2 from 256 of 128x128 on, else 1.
  * 13 and 14 name the kernel for K = 256 e4m3 elements whose workgroups keep 256 rows of A in registers and walk N (the
  * attention-bias generator's product): a bare scaled product (no bias, activation, residual or amax; alpha = 1) into a
  * bf16/f16 output of more than 64 MB, M a multiple of 256, N of 128; anything else is CRL_ERR_ARG. 13 writes C row-major
@@ -262,8 +263,9 @@ int crl_model_forward_tokens(crl_model* m, const float* planes, const int64_t* i
  * crl_model_set_decode_graph(m, 1) records the per-token launches once into a HIP graph (from the second token on;
  * the kernels then read the token index from a device counter) and replays it; results are bit-identical, the call
  * returns after the stream has drained, and the stream must not itself be under capture. It is off by default: a
- * token step is bound by its kernels' run time on the device, not by the host's launches (measured: no gain at 128
- * sequences), so the option is for hosts that cannot keep up. The profiling mode always launches plainly. */
+ * token step is bound by its kernels' run time on the device, not by the host's launches (measured at 128 sequences:
+ * 60.8 ms plain, 64.4 ms replayed, where storing keys and values and advancing the counter are launches of their own), so
+ * the option is for hosts that cannot keep up. The profiling mode always launches plainly. */
 int crl_model_generate(crl_model* m, const float* planes, int B, int steps, float temperature, uint64_t seed, int rules,
                        int64_t* sequences, float* step_out, int out_logits, void* stream);
 int crl_model_set_decode_graph(crl_model* m, int on);
