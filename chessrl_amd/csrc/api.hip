@@ -4,6 +4,7 @@
 #include <condition_variable>
 #include <cstring>
 #include <mutex>
+#include <exception>
 #include <system_error>
 #include <thread>
 
@@ -56,7 +57,10 @@ int parallel_for(int n, int threads, Fn fn, int grain = 64) {
     }
   };
   std::vector<std::thread> pool;
-  for (int t = 1; t < threads; ++t) pool.emplace_back(work);
+  try {
+    pool.reserve((size_t)threads - 1);
+    for (int t = 1; t < threads; ++t) pool.emplace_back(work);
+  } catch (const std::exception&) {}   // (no more threads to be had: the ones there are and this one do the work)
   work();
   for (auto& th : pool) th.join();
   if (bad_rc) set_error(bad_err);

@@ -4,6 +4,9 @@ import ctypes
 import hashlib
 import os
 import re
+import resource
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -31,6 +34,33 @@ def test_header_symbols_exported():
     for name in declared:
         assert hasattr(lib, name), name
     assert b"gfx950" in _lib.lib().crl_version()
+
+
+def test_threads_that_cannot_be_started_are_done_without():
+    """A host function asked for more threads than the process may have does its work on those it gets (no exception leaves a C
+    entry): stacks of 256 MB in 700 MB of address space."""
+    code = """
+import resource, numpy as np
+from chessrl_amd import _lib, board
+fens = board.random_positions(3, 100, fens=True)["fens"] * 100
+n, arr, one, many = len(fens), _lib.str_array(fens), np.zeros((len(fens), 64), np.uint8), np.zeros((len(fens), 64), np.uint8)
+flags = np.zeros((n, 4), np.uint8)
+lib = _lib.lib()
+assert lib.crl_encode_fens_compact(arr, n, one.ctypes.data, flags.ctypes.data, 1) == 0
+top = int(open("/proc/self/statm").read().split()[0]) * resource.getpagesize() + (700 << 20)
+resource.setrlimit(resource.RLIMIT_AS, (top, top))
+assert lib.crl_encode_fens_compact(arr, n, many.ctypes.data, flags.ctypes.data, 32) == 0
+assert (one == many).all() and one.any()
+print("done")
+"""
+
+    def big_stacks():
+        hard = resource.getrlimit(resource.RLIMIT_STACK)[1]
+        resource.setrlimit(resource.RLIMIT_STACK, (256 << 20, hard))
+
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, preexec_fn=big_stacks, timeout=120,
+                       cwd=os.path.join(os.path.dirname(_lib.LIB_PATH), ".."))
+    assert r.returncode == 0 and r.stdout.strip() == "done", (r.returncode, r.stderr[-500:])
 
 
 def test_vocab_pinned():
