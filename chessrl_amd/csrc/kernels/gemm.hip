@@ -387,9 +387,9 @@ __global__ void __launch_bounds__(256) splitk_reduce_ln_kernel(const GemmArgs a,
 // Measured on MI355X (M=65536, N=1024..3072, K=1024..8192, fp8 and bf16, same job): the 256x256
 // tile fed by direct-to-LDS loads with 128-byte rows and two stages (DmaCfg2) is 10-20 % faster
 // than the same 8-wave tile with register staging; a 256x128 single-stage tile at two workgroups per
-// CU, a 4-stage ring of 64-byte rows (twice the barriers) and a one-workgroup-per-CU loop over several
-// tiles (with bare barriers and a counted wait past the previous tile's stores too) were slower or equal.
-// The register-staged kernel serves the small tiles.
+// CU and a 4-stage ring of 64-byte rows (twice the barriers) were slower or equal. (The kernels for K in whole slabs
+// have gone further: gemm_dmaf_kernel.hpp, gemm_dmam_kernel.hpp, gemm_dmas_kernel.hpp.)
+// The register-staged kernel serves the small tiles of every other call.
 typedef GemmCfg<128, 128, 2, 2, 2, 0, 2> CfgMid;    // 4 waves, 64x64 per wave, two workgroups per CU
 typedef GemmCfg<64, 64, 2, 2, 2, 0, 2> CfgSmall;    // 4 waves, 32x32 per wave
 typedef GemmCfg<64, 64, 2, 2, 2, 0, 2, 4> CfgSmallK4;   // the same tile walked by 4 groups of 4 waves, K slabs in turn

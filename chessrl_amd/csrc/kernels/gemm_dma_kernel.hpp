@@ -1,5 +1,5 @@
-// C[M,N] = epilogue(A[M,K] · W[N,K]^T) on the 256x256 workgroup tile: the GEMM of the large batches (every trunk linear
-// of a 4096-position forward). The call sites, operand layout and epilogue are those described in gemm.hip. The kernel
+// C[M,N] = epilogue(A[M,K] · W[N,K]^T) on the 256x256 workgroup tile, any K and every type combination: the large products
+// that gemm_dmaf_kernel.hpp does not take. The call sites, operand layout and epilogue are those described in gemm.hip. The kernel
 // is a header because its instances are spread over two translation units (gemm_dma.hip, gemm_dma_resnorm.hip): a
 // kernel added to a code object moves the others in it, and their speed depends measurably on where they land.
 #pragma once
