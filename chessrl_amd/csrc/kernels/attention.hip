@@ -1,4 +1,4 @@
-// Fused 64-token multi-head attention: one 64-lane wave per (position, head).
+// Fused 64-token multi-head attention: one 64-lane wave per unit, i.e. (position, head); two where there are few of them.
 //
 // Replaces F.scaled_dot_product_attention(q,k,v,is_causal=True) of model_bis.py:71 and
 // the score/softmax/context chain of RelativeMultiHeadAttention2.forward
@@ -14,6 +14,8 @@
 // re-used in place as the column operand of the second product O^T = V^T · P^T; only V
 // needs a transpose, which goes through a wave-private LDS patch.
 #include "common.hpp"
+
+#include <type_traits>
 
 namespace crl {
 
@@ -87,14 +89,15 @@ struct AttnMinWaves { static constexpr int N = (HS == 32 && MODE == ATTN_BIAS) ?
 
 // OUT_FP8: write e4m3 (value*out_scale) instead of the input element type.
 // COOP: the workgroup's outputs leave through an LDS tile as whole row segments (see s_out below; the launcher says when).
+// SPLIT: a workgroup is one unit, its two waves take a query tile each and transpose half of V each.
 // LAST (ATTN_CAUSAL): only token 63's output is wanted: the query tile of tokens 32..63 alone runs and that one row is stored, at row b.
-template <int HS, int MODE, int OUT_FP8, int IN_DT, int COOP = 0, int LAST = 0>
-__global__ void __launch_bounds__(64 * AttnWaves<MODE>::N, (AttnMinWaves<HS, MODE>::N)) attention_kernel(const AttnArgs a) {
+template <int HS, int MODE, int OUT_FP8, int IN_DT, int COOP = 0, int LAST = 0, int SPLIT = 0>
+__global__ void __launch_bounds__(SPLIT ? 128 : 64 * AttnWaves<MODE>::N, (SPLIT ? 0 : AttnMinWaves<HS, MODE>::N)) attention_kernel(const AttnArgs a) {
   typedef Half16<IN_DT> H16;
   typedef typename H16::vec hvec;
   constexpr int KS = HS / 16;   // k-steps of the score product
   constexpr int DT_TILES = HS / 32;
-  constexpr int NW = AttnWaves<MODE>::N;
+  constexpr int NW = SPLIT ? 1 : AttnWaves<MODE>::N;   // units of the workgroup
   __shared__ __align__(16) uint16_t s_vt[NW][HS * VT_STRIDE];
   __shared__ float s_sp[MODE == ATTN_RELSHIFT ? NW : 1][MODE == ATTN_RELSHIFT ? 64 * SP_STRIDE : 1];
   // Output tile of the workgroup's NW heads (head size 32): 64 rows of NW * HS elements, 16 bytes of padding
@@ -102,7 +105,8 @@ __global__ void __launch_bounds__(64 * AttnWaves<MODE>::N, (AttnMinWaves<HS, MOD
   // lane and row, a quarter or an eighth of a line at a time; gathered here, the workgroup stores whole lines (measured
   // on 4096 positions x 32 heads in e4m3: the stores were 9 % of the kernel's bytes and 21 % of its time).
   static_assert(!LAST || (MODE == ATTN_CAUSAL && !COOP), "one-row form");
-  constexpr int IT0 = LAST ? 1 : 0;   // first query tile
+  static_assert(!SPLIT || (MODE != ATTN_RELSHIFT && !COOP && !LAST), "one query tile per wave");
+  constexpr int NIT = LAST || SPLIT ? 1 : 2;   // query tiles of a wave
   static_assert(!COOP || (HS == 32 && (NW == 4 || NW == 8 || NW == 16)), "the output tile is laid out for head size 32");
   constexpr int OSZ = OUT_FP8 ? 1 : 2;
   constexpr int OROW = NW * HS * OSZ, OSTRIDE = OROW + 16;
@@ -119,7 +123,8 @@ __global__ void __launch_bounds__(64 * AttnWaves<MODE>::N, (AttnMinWaves<HS, MOD
     const int per = gridDim.x >> 3;
     if (bid < (per << 3)) bid = (bid & 7) * per + (bid >> 3);
   }
-  const int unit = bid * NW + wave;
+  const int unit = SPLIT ? bid : bid * NW + wave;
+  const int it0 = LAST ? 1 : SPLIT ? wave : 0;   // the first of them
   if (unit >= a.B * a.H) return;
   const int b = unit / a.H, h = unit - b * a.H;
   constexpr bool coop = COOP != 0;
@@ -131,7 +136,7 @@ __global__ void __launch_bounds__(64 * AttnWaves<MODE>::N, (AttnMinWaves<HS, MOD
   const uint16_t* vp = reinterpret_cast<const uint16_t*>(a.v) + (long)b * 64 * a.ldv + h * HS;
 
   // ---- V -> V^T in LDS ------------------------------------------------------------
-  uint16_t* vt = s_vt[wave];
+  uint16_t* vt = s_vt[SPLIT ? 0 : wave];
   // VPAIR: the two waves of a pair of neighbouring heads (a token's V rows of the two are one whole 128-byte line) take
   // half the tokens each, for both heads: every line is read by one wave, once, with the non-temporal hint, and lands
   // transposed in the patch of the head it belongs to; the workgroup meets at a barrier before the second product.
@@ -160,8 +165,10 @@ __global__ void __launch_bounds__(64 * AttnWaves<MODE>::N, (AttnMinWaves<HS, MOD
     constexpr int DC = HS / 8;            // 16-byte chunks per V row
     constexpr int PASSES = (16 * DC) / 64;
 #pragma unroll
-    for (int p = 0; p < PASSES; ++p) {
-      const int id = p * 64 + lane;
+    for (int p = 0; p < (SPLIT && PASSES > 1 ? PASSES / 2 : PASSES); ++p) {
+      // (SPLIT: half of the rows each; with a single pass half the lanes of each wave)
+      if (SPLIT && PASSES == 1 && g) break;
+      const int id = SPLIT ? (PASSES == 1 ? 32 * wave + lr : (wave * (PASSES / 2) + p) * 64 + lane) : p * 64 + lane;
       const int jq = id / DC, dc = id - jq * DC;
       uint4 rows[4];
 #pragma unroll
@@ -182,27 +189,22 @@ __global__ void __launch_bounds__(64 * AttnWaves<MODE>::N, (AttnMinWaves<HS, MOD
   }
 
   // ---- scores -----------------------------------------------------------------------
-  hvec qf[2][KS], kf[2][KS];
+  hvec qf[NIT][KS], kf[2][KS];
 #pragma unroll
   for (int t = 0; t < 2; ++t)
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
-      const uint16_t* qa = qp + (long)(32 * t + lr) * a.ldq + 16 * ks + 8 * g;
       const uint16_t* ka = kp + (long)(32 * t + lr) * a.ldk + 16 * ks + 8 * g;
-      if (LAST && t < IT0) {
-        kf[t][ks] = *reinterpret_cast<const hvec*>(ka);
-      } else if (qk_once) {
-        qf[t][ks] = __builtin_bit_cast(hvec, attn_load_once(qa));
-        kf[t][ks] = __builtin_bit_cast(hvec, attn_load_once(ka));
-      } else {
-        qf[t][ks] = *reinterpret_cast<const hvec*>(qa);
-        kf[t][ks] = *reinterpret_cast<const hvec*>(ka);
+      if (t < NIT) {
+        const uint16_t* qa = qp + (long)(32 * (it0 + t) + lr) * a.ldq + 16 * ks + 8 * g;
+        qf[t][ks] = qk_once ? __builtin_bit_cast(hvec, attn_load_once(qa)) : *reinterpret_cast<const hvec*>(qa);
       }
+      kf[t][ks] = qk_once ? __builtin_bit_cast(hvec, attn_load_once(ka)) : *reinterpret_cast<const hvec*>(ka);
     }
 
   // The bias tile (8 KB per wave), requested behind V, q and k: loads return in the order of their issue, which is now
   // the order of their use, and all twenty are out before the first of them is waited for.
-  uint4 braw[2][2][2];
+  uint4 braw[NIT][2][2];
   if constexpr (MODE == ATTN_BIAS) {
     // Element k = 512 L + 8 lane + e of the unit's 4096 (L = (it, jt, rh)): row-major, or in blocks of 256 units x 128
     // elements (the layout the bias generator's GEMM writes fastest), where a load of 1 KB is four pieces of 256 bytes.
@@ -215,20 +217,20 @@ __global__ void __launch_bounds__(64 * AttnWaves<MODE>::N, (AttnMinWaves<HS, MOD
       bp += (long)unit * 4096 + (lane << 3);
     }
 #pragma unroll
-    for (int it = IT0; it < 2; ++it)
+    for (int it = 0; it < NIT; ++it)
 #pragma unroll
       for (int jt = 0; jt < 2; ++jt)
 #pragma unroll
         for (int rh = 0; rh < 2; ++rh)
-          braw[it][jt][rh] = attn_load_once(bp + ((it * 2 + jt) * 2 + rh) * lstride);
+          braw[it][jt][rh] = attn_load_once(bp + (((it0 + it) * 2 + jt) * 2 + rh) * lstride);
   }
 
   if constexpr (MODE == ATTN_BIAS) __builtin_amdgcn_s_setprio(0);
-  f32x16_t s[2][2];  // [jt][it]
+  f32x16_t s[2][NIT];  // [jt][it]
 #pragma unroll
   for (int jt = 0; jt < 2; ++jt)
 #pragma unroll
-    for (int it = IT0; it < 2; ++it)
+    for (int it = 0; it < NIT; ++it)
 #pragma unroll
       for (int r = 0; r < 16; ++r) s[jt][it][r] = 0.f;
 
@@ -236,11 +238,11 @@ __global__ void __launch_bounds__(64 * AttnWaves<MODE>::N, (AttnMinWaves<HS, MOD
     // content = (q+u)·k, position = (q+v)·p, both with the bias folded into the query.
     const uint16_t* pp = reinterpret_cast<const uint16_t*>(a.pos) + h * HS;
     const long ldp = (long)a.H * HS;
-    f32x16_t sp[2][2];
+    f32x16_t sp[2][NIT];
 #pragma unroll
     for (int jt = 0; jt < 2; ++jt)
 #pragma unroll
-      for (int it = IT0; it < 2; ++it)
+      for (int it = 0; it < NIT; ++it)
 #pragma unroll
         for (int r = 0; r < 16; ++r) sp[jt][it][r] = 0.f;
 #pragma unroll
@@ -255,7 +257,7 @@ __global__ void __launch_bounds__(64 * AttnWaves<MODE>::N, (AttnMinWaves<HS, MOD
 #pragma unroll
       for (int t = 0; t < 2; ++t) pf[t] = *reinterpret_cast<const hvec*>(pp + (long)(32 * t + lr) * ldp + 16 * ks + 8 * g);
 #pragma unroll
-      for (int it = IT0; it < 2; ++it) {
+      for (int it = 0; it < NIT; ++it) {
         const hvec qu = add_bias_h<H16>(qf[it][ks], ub);
         const hvec qv = add_bias_h<H16>(qf[it][ks], vb);
 #pragma unroll
@@ -271,7 +273,7 @@ __global__ void __launch_bounds__(64 * AttnWaves<MODE>::N, (AttnMinWaves<HS, MOD
 #pragma unroll
     for (int jt = 0; jt < 2; ++jt)
 #pragma unroll
-      for (int it = IT0; it < 2; ++it)
+      for (int it = 0; it < NIT; ++it)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const int m = 32 * jt + 8 * (r >> 2) + 4 * g + (r & 3);
@@ -283,7 +285,7 @@ __global__ void __launch_bounds__(64 * AttnWaves<MODE>::N, (AttnMinWaves<HS, MOD
 #pragma unroll
     for (int jt = 0; jt < 2; ++jt)
 #pragma unroll
-      for (int it = IT0; it < 2; ++it)
+      for (int it = 0; it < NIT; ++it)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const int j = 32 * jt + 8 * (r >> 2) + 4 * g + (r & 3);
@@ -299,12 +301,12 @@ __global__ void __launch_bounds__(64 * AttnWaves<MODE>::N, (AttnMinWaves<HS, MOD
 #pragma unroll
       for (int jt = 0; jt < 2; ++jt)
 #pragma unroll
-        for (int it = IT0; it < 2; ++it)
+        for (int it = 0; it < NIT; ++it)
           s[jt][it] = H16::mfma(kf[jt][ks], qf[it][ks], s[jt][it]);
 
     if constexpr (MODE == ATTN_BIAS) {
 #pragma unroll
-      for (int it = IT0; it < 2; ++it)
+      for (int it = 0; it < NIT; ++it)
 #pragma unroll
         for (int jt = 0; jt < 2; ++jt)
 #pragma unroll
@@ -317,69 +319,81 @@ __global__ void __launch_bounds__(64 * AttnWaves<MODE>::N, (AttnMinWaves<HS, MOD
               s[jt][it][8 * rh + e] = s[jt][it][8 * rh + e] * a.scale + bv;
             }
           }
-    } else {
-#pragma unroll
-      for (int jt = 0; jt < 2; ++jt)
-#pragma unroll
-        for (int it = IT0; it < 2; ++it)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            float x = s[jt][it][r] * a.scale;
-            if constexpr (MODE == ATTN_CAUSAL) {
-              const int j = 32 * jt + 8 * (r >> 2) + 4 * g + (r & 3);
-              const int i = 32 * it + lr;
-              if (j > i) x = -INFINITY;
-            }
-            s[jt][it][r] = x;
-          }
     }
   }
 
   // ---- softmax over keys (registers + lane^32) ------------------------------------------
-  float inv_l[2];
-#pragma unroll
-  for (int it = IT0; it < 2; ++it) {
+  // tc: the query tile, which the causal test wants as a constant: keys of a later tile than the queries' have no weight, those of an earlier one are all
+  // seen, and only in between is there anything to test. Every instance multiplies and subtracts in the same steps (a fused multiply-add where
+  // the scaled score is not changed in between), so that a row does not depend on the instance.
+  float inv_l[NIT];
+  auto softmax = [&](int it, auto tc) {
+    constexpr int TILE = decltype(tc)::value;
+    constexpr bool SCALED = MODE == ATTN_BIAS || MODE == ATTN_RELSHIFT;   // (the scores are finished)
+    constexpr int JT = MODE == ATTN_CAUSAL ? TILE + 1 : 2;
     float mx = -INFINITY;
 #pragma unroll
-    for (int jt = 0; jt < 2; ++jt)
+    for (int jt = 0; jt < JT; ++jt)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[jt][it][r]);
+      for (int r = 0; r < 16; ++r) {
+        float x = s[jt][it][r];
+        if constexpr (!SCALED) {
+          x *= a.scale;
+          if (MODE == ATTN_CAUSAL && jt == TILE) {
+            const int j = 8 * (r >> 2) + 4 * g + (r & 3);   // (within the tile)
+            if (j > lr) x = -INFINITY;
+            s[jt][it][r] = x;
+          }
+        }
+        mx = fmaxf(mx, x);
+      }
     mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
     float sum = 0.f;
 #pragma unroll
     for (int jt = 0; jt < 2; ++jt)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const float p = __expf(s[jt][it][r] - mx);
+        float p = 0.f;
+        if (jt < JT) p = __expf(SCALED || (MODE == ATTN_CAUSAL && jt == TILE) ? s[jt][it][r] - mx : fmaf(s[jt][it][r], a.scale, -mx));
         s[jt][it][r] = p;
         sum += p;
       }
     sum += __shfl_xor(sum, 32, 64);
     inv_l[it] = 1.0f / sum;
+  };
+  typedef std::integral_constant<int, 0> T0;
+  typedef std::integral_constant<int, 1> T1;
+  if constexpr (NIT == 2) {
+    softmax(0, T0{});
+    softmax(1, T1{});
+  } else if (it0 == 1 && MODE == ATTN_CAUSAL) {
+    softmax(0, T1{});
+  } else {
+    softmax(0, T0{});
   }
 
   // ---- O^T = V^T · P^T ------------------------------------------------------------------
-  if constexpr (VPAIR) {
+  if constexpr (VPAIR || SPLIT) {
     __syncthreads();   // (the other wave of the pair wrote half of this head's V^T)
   } else {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   }
-  f32x16_t o[DT_TILES][2];
+  f32x16_t o[DT_TILES][NIT];
 #pragma unroll
   for (int dt = 0; dt < DT_TILES; ++dt)
 #pragma unroll
-    for (int it = IT0; it < 2; ++it)
+    for (int it = 0; it < NIT; ++it)
 #pragma unroll
       for (int r = 0; r < 16; ++r) o[dt][it][r] = 0.f;
 
 #pragma unroll
   for (int kb = 0; kb < 4; ++kb) {
     const int jt = kb >> 1, kh = kb & 1;
-    hvec pf[2];
+    hvec pf[NIT];
 #pragma unroll
-    for (int it = IT0; it < 2; ++it)
+    for (int it = 0; it < NIT; ++it)
 #pragma unroll
       for (int e = 0; e < 8; ++e) pf[it][e] = (typename H16::elem)s[jt][it][8 * kh + e];
 #pragma unroll
@@ -390,15 +404,15 @@ __global__ void __launch_bounds__(64 * AttnWaves<MODE>::N, (AttnMinWaves<HS, MOD
       const uint4 packed = make_uint4(lo.x, lo.y, hi.x, hi.y);
       const hvec vf = __builtin_bit_cast(hvec, packed);
 #pragma unroll
-      for (int it = IT0; it < 2; ++it) o[dt][it] = H16::mfma(vf, pf[it], o[dt][it]);
+      for (int it = 0; it < NIT; ++it) o[dt][it] = H16::mfma(vf, pf[it], o[dt][it]);
     }
   }
 
   // ---- normalise and store ----------------------------------------------------------------
   float am = 0.f;
 #pragma unroll
-  for (int it = IT0; it < 2; ++it) {
-    const long row = LAST ? (long)b : (long)b * 64 + 32 * it + lr;
+  for (int it = 0; it < NIT; ++it) {
+    const long row = LAST ? (long)b : (long)b * 64 + 32 * (it0 + it) + lr;
     const bool keep_row = !LAST || lr == 31;
 #pragma unroll
     for (int dt = 0; dt < DT_TILES; ++dt)
@@ -688,6 +702,19 @@ template <int HS, int MODE, int IN_DT>
 static hipError_t launch_attn_dt(const AttnArgs& a, hipStream_t st) {
   constexpr int NW = AttnWaves<MODE>::N;
   const dim3 grid((a.B * a.H + NW - 1) / NW), block(64 * NW);
+  // Few units: two waves for each, one per query tile (bit-equal; the shift of the relative mode crosses the tiles). The wave's chain of loads, scores,
+  // softmax and output bounds a call that does not fill the chip, and this halves all of it but the loads: 15 layers of 32 heads of 32, one
+  // position 6.8 -> 4.2 us a launch, 8 positions 7.2 -> 4.5, 33 9.0 -> 7.9, 64 the same, 250 +10 %; 6 layers of 12 heads of 64, one position 6.9 -> 4.8 us,
+  // 16 7.2 -> 5.0, 32 -0.6 us, 64 +0.4, 256 +9. Beyond the lines the second reading of the keys costs more than the shorter chain gives.
+  if constexpr (MODE != ATTN_RELSHIFT) {
+    if (!a.last_row && 2L * a.B * a.H <= (HS == 32 ? 9L : 4L) * device_cus()) {
+      const dim3 units(a.B * a.H), two(128);
+      if (a.out_dtype == DT_FP8) hipLaunchKernelGGL((attention_kernel<HS, MODE, 1, IN_DT, 0, 0, 1>), units, two, 0, st, a);
+      else if (a.out_dtype == IN_DT) hipLaunchKernelGGL((attention_kernel<HS, MODE, 0, IN_DT, 0, 0, 1>), units, two, 0, st, a);
+      else return hipErrorInvalidValue;
+      return hipGetLastError();
+    }
+  }
   if constexpr (HS == 32 && (NW == 4 || NW == 8 || NW == 16)) {
     // Whole workgroups only: H a multiple of 4 puts four heads of one position in every workgroup and leaves none partly
     // filled; 16-byte stores need rows and base aligned to that.

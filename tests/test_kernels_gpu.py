@@ -573,6 +573,25 @@ def test_attention_whole_line_stores_equal_per_wave_stores(cuda, mode, dtype):
         assert whole.float().abs().max() > 0
 
 
+@pytest.mark.parametrize("mode", [_lib.ATTN_PLAIN, _lib.ATTN_CAUSAL, _lib.ATTN_BIAS])
+@pytest.mark.parametrize("hs,out_dt", [(32, None), (32, _lib.FP8), (64, None), (64, _lib.FP8)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_attention_of_few_units_equals_its_rows_of_many(cuda, mode, hs, out_dt, dtype):
+    """Few (position, head) units run on two waves each, one per query tile; many on one. Bit-equal, from one unit to the last count on
+    either side of the line (4.5 units a compute unit at head size 32, 2 at 64), with an odd number of heads too."""
+    cus = torch.cuda.get_device_properties(cuda).multi_processor_count
+    H = 5
+    line = (9 if hs == 32 else 4) * cus // 2 // H
+    B = line + 3
+    qkv, Cm = make_qkv(B, H, hs, cuda, 17 + mode, dtype)
+    bias = torch.randn(B, H, 4096, device=cuda).to(dtype) if mode == _lib.ATTN_BIAS else None
+    many = run_attn(qkv, B, H, hs, mode, 1 / math.sqrt(hs), bias=bias, out_dt=out_dt, out_scale=37.0)
+    assert many.float().abs().max() > 0
+    for few in (1, 2, line, line + 1):
+        got = run_attn(qkv[:few * 64].contiguous(), few, H, hs, mode, 1 / math.sqrt(hs), bias=None if bias is None else bias[:few].contiguous(), out_dt=out_dt, out_scale=37.0)
+        assert torch.equal(got, many[:few * 64]), (few, mode, hs, out_dt)
+
+
 def test_attention_relshift(cuda):
     from oracle.models import rel_shift
     B, H, hs = 4, 8, 64
