@@ -24,6 +24,7 @@ SOURCES = [
     "kernels/gemm_dmas.hip",
     "kernels/gemm_shortk.hip",
     "kernels/gemm_norm.hip",
+    "kernels/gemm_norm256.hip",
     "kernels/norm_embed.hip",
     "kernels/attention.hip",
     "kernels/heads.hip",

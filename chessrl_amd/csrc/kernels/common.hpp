@@ -172,6 +172,19 @@ struct NormGemmArgs {
   int M, N, K, nsplit, act, out_dtype, vec_ok;
   float descale, out_scale;
 };
+// Norm of 256-column rows and the product behind it, one launch (gemm_norm256_kernel.hpp).
+struct Norm256Args {
+  const void* x; long ldx; int x_dtype;        // [M, 256] bf16 or f16, also the output's type
+  int grouped;                                 // 0: every row its own norm, gamma and beta [256], out = swish(norm(X) · W^T + bias)
+                                               // 1: 32 rows (dense) are normalised together, [8192], out = descale * norm(X) · W^T
+  const float* gamma; const float* beta; float eps;
+  const void* W; int in_dtype; float x_scale;  // [N, 256] dense, of x's type or e4m3 (grouped only), for which the normalised values are multiplied by x_scale
+  const float* bias;                           // [N], row by row only
+  void* out; long ldo; int M, N;
+  float descale;
+};
+bool gemm_norm256_can(const Norm256Args& a);
+hipError_t launch_gemm_norm256(const Norm256Args& a, hipStream_t st);
 int device_cus();   // compute units of the current device (gemm.hip)
 int gemm_norm_width(int M, int N, int K, int in_dt, int cus);
 hipError_t launch_gemm_norm(NormGemmArgs a, int in_dt, int width, bool k_parallel, hipStream_t st);

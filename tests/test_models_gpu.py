@@ -208,6 +208,25 @@ def test_bt4class_batch_invariance(cuda, fp8):
     assert torch.equal(p3.cpu(), pol.cpu()[perm]) and torch.equal(w3.cpu(), wdl.cpu()[perm])
 
 
+@pytest.mark.parametrize("act,fp8", [("bf16", False), ("f16", False), ("bf16", True)])
+def test_bt4class_bias_generator_norms_inside_their_products(cuda, act, fp8):
+    """Full width, the only one whose second bias-generator norm (over a position's 32 rows of 256) runs inside the product behind it: on 32 rows and one
+    tile up to 2 and 4 positions, on 64 rows and slices of N beyond, as a launch of its own from one position per compute unit on; the first norm on 32 rows up
+    to 64 positions. Odd positions leave a row block half empty. Same bits on all of them."""
+    m = models.BT4Class(2, 1024, 1536, 32, fp8=fp8, act_dtype=act)
+    m.load_state_dict(om.test_init_(om.BT4ClassOracle(policy_leela, 2, 1024, 1536, 32), seed=6).state_dict())
+    cus = torch.cuda.get_device_properties(cuda).multi_processor_count
+    x = positions(cus + 47, seed=14, leela=True)[0].to(cuda)
+    if fp8:
+        m.calibrate(x[:128].contiguous())
+    pol, wdl = m(x)
+    assert pol.abs().max() > 0
+    for B in (1, 2, 3, 4, 5, 8, 31, 33, 64, 65, 96, 127, cus - 1, cus, cus + 1):
+        p2, w2 = m(x[47 - B % 47:47 - B % 47 + B].contiguous())
+        lo = 47 - B % 47
+        assert torch.equal(p2, pol[lo:lo + B]) and torch.equal(w2, wdl[lo:lo + B]), B
+
+
 def test_bt4class_fp8_residuals_normalised_on_ragged_persistent_tiles(cuda):
     """Full width in e4m3: 33, 65, 129 and 131 positions end inside a 128-row tile, the last two on workgroups that walk several
     tiles; 1025 end inside a 256-row one. The residual that is normalised in the epilogue has the same bits on all of them and alone."""
