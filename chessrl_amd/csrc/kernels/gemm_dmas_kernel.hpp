@@ -23,14 +23,16 @@ namespace crl {
 // BT = 64: eight stages of 16 KB, four computing waves of 32x32; BT = 32: sixteen stages of 8 KB, one. Eight loading waves either
 // way, which keep AHEAD slabs requested (at the CU's load rate a slab of 8 KB takes 128 cycles, and memory some 1000; twelve of them delay the first: GPT one position 217 -> 228 us), and one
 // wave that fetches what the epilogue needs.
-// KP > 1 (token steps, whose sums may be added in another order): KP computing waves per 32x32 take the slabs in turn.
+// KP > 1 (token steps, whose sums may be added in another order): KP computing waves per 32x32 take the slabs in turn, a round of KP slabs to a barrier and
+// three rounds requested ahead. With a barrier to each slab every wave waited for the one that had it: 128 rows, N = 768, K = 768 4.8 -> 4.1 us,
+// K = 3072 11.9 -> 9.4 (a token step of 128 sequences 311 -> 291).
 template <int BT, int KP_ = 1>
 struct DmasCfg {
   static_assert(BT == 64 || BT == 32, "two tile sizes");
   static_assert(KP_ == 1 || (BT == 32 && KP_ <= 4), "patches of the K groups lie in stages nothing is loaded into any more");
   static constexpr int BM = BT, BN = BT, WGM = BT / 32, WGN = BT / 32;
   static constexpr int KP = KP_, NCOMP = WGM * WGN * KP, NLOAD = 8, NT = 64 * (NCOMP + NLOAD + 1);
-  static constexpr int ROWB = 128, NSTAGE = 512 / BT, AHEAD = 6;
+  static constexpr int ROWB = 128, NSTAGE = 512 / BT, AHEAD = KP > 1 ? 3 * KP : 6;
   static constexpr int LOADS = 2 * BT / (8 * NLOAD);           // load instructions (8 rows each) of a wave per stage
   static constexpr int STAGE = BN * ROWB;                      // bytes of one operand's rows in one stage
   static constexpr int PART_BYTES = NSTAGE * STAGE;            // 64 KB: the weight rows of all stages, then the activation rows
@@ -43,6 +45,8 @@ struct DmasCfg {
   static __device__ __forceinline__ int patch_off(int nslab, int w) {
     return ((nslab + w * 4096 / STAGE) & (NSTAGE - 1)) * STAGE + w * 4096 % STAGE;
   }
+  static constexpr int PER = KP;   // slabs a barrier announces
+  static_assert(KP == 1 || 4 * KP <= NSTAGE, "a round in work, three requested");
   static_assert(AHEAD * LOADS < 64 && AHEAD + 2 <= NSTAGE, "the counted waits fit the counter; a stage is read before it is refilled");
   static_assert(LDS_BYTES <= 160 * 1024, "LDS of a CU");
 };
@@ -54,7 +58,8 @@ struct SmallArgs {
   int M, N, nslab, nsplit;
   int act, res_dtype, res_rows, vec_ok;
   float descale, alpha, out_scale;
-  int tiles_n; uint32_t m_tn;  // columns of tiles and the magic of dividing by them
+  int inner; uint32_t m_inner; // tiles along the direction that is walked first, and the magic of dividing by them
+  int by_cols;                 // 1: that direction is down a column of tiles
   int per_xcd;                 // workgroups per XCD
 };
 
@@ -204,14 +209,16 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_dmas_kernel(const SmallArgs s) {
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int nslab = s.nslab;
 
-  // Workgroup b runs on XCD b & 7, which owns a contiguous range of the row-major tile order.
+  // Workgroup b runs on XCD b & 7, which owns a contiguous range of the tile order (rows or columns first, see the launch).
   int pid = blockIdx.x;
   if (pid < (s.per_xcd << 3)) pid = (pid & 7) * s.per_xcd + (pid >> 3);
-  const int tile_m = dmaf_div(pid, s.m_tn), tile_n = pid - tile_m * s.tiles_n;
+  const int outer = dmaf_div(pid, s.m_inner), inner = pid - outer * s.inner;
+  const int tile_m = s.by_cols ? inner : outer, tile_n = s.by_cols ? outer : inner;
   const int m0 = tile_m * BM, n0 = tile_n * BN;
 
-  // Barrier i (0 .. nslab - 1) of the workgroup says that slab i has landed, barrier nslab that sums, residual and bias lie in LDS.
-  // Every wave passes all of them.
+  // Barrier i (0 .. nbar - 1) of the workgroup says that slab i (KP > 1: slabs KP i .. KP i + KP - 1) has landed, barrier nbar that sums, residual and bias
+  // lie in LDS. Every wave passes all of them.
+  const int nbar = (nslab + Cfg::PER - 1) / Cfg::PER;
   if (wave == Cfg::NCOMP + Cfg::NLOAD) {
     if (small_tile_full(s, n0, BN)) {
       if (s.bias) {
@@ -236,7 +243,7 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_dmas_kernel(const SmallArgs s) {
       }
     }
 #pragma unroll 1
-    for (int slab = 0; slab < nslab; ++slab) dmas_barrier();
+    for (int i = 0; i < nbar; ++i) dmas_barrier();
     wait_vmcnt<0>();
     dmas_barrier();
     return;
@@ -271,23 +278,48 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_dmas_kernel(const SmallArgs s) {
 #pragma unroll
     for (int s0 = 0; s0 < AHEAD; ++s0)
       if (s0 < nslab) issue_slab(s0);
-    int slab = 0;
+    if constexpr (Cfg::KP > 1) {
+      constexpr int KP = Cfg::KP;
+      int r = 0;
 #pragma unroll 1
-    for (; slab + AHEAD < nslab; ++slab) {
-      wait_vmcnt<(AHEAD - 1) * LOADS>();
-      dmas_barrier();
-      // (stage slab + AHEAD - NSTAGE <= slab - 2, whose fragments the computing waves had in registers before they came here)
-      issue_slab(slab + AHEAD);
-    }
-    // The last AHEAD slabs, or all there are: nothing is issued any more, so each wait leaves one slab less in flight.
-    static_for<0, AHEAD>([&](auto ic) {
-      constexpr int left = AHEAD - decltype(ic)::value;   // slabs still to be announced
-      if (nslab - slab >= left) {
-        wait_vmcnt<(left - 1) * LOADS>();
+      for (; r + 3 < nbar; ++r) {
+        wait_vmcnt<2 * KP * LOADS>();
         dmas_barrier();
-        ++slab;
+        // (into the stages of round r - 1, which the computing waves had in registers before they came here)
+#pragma unroll
+        for (int i = 0; i < KP; ++i)
+          if ((r + 3) * KP + i < nslab) issue_slab((r + 3) * KP + i);
       }
-    });
+      // The last three rounds, or all there are; where the last one is short its slabs are waited for with the round before.
+      const bool full = nslab % KP == 0;
+      static_for<0, 3>([&](auto ic) {
+        constexpr int left = 3 - decltype(ic)::value;
+        if (nbar - r >= left) {
+          if (full) wait_vmcnt<(left - 1) * KP * LOADS>();
+          else wait_vmcnt<(left > 2 ? left - 2 : 0) * KP * LOADS>();
+          dmas_barrier();
+          ++r;
+        }
+      });
+    } else {
+      int slab = 0;
+#pragma unroll 1
+      for (; slab + AHEAD < nslab; ++slab) {
+        wait_vmcnt<(AHEAD - 1) * LOADS>();
+        dmas_barrier();
+        // (stage slab + AHEAD - NSTAGE <= slab - 2, whose fragments the computing waves had in registers before they came here)
+        issue_slab(slab + AHEAD);
+      }
+      // The last AHEAD slabs, or all there are: nothing is issued any more, so each wait leaves one slab less in flight.
+      static_for<0, AHEAD>([&](auto ic) {
+        constexpr int left = AHEAD - decltype(ic)::value;   // slabs still to be announced
+        if (nslab - slab >= left) {
+          wait_vmcnt<(left - 1) * LOADS>();
+          dmas_barrier();
+          ++slab;
+        }
+      });
+    }
     dmas_barrier();
     // This thread's part of the epilogue: row er, columns ec .. ec + EV - 1 of the tile.
     constexpr int TPR = BN / EV;   // threads per row
@@ -319,7 +351,7 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_dmas_kernel(const SmallArgs s) {
 
   const int wm = wave % Cfg::WGM, wn = wave / Cfg::WGM % Cfg::WGN;
   if (m0 + wm * 32 >= s.M || n0 + wn * 32 >= s.N) {
-    for (int slab = 0; slab <= nslab; ++slab) dmas_barrier();
+    for (int i = 0; i <= nbar; ++i) dmas_barrier();
     return;
   }
   // Fragment addresses, as in gemm_dmaf_kernel.hpp: chunk Kc ^ L with L = (2g or g) ^ swizzle(row) per lane and a
@@ -357,12 +389,12 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_dmas_kernel(const SmallArgs s) {
     static_for<0, KSTEPS>([&](auto ksc) { constexpr int ks = decltype(ksc)::value; acc = mfma_frag<IN_DT>(cur.w[ks], cur.x[ks], acc); });
   };
   if constexpr (Cfg::KP > 1) {
-    // This wave's slabs are kp, kp + KP, ...: read from LDS and multiplied when they have landed.
+    // This wave's slabs are kp, kp + KP, ...: one of every round.
     const int kp = wave / (Cfg::WGM * Cfg::WGN);
 #pragma unroll 1
-    for (int slab = 0; slab < nslab; ++slab) {
+    for (int slab = kp, i = 0; i < nbar; ++i, slab += Cfg::KP) {
       dmas_barrier();
-      if (slab % Cfg::KP != kp) continue;
+      if (slab >= nslab) continue;
       static_for<0, KSTEPS>([&](auto ksc) { read_step((slab & (NSTAGE - 1)) * STAGE, f0, ksc); });
       last_step(f0);
     }
@@ -425,7 +457,14 @@ static hipError_t launch_dmas(const GemmArgs& a, hipStream_t st) {
   s.M = a.M; s.N = a.N; s.nslab = a.K * ESZ / Cfg::ROWB; s.nsplit = a.nsplit;
   s.act = a.act; s.res_dtype = a.res_dtype; s.res_rows = a.res_rows; s.vec_ok = a.vec_ok;
   s.descale = a.descale; s.alpha = a.alpha; s.out_scale = a.out_scale;
-  s.tiles_n = tiles_n; s.m_tn = dmaf_magic(tiles_n); s.per_xcd = tiles >> 3;
+  // Rows or columns of tiles first, whichever lets an XCD read fewer rows of both operands: each XCD's L2 fetches its own copy (BT4-class bf16, whole calls
+  // of 2, 4 and 8 positions: 850 -> 835, 912 -> 868, 1083 -> 1065 us). Two rows of tiles gain nothing, and the K-shared form of 128 rows, 768
+  // columns, K = 3072 loses 0.5 us a launch: rows first there.
+  const int tiles_m = tiles / tiles_n, per = std::max(tiles >> 3, 1);
+  const int by_rows = (per + tiles_n - 1) / tiles_n + std::min(per, tiles_n), by_cols = (per + tiles_m - 1) / tiles_m + std::min(per, tiles_m);
+  s.by_cols = Cfg::KP == 1 && tiles_m >= 4 && by_cols < by_rows;
+  s.inner = s.by_cols ? tiles_m : tiles_n;
+  s.m_inner = dmaf_magic(s.inner); s.per_xcd = tiles >> 3;
   hipLaunchKernelGGL(kern, dim3(tiles), dim3(Cfg::NT), Cfg::LDS_BYTES, st, s);
   return hipGetLastError();
 }
