@@ -158,6 +158,8 @@ struct GemmArgs {
   // 1: C (ldc == N) is written in contiguous blocks of 256 rows x 128 columns, block (m / 256, n / 128) at index
   // (m / 256) * (N / 128) + n / 128, instead of row-major (only where gemm_shortk_can says so).
   int c_blocked;
+  // 1: the weights are read with the non-temporal hint: they will not be met in the memory-side cache again (Model::mark_streamed; gemm_dmas_kernel.hpp alone heeds it).
+  int w_once;
 };
 
 // LayerNorm (or RMSNorm) of X's rows and the product with W behind it, one launch (gemm_norm_kernel.hpp).

@@ -86,6 +86,9 @@ __device__ __forceinline__ void dmaf_barrier() { asm volatile("s_barrier" ::: "m
 __device__ __forceinline__ void dmaf_load16(__amdgpu_buffer_rsrc_t r, uint8_t* dst, int voff, int soff) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, voff, soff, 0, 0);
 }
+__device__ __forceinline__ void dmaf_load16_nt(__amdgpu_buffer_rsrc_t r, uint8_t* dst, int voff, int soff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, voff, soff, 0, 2);
+}
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t dmaf_rsrc(const void* base, long span) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)(span < 0x7fffffffL ? span : 0x7fffffffL), 0x00020000);
 }

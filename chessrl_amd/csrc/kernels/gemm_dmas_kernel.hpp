@@ -64,10 +64,6 @@ struct SmallArgs {
 };
 
 __device__ __forceinline__ void dmas_barrier() { asm volatile("s_barrier" ::: "memory"); }
-// (a function of its own, like dmaf_load16: inside a kernel template this builtin makes the host pass drop the kernel's stub)
-__device__ __forceinline__ void dmas_load16(__amdgpu_buffer_rsrc_t r, uint8_t* dst, int voff, int soff) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, voff, soff, 0, 0);
-}
 
 // The epilogue of one thread: EV consecutive columns of one row, arithmetic as in gemm_epilogue. small_full: the tile's columns
 // lie inside C and on one side of the column split, with aligned rows (uniform): vector accesses, residual and bias from LDS.
@@ -197,7 +193,8 @@ __device__ __forceinline__ void small_full(const SmallArgs& s, const float (&acc
   }
 }
 
-template <typename Cfg, int IN_DT, int OUT_DT>
+// ONCE: GemmArgs::w_once (an instance of its own: a branch at every load cost a call of one position 2 %)
+template <typename Cfg, int IN_DT, int OUT_DT, int ONCE = 0>
 __global__ void __launch_bounds__(Cfg::NT) gemm_dmas_kernel(const SmallArgs s) {
   constexpr int KSTEPS = Cfg::ROWB / (IN_DT == DT_FP8 ? 64 : 32);   // MFMA K steps per slab
   constexpr int BM = Cfg::BM, BN = Cfg::BN, LOADS = Cfg::LOADS, NSTAGE = Cfg::NSTAGE, AHEAD = Cfg::AHEAD, EV = Cfg::EV;
@@ -272,7 +269,8 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_dmas_kernel(const SmallArgs s) {
       uint8_t* dst = smem + lds_load0 + (slab & (NSTAGE - 1)) * STAGE;
       static_for<0, LOADS>([&](auto ic) {
         constexpr int i = decltype(ic)::value;
-        dmas_load16(rsrc_mine, dst + i * 1024, (int)voff[i], slab * Cfg::ROWB);
+        if (ONCE && !loads_a) dmaf_load16_nt(rsrc_mine, dst + i * 1024, (int)voff[i], slab * Cfg::ROWB);
+        else dmaf_load16(rsrc_mine, dst + i * 1024, (int)voff[i], slab * Cfg::ROWB);
       });
     };
 #pragma unroll
@@ -433,8 +431,12 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_dmas_kernel(const SmallArgs s) {
   dmas_barrier();
 }
 
-template <typename Cfg, int IN_DT, int OUT_DT>
+template <typename Cfg, int IN_DT, int OUT_DT, int ONCE = 0>
 static hipError_t launch_dmas(const GemmArgs& a, hipStream_t st) {
+  if constexpr (Cfg::KP == 1 && !ONCE) {
+    // (up to 512 rows: the weight rows that more tiles share do better kept in L2; 8 positions 1062 -> 1013 us, 12 the same, 16 1222 -> 1262)
+    if (a.w_once && a.M <= 512) return launch_dmas<Cfg, IN_DT, OUT_DT, 1>(a, st);
+  }
   static std::atomic<bool> attr_set[16] = {};
   constexpr int ESZ = IN_DT == DT_FP8 ? 1 : 2;
   auto fits = [](long v) { return v >= 0 && v < (1L << 31); };
@@ -442,7 +444,7 @@ static hipError_t launch_dmas(const GemmArgs& a, hipStream_t st) {
     return hipErrorInvalidValue;
   int dev = 0;
   (void)hipGetDevice(&dev);
-  auto kern = gemm_dmas_kernel<Cfg, IN_DT, OUT_DT>;
+  auto kern = gemm_dmas_kernel<Cfg, IN_DT, OUT_DT, ONCE>;
   if (dev < 0 || dev >= 16 || !attr_set[dev]) {
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::LDS_BYTES);
     if (e != hipSuccess) return e;

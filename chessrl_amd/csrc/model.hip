@@ -193,6 +193,24 @@ int Model::make_ffn(Layer& ly, const std::vector<float>& w1, const std::vector<f
   return make_lin(ly.ff2, pad_to(w2, C, F, C, FP), &b2, C, FP, ad, cfg.fp8 != 0);
 }
 
+// Weights that a pass reads beyond what the 256 MB memory-side cache keeps from one pass to the next. Read in turn, 311 MB of them (BT4-class, bf16) never
+// meet themselves there again: every line is gone by the time it is asked for. The layers that go beyond the share below are read with the non-temporal
+// hint, which leaves the others where they are. One bf16 position of the 15 x 1024 model, layers kept: all 789 us, 11 759, 9 (208 MB with what is
+// not a layer's) 737, 7 749, 5 763, none 795; with the share below 792 -> 740, 4 positions 867 -> 827, 8 1062 -> 1013. Larger batches replace the
+// cache's contents themselves, and the kernels of their products share weight rows between many tiles.
+void Model::mark_streamed() {
+  constexpr size_t KEEP = 200u << 20;
+  auto bytes = [](const Lin& l) -> size_t { return (size_t)l.N * l.K * (l.w8 ? 1 : dtype_size(l.dt)); };
+  auto each = [](Layer& y, auto f) { for (Lin* l : {&y.qkv, &y.proj, &y.ff1, &y.ff2, &y.sm_hidden}) f(*l); };
+  size_t sum = 0;
+  for (const Lin* l : {&lm_head, &pol_tok, &pol_qk, &pol_head, &val1, &val2, &val3, &sm_weight_gen}) sum += bytes(*l);
+  for (Layer& y : layers) sum += bytes(y.sm_gen);   // (their kernel has no such reads)
+  for (Layer& y : layers) {
+    each(y, [&](Lin& l) { sum += bytes(l); });
+    if (sum > KEEP) each(y, [](Lin& l) { l.once = true; });
+  }
+}
+
 int Model::finalize() {
   for (auto& e : expected)
     if (!host.count(e.first)) { set_error("finalize: missing weight " + e.first); return CRL_ERR_STATE; }
@@ -353,6 +371,7 @@ int Model::finalize() {
   HIPCHK(hipMemset(amax_dev, 0, sizeof(float) * amax_host.size()));
 #undef UP
 #undef LIN
+  mark_streamed();
   finalized = true;
   return CRL_OK;
 }
@@ -469,6 +488,7 @@ int Model::gemm(const Lin& L, const void* A, long lda, int in_dt, void* C, long 
   // Few rows: K spread over more waves (another summation order; the token steps of generation always, the forward pass
   // only where the model was told that a position's bits may depend on the batch it travels in).
   g.k_parallel = o.k_parallel ? 1 : 0;
+  g.w_once = L.once ? 1 : 0;
   g.splitk_ws = ws.splitk; g.splitk_ws_bytes = Workspace::SPLITK_BYTES;
   if (o.ln_out) {
     g.nsplit = g.N;

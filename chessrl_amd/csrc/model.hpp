@@ -21,6 +21,7 @@ struct Lin {
   void* w8 = nullptr;
   float* b = nullptr;
   int N = 0, K = 0, dt = DT_BF16;
+  bool once = false;          // GemmArgs::w_once
   int pad_N = 0, pad_K = 0;   // of which rows and columns of zeros (Model::ff_cols), left out of the profile's operation counts
   float wscale = 1.f;
   // Output rows [first, first + count) of this layer, as a layer of its own on the same memory.
@@ -165,6 +166,7 @@ struct Model {
   int norm_gemm(const void* x, long ldx, const float* g, const float* b, const Lin& L, int in_dt, void* C, long ldc, int out_dt, int M, const GOpt& o, hipStream_t st);
   // One of the bias generator's norms (grouped: over a position's 32 rows of 256) and the product behind it in one launch.
   int norm256(const void* x, long ldx, int grouped, const float* g, const float* b, const Lin& L, int in_dt, float x_scale, void* C, long ldc, int M, hipStream_t st);
+  void mark_streamed();
   int finish_last_layer(hipStream_t st);
   float act_scale(int layer, int slot) const;
   void prof_begin(int fam, hipStream_t st);
