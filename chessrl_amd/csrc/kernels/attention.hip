@@ -22,7 +22,7 @@ namespace crl {
 constexpr int VT_STRIDE = 68;   // bf16 elements per V^T row (64 keys + 4 padding: rows 8 apart land 16 banks apart, so the transposing
                                 // 8-byte writes and the fragment reads of a wave touch every bank twice, the minimum; with 72 it was eight and four times)
 constexpr int SP_STRIDE = 66;   // floats per row of the positional score patch: the shifted read-back of a wave walks it in steps of one less, an odd number
-                                // (with 65 all 32 rows of a read lay in one bank: 71 us per layer of 496 positions of 8 heads, 49 us now)
+                                // (with 65 all 32 rows of a read lay in one bank: 71 us per layer of 496 positions of 8 heads, 49 with the other)
 
 // Storage order of a 64x64 bias tile so that each lane reads its accumulator
 // registers as 16-byte vectors: element (query i, key j) lives at
@@ -56,6 +56,13 @@ struct Half16<DT_F16> {
   static __device__ __forceinline__ uint32_t pack2(float lo, float hi) { return (uint32_t)f32_to_f16_bits(lo) | ((uint32_t)f32_to_f16_bits(hi) << 16); }
 };
 
+// This wave's LDS writes are done and seen by its later reads.
+__device__ __forceinline__ void wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 template <typename H>
 __device__ __forceinline__ typename H::vec add_bias_h(typename H::vec q, const float* bias8) {
   typename H::vec r;
@@ -64,13 +71,12 @@ __device__ __forceinline__ typename H::vec add_bias_h(typename H::vec q, const f
   return r;
 }
 
-// Waves per workgroup: the relative-shift mode needs a 16.6 KB score patch per wave,
-// so it runs two waves per workgroup to stay inside 64 KB of static LDS. With a generated bias a workgroup takes eight
+// Waves per workgroup (of the form with one wave per unit). With a generated bias a workgroup takes eight
 // heads of a position (eight waves): per token row it then reads 512 contiguous bytes of each of q, k and v, its bias is
 // 2 KB pieces of the blocked layout and its e4m3 output rows are two whole lines (measured 9.07 -> 8.53 ms per
 // 4096-position forward against four waves; sixteen waves, one workgroup per CU, 9.71 ms).
 template <int MODE>
-struct AttnWaves { static constexpr int N = MODE == ATTN_RELSHIFT ? 2 : MODE == ATTN_BIAS ? 8 : 4; };
+struct AttnWaves { static constexpr int N = MODE == ATTN_BIAS ? 8 : 4; };
 
 // Waves per SIMD the register allocation is held to (0: the compiler's own choice). The kernel is a chain of load,
 // compute and store phases, so resident waves are what hides its memory latency: at head size 32 with a generated
@@ -99,13 +105,15 @@ __global__ void __launch_bounds__(SPLIT ? 128 : 64 * AttnWaves<MODE>::N, (SPLIT 
   constexpr int DT_TILES = HS / 32;
   constexpr int NW = SPLIT ? 1 : AttnWaves<MODE>::N;   // units of the workgroup
   __shared__ __align__(16) uint16_t s_vt[NW][HS * VT_STRIDE];
-  __shared__ float s_sp[MODE == ATTN_RELSHIFT ? NW : 1][MODE == ATTN_RELSHIFT ? 64 * SP_STRIDE : 1];
+  __shared__ float s_sp[MODE == ATTN_RELSHIFT ? 64 * SP_STRIDE : 1];
+  __shared__ __align__(16) float s_uv[MODE == ATTN_RELSHIFT ? 2 : 1][MODE == ATTN_RELSHIFT ? 2 * HS : 1];
   // Output tile of the workgroup's NW heads (head size 32): 64 rows of NW * HS elements, 16 bytes of padding
   // per row. A wave's own output is 64 row pieces of 32 (e4m3) or 64 bytes, which it would have to store 16 bytes per
   // lane and row, a quarter or an eighth of a line at a time; gathered here, the workgroup stores whole lines (measured
   // on 4096 positions x 32 heads in e4m3: the stores were 9 % of the kernel's bytes and 21 % of its time).
   static_assert(!LAST || (MODE == ATTN_CAUSAL && !COOP), "one-row form");
-  static_assert(!SPLIT || (MODE != ATTN_RELSHIFT && !COOP && !LAST), "one query tile per wave");
+  static_assert(!SPLIT || (!COOP && !LAST), "one query tile per wave");
+  static_assert(SPLIT || MODE != ATTN_RELSHIFT, "the relative mode has one form");
   constexpr int NIT = LAST || SPLIT ? 1 : 2;   // query tiles of a wave
   static_assert(!COOP || (HS == 32 && (NW == 4 || NW == 8 || NW == 16)), "the output tile is laid out for head size 32");
   constexpr int OSZ = OUT_FP8 ? 1 : 2;
@@ -137,6 +145,35 @@ __global__ void __launch_bounds__(SPLIT ? 128 : 64 * AttnWaves<MODE>::N, (SPLIT 
 
   // ---- V -> V^T in LDS ------------------------------------------------------------
   uint16_t* vt = s_vt[SPLIT ? 0 : wave];
+  // V rows of this wave (SPLIT: half of the unit's each; with a single pass half the lanes of each wave), four of one 16-byte chunk a lane and pass.
+  constexpr int DC = HS / 8;            // 16-byte chunks per V row
+  constexpr int PASSES = (16 * DC) / 64, MYP = SPLIT && PASSES > 1 ? PASSES / 2 : PASSES;
+  i32x4_t vrow4[MYP][4];
+  const bool v_mine = !(SPLIT && PASSES == 1 && g);
+  auto v_id = [&](int p) { return SPLIT ? (PASSES == 1 ? 32 * wave + lr : (wave * MYP + p) * 64 + lane) : p * 64 + lane; };
+  auto v_load = [&]() {
+#pragma unroll
+    for (int p = 0; p < MYP; ++p)
+      if (v_mine) {
+        const int id = v_id(p), jq = id / DC, dc = id - jq * DC;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) vrow4[p][t] = *reinterpret_cast<const i32x4_t*>(vp + (long)(4 * jq + t) * a.ldv + 8 * dc);
+      }
+  };
+  auto v_write = [&]() {
+#pragma unroll
+    for (int p = 0; p < MYP; ++p)
+      if (v_mine) {
+        const int id = v_id(p), jq = id / DC, dc = id - jq * DC;
+#pragma unroll
+        for (int e2 = 0; e2 < 4; ++e2) {
+          // d = 8dc + 2e2 (low halves) and d+1 (high halves)
+          const uint32_t w0 = (uint32_t)vrow4[p][0][e2], w1 = (uint32_t)vrow4[p][1][e2], w2 = (uint32_t)vrow4[p][2][e2], w3 = (uint32_t)vrow4[p][3][e2];
+          *reinterpret_cast<uint2*>(vt + (8 * dc + 2 * e2) * VT_STRIDE + 4 * jq) = make_uint2((w0 & 0xffffu) | (w1 << 16), (w2 & 0xffffu) | (w3 << 16));
+          *reinterpret_cast<uint2*>(vt + (8 * dc + 2 * e2 + 1) * VT_STRIDE + 4 * jq) = make_uint2((w0 >> 16) | (w1 & 0xffff0000u), (w2 >> 16) | (w3 & 0xffff0000u));
+        }
+      }
+  };
   // VPAIR: the two waves of a pair of neighbouring heads (a token's V rows of the two are one whole 128-byte line) take
   // half the tokens each, for both heads: every line is read by one wave, once, with the non-temporal hint, and lands
   // transposed in the patch of the head it belongs to; the workgroup meets at a barrier before the second product.
@@ -161,31 +198,9 @@ __global__ void __launch_bounds__(SPLIT ? 128 : 64 * AttnWaves<MODE>::N, (SPLIT 
       *reinterpret_cast<uint2*>(vt2 + (8 * dc + 2 * e2) * VT_STRIDE + 4 * jq) = lo;
       *reinterpret_cast<uint2*>(vt2 + (8 * dc + 2 * e2 + 1) * VT_STRIDE + 4 * jq) = hi;
     }
-  } else {
-    constexpr int DC = HS / 8;            // 16-byte chunks per V row
-    constexpr int PASSES = (16 * DC) / 64;
-#pragma unroll
-    for (int p = 0; p < (SPLIT && PASSES > 1 ? PASSES / 2 : PASSES); ++p) {
-      // (SPLIT: half of the rows each; with a single pass half the lanes of each wave)
-      if (SPLIT && PASSES == 1 && g) break;
-      const int id = SPLIT ? (PASSES == 1 ? 32 * wave + lr : (wave * (PASSES / 2) + p) * 64 + lane) : p * 64 + lane;
-      const int jq = id / DC, dc = id - jq * DC;
-      uint4 rows[4];
-#pragma unroll
-      for (int t = 0; t < 4; ++t) rows[t] = *reinterpret_cast<const uint4*>(vp + (long)(4 * jq + t) * a.ldv + 8 * dc);
-      const uint32_t* w0 = reinterpret_cast<const uint32_t*>(&rows[0]);
-      const uint32_t* w1 = reinterpret_cast<const uint32_t*>(&rows[1]);
-      const uint32_t* w2 = reinterpret_cast<const uint32_t*>(&rows[2]);
-      const uint32_t* w3 = reinterpret_cast<const uint32_t*>(&rows[3]);
-#pragma unroll
-      for (int e2 = 0; e2 < 4; ++e2) {
-        // d = 8dc + 2e2 (low halves) and d+1 (high halves)
-        uint2 lo = make_uint2((w0[e2] & 0xffffu) | (w1[e2] << 16), (w2[e2] & 0xffffu) | (w3[e2] << 16));
-        uint2 hi = make_uint2((w0[e2] >> 16) | (w1[e2] & 0xffff0000u), (w2[e2] >> 16) | (w3[e2] & 0xffff0000u));
-        *reinterpret_cast<uint2*>(vt + (8 * dc + 2 * e2) * VT_STRIDE + 4 * jq) = lo;
-        *reinterpret_cast<uint2*>(vt + (8 * dc + 2 * e2 + 1) * VT_STRIDE + 4 * jq) = hi;
-      }
-    }
+  } else if constexpr (MODE != ATTN_RELSHIFT) {
+    v_load();
+    v_write();
   }
 
   // ---- scores -----------------------------------------------------------------------
@@ -235,66 +250,67 @@ __global__ void __launch_bounds__(SPLIT ? 128 : 64 * AttnWaves<MODE>::N, (SPLIT 
       for (int r = 0; r < 16; ++r) s[jt][it][r] = 0.f;
 
   if constexpr (MODE == ATTN_RELSHIFT) {
-    // content = (q+u)·k, position = (q+v)·p, both with the bias folded into the query.
+    // content = (q+u)·k, position = (q+v)·p, both with the bias folded into the query. Everything the wave reads is requested up front (left alone, the
+    // compiler asks for the positional table and the biases step by step, a memory round trip each), V last, which is wanted last. With the shift's
+    // reads in one go too, and a wave per query tile, a layer of 496 positions of 8 heads takes 41 us instead of 51 and one of 1488 126 instead of 150 (bytes:
+    // 26 and 77 us); held to three waves per SIMD (158 registers instead of 192) the same.
     const uint16_t* pp = reinterpret_cast<const uint16_t*>(a.pos) + h * HS;
     const long ldp = (long)a.H * HS;
-    f32x16_t sp[2][NIT];
+    hvec pf[2][KS];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) pf[t][ks] = *reinterpret_cast<const hvec*>(pp + (long)(32 * t + lr) * ldp + 16 * ks + 8 * g);
+    const float ul = a.u_bias[h * HS + lane % HS], vl = a.v_bias[h * HS + lane % HS];
+    v_load();
+    __builtin_amdgcn_sched_barrier(0);
+    float* const uv = s_uv[wave];   // u, then v (a wave's own copy)
+    if (lane < HS) { uv[lane] = ul; uv[HS + lane] = vl; }
+    wave_fence();
+    f32x16_t sp[2];
 #pragma unroll
     for (int jt = 0; jt < 2; ++jt)
 #pragma unroll
-      for (int it = 0; it < NIT; ++it)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) sp[jt][it][r] = 0.f;
+      for (int r = 0; r < 16; ++r) sp[jt][r] = 0.f;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       float ub[8], vb[8];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        ub[e] = a.u_bias[h * HS + 16 * ks + 8 * g + e];
-        vb[e] = a.v_bias[h * HS + 16 * ks + 8 * g + e];
-      }
-      hvec pf[2];
+      for (int e = 0; e < 8; ++e) { ub[e] = uv[16 * ks + 8 * g + e]; vb[e] = uv[HS + 16 * ks + 8 * g + e]; }
+      const hvec qu = add_bias_h<H16>(qf[0][ks], ub);
+      const hvec qv = add_bias_h<H16>(qf[0][ks], vb);
 #pragma unroll
-      for (int t = 0; t < 2; ++t) pf[t] = *reinterpret_cast<const hvec*>(pp + (long)(32 * t + lr) * ldp + 16 * ks + 8 * g);
-#pragma unroll
-      for (int it = 0; it < NIT; ++it) {
-        const hvec qu = add_bias_h<H16>(qf[it][ks], ub);
-        const hvec qv = add_bias_h<H16>(qf[it][ks], vb);
-#pragma unroll
-        for (int jt = 0; jt < 2; ++jt) {
-          s[jt][it] = H16::mfma(kf[jt][ks], qu, s[jt][it]);
-          sp[jt][it] = H16::mfma(pf[jt], qv, sp[jt][it]);
-        }
+      for (int jt = 0; jt < 2; ++jt) {
+        s[jt][0] = H16::mfma(kf[jt][ks], qu, s[jt][0]);
+        sp[jt] = H16::mfma(pf[jt][ks], qv, sp[jt]);
       }
     }
+    v_write();
     // Shifted read-back (new_paradigm/attn.py:525-533): with T=64,
     //   out[i][j] = P[i][63-i+j] (j<=i), 0 (j==i+1), P[i+1][j-i-2] (j>i+1).
-    float* spm = s_sp[wave];
+    const int i = 32 * it0 + lr;
 #pragma unroll
     for (int jt = 0; jt < 2; ++jt)
 #pragma unroll
-      for (int it = 0; it < NIT; ++it)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int m = 32 * jt + 8 * (r >> 2) + 4 * g + (r & 3);
-          spm[(32 * it + lr) * SP_STRIDE + m] = sp[jt][it][r];
-        }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      for (int r = 0; r < 16; ++r) s_sp[i * SP_STRIDE + 32 * jt + 8 * (r >> 2) + 4 * g + (r & 3)] = sp[jt][r];
+    __syncthreads();   // (row 32 of the shift is the other wave's, as is half of V^T)
+    // (both cases at one address but for a constant; the element between them is zero; all reads ahead of their use)
+    const float* const back = s_sp + i * (SP_STRIDE - 1) + 63 + 4 * g;
 #pragma unroll
     for (int jt = 0; jt < 2; ++jt)
 #pragma unroll
-      for (int it = 0; it < NIT; ++it)
+      for (int r = 0; r < 16; ++r) {
+        const int j0 = 32 * jt + 8 * (r >> 2) + (r & 3);
+        sp[jt][r] = back[j0 + (j0 + 4 * g > i ? SP_STRIDE - 65 : 0)];
+      }
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int j = 32 * jt + 8 * (r >> 2) + 4 * g + (r & 3);
-          const int i = 32 * it + lr;
-          // (both cases at one address but for a constant; the element between them is zero)
-          const float at = spm[i * (SP_STRIDE - 1) + 63 + j + (j > i ? SP_STRIDE - 65 : 0)];
-          const float pv = j == i + 1 ? 0.f : at;
-          s[jt][it][r] = (s[jt][it][r] + pv) * a.scale;
-        }
+    for (int jt = 0; jt < 2; ++jt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const float pv = 32 * jt + 8 * (r >> 2) + 4 * g + (r & 3) == i + 1 ? 0.f : sp[jt][r];
+        s[jt][0][r] = (s[jt][0][r] + pv) * a.scale;
+      }
   } else {
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks)
@@ -373,7 +389,7 @@ __global__ void __launch_bounds__(SPLIT ? 128 : 64 * AttnWaves<MODE>::N, (SPLIT 
   }
 
   // ---- O^T = V^T · P^T ------------------------------------------------------------------
-  if constexpr (VPAIR || SPLIT) {
+  if constexpr (VPAIR || (SPLIT && MODE != ATTN_RELSHIFT)) {
     __syncthreads();   // (the other wave of the pair wrote half of this head's V^T)
   } else {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -706,16 +722,15 @@ static hipError_t launch_attn_dt(const AttnArgs& a, hipStream_t st) {
   // softmax and output bounds a call that does not fill the chip, and this halves all of it but the loads: 15 layers of 32 heads of 32, one
   // position 6.8 -> 4.2 us a launch, 8 positions 7.2 -> 4.5, 33 9.0 -> 7.9, 64 the same, 250 +10 %; 6 layers of 12 heads of 64, one position 6.9 -> 4.8 us,
   // 16 7.2 -> 5.0, 32 -0.6 us, 64 +0.4, 256 +9. Beyond the lines the second reading of the keys costs more than the shorter chain gives.
-  if constexpr (MODE != ATTN_RELSHIFT) {
-    if (!a.last_row && 2L * a.B * a.H <= (HS == 32 ? 9L : 4L) * device_cus()) {
-      const dim3 units(a.B * a.H), two(128);
-      if (a.out_dtype == DT_FP8) hipLaunchKernelGGL((attention_kernel<HS, MODE, 1, IN_DT, 0, 0, 1>), units, two, 0, st, a);
-      else if (a.out_dtype == IN_DT) hipLaunchKernelGGL((attention_kernel<HS, MODE, 0, IN_DT, 0, 0, 1>), units, two, 0, st, a);
-      else return hipErrorInvalidValue;
-      return hipGetLastError();
-    }
+  // The relative mode has no other form.
+  if (MODE == ATTN_RELSHIFT || (!a.last_row && 2L * a.B * a.H <= (HS == 32 ? 9L : 4L) * device_cus())) {
+    const dim3 units(a.B * a.H), two(128);
+    if (a.out_dtype == DT_FP8) hipLaunchKernelGGL((attention_kernel<HS, MODE, 1, IN_DT, 0, 0, 1>), units, two, 0, st, a);
+    else if (a.out_dtype == IN_DT) hipLaunchKernelGGL((attention_kernel<HS, MODE, 0, IN_DT, 0, 0, 1>), units, two, 0, st, a);
+    else return hipErrorInvalidValue;
+    return hipGetLastError();
   }
-  if constexpr (HS == 32 && (NW == 4 || NW == 8 || NW == 16)) {
+  if constexpr (HS == 32 && MODE != ATTN_RELSHIFT && (NW == 4 || NW == 8 || NW == 16)) {
     // Whole workgroups only: H a multiple of 4 puts four heads of one position in every workgroup and leaves none partly
     // filled; 16-byte stores need rows and base aligned to that.
     const int osz = a.out_dtype == DT_FP8 ? 1 : 2;
@@ -734,9 +749,11 @@ static hipError_t launch_attn_dt(const AttnArgs& a, hipStream_t st) {
       return hipGetLastError();
     }
   }
-  if (a.out_dtype == DT_FP8) hipLaunchKernelGGL((attention_kernel<HS, MODE, 1, IN_DT>), grid, block, 0, st, a);
-  else if (a.out_dtype == IN_DT) hipLaunchKernelGGL((attention_kernel<HS, MODE, 0, IN_DT>), grid, block, 0, st, a);
-  else return hipErrorInvalidValue;
+  if constexpr (MODE != ATTN_RELSHIFT) {
+    if (a.out_dtype == DT_FP8) hipLaunchKernelGGL((attention_kernel<HS, MODE, 1, IN_DT>), grid, block, 0, st, a);
+    else if (a.out_dtype == IN_DT) hipLaunchKernelGGL((attention_kernel<HS, MODE, 0, IN_DT>), grid, block, 0, st, a);
+    else return hipErrorInvalidValue;
+  }
   return hipGetLastError();
 }
 

@@ -610,6 +610,29 @@ def test_attention_relshift(cuda):
     assert torch.allclose(out.float(), ref, rtol=2 ** -6, atol=2 ** -6), (out.float() - ref).abs().max()
 
 
+@pytest.mark.parametrize("B,H,hs", [(1, 1, 32), (3, 5, 32), (1, 1, 64), (9, 3, 64)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_attention_relshift_sizes_and_types(cuda, B, H, hs, dtype):
+    """Both head sizes, both 16-bit types and the e4m3 output: the shift crosses the two waves of a unit, which at head size 32 fill V's transpose with
+    half their lanes. Bounds as above for bf16, 2^-9 for f16 (its 2^-11 per rounding, twice), and half a step of e4m3."""
+    from oracle.models import rel_shift
+    qkv, Cm = make_qkv(B, H, hs, cuda, 19 + hs, dtype)
+    pos = torch.randn(64, Cm, device=cuda).to(dtype)
+    u, vb = torch.randn(Cm, device=cuda) * 0.3, torch.randn(Cm, device=cuda) * 0.3
+    q, k, v = split_heads(qkv, B, H, hs)
+    qu = (q + u.view(1, H, 1, hs)).to(dtype).float()
+    qv = (q + vb.view(1, H, 1, hs)).to(dtype).float()
+    pm = pos.float().view(64, H, hs).permute(1, 2, 0).contiguous()
+    s = (qu @ k.transpose(-1, -2).contiguous() + rel_shift((qv @ pm).cpu()).to(cuda)) / math.sqrt(Cm)
+    ref = (s.softmax(-1) @ v).transpose(1, 2).reshape(B * 64, Cm)
+    tol = 2 ** -6 if dtype == torch.bfloat16 else 2 ** -9
+    out = run_attn(qkv, B, H, hs, _lib.ATTN_RELSHIFT, 1 / math.sqrt(Cm), pos=pos, u=u, v=vb)
+    assert torch.allclose(out.float(), ref, rtol=tol, atol=tol), (out.float() - ref).abs().max()
+    so = 448.0 / ref.abs().max().item()
+    o8 = run_attn(qkv, B, H, hs, _lib.ATTN_RELSHIFT, 1 / math.sqrt(Cm), pos=pos, u=u, v=vb, out_dt=_lib.FP8, out_scale=so)
+    assert (o8.view(torch.float8_e4m3fn).float() / so - ref).abs().max() <= ref.abs().max() * 2 ** -3
+
+
 @pytest.mark.parametrize("T", [1.0, 0.5, 0.0])
 def test_masked_softmax(cuda, T):
     torch.manual_seed(3)
