@@ -613,8 +613,10 @@ __global__ void __launch_bounds__(256) causal_long_kernel(const AttnArgs a) {
         for (int r = 0; r < 16; ++r) {
           const int j = 64 * kb + 32 * jt + 8 * (r >> 2) + 4 * g + (r & 3);
           float x = s[jt][it][r] * a.scale;
-          if (edge && (j > i || j >= T)) x = -INFINITY;
-          s[jt][it][r] = x;
+          if constexpr (edge) {
+            if (j > i || j >= T) x = -INFINITY;
+            s[jt][it][r] = x;
+          }
           mx = fmaxf(mx, x);
         }
       mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
@@ -625,7 +627,7 @@ __global__ void __launch_bounds__(256) causal_long_kernel(const AttnArgs a) {
       for (int jt = 0; jt < 2; ++jt)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          const float p = __expf(s[jt][it][r] - mx);
+          const float p = __expf(edge ? s[jt][it][r] - mx : fmaf(s[jt][it][r], a.scale, -mx));
           s[jt][it][r] = p;
           sum += p;
         }
@@ -698,8 +700,207 @@ __global__ void __launch_bounds__(256) causal_long_kernel(const AttnArgs a) {
   }
 }
 
+// The same for up to 256 tokens, all rows wanted: one workgroup of four waves per (position, head). V is transposed into LDS once for all of them, a block of
+// 64 keys per wave; then every wave takes two tiles of 32 queries, the wave-th from the end and, of what is left, the one that makes the waves' key
+// blocks equal (256 tokens: 5 each). A wave's state is half of the other form's, which at 402 registers left a SIMD with one wave that waited for its own
+// chain: 128 sequences of 256 tokens, 12 heads of 64, 80.6 us a launch there, 68 here (71 at the compiler's own 248 registers, 101 held to 128; leaving out the half
+// of a diagonal block that an even tile cannot see changes nothing); of 65 tokens 27 and 21. Vector instructions are 36 % of it, the rest is waits between
+// dependent ones; bytes 40 us at the rate of a large copy.
+constexpr int CG_BLOCKS = 4;
+template <int HS, int OUT_FP8, int IN_DT>
+__global__ void __launch_bounds__(256, 3) causal_group_kernel(const AttnArgs a) {
+  typedef Half16<IN_DT> H16;
+  typedef typename H16::vec hvec;
+  constexpr int KS = HS / 16, DT_TILES = HS / 32;
+  __shared__ __align__(16) uint16_t s_vt[CG_BLOCKS][HS * VT_STRIDE];
+
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int lr = lane & 31, g = lane >> 5;
+  const int T = a.T, nblk = (T + 63) >> 6, ntile = (T + 31) >> 5;
+  int unit = blockIdx.x;   // (as in attention_kernel: each XCD walks a contiguous range)
+  {
+    const int per = gridDim.x >> 3;
+    if (unit < (per << 3)) unit = (unit & 7) * per + (unit >> 3);
+  }
+  const int b = unit / a.H, h = unit - b * a.H;
+  const long row0 = (long)b * T;
+  const uint16_t* qp = reinterpret_cast<const uint16_t*>(a.q) + row0 * a.ldq + h * HS;
+  const uint16_t* kp = reinterpret_cast<const uint16_t*>(a.k) + row0 * a.ldk + h * HS;
+  const uint16_t* vp = reinterpret_cast<const uint16_t*>(a.v) + row0 * a.ldv + h * HS;
+  auto clampT = [&](int t) { return t < T ? t : T - 1; };   // rows past the end re-read the last token
+
+  hvec qf[KS], kf[2][KS];
+  auto request_q = [&](int tile) {
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) qf[ks] = *reinterpret_cast<const hvec*>(qp + (long)clampT(32 * tile + lr) * a.ldq + 16 * ks + 8 * g);
+  };
+  auto request_k = [&](int kb) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) kf[t][ks] = *reinterpret_cast<const hvec*>(kp + (long)clampT(64 * kb + 32 * t + lr) * a.ldk + 16 * ks + 8 * g);
+  };
+  int tile = ntile - 1 - wave;
+  constexpr int DC = HS / 8, PASSES = (16 * DC) / 64;
+  i32x4_t vrow4[PASSES][4];
+  if (wave < nblk) {
+#pragma unroll
+    for (int p = 0; p < PASSES; ++p) {
+      const int id = p * 64 + lane, jq = id / DC, dc = id - jq * DC;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) vrow4[p][t] = *reinterpret_cast<const i32x4_t*>(vp + (long)clampT(64 * wave + 4 * jq + t) * a.ldv + 8 * dc);
+    }
+  }
+  if (tile >= 0) { request_q(tile); request_k(0); }
+  __builtin_amdgcn_sched_barrier(0);
+  if (wave < nblk) {
+    uint16_t* vt = s_vt[wave];
+#pragma unroll
+    for (int p = 0; p < PASSES; ++p) {
+      const int id = p * 64 + lane, jq = id / DC, dc = id - jq * DC;
+#pragma unroll
+      for (int e2 = 0; e2 < 4; ++e2) {
+        const uint32_t w0 = (uint32_t)vrow4[p][0][e2], w1 = (uint32_t)vrow4[p][1][e2], w2 = (uint32_t)vrow4[p][2][e2], w3 = (uint32_t)vrow4[p][3][e2];
+        *reinterpret_cast<uint2*>(vt + (8 * dc + 2 * e2) * VT_STRIDE + 4 * jq) = make_uint2((w0 & 0xffffu) | (w1 << 16), (w2 & 0xffffu) | (w3 << 16));
+        *reinterpret_cast<uint2*>(vt + (8 * dc + 2 * e2 + 1) * VT_STRIDE + 4 * jq) = make_uint2((w0 >> 16) | (w1 & 0xffff0000u), (w2 >> 16) | (w3 & 0xffff0000u));
+      }
+    }
+  }
+  __syncthreads();
+
+  float am = 0.f;
+#pragma unroll 1
+  for (int part = 0; part < 2; ++part) {
+    if (part == 1) {
+      tile = wave + ntile - 8;
+      if (tile >= 0) { request_q(tile); request_k(0); }
+    }
+    if (tile < 0) continue;
+    const int qb = tile >> 1, i = 32 * tile + lr;
+    float run_m = -INFINITY, run_l = 0.f;
+    f32x16_t o[DT_TILES];
+#pragma unroll
+    for (int dt = 0; dt < DT_TILES; ++dt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o[dt][r] = 0.f;
+    // (the diagonal block alone needs the causal test; keys past T sit in it too)
+    auto key_block = [&](int kb, auto edge_c) {
+      constexpr bool edge = decltype(edge_c)::value;
+      f32x16_t s[2];
+#pragma unroll
+      for (int jt = 0; jt < 2; ++jt) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[jt][r] = 0.f;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) s[jt] = H16::mfma(kf[jt][ks], qf[ks], s[jt]);
+      }
+      if constexpr (!edge) request_k(kb + 1);
+      __builtin_amdgcn_sched_barrier(0);   // (the requests stay above the softmax)
+      float mx = run_m;
+#pragma unroll
+      for (int jt = 0; jt < 2; ++jt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          float x = s[jt][r] * a.scale;
+          if constexpr (edge) {
+            const int j = 64 * kb + 32 * jt + 8 * (r >> 2) + 4 * g + (r & 3);
+            if (j > i || j >= T) x = -INFINITY;
+            s[jt][r] = x;
+          }
+          mx = fmaxf(mx, x);
+        }
+      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+      // Key 0 is visible to every query, so mx is finite from the first block on.
+      const float alpha = __expf(run_m - mx);
+      float sum = 0.f;
+#pragma unroll
+      for (int jt = 0; jt < 2; ++jt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const float p = __expf(edge ? s[jt][r] - mx : fmaf(s[jt][r], a.scale, -mx));
+          s[jt][r] = p;
+          sum += p;
+        }
+      sum += __shfl_xor(sum, 32, 64);
+      run_l = run_l * alpha + sum;
+      run_m = mx;
+#pragma unroll
+      for (int dt = 0; dt < DT_TILES; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[dt][r] *= alpha;
+      // ---- O^T += V^T · P^T
+#pragma unroll
+      for (int k4 = 0; k4 < 4; ++k4) {
+        const int jt = k4 >> 1, kh = k4 & 1;
+        hvec pf;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) pf[e] = (typename H16::elem)s[jt][8 * kh + e];
+#pragma unroll
+        for (int dt = 0; dt < DT_TILES; ++dt) {
+          const uint16_t* vrow = s_vt[kb] + (32 * dt + lr) * VT_STRIDE + 16 * k4 + 4 * g;
+          const uint2 lo = *reinterpret_cast<const uint2*>(vrow);
+          const uint2 hi = *reinterpret_cast<const uint2*>(vrow + 8);
+          const uint4 packed = make_uint4(lo.x, lo.y, hi.x, hi.y);
+          o[dt] = H16::mfma(__builtin_bit_cast(hvec, packed), pf, o[dt]);
+        }
+      }
+    };
+#pragma unroll 1
+    for (int kb = 0; kb < qb; ++kb) key_block(kb, std::false_type{});
+    key_block(qb, std::true_type{});
+
+    // Two lanes of a row exchange halves, as in attention_kernel: each stores eight consecutive dims. (Rows past the end take part and store nothing.)
+    const float inv_l = 1.0f / run_l;
+    const bool keep_row = i < T;
+#pragma unroll
+    for (int dt = 0; dt < DT_TILES; ++dt)
+#pragma unroll
+      for (int rp = 0; rp < 2; ++rp) {
+        uint32_t pk[2][2];
+#pragma unroll
+        for (int q2 = 0; q2 < 2; ++q2) {
+          float v[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            v[e] = o[dt][4 * (2 * rp + q2) + e] * inv_l;
+            if (keep_row) am = fmaxf(am, fabsf(v[e]));
+          }
+          if constexpr (OUT_FP8) {
+            pk[q2][0] = pack_fp8x4(v[0] * a.out_scale, v[1] * a.out_scale, v[2] * a.out_scale, v[3] * a.out_scale);
+            pk[q2][1] = 0;
+          } else {
+            pk[q2][0] = H16::pack2(v[0], v[1]);
+            pk[q2][1] = H16::pack2(v[2], v[3]);
+          }
+        }
+        const uint32_t keep0 = g ? pk[1][0] : pk[0][0], keep1 = g ? pk[1][1] : pk[0][1];
+        const uint32_t r0 = __shfl_xor(g ? pk[0][0] : pk[1][0], 32, 64);
+        const long off = (row0 + i) * a.ldo + h * HS + 32 * dt + 16 * rp + 8 * g;
+        if constexpr (OUT_FP8) {
+          if (keep_row) *reinterpret_cast<uint2*>(reinterpret_cast<uint8_t*>(a.out) + off) = g ? make_uint2(r0, keep0) : make_uint2(keep0, r0);
+        } else {
+          const uint32_t r1 = __shfl_xor(g ? pk[0][1] : pk[1][1], 32, 64);
+          if (keep_row) *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(a.out) + off) = g ? make_uint4(r0, r1, keep0, keep1) : make_uint4(keep0, keep1, r0, r1);
+        }
+      }
+  }
+  if (a.amax) {
+    am = wave_max(am);
+    if (lane == 0) atomic_amax(a.amax, am);
+  }
+}
+
 template <int HS, int IN_DT>
 static hipError_t launch_causal_long_dt(const AttnArgs& a, hipStream_t st) {
+  // (16-byte stores of the one with the shared V need rows and base aligned to that)
+  const int osz = a.out_dtype == DT_FP8 ? 1 : 2;
+  if (a.T > 64 && a.T <= 64 * CG_BLOCKS && !a.last_row && (a.ldo * osz) % 16 == 0 && (reinterpret_cast<uintptr_t>(a.out) & 15) == 0) {
+    const dim3 grid((unsigned)(a.B * a.H)), block(256);
+    if (a.out_dtype == DT_FP8) hipLaunchKernelGGL((causal_group_kernel<HS, 1, IN_DT>), grid, block, 0, st, a);
+    else if (a.out_dtype == IN_DT) hipLaunchKernelGGL((causal_group_kernel<HS, 0, IN_DT>), grid, block, 0, st, a);
+    else return hipErrorInvalidValue;
+    return hipGetLastError();
+  }
   const long units = (long)a.B * a.H * (a.last_row ? 1 : (a.T + 63) / 64);   // (the last token sits in the block that is walked first)
   const dim3 grid((unsigned)((units + 3) / 4)), block(256);
   if (a.out_dtype == DT_FP8) hipLaunchKernelGGL((causal_long_kernel<HS, 1, IN_DT>), grid, block, 0, st, a);

@@ -610,6 +610,29 @@ def test_attention_relshift(cuda):
     assert torch.allclose(out.float(), ref, rtol=2 ** -6, atol=2 ** -6), (out.float() - ref).abs().max()
 
 
+@pytest.mark.parametrize("T", [65, 96, 97, 128, 129, 160, 161, 191, 224, 255, 256])
+@pytest.mark.parametrize("hs", [32, 64])
+@pytest.mark.parametrize("dtype,fp8", [(torch.bfloat16, False), (torch.float16, False), (torch.bfloat16, True)])
+def test_attention_causal_on_shared_values_equals_a_wave_alone(cuda, T, hs, dtype, fp8):
+    """Up to 256 tokens the four waves of a head share V and take two tiles of 32 queries each; an output stride that is not a multiple of 16 bytes goes to the
+    form with a wave for every 64 queries. Same bits, at lengths on either side of every tile and block."""
+    B, H = 3, 3
+    Cm = H * hs
+    torch.manual_seed(T)
+    qkv = torch.randn(B * T, 3 * Cm, device=cuda).to(dtype)
+    in_dt = _lib.F16 if dtype == torch.float16 else _lib.BF16
+    base, out_dt = qkv.data_ptr(), _lib.FP8 if fp8 else in_dt
+    outs = []
+    for ldo in (Cm + (16 if fp8 else 8), Cm + 4):
+        out = torch.zeros(B * T, ldo, dtype=torch.uint8 if fp8 else dtype, device=cuda)
+        check(lib().crl_attention_causal(C.c_void_p(base), 3 * Cm, C.c_void_p(base + 2 * Cm), 3 * Cm, C.c_void_p(base + 4 * Cm), 3 * Cm, in_dt,
+                                         p(out), ldo, out_dt, 37.0, B, H, hs, T, 1 / math.sqrt(hs), None, stream()), "causal")
+        torch.cuda.synchronize()
+        assert not out[:, Cm:].any()
+        outs.append(out[:, :Cm].float())
+    assert outs[0].abs().max() > 0 and torch.equal(outs[0], outs[1])
+
+
 @pytest.mark.parametrize("B,H,hs", [(1, 1, 32), (3, 5, 32), (1, 1, 64), (9, 3, 64)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_attention_relshift_sizes_and_types(cuda, B, H, hs, dtype):
