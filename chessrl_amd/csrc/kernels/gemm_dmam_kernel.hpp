@@ -172,6 +172,7 @@ __global__ void __launch_bounds__(DmamCfg::NT) gemm_dmam_kernel(const GemmArgs a
       n = n < a.N ? n : a.N - 1;
       uint8_t* c = smem + Cfg::COLS_OFF + wave * (3 * 64 * 4);
       if (a.bias) __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(a.bias + n), (__attribute__((address_space(3))) void*)c, 4, 0, 0);
+      else if constexpr (PERSIST) reinterpret_cast<float*>(c)[lane] = 0.f;   // (so that the epilogue reads the constants without asking)
       if constexpr (EPI == DMAF_RESNORM || EPI == DMAF_GENERAL_NORM) {
         __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(a.res_gamma + n), (__attribute__((address_space(3))) void*)(c + 256), 4, 0, 0);
         if (a.res_beta)
@@ -244,17 +245,23 @@ __global__ void __launch_bounds__(DmamCfg::NT) gemm_dmam_kernel(const GemmArgs a
       left = left < BN ? left : BN;
       const __amdgpu_buffer_rsrc_t rsrc_o = dmaf_rsrc(reinterpret_cast<char*>(first ? a.C : a.C2) + (long)m0 * ldob + (long)(first ? n0 : n0 - a.nsplit) * OSZ,
                                                       (long)(rows - 1) * ldob + (long)left * OSZ);
-      constexpr int NOWHERE = (int)0x80000000u, CPL = 16 / OSZ;     // columns per lane in the store layout
+      constexpr int NOWHERE = (int)0x80000000u, CPL = 16 / OSZ, NST = OUT_DT == DT_FP8 ? 1 : 2;     // columns per lane in the store layout, stores of a row block
       const bool nt = a.stream_out != 0 && (OUT_DT != DT_F32 || ldob % 128 == 0);
-      auto put = [&](u32x4_t v, int row, int col) {
+      // (one branch on the hint per row block, as in gemm_dmaf_kernel.hpp)
+      auto put = [&](const u32x4_t (&v)[NST], int row, int col) {
         const int off = wn * Cfg::WN + col + (OUT_DT == DT_F32 && !HAS_RES ? 3 : 0) < left ? (wm * Cfg::WM + row) * ldob + (wn * Cfg::WN + col) * OSZ : NOWHERE;
-        if (nt) dmaf_put16_nt(v, rsrc_o, off);
-        else dmaf_put16(v, rsrc_o, off);
+        if (nt) {
+#pragma unroll
+          for (int it = 0; it < NST; ++it) dmaf_put16_nt(v[it], rsrc_o, off + it * (64 / EPR) * ldob);
+        } else {
+#pragma unroll
+          for (int it = 0; it < NST; ++it) dmaf_put16(v[it], rsrc_o, off + it * (64 / EPR) * ldob);
+        }
       };
-      auto col_const = [&](const float* c, bool have, float (&o)[16]) {
+      auto col_const = [&](const float* c, float (&o)[16]) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          const f32x4_t v = have ? *reinterpret_cast<const f32x4_t*>(c + 8 * q + 4 * eg) : f32x4_t{0.f, 0.f, 0.f, 0.f};
+          const f32x4_t v = *reinterpret_cast<const f32x4_t*>(c + 8 * q + 4 * eg);
 #pragma unroll
           for (int e = 0; e < 4; ++e) o[4 * q + e] = v[e];
         }
@@ -268,40 +275,42 @@ __global__ void __launch_bounds__(DmamCfg::NT) gemm_dmam_kernel(const GemmArgs a
         // raw sums through the patch, 16 columns at a time; the rest in the store layout (4 columns per lane)
         static_for<0, 2 * TM>([&](auto sc) {
           constexpr int st = decltype(sc)::value, half = st / TM, t = st % TM;
-          const f32x4_t bv = a.bias ? *reinterpret_cast<const f32x4_t*>(cols + half * 16 + ec * 4) : f32x4_t{0.f, 0.f, 0.f, 0.f};
+          const f32x4_t bv = *reinterpret_cast<const f32x4_t*>(cols + half * 16 + ec * 4);
 #pragma unroll
           for (int qq = 0; qq < 2; ++qq) {
             const int r0 = 4 * (2 * half + qq);
             *reinterpret_cast<f32x4_t*>(at(el, 2 * qq + eg)) = f32x4_t{acc[0][t][r0], acc[0][t][r0 + 1], acc[0][t][r0 + 2], acc[0][t][r0 + 3]};
           }
           wave_lds_fence();
+          u32x4_t o[2];
 #pragma unroll
-          for (int it = 0; it < 2; ++it) {
-            const f32x4_t s = *reinterpret_cast<const f32x4_t*>(at(er + 16 * it, ec));
-            u32x4_t o;
+          for (int it = 0; it < 2; ++it) o[it] = *reinterpret_cast<const u32x4_t*>(at(er + 16 * it, ec));
+#pragma unroll
+          for (int it = 0; it < 2; ++it)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-              float v = activate(fmaf(s[e], a.descale, bv[e]));
+              float v = activate(fmaf(__uint_as_float(o[it][e]), a.descale, bv[e]));
               if constexpr (HAS_RES) v = fmaf(v, a.alpha, __uint_as_float(res[(half * TM + t) * 2 + it][e]));
-              o[e] = __float_as_uint(v);
+              o[it][e] = __float_as_uint(v);
             }
-            put(o, t * 32 + er + 16 * it, half * 16 + ec * 4);
-            if constexpr (!HAS_RES) {
-              const int col = wn * Cfg::WN + half * 16 + ec * 4;
-              if (left & 3) dmaf_put_part(o, rsrc_o, (wm * Cfg::WM + t * 32 + er + 16 * it) * ldob + col * 4, left - col);
-            }
+          put(o, t * 32 + er, half * 16 + ec * 4);
+          if constexpr (!HAS_RES) {
+            const int col = wn * Cfg::WN + half * 16 + ec * 4;
+            if (left & 3)
+#pragma unroll
+              for (int it = 0; it < 2; ++it) dmaf_put_part(o[it], rsrc_o, (wm * Cfg::WM + t * 32 + er + 16 * it) * ldob + col * 4, left - col);
           }
           wave_lds_fence();
         });
       } else {
         float bias16[16], gain16[16];
-        col_const(cols, a.bias != nullptr, bias16);
+        col_const(cols, bias16);
         if constexpr (EPI == DMAF_RESNORM) {
-          col_const(cols + 64, true, gain16);
+          col_const(cols + 64, gain16);
           if (a.res_beta) {   // the offset joins the bias (which is multiplied by alpha)
             const float inv_alpha = 1.0f / a.alpha;
             float off16[16];
-            col_const(cols + 128, true, off16);
+            col_const(cols + 128, off16);
 #pragma unroll
             for (int i = 0; i < 16; ++i) bias16[i] += off16[i] * inv_alpha;
           }
@@ -360,8 +369,10 @@ __global__ void __launch_bounds__(DmamCfg::NT) gemm_dmam_kernel(const GemmArgs a
             }
           }
           wave_lds_fence();
+          u32x4_t o[NST];
 #pragma unroll
-          for (int it = 0; it < (OUT_DT == DT_FP8 ? 1 : 2); ++it) put(*reinterpret_cast<const u32x4_t*>(at(er + (64 / EPR) * it, ec)), t * 32 + er + (64 / EPR) * it, ec * CPL);
+          for (int it = 0; it < NST; ++it) o[it] = *reinterpret_cast<const u32x4_t*>(at(er + (64 / EPR) * it, ec));
+          put(o, t * 32 + er, ec * CPL);
           wave_lds_fence();
         });
       }
