@@ -363,7 +363,7 @@ __global__ void __launch_bounds__(SPLIT ? 128 : 64 * AttnWaves<MODE>::N, (SPLIT 
         }
         mx = fmaxf(mx, x);
       }
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    mx = max_xor32(mx);
     float sum = 0.f;
 #pragma unroll
     for (int jt = 0; jt < 2; ++jt)
@@ -374,7 +374,7 @@ __global__ void __launch_bounds__(SPLIT ? 128 : 64 * AttnWaves<MODE>::N, (SPLIT 
         s[jt][it][r] = p;
         sum += p;
       }
-    sum += __shfl_xor(sum, 32, 64);
+    sum = add_xor32(sum);
     inv_l[it] = 1.0f / sum;
   };
   typedef std::integral_constant<int, 0> T0;
@@ -456,17 +456,16 @@ __global__ void __launch_bounds__(SPLIT ? 128 : 64 * AttnWaves<MODE>::N, (SPLIT 
           }
         }
         // g = 0 keeps group 2rp and receives the partner's half of it; g = 1 keeps group 2rp+1.
-        const int keep = g, give = 1 - g;
-        const uint32_t r0 = __shfl_xor(pk[give][0], 32, 64);
+        lanes_swap32(pk[0][0], pk[1][0]);
         const int d = 32 * dt + 16 * rp + 8 * g;
         const long off = row * a.ldo + h * HS + d;
         if constexpr (OUT_FP8) {
-          const uint2 w = g ? make_uint2(r0, pk[keep][0]) : make_uint2(pk[keep][0], r0);
+          const uint2 w = make_uint2(pk[0][0], pk[1][0]);
           if constexpr (coop) *reinterpret_cast<uint2*>(s_out + (32 * it + lr) * OSTRIDE + (wave * HS + d) * OSZ) = w;
           else if (keep_row) *reinterpret_cast<uint2*>(reinterpret_cast<uint8_t*>(a.out) + off) = w;
         } else {
-          const uint32_t r1 = __shfl_xor(pk[give][1], 32, 64);
-          const uint4 w = g ? make_uint4(r0, r1, pk[keep][0], pk[keep][1]) : make_uint4(pk[keep][0], pk[keep][1], r0, r1);
+          lanes_swap32(pk[0][1], pk[1][1]);
+          const uint4 w = make_uint4(pk[0][0], pk[0][1], pk[1][0], pk[1][1]);
           if constexpr (coop) *reinterpret_cast<uint4*>(s_out + (32 * it + lr) * OSTRIDE + (wave * HS + d) * OSZ) = w;
           else if (keep_row) *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(a.out) + off) = w;
         }
@@ -619,7 +618,7 @@ __global__ void __launch_bounds__(256) causal_long_kernel(const AttnArgs a) {
           }
           mx = fmaxf(mx, x);
         }
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+      mx = max_xor32(mx);
       // Key 0 is visible to every query, so mx is finite from the first block on.
       const float alpha = __expf(run_m[it] - mx);
       float sum = 0.f;
@@ -631,7 +630,7 @@ __global__ void __launch_bounds__(256) causal_long_kernel(const AttnArgs a) {
           s[jt][it][r] = p;
           sum += p;
         }
-      sum += __shfl_xor(sum, 32, 64);
+      sum = add_xor32(sum);
       run_l[it] = run_l[it] * alpha + sum;
       run_m[it] = mx;
 #pragma unroll
@@ -809,7 +808,7 @@ __global__ void __launch_bounds__(256, 3) causal_group_kernel(const AttnArgs a) 
           }
           mx = fmaxf(mx, x);
         }
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+      mx = max_xor32(mx);
       // Key 0 is visible to every query, so mx is finite from the first block on.
       const float alpha = __expf(run_m - mx);
       float sum = 0.f;
@@ -821,7 +820,7 @@ __global__ void __launch_bounds__(256, 3) causal_group_kernel(const AttnArgs a) 
           s[jt][r] = p;
           sum += p;
         }
-      sum += __shfl_xor(sum, 32, 64);
+      sum = add_xor32(sum);
       run_l = run_l * alpha + sum;
       run_m = mx;
 #pragma unroll
@@ -873,14 +872,13 @@ __global__ void __launch_bounds__(256, 3) causal_group_kernel(const AttnArgs a) 
             pk[q2][1] = H16::pack2(v[2], v[3]);
           }
         }
-        const uint32_t keep0 = g ? pk[1][0] : pk[0][0], keep1 = g ? pk[1][1] : pk[0][1];
-        const uint32_t r0 = __shfl_xor(g ? pk[0][0] : pk[1][0], 32, 64);
+        lanes_swap32(pk[0][0], pk[1][0]);
         const long off = (row0 + i) * a.ldo + h * HS + 32 * dt + 16 * rp + 8 * g;
         if constexpr (OUT_FP8) {
-          if (keep_row) *reinterpret_cast<uint2*>(reinterpret_cast<uint8_t*>(a.out) + off) = g ? make_uint2(r0, keep0) : make_uint2(keep0, r0);
+          if (keep_row) *reinterpret_cast<uint2*>(reinterpret_cast<uint8_t*>(a.out) + off) = make_uint2(pk[0][0], pk[1][0]);
         } else {
-          const uint32_t r1 = __shfl_xor(g ? pk[0][1] : pk[1][1], 32, 64);
-          if (keep_row) *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(a.out) + off) = g ? make_uint4(r0, r1, keep0, keep1) : make_uint4(keep0, keep1, r0, r1);
+          lanes_swap32(pk[0][1], pk[1][1]);
+          if (keep_row) *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(a.out) + off) = make_uint4(pk[0][0], pk[0][1], pk[1][0], pk[1][1]);
         }
       }
   }

@@ -89,33 +89,48 @@ __device__ __forceinline__ float apply_act(float x, int act) {
 }
 
 // ---- wave reductions (64 lanes) ---------------------------------------------------
-// An xor butterfly over lane distances 1, 2, 4, 8, 16, 32. The four short distances are data-parallel-primitive moves
-// inside a row of 16 lanes (no trip through the LDS crossbar, which is what __shfl_xor compiles to: six dependent ones per
-// reduction were most of a LayerNorm wave's latency). At distance 4 and 8 the partner is the mirrored lane of the half row
+// An xor butterfly over lane distances 1, 2, 4, 8, 16, 32, without a trip through the LDS crossbar (which is what __shfl_xor compiles to: six
+// dependent ones per reduction were most of a LayerNorm wave's latency). The four short distances are data-parallel-primitive moves
+// inside a row of 16 lanes, the two long ones exchanges of whole rows: v with itself leaves every lane with its own value in one result
+// and its partner's in the other, so the two are added as they are (1 leaf position 740 -> 726 us, a 71-token move 192.1 -> 188.4).
+// At distance 4 and 8 the partner is the mirrored lane of the half row
 // or row: after the shorter steps every lane of a group of 4 or 8 holds the group's partial result, so the mirrored lane
 // holds exactly what the xor partner holds.
 template <int CTRL>
 __device__ __forceinline__ float dpp_move(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false));
 }
-constexpr int DPP_XOR1 = 0xB1, DPP_XOR2 = 0x4E, DPP_HALF_MIRROR = 0x141, DPP_MIRROR = 0x140;
+constexpr int DPP_XOR1 = 0xB1, DPP_XOR2 = 0x4E, DPP_HALF_MIRROR = 0x141, DPP_MIRROR = 0x140, DPP_XOR8 = 0x128;
+__device__ __forceinline__ void lanes_xor16(float v, float& a, float& b) {   // {a, b} = {v, v of lane ^ 16}, in lane order
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  a = __uint_as_float(r[0]); b = __uint_as_float(r[1]);
+}
+__device__ __forceinline__ void lanes_xor32(float v, float& a, float& b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  a = __uint_as_float(r[0]); b = __uint_as_float(r[1]);
+}
+// The upper half of a wave trades a with the lower half's b.
+__device__ __forceinline__ void lanes_swap32(uint32_t& a, uint32_t& b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+  a = r[0]; b = r[1];
+}
+__device__ __forceinline__ float add_xor16(float v) { float a, b; lanes_xor16(v, a, b); return a + b; }
+__device__ __forceinline__ float add_xor32(float v) { float a, b; lanes_xor32(v, a, b); return a + b; }
+__device__ __forceinline__ float max_xor16(float v) { float a, b; lanes_xor16(v, a, b); return fmaxf(a, b); }
+__device__ __forceinline__ float max_xor32(float v) { float a, b; lanes_xor32(v, a, b); return fmaxf(a, b); }
 __device__ __forceinline__ float wave_sum(float v) {
   v += dpp_move<DPP_XOR1>(v);
   v += dpp_move<DPP_XOR2>(v);
   v += dpp_move<DPP_HALF_MIRROR>(v);
   v += dpp_move<DPP_MIRROR>(v);
-  v += __shfl_xor(v, 16, 64);
-  v += __shfl_xor(v, 32, 64);
-  return v;
+  return add_xor32(add_xor16(v));
 }
 __device__ __forceinline__ float wave_max(float v) {
   v = fmaxf(v, dpp_move<DPP_XOR1>(v));
   v = fmaxf(v, dpp_move<DPP_XOR2>(v));
   v = fmaxf(v, dpp_move<DPP_HALF_MIRROR>(v));
   v = fmaxf(v, dpp_move<DPP_MIRROR>(v));
-  v = fmaxf(v, __shfl_xor(v, 16, 64));
-  v = fmaxf(v, __shfl_xor(v, 32, 64));
-  return v;
+  return max_xor32(max_xor16(v));
 }
 
 // amax is kept as the bit pattern of a non-negative float so integer max orders it.

@@ -66,6 +66,7 @@ template <int HS, int IN_DT>
 __global__ void __launch_bounds__(256) decode_attention_kernel(const uint16_t* q, long ldq, const uint16_t* cache, int Tmax, int C, int n_arg,
                                                                const int* dyn_k, uint16_t* out, long ldo, int B, int H, float scale) {
   constexpr int LPK = HS / 8, KPI = 64 / LPK;    // lanes per key row, key rows per wave instruction
+  static_assert(LPK == 4 || LPK == 8, "head sizes 32 and 64");
   __shared__ float s_p[DEC_TMAX];
   __shared__ float s_acc[4][HS];
   const int n = dyn_k ? 65 + dyn_k[0] : n_arg;
@@ -95,8 +96,9 @@ __global__ void __launch_bounds__(256) decode_attention_kernel(const uint16_t* q
 #pragma unroll
       for (int e = 0; e < 8; ++e) s = fmaf(qv[e], kv[e], s);
     }
-#pragma unroll
-    for (int o = 1; o < LPK; o <<= 1) s += __shfl_xor(s, o, 64);
+    s += dpp_move<DPP_XOR1>(s);
+    s += dpp_move<DPP_XOR2>(s);
+    if constexpr (LPK == 8) s += dpp_move<DPP_HALF_MIRROR>(s);
     if (sub == 0 && j < n) s_p[j] = s * scale;
   }
   __syncthreads();
@@ -123,9 +125,12 @@ __global__ void __launch_bounds__(256) decode_attention_kernel(const uint16_t* q
     }
   }
 #pragma unroll
-  for (int o = LPK; o < 64; o <<= 1)
-#pragma unroll
-    for (int e = 0; e < 8; ++e) acc[e] += __shfl_xor(acc[e], o, 64);
+  for (int e = 0; e < 8; ++e) {
+    // (distances LPK = 4 or 8, then 8, 16 and 32; at distance 4 the sums of a lane's neighbours are other dims', so no mirrored lane)
+    if constexpr (LPK == 4) acc[e] += __shfl_xor(acc[e], 4, 64);
+    acc[e] += dpp_move<DPP_XOR8>(acc[e]);
+    acc[e] = add_xor32(add_xor16(acc[e]));
+  }
   if (kin == 0) {
 #pragma unroll
     for (int e = 0; e < 8; ++e) s_acc[wave][sub * 8 + e] = acc[e];

@@ -35,8 +35,7 @@ __device__ __forceinline__ float half_wave_sum(float v) {
   v += dpp_move<DPP_XOR2>(v);
   v += dpp_move<DPP_HALF_MIRROR>(v);
   v += dpp_move<DPP_MIRROR>(v);
-  v += __shfl_xor(v, 16, 64);
-  return v;
+  return add_xor16(v);
 }
 
 // X_DT: type of X and of the output; IN_DT: operand type (X_DT or e4m3); RB: row blocks of 32 per workgroup.

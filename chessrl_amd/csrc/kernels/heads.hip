@@ -138,9 +138,9 @@ __global__ void __launch_bounds__(256) policy_qk_kernel(const PolicyQKArgs a) {
         }
       }
     }
-    sum += __shfl_xor(sum, 1, 64);
-    sum += __shfl_xor(sum, 2, 64);
-    sum += __shfl_xor(sum, 4, 64);
+    sum += dpp_move<DPP_XOR1>(sum);
+    sum += dpp_move<DPP_XOR2>(sum);
+    sum += dpp_move<DPP_HALF_MIRROR>(sum);
     if (part == 0) s_off[file][piece] = sum;
   }
   __syncthreads();
