@@ -18,9 +18,16 @@ namespace crl {
 // from rows it alone reads (a row's 512 bytes of that quarter are four whole lines; with the channels shared and the
 // output split over the waves instead, every row was fetched by two waves in 32-byte pieces: 2.4 TB/s); the partial
 // tiles meet in LDS and are added in a fixed order, (w0 + w2) + (w1 + w3).
+// Bound by the reads of Q and K (256 KB a position at 1024 channels) and, at few positions, by how many wait for one another: the loop
+// over steps of 16 channels, the promotion dots and the move tables each took a trip to memory per iteration. Slabs of four steps in two
+// register sets, dots with eight iterations requested at once and tables read ahead of the product make it 17.8 -> 12.7 us for one
+// position, 32 -> 14 for 496 of 512 channels, 118 -> 58 for 1000 of 1024 and 340 -> 219 for 4096 (5.0 TB/s). The second launch bound keeps
+// two workgroups on a compute unit (left alone the compiler takes 276 registers and one: 261 us); one register set instead of two is
+// 358 us, and four workgroups with less in flight 508.
+constexpr int PQK_MOVES = 8;     // moves per thread whose table entries are requested together
 constexpr int PQK_STRIDE = 68;   // floats per row of a partial tile: 16 lanes' 16-byte stores cover 64 banks
 template <int IN_DT>
-__global__ void __launch_bounds__(256) policy_qk_kernel(const PolicyQKArgs a) {
+__global__ void __launch_bounds__(256, 2) policy_qk_kernel(const PolicyQKArgs a) {
   __shared__ __align__(16) float s_part[2][64 * PQK_STRIDE];
   __shared__ float s_off[8][4];
   float* const s_a = s_part[0];   // after the sum: the scaled 64x64 tile, row stride 65 (the gather's bank spread)
@@ -32,6 +39,65 @@ __global__ void __launch_bounds__(256) policy_qk_kernel(const PolicyQKArgs a) {
   const uint16_t* kp = reinterpret_cast<const uint16_t*>(a.k) + ((long)b * 64 + lr) * a.ldk + wave * kq + 8 * g;
   const long q32 = 32 * a.ldq, k32 = 32 * a.ldk;
 
+  // Four steps of 16 channels form a slab: a slab's 16 pieces are requested together, a row's four one after another (they are one
+  // 128-byte line), and the next slab's while this one is multiplied.
+  using piece_t = i32x4_t;
+  piece_t qa[2][4], ka[2][4], qb[2][4], kb[2][4];
+  const int steps = kq / 16, slabs = steps / 4;
+  auto slab_load = [&](piece_t (&qv)[2][4], piece_t (&kv)[2][4], int c) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+#pragma unroll
+      for (int s = 0; s < 4; ++s) qv[t][s] = *reinterpret_cast<const piece_t*>(qp + t * q32 + 64 * c + 16 * s);
+#pragma unroll
+      for (int s = 0; s < 4; ++s) kv[t][s] = *reinterpret_cast<const piece_t*>(kp + t * k32 + 64 * c + 16 * s);
+    }
+  };
+  if (slabs > 0) slab_load(qa, ka, 0);
+
+  // Promotion offsets from the keys of the promotion rank: tokens 0..7 when white is
+  // to move, 56..63 (rank 1) when black is. 32 dot products, 8 threads each.
+  const int white = a.white_to_move ? a.white_to_move[b] : 1;
+  const bool gather = a.logits && a.nmoves > 0;
+  const int16_t* gi = a.gidx + (white ? a.nmoves : 0);
+  int ft[PQK_MOVES], pr[PQK_MOVES];
+  auto tables = [&](int v0) {   // this thread's moves of [v0, v0 + 256 * PQK_MOVES): read ahead, not between the stores
+#pragma unroll
+    for (int m = 0; m < PQK_MOVES; ++m) {
+      const int v = min(v0 + 256 * m + (int)threadIdx.x, a.nmoves - 1);
+      ft[m] = gi[v];
+      pr[m] = a.gpromo[v];
+    }
+  };
+  if (gather) {
+    tables(0);
+    const int dot = threadIdx.x >> 3, part = threadIdx.x & 7;
+    const int file = dot >> 2, piece = dot & 3;
+    const int tok = (white ? 0 : 56) + file;
+    const uint16_t* krow = reinterpret_cast<const uint16_t*>(a.k) + ((long)b * 64 + tok) * a.ldk;
+    const float* wrow = a.wpromo + (long)piece * a.C;
+    float sum = 0.f;
+    if (a.wpromo) {
+      // (eight channels per thread and step: a 16-byte piece of the key row against two vectors of the weight row)
+#pragma unroll 8
+      for (int c = part * 8; c < a.C; c += 64) {
+        const uint4 kraw = *reinterpret_cast<const uint4*>(krow + c);
+        const float4 w0 = *reinterpret_cast<const float4*>(wrow + c), w1 = *reinterpret_cast<const float4*>(wrow + c + 4);
+        const uint32_t kw[4] = {kraw.x, kraw.y, kraw.z, kraw.w};
+        const float wv[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const uint16_t bits = (uint16_t)((e & 1) ? (kw[e >> 1] >> 16) : (kw[e >> 1] & 0xffff));
+          sum = fmaf((IN_DT == DT_BF16) ? bf16_bits_to_f32(bits) : f16_bits_to_f32(bits), wv[e], sum);
+        }
+      }
+    }
+    sum += dpp_move<DPP_XOR1>(sum);
+    sum += dpp_move<DPP_XOR2>(sum);
+    sum += dpp_move<DPP_HALF_MIRROR>(sum);
+    if (part == 0) s_off[file][piece] = sum;
+  }
+
   f32x16_t acc[2][2];   // [jt][it]
 #pragma unroll
   for (int jt = 0; jt < 2; ++jt)
@@ -39,24 +105,30 @@ __global__ void __launch_bounds__(256) policy_qk_kernel(const PolicyQKArgs a) {
     for (int it = 0; it < 2; ++it)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[jt][it][r] = 0.f;
-  const int steps = kq / 16;
-#pragma unroll 4
-  for (int s = 0; s < steps; ++s) {
-    uint4 qv[2], kv[2];
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      qv[t] = *reinterpret_cast<const uint4*>(qp + t * q32 + 16 * s);
-      kv[t] = *reinterpret_cast<const uint4*>(kp + t * k32 + 16 * s);
-    }
+  auto multiply = [&](const piece_t& q0, const piece_t& q1, const piece_t& k0, const piece_t& k1) {
 #pragma unroll
     for (int jt = 0; jt < 2; ++jt)
 #pragma unroll
       for (int it = 0; it < 2; ++it) {
+        const piece_t kv = jt ? k1 : k0, qv = it ? q1 : q0;
         if constexpr (IN_DT == DT_BF16)
-          acc[jt][it] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, kv[jt]), __builtin_bit_cast(bf16x8_t, qv[it]), acc[jt][it], 0, 0, 0);
+          acc[jt][it] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, kv), __builtin_bit_cast(bf16x8_t, qv), acc[jt][it], 0, 0, 0);
         else
-          acc[jt][it] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, kv[jt]), __builtin_bit_cast(f16x8_t, qv[it]), acc[jt][it], 0, 0, 0);
+          acc[jt][it] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, kv), __builtin_bit_cast(f16x8_t, qv), acc[jt][it], 0, 0, 0);
       }
+  };
+  for (int c = 0; c < slabs; c += 2) {
+    if (c + 1 < slabs) slab_load(qb, kb, c + 1);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) multiply(qa[0][s], qa[1][s], ka[0][s], ka[1][s]);
+    if (c + 1 >= slabs) break;
+    if (c + 2 < slabs) slab_load(qa, ka, c + 2);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) multiply(qb[0][s], qb[1][s], kb[0][s], kb[1][s]);
+  }
+  for (int s = 4 * slabs; s < steps; ++s) {
+    auto piece = [](const uint16_t* p) { return *reinterpret_cast<const piece_t*>(p); };
+    multiply(piece(qp + 16 * s), piece(qp + q32 + 16 * s), piece(kp + 16 * s), piece(kp + k32 + 16 * s));
   }
   // acc[jt][it][r]: key j = 32jt + 8(r/4) + 4g + r%4, query i = 32it + lr.
   // Waves 0 and 1 lay their tiles down, waves 2 and 3 add theirs on top (same lane, same element).
@@ -106,7 +178,7 @@ __global__ void __launch_bounds__(256) policy_qk_kernel(const PolicyQKArgs a) {
       }
     }
   }
-  if (!a.logits) return;  // uniform across the workgroup
+  if (!gather) return;  // uniform across the workgroup
 
   __syncthreads();   // every thread has read its partials: their first tile becomes the summed one
   {
@@ -114,43 +186,16 @@ __global__ void __launch_bounds__(256) policy_qk_kernel(const PolicyQKArgs a) {
 #pragma unroll
     for (int e = 0; e < 16; ++e) s_a[i * 65 + j0 + e] = tot[e];
   }
-  // Promotion offsets from the keys of the promotion rank: tokens 0..7 when white is
-  // to move, 56..63 (rank 1) when black is. 32 dot products, 8 threads each.
-  const int white = a.white_to_move ? a.white_to_move[b] : 1;
-  {
-    const int dot = threadIdx.x >> 3, part = threadIdx.x & 7;
-    const int file = dot >> 2, piece = dot & 3;
-    const int tok = (white ? 0 : 56) + file;
-    const uint16_t* krow = reinterpret_cast<const uint16_t*>(a.k) + ((long)b * 64 + tok) * a.ldk;
-    const float* wrow = a.wpromo + (long)piece * a.C;
-    float sum = 0.f;
-    if (a.wpromo) {
-      // (eight channels per thread and step: a 16-byte piece of the key row against two vectors of the weight row)
-      for (int c = part * 8; c < a.C; c += 64) {
-        const uint4 kraw = *reinterpret_cast<const uint4*>(krow + c);
-        const float4 w0 = *reinterpret_cast<const float4*>(wrow + c), w1 = *reinterpret_cast<const float4*>(wrow + c + 4);
-        const uint32_t kw[4] = {kraw.x, kraw.y, kraw.z, kraw.w};
-        const float wv[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const uint16_t bits = (uint16_t)((e & 1) ? (kw[e >> 1] >> 16) : (kw[e >> 1] & 0xffff));
-          sum = fmaf((IN_DT == DT_BF16) ? bf16_bits_to_f32(bits) : f16_bits_to_f32(bits), wv[e], sum);
-        }
-      }
-    }
-    sum += dpp_move<DPP_XOR1>(sum);
-    sum += dpp_move<DPP_XOR2>(sum);
-    sum += dpp_move<DPP_HALF_MIRROR>(sum);
-    if (part == 0) s_off[file][piece] = sum;
-  }
   __syncthreads();
-  const int16_t* gi = a.gidx + (white ? a.nmoves : 0);
-  for (int v = threadIdx.x; v < a.nmoves; v += 256) {
-    const int ft = gi[v];
-    float x = s_a[(ft >> 6) * 65 + (ft & 63)];
-    const int pr = a.gpromo[v];
-    if (pr >= 0) x += s_off[pr >> 2][pr & 3] + s_off[pr >> 2][3];
-    a.logits[(long)b * a.ldl + v] = x;
+  for (int v0 = 0; v0 < a.nmoves; v0 += 256 * PQK_MOVES) {
+#pragma unroll
+    for (int m = 0; m < PQK_MOVES; ++m) {
+      const int v = v0 + 256 * m + (int)threadIdx.x;
+      float x = s_a[(ft[m] >> 6) * 65 + (ft[m] & 63)];
+      if (pr[m] >= 0) x += s_off[pr[m] >> 2][pr[m] & 3] + s_off[pr[m] >> 2][3];
+      if (v < a.nmoves) a.logits[(long)b * a.ldl + v] = x;
+    }
+    if (v0 + 256 * PQK_MOVES < a.nmoves) tables(v0 + 256 * PQK_MOVES);
   }
 }
 

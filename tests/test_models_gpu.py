@@ -227,6 +227,20 @@ def test_bt4class_bias_generator_norms_inside_their_products(cuda, act, fp8):
         assert torch.equal(p2, pol[lo:lo + B]) and torch.equal(w2, wdl[lo:lo + B]), B
 
 
+@pytest.mark.parametrize("act", ["bf16", "f16"])
+@pytest.mark.parametrize("Cm", [64, 128, 192, 256, 320, 512, 832])
+def test_bt4class_policy_product_channel_slabs(cuda, Cm, act):
+    """The policy product's walk over a wave's quarter of the channels: steps of 16 without a slab of four, one, two and three slabs, and slabs with steps left."""
+    oracle = om.test_init_(om.BT4ClassOracle(policy_leela, 1, Cm, 2 * Cm, Cm // 32), seed=8)
+    planes, mask = positions(5, seed=15, leela=True)
+    rpol, _ = oracle.forward_pv(planes)
+    m = models.BT4Class(1, Cm, 2 * Cm, Cm // 32, act_dtype=act)
+    m.load_state_dict(oracle.state_dict())
+    pol = m(planes.to(cuda))[0].cpu()
+    report("channels %d %s" % (Cm, act), pol, rpol, mask)
+    assert rel_rms(pol, rpol) < (2e-2 if act == "bf16" else 4e-3)
+
+
 def test_bt4class_fp8_residuals_normalised_on_ragged_persistent_tiles(cuda):
     """Full width in e4m3: 33, 65, 129 and 131 positions end inside a 128-row tile, the last two on workgroups that walk several
     tiles; 1025 end inside a 256-row one. The residual that is normalised in the epilogue has the same bits on all of them and alone."""
