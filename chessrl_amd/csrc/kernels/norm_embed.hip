@@ -147,7 +147,7 @@ __global__ void __launch_bounds__(256) layernorm_kernel(const LayerNormArgs a) {
 template <bool OUT16, bool OUT8, int RPW>
 __global__ void __launch_bounds__(256) layernorm_trunk_kernel(const LayerNormArgs a) {
   const int lane = threadIdx.x & 63;
-  const long row0 = ((long)blockIdx.x * 4 + (threadIdx.x >> 6)) * RPW;
+  const long row0 = ((long)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * RPW;
   if (row0 >= a.rows) return;
   float x[RPW][2][8], g[2][8], b[2][8];
 #pragma unroll
@@ -211,12 +211,11 @@ __global__ void __launch_bounds__(256) layernorm_trunk_kernel(const LayerNormArg
 }
 
 template <int RPW>
-static bool launch_ln_trunk(const LayerNormArgs& a, hipStream_t st) {
-  const dim3 grid((a.rows / RPW + 3) / 4), block(256);
+static void launch_ln_trunk(const LayerNormArgs& a, int waves, hipStream_t st) {
+  const dim3 grid((a.rows / RPW + waves - 1) / waves), block(64 * waves);
   if (a.out && a.out_fp8) hipLaunchKernelGGL((layernorm_trunk_kernel<true, true, RPW>), grid, block, 0, st, a);
   else if (a.out) hipLaunchKernelGGL((layernorm_trunk_kernel<true, false, RPW>), grid, block, 0, st, a);
   else hipLaunchKernelGGL((layernorm_trunk_kernel<false, true, RPW>), grid, block, 0, st, a);
-  return true;
 }
 
 // Rows longer than 2048 elements (the 8192-wide norm of the bias generator): the four waves of a workgroup share one
@@ -290,8 +289,12 @@ static hipError_t launch_ln_dt(const LayerNormArgs& a, hipStream_t st) {
   if constexpr (IN_DT == DT_BF16) {
     if (a.C == 1024 && !a.rms && a.beta && !a.out_b && (a.out || a.out_fp8) && (!a.out || a.out_dtype == DT_BF16)) {
       // (two rows per wave: 18 % faster than one at 262144 rows, and no slower than four; per-row arithmetic is the same)
-      if (a.rows % 2 == 0) launch_ln_trunk<2>(a, st);
-      else launch_ln_trunk<1>(a, st);
+      // (few rows: the launch is one wave's chain of latencies, and a row's wave alone on its compute unit has the shortest; 64 rows 3.45 us with
+      // two rows per wave, 3.0 with one, 2.7 in workgroups of one wave)
+      const int cus = device_cus();
+      if (a.rows <= 2 * cus) launch_ln_trunk<1>(a, 1, st);
+      else if (a.rows % 2 || a.rows <= 16 * cus) launch_ln_trunk<1>(a, 4, st);
+      else launch_ln_trunk<2>(a, 4, st);
       return hipGetLastError();
     }
   }

@@ -815,6 +815,29 @@ def test_sample_distribution_and_argmax(cuda):
     assert bool((t0 == 7).all())
 
 
+def test_layernorm_trunk_width_workgroups_by_row_count(cuda):
+    """The instance for bf16 rows of 1024 elements takes workgroups of one wave, four waves of a row each or four of two rows by the number of rows: the
+    same bits and the same maximum on both sides of each line, and nothing past the last row."""
+    torch.manual_seed(3)
+    C_, cus = 1024, torch.cuda.get_device_properties(cuda).multi_processor_count
+    most = 16 * cus + 2
+    x = (torch.randn(most, C_, device=cuda) * 3 + 0.5).bfloat16()
+    g, b = torch.randn(C_, device=cuda), torch.randn(C_, device=cuda)
+
+    def run(n):
+        out, out8, amax = torch.full((n + 2, C_), 7.0, dtype=torch.bfloat16, device=cuda), torch.full((n + 2, C_), 1, dtype=torch.uint8, device=cuda), torch.zeros(1, device=cuda)
+        check(lib().crl_layernorm(p(x), C_, _lib.BF16, p(g), p(b), p(out), _lib.BF16, p(out8), 0.7, C_, n, C_, 1e-5, p(amax), stream()), "ln")
+        torch.cuda.synchronize()
+        assert bool((out[n:] == 7).all()) and bool((out8[n:] == 1).all())
+        return out[:n], out8[:n], amax.item()
+
+    ref, ref8, _ = run(most)
+    for n in (1, 2, 3, 64, 2 * cus - 1, 2 * cus, 2 * cus + 1, 2 * cus + 2, 16 * cus - 1, 16 * cus, 16 * cus + 1):
+        out, out8, amax = run(n)
+        assert torch.equal(out, ref[:n]) and torch.equal(out8, ref8[:n]), n
+        assert abs(amax - ref[:n].float().abs().max().item()) <= 2 ** -8 * amax, n
+
+
 @pytest.mark.parametrize("C_,in_dt", [(256, _lib.F32), (1024, _lib.BF16), (8192, _lib.BF16), (1536, _lib.F16)])
 def test_rmsnorm(cuda, C_, in_dt):
     """crl_rmsnorm against torch.nn.functional.rms_norm on the same (rounded) input."""
