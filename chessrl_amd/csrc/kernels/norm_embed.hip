@@ -17,48 +17,6 @@
 
 namespace crl {
 
-// Normalise the VPL*8 values a lane holds (columns col0(i) = (i*64+lane)*8) and write them.
-// rms: RMSNorm (mean taken as zero, no offset): y = x * rsqrt(mean(x^2) + eps) * gamma.
-// FULL: C == VPL * 512, every lane holds VPL whole vectors (no column guards in the instruction stream).
-template <int VPL, bool FULL = false>
-__device__ __forceinline__ void ln_finish(float (&x)[VPL][8], int lane, int C, const float* gamma, const float* beta,
-                                           float eps, float (&y)[VPL][8], float* stats = nullptr, bool rms = false) {
-  float s = 0.f;
-#pragma unroll
-  for (int i = 0; i < VPL; ++i) {
-    if (FULL || (i * 64 + lane) * 8 < C) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) s += x[i][e];
-    }
-  }
-  // (1 / C by the hardware reciprocal, exact for the power-of-two widths and within one unit in the last place otherwise:
-  // two IEEE divisions are 22 of a row's ~400 instructions)
-  const float inv_c = fast_rcp((float)C);
-  const float mean = rms ? 0.f : wave_sum(s) * inv_c;
-  if (rms) beta = nullptr;
-  float q = 0.f;
-#pragma unroll
-  for (int i = 0; i < VPL; ++i) {
-    if (FULL || (i * 64 + lane) * 8 < C) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) { const float d = x[i][e] - mean; q += d * d; }
-    }
-  }
-  const float rstd = rsqrtf(wave_sum(q) * inv_c + eps);
-  if (stats && lane == 0) *reinterpret_cast<float2*>(stats) = make_float2(rstd, -mean * rstd);   // (x - mean) * rstd = x * s0 + s1
-#pragma unroll
-  for (int i = 0; i < VPL; ++i) {
-    const int col = (i * 64 + lane) * 8;
-    if (FULL || col < C) {
-      float gv[8], bv[8];
-      load8<DT_F32>(gamma, col, gv);
-      if (beta) load8<DT_F32>(beta, col, bv);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) y[i][e] = (x[i][e] - mean) * rstd * gv[e] + (beta ? bv[e] : 0.f);
-    }
-  }
-}
-
 // (fp32 rows: a lane's columns are two groups of four per vector, see norm_column; 16-bit rows: eight consecutive ones)
 template <int IN_DT, int VPL, bool FULL = false>
 __global__ void __launch_bounds__(256) layernorm_kernel(const LayerNormArgs a) {
@@ -321,76 +279,109 @@ hipError_t launch_layernorm(const LayerNormArgs& a, hipStream_t st) {
 }
 
 // ---- embedding ------------------------------------------------------------------------
+// A wave per token; lane p holds feature p. At few tokens the launch is one wave's trips to memory, beyond them the activation and the
+// norm on the vector units. The weight rows of the features that are not zero (3 to 8 of 19) are requested EMB_ROWS at a time, all vectors of
+// a row together (one by one, each behind a branch and its own wait: 8.6 us for 64 tokens of 1024, 12.2 for 4096, 89 for 64000; now 6.4,
+// 9.7 and 81). Two rows at a time and scale, offset and gates read where they are used keep six or more waves on a SIMD: with four rows and
+// those reads up front 64 tokens take 6.1 but 64000 105 us; a wave that keeps them in registers and walks a square of several
+// positions was no faster anywhere.
+constexpr int EMB_ROWS = 2;
 template <int VPL>
 __global__ void __launch_bounds__(256) embed_kernel(const EmbedArgs a) {
   const int lane = threadIdx.x & 63;
-  const int tok = blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int tok = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
   if (tok >= a.tokens) return;
   const int sqr = tok & 63;
-
-  // The 19 input features of this token (uniform across the wave).
-  float f[19];
+  float f = 0.f;
   if (a.planes) {
-#pragma unroll
-    for (int p = 0; p < 19; ++p) f[p] = a.planes[(long)tok * 19 + p];
+    if (lane < 19) f = a.planes[(long)tok * 19 + lane];
   } else {
-    const int b = tok >> 6;
     const int id = a.ids[tok];
-    const uint8_t* fl = a.flags + b * 4;
-#pragma unroll
-    for (int p = 0; p < 12; ++p) f[p] = (id == p + 1) ? 1.f : 0.f;
-    f[12] = fl[0] ? 1.f : 0.f;
-    f[13] = (fl[2] == sqr) ? 1.f : 0.f;
-    f[14] = (fl[1] & 1) ? 1.f : 0.f;
-    f[15] = (fl[1] & 2) ? 1.f : 0.f;
-    f[16] = (fl[1] & 4) ? 1.f : 0.f;
-    f[17] = (fl[1] & 8) ? 1.f : 0.f;
-    f[18] = fminf((float)fl[3] / 100.0f, 1.0f);
+    const uint8_t* fl = a.flags + (tok >> 6) * 4;
+    if (lane < 12) f = id == lane + 1 ? 1.f : 0.f;
+    else if (lane == 12) f = fl[0] ? 1.f : 0.f;
+    else if (lane == 13) f = fl[2] == sqr ? 1.f : 0.f;
+    else if (lane < 18) f = (fl[1] >> (lane - 14)) & 1 ? 1.f : 0.f;
+    else if (lane == 18) f = fminf((float)fl[3] / 100.0f, 1.0f);
   }
-
-  float x[VPL][8], y[VPL][8];
+  float x[VPL][8];
 #pragma unroll
   for (int i = 0; i < VPL; ++i) {
     const int col = (i * 64 + lane) * 8;
-    if (col < a.C) {
-      load8<DT_F32>(a.b1, col, x[i]);
+    if (col < a.C) load8<DT_F32>(a.b1, col, x[i]);
+  }
+  uint32_t left = (uint32_t)__ballot(f != 0.f);   // the features that are not zero, added in their order
+  while (left) {
+    float w[EMB_ROWS][VPL][8], fv[EMB_ROWS];
+    int cnt = 0;
 #pragma unroll
-      for (int p = 0; p < 19; ++p) {
-        if (f[p] != 0.f) {  // uniform branch: most planes are zero for a given token
-          float w[8];
-          load8<DT_F32>(a.w1t, (long)p * a.C + col, w);
+    for (int k = 0; k < EMB_ROWS; ++k)
+      if (left) {
+        const int p = __builtin_ctz(left);
+        left &= left - 1;
+        cnt = k + 1;
+        fv[k] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(f), p));
 #pragma unroll
-          for (int e = 0; e < 8; ++e) x[i][e] = fmaf(f[p], w[e], x[i][e]);
+        for (int i = 0; i < VPL; ++i) {
+          const int col = (i * 64 + lane) * 8;
+          if (col < a.C) load8<DT_F32>(a.w1t, (long)p * a.C + col, w[k][i]);
         }
       }
 #pragma unroll
-      for (int e = 0; e < 8; ++e) x[i][e] = apply_act(x[i][e], a.act);
-    }
+    for (int k = 0; k < EMB_ROWS; ++k)
+      if (k < cnt) {
+#pragma unroll
+        for (int i = 0; i < VPL; ++i)
+          if ((i * 64 + lane) * 8 < a.C) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) x[i][e] = fmaf(fv[k], w[k][i][e], x[i][e]);
+          }
+      }
   }
-  ln_finish<VPL>(x, lane, a.C, a.ln_g, a.ln_b, a.eps, y);
+  float s = 0.f;
+#pragma unroll
+  for (int i = 0; i < VPL; ++i)
+    if ((i * 64 + lane) * 8 < a.C) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) { x[i][e] = apply_act(x[i][e], a.act); s += x[i][e]; }
+    }
+  // (1 / C by the hardware reciprocal, exact for the power-of-two widths and within one unit in the last place otherwise)
+  const float inv_c = fast_rcp((float)a.C);
+  const float mean = wave_sum(s) * inv_c;
+  float q = 0.f;
+#pragma unroll
+  for (int i = 0; i < VPL; ++i)
+    if ((i * 64 + lane) * 8 < a.C) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) { const float d = x[i][e] - mean; q += d * d; }
+    }
+  const float rstd = rsqrtf(wave_sum(q) * inv_c + a.eps);
   const long orow = a.out_T > 64 ? (long)(tok >> 6) * a.out_T + sqr : (long)tok;
   float am = 0.f;
 #pragma unroll
   for (int i = 0; i < VPL; ++i) {
     const int col = (i * 64 + lane) * 8;
     if (col < a.C) {
-      float ga[8], gb[8];
+      float y[8];
+      float lg[8], lb[8], ga[8], gb[8];
+      load8<DT_F32>(a.ln_g, col, lg);
+      load8<DT_F32>(a.ln_b, col, lb);
       load8<DT_F32>(a.gate_a_exp, (long)sqr * a.C + col, ga);
       load8<DT_F32>(a.gate_b, (long)sqr * a.C + col, gb);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) y[i][e] = y[i][e] * ga[e] + gb[e];
+      for (int e = 0; e < 8; ++e) y[e] = ((x[i][e] - mean) * rstd * lg[e] + lb[e]) * ga[e] + gb[e];
       if (a.pe) {
         float pe[8];
         load8<DT_F32>(a.pe, (long)sqr * a.C + col, pe);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) y[i][e] += pe[e];
+        for (int e = 0; e < 8; ++e) y[e] += pe[e];
       }
-      store8(a.out, orow * a.C + col, y[i], a.out_dtype);
-      if (a.out_b) store8(a.out_b, orow * a.C + col, y[i], a.out_b_dtype);
-      if (a.out_fp8) store8_fp8(a.out_fp8, orow * a.C + col, y[i], a.fp8_scale);
+      store8(a.out, orow * a.C + col, y, a.out_dtype);
+      if (a.out_b) store8(a.out_b, orow * a.C + col, y, a.out_b_dtype);
+      if (a.out_fp8) store8_fp8(a.out_fp8, orow * a.C + col, y, a.fp8_scale);
       if (a.amax) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) am = fmaxf(am, fabsf(y[i][e]));
+        for (int e = 0; e < 8; ++e) am = fmaxf(am, fabsf(y[e]));
       }
     }
   }
@@ -426,8 +417,9 @@ hipError_t launch_token_embed(const TokenEmbedArgs& a, hipStream_t st) {
 hipError_t launch_embed(const EmbedArgs& a, hipStream_t st) {
   if (a.tokens <= 0) return hipSuccess;
   if (a.C % 8 || a.C > 2048) return hipErrorInvalidValue;
-  const dim3 grid((a.tokens + 3) / 4), block(256);
   const int vecs = (a.C / 8 + 63) / 64;
+  const int waves = a.tokens <= 2 * device_cus() ? 1 : 4;   // (few tokens: a wave alone on its compute unit has the shortest chain)
+  const dim3 grid((a.tokens + waves - 1) / waves), block(64 * waves);
   if (vecs <= 1) hipLaunchKernelGGL((embed_kernel<1>), grid, block, 0, st, a);
   else if (vecs <= 2) hipLaunchKernelGGL((embed_kernel<2>), grid, block, 0, st, a);
   else hipLaunchKernelGGL((embed_kernel<4>), grid, block, 0, st, a);

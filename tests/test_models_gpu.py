@@ -71,6 +71,24 @@ def test_gpt_plumbing_config(cuda):
     assert torch.equal(shuf[:, 0].cpu(), pol[perm])
 
 
+def test_embedding_adds_any_number_of_features(cuda):
+    """Tokens with 0 to 19 features that are not zero, of any value, at row counts on both sides of the launch's line: against the oracle, and each position's
+    bits alone and in the batch."""
+    oracle = om.test_init_(om.GPTOracle(1, 4, 256), seed=4)
+    g = torch.Generator().manual_seed(7)
+    planes = torch.randn(12, 64, 19, generator=g)
+    keep = torch.rand(12, 64, 19, generator=g).argsort(-1) < torch.arange(12 * 64).remainder(20).view(12, 64, 1)
+    planes = planes * keep
+    planes[3] = 0.0
+    ref = oracle.forward_last(planes)
+    m = models.GPT(models.GPTConfig(block_size=256, vocab_size=1929, n_layer=1, n_head=4, n_embd=256))
+    m.load_state_dict(oracle.state_dict())
+    out = m.forward((planes.to(cuda), None))[0][:, 0]
+    assert rel_rms(out.cpu(), ref) < 1e-2
+    for i in range(12):
+        assert torch.equal(m.forward((planes[i:i + 1].to(cuda), None))[0][0, 0], out[i])
+
+
 def test_gpt_state_dict_roundtrip_and_move(cuda):
     m = models.GPT(models.GPTConfig(block_size=256, vocab_size=1929, n_layer=2, n_head=8, n_embd=256))
     sd = m.state_dict()
