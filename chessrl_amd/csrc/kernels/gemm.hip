@@ -266,12 +266,21 @@ __global__ void __launch_bounds__(Cfg::NT_ALL, Cfg::MIN_WAVES) gemm_kernel(const
 // epilogue of the one-pass kernels: C = res + alpha*act(descale*sum + bias), amax, the fp8 output scale, the C/C2 split.
 // The four columns n..n+3 of row m: slices added in order, epilogue applied, result stored; v receives the values
 // (as stored: rounded to the output type) and the return value their largest magnitude.
-template <int OUT_DT>
+template <int OUT_DT, int GROUPS = 1>
 __device__ __forceinline__ float reduce_columns4(const GemmArgs& a, const float* partial, int ks, long ldp, int m, int n, float (&v)[4]) {
   f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
-  const float* pp = partial + (long)m * ldp + n;
+  const float* pp = partial + (long)m * ldp + n;   // ldp is a multiple of 4 and >= N rounded up
+  auto share = [&](int y) { return *reinterpret_cast<const f32x4_t*>(pp + (long)y * a.M * ldp); };
+  if constexpr (GROUPS == 4) {
+#pragma unroll 4
+    for (int s = 0; s < ks; ++s) {
+      const f32x4_t g0 = share(4 * s), g1 = share(4 * s + 1), g2 = share(4 * s + 2), g3 = share(4 * s + 3);
+      acc += g0 + g1 + g2 + g3;
+    }
+  } else {
 #pragma unroll 8
-  for (int s = 0; s < ks; ++s) acc += *reinterpret_cast<const f32x4_t*>(pp + (long)s * a.M * ldp);   // ldp is a multiple of 4 and >= N rounded up
+    for (int s = 0; s < ks; ++s) acc += share(s);
+  }
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const float b = (a.bias && n + i < a.N) ? a.bias[n + i] : 0.f;
@@ -309,7 +318,7 @@ __device__ __forceinline__ float reduce_columns4(const GemmArgs& a, const float*
   return amax;
 }
 
-template <int OUT_DT>
+template <int OUT_DT, int GROUPS = 1>
 __global__ void __launch_bounds__(256) splitk_reduce_kernel(const GemmArgs a, const float* partial, int ks, long ldp) {
   const int groups = (a.N + 3) / 4;
   const long idx = (long)blockIdx.x * 256 + threadIdx.x;
@@ -317,7 +326,7 @@ __global__ void __launch_bounds__(256) splitk_reduce_kernel(const GemmArgs a, co
   float local_amax = 0.f;
   if (m < a.M) {
     float v[4];
-    local_amax = reduce_columns4<OUT_DT>(a, partial, ks, ldp, m, n, v);
+    local_amax = reduce_columns4<OUT_DT, GROUPS>(a, partial, ks, ldp, m, n, v);
   }
   if (a.amax) {
     local_amax = wave_max(local_amax);
@@ -530,6 +539,33 @@ static int splitk_plan_fixed(const GemmArgs& a, int esz, int* slabs_per_slice) {
   return ks;
 }
 
+// At few rows the walk above waits for memory slab by slab on a fraction of the chip. There every (slice, group) is a workgroup of the ring kernel,
+// and the second pass adds four groups to a slice's sum and then the slices, as above: the same bits. Needs slices of equal length in whole rounds of the
+// groups. 8192 -> 128 behind cold caches, both passes: 1 row 21.7 -> 10.7 us, 64 24.1 -> 11.8, 496 23.8 -> 15.0, 1000 24.6 -> 20.4; 1521 and more the same
+// or slower. A second workgroup on a CU pays with eight slabs each (4096 -> 200, four: 256 rows 17.5 -> 15.0 us, but 400 17.6 -> 19.6).
+static bool ring_shares(const GemmArgs& a, int in_dt, int ks, int per) {
+  const long ldp = (a.N + 7) / 8 * 8, tiles = (long)((a.M + 63) / 64) * ((a.N + 63) / 64) * ks * 4;
+  return (in_dt == DT_BF16 || in_dt == DT_F16) && (long)a.K * 2 == 128L * ks * per && per % 4 == 0 && tiles <= (per >= 32 ? 2 : 1) * device_cus() && a.lda < 1L << 24 && a.ldw < 1L << 24 &&
+         (size_t)ks * 4 * a.M * ldp * sizeof(float) <= (a.splitk_ws ? (size_t)a.splitk_ws_bytes : SPLITK_WS_BYTES);
+}
+
+template <int OUT_DT>
+static hipError_t launch_ring_shares(const GemmArgs& a, int in_dt, int ks, hipStream_t st) {
+  float* ws = a.splitk_ws;
+  hipError_t e = ws ? hipSuccess : workspace_for(st, &ws);
+  if (e != hipSuccess) return e;
+  const long ldp = (a.N + 7) / 8 * 8;
+  GemmArgs b = a;
+  b.C = b.C2 = ws; b.ldc = b.ldc2 = ldp; b.nsplit = a.N; b.vec_ok = 1;
+  b.bias = nullptr; b.res = nullptr; b.amax = nullptr; b.act = ACT_NONE; b.descale = 1.f; b.alpha = 1.f; b.out_scale = 1.f; b.w_once = 0;
+  const long small = (long)((a.M + 31) / 32) * ((a.N + 31) / 32) * ks * 4;
+  e = launch_gemm_dmas_sliced(b, in_dt, st, small <= device_cus() ? 32 : 64, 4 * ks);
+  if (e != hipSuccess) return e;
+  const long threads = (long)a.M * ((a.N + 3) / 4);
+  hipLaunchKernelGGL((splitk_reduce_kernel<OUT_DT, 4>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st, a, ws, ks, ldp);
+  return hipGetLastError();
+}
+
 bool gemm_folds_layernorm(const GemmArgs& a, int in_dt) {
   int per = 0;
   return a.k_parallel && a.N <= 4096 && (a.nsplit <= 0 || a.nsplit >= a.N || !a.C2) && splitk_plan(a, in_dt == DT_FP8 ? 1 : 2, false, &per) > 1;
@@ -605,6 +641,7 @@ static hipError_t launch_in_out(const GemmArgs& a, int tile, hipStream_t st) {
     if (tile == 1 && !a.k_parallel && !a.res_stats) {
       int per = 0;
       const int ks = splitk_plan_fixed(a, IN_DT == DT_FP8 ? 1 : 2, &per);
+      if (ks > 1 && !a.ln_out && ring_shares(a, IN_DT, ks, per)) return launch_ring_shares<OUT_DT>(a, IN_DT, ks, st);
       if (ks > 1) return launch_splitk<CfgSmallK4, IN_DT, OUT_DT>(a, ks, per, st);
     }
     // K in whole slabs: the kernels with direct-to-LDS rings (bit-equal). 32x32 tiles while every such tile has a CU of its own

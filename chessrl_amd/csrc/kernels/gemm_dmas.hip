@@ -24,4 +24,13 @@ hipError_t launch_gemm_dmas(const GemmArgs& a, int in_dt, int out_dt, hipStream_
   return a.k_parallel ? launch_small<DmasCfg<32, 4>>(a, in_dt, out_dt, st) : launch_small<DmasCfg<32>>(a, in_dt, out_dt, st);
 }
 
+// K in 4 n equal shares (SLICED), 16-bit operands: the raw fp32 sums of share y in rows y M .. of C.
+hipError_t launch_gemm_dmas_sliced(const GemmArgs& a, int in_dt, hipStream_t st, int tile_size, int shares) {
+  if (in_dt == DT_BF16)
+    return tile_size == 64 ? launch_dmas<DmasCfg<64>, DT_BF16, DT_F32, 0, 1>(a, st, shares) : launch_dmas<DmasCfg<32>, DT_BF16, DT_F32, 0, 1>(a, st, shares);
+  if (in_dt == DT_F16)
+    return tile_size == 64 ? launch_dmas<DmasCfg<64>, DT_F16, DT_F32, 0, 1>(a, st, shares) : launch_dmas<DmasCfg<32>, DT_F16, DT_F32, 0, 1>(a, st, shares);
+  return hipErrorInvalidValue;
+}
+
 }  // namespace crl

@@ -194,8 +194,12 @@ __device__ __forceinline__ void small_full(const SmallArgs& s, const float (&acc
 }
 
 // ONCE: GemmArgs::w_once (an instance of its own: a branch at every load cost a call of one position 2 %)
-template <typename Cfg, int IN_DT, int OUT_DT, int ONCE = 0>
-__global__ void __launch_bounds__(Cfg::NT) gemm_dmas_kernel(const SmallArgs s) {
+// SLICED: the fp32 sums of K share y = blockIdx.y go to rows y M .. y M + M - 1 of C. Share y is what group y % 4 of a four-group workgroup walks of slice
+// y / 4 of K: nslab slabs, every fourth one.
+template <typename Cfg, int IN_DT, int OUT_DT, int ONCE = 0, int SLICED = 0>
+__global__ void __launch_bounds__(Cfg::NT) gemm_dmas_kernel(const SmallArgs s_in) {
+  SmallArgs s = s_in;
+  if constexpr (SLICED) s.C = reinterpret_cast<float*>(s.C) + (long)blockIdx.y * s.M * s.ldc;
   constexpr int KSTEPS = Cfg::ROWB / (IN_DT == DT_FP8 ? 64 : 32);   // MFMA K steps per slab
   constexpr int BM = Cfg::BM, BN = Cfg::BN, LOADS = Cfg::LOADS, NSTAGE = Cfg::NSTAGE, AHEAD = Cfg::AHEAD, EV = Cfg::EV;
   constexpr int STAGE = Cfg::STAGE;
@@ -262,15 +266,16 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_dmas_kernel(const SmallArgs s) {
       voff[i] = (uint32_t)r * (uint32_t)ld + (((lane & 7) ^ (lane >> 3) ^ ((rbase / 8 + i) & 7)) << 4);
     }
     // (the rows of a tile span less than 2 GB: the launcher checks)
-    const uint8_t* origin = reinterpret_cast<const uint8_t*>(loads_a ? s.A : s.W) + (long)(loads_a ? m0 : n0) * ld;
+    const uint8_t* origin = reinterpret_cast<const uint8_t*>(loads_a ? s.A : s.W) + (long)(loads_a ? m0 : n0) * ld + (SLICED ? (long)((blockIdx.y >> 2) * 4 * nslab + (blockIdx.y & 3)) * Cfg::ROWB : 0);
     const __amdgpu_buffer_rsrc_t rsrc_mine = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(origin), 0, (rows_left < BM ? rows_left : BM) * ld, 0x00020000);
     const uint32_t lds_load0 = (loads_a ? Cfg::PART_BYTES : 0) + rbase * Cfg::ROWB;   // stage 0
     auto issue_slab = [&](int slab) {
       uint8_t* dst = smem + lds_load0 + (slab & (NSTAGE - 1)) * STAGE;
       static_for<0, LOADS>([&](auto ic) {
         constexpr int i = decltype(ic)::value;
-        if (ONCE && !loads_a) dmaf_load16_nt(rsrc_mine, dst + i * 1024, (int)voff[i], slab * Cfg::ROWB);
-        else dmaf_load16(rsrc_mine, dst + i * 1024, (int)voff[i], slab * Cfg::ROWB);
+        constexpr int STEP = SLICED ? 4 * Cfg::ROWB : Cfg::ROWB;
+        if (ONCE && !loads_a) dmaf_load16_nt(rsrc_mine, dst + i * 1024, (int)voff[i], slab * STEP);
+        else dmaf_load16(rsrc_mine, dst + i * 1024, (int)voff[i], slab * STEP);
       });
     };
 #pragma unroll
@@ -431,20 +436,21 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_dmas_kernel(const SmallArgs s) {
   dmas_barrier();
 }
 
-template <typename Cfg, int IN_DT, int OUT_DT, int ONCE = 0>
-static hipError_t launch_dmas(const GemmArgs& a, hipStream_t st) {
-  if constexpr (Cfg::KP == 1 && !ONCE) {
+template <typename Cfg, int IN_DT, int OUT_DT, int ONCE = 0, int SLICED = 0>
+static hipError_t launch_dmas(const GemmArgs& a, hipStream_t st, int shares = 1) {
+  static_assert(!SLICED || (Cfg::KP == 1 && OUT_DT == DT_F32), "a share's sums as they are");
+  if constexpr (Cfg::KP == 1 && !ONCE && !SLICED) {
     // (up to 512 rows: the weight rows that more tiles share do better kept in L2; 8 positions 1062 -> 1013 us, 12 the same, 16 1222 -> 1262)
     if (a.w_once && a.M <= 512) return launch_dmas<Cfg, IN_DT, OUT_DT, 1>(a, st);
   }
   static std::atomic<bool> attr_set[16] = {};
   constexpr int ESZ = IN_DT == DT_FP8 ? 1 : 2;
   auto fits = [](long v) { return v >= 0 && v < (1L << 31); };
-  if ((a.K * ESZ) % Cfg::ROWB != 0 || a.K <= 0 || a.res_stats || !fits(a.lda * ESZ * 64) || !fits(a.ldw * ESZ * 64) || !fits(a.ldc) || !fits(a.ldc2) || (a.res && !fits(a.ldr)))
+  if ((a.K * ESZ) % (Cfg::ROWB * shares) != 0 || a.K <= 0 || a.res_stats || !fits(a.lda * ESZ * 64) || !fits(a.ldw * ESZ * 64) || !fits(a.ldc) || !fits(a.ldc2) || (a.res && !fits(a.ldr)))
     return hipErrorInvalidValue;
   int dev = 0;
   (void)hipGetDevice(&dev);
-  auto kern = gemm_dmas_kernel<Cfg, IN_DT, OUT_DT, ONCE>;
+  auto kern = gemm_dmas_kernel<Cfg, IN_DT, OUT_DT, ONCE, SLICED>;
   if (dev < 0 || dev >= 16 || !attr_set[dev]) {
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::LDS_BYTES);
     if (e != hipSuccess) return e;
@@ -456,7 +462,7 @@ static hipError_t launch_dmas(const GemmArgs& a, hipStream_t st) {
   SmallArgs s{};
   s.A = a.A; s.W = a.W; s.C = a.C; s.C2 = a.C2; s.bias = a.bias; s.res = a.res; s.amax = a.amax;
   s.lda_b = (int)(a.lda * ESZ); s.ldw_b = (int)(a.ldw * ESZ); s.ldc = (int)a.ldc; s.ldc2 = (int)a.ldc2; s.ldr = (int)a.ldr;
-  s.M = a.M; s.N = a.N; s.nslab = a.K * ESZ / Cfg::ROWB; s.nsplit = a.nsplit;
+  s.M = a.M; s.N = a.N; s.nslab = a.K * ESZ / Cfg::ROWB / shares; s.nsplit = a.nsplit;
   s.act = a.act; s.res_dtype = a.res_dtype; s.res_rows = a.res_rows; s.vec_ok = a.vec_ok;
   s.descale = a.descale; s.alpha = a.alpha; s.out_scale = a.out_scale;
   // Rows or columns of tiles first, whichever lets an XCD read fewer rows of both operands: each XCD's L2 fetches its own copy (BT4-class bf16, whole calls
@@ -467,7 +473,7 @@ static hipError_t launch_dmas(const GemmArgs& a, hipStream_t st) {
   s.by_cols = Cfg::KP == 1 && tiles_m >= 4 && by_cols < by_rows;
   s.inner = s.by_cols ? tiles_m : tiles_n;
   s.m_inner = dmaf_magic(s.inner); s.per_xcd = tiles >> 3;
-  hipLaunchKernelGGL(kern, dim3(tiles), dim3(Cfg::NT), Cfg::LDS_BYTES, st, s);
+  hipLaunchKernelGGL(kern, dim3(tiles, shares), dim3(Cfg::NT), Cfg::LDS_BYTES, st, s);
   return hipGetLastError();
 }
 

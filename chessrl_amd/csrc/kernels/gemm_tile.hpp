@@ -527,6 +527,7 @@ bool gemm_dmam_has(int in_dt, int out_dt);
 hipError_t launch_gemm_dmam(const GemmArgs& a, int in_dt, int out_dt, int cus, hipStream_t st);
 // gemm_dmas.hip: the 64x64 and 32x32 tiles of products that leave every tile a CU (the operand types of gemm_dmam_has).
 hipError_t launch_gemm_dmas(const GemmArgs& a, int in_dt, int out_dt, hipStream_t st, int tile_size);
+hipError_t launch_gemm_dmas_sliced(const GemmArgs& a, int in_dt, hipStream_t st, int tile_size, int shares);
 // gemm_shortk.hip: K = 256 e4m3 operands, bare scaled product: a workgroup keeps 256 rows of A in registers and walks N.
 bool gemm_shortk_can(const GemmArgs& a, int in_dt, int out_dt);
 hipError_t launch_gemm_shortk(const GemmArgs& a, int in_dt, int out_dt, hipStream_t st);

@@ -441,6 +441,32 @@ def test_gemm_short_k_rows_resident_rejects_what_it_cannot_do(cuda):
     torch.cuda.synchronize()
 
 
+@pytest.mark.parametrize("N,K,in_dt,out_dt", [(128, 8192, _lib.BF16, _lib.BF16), (128, 8192, _lib.F16, _lib.F16), (200, 4096, _lib.BF16, _lib.F32), (72, 4608, _lib.BF16, _lib.BF16)])
+def test_gemm_narrow_output_long_k_at_few_rows(cuda, N, K, in_dt, out_dt):
+    """A narrow output with a long K, where few rows take a workgroup per slice and group of K and more rows one per slice: the same bits on both sides of the
+    line (72 columns of K = 4608: slices that are not whole rounds of the groups stay on one path), and the fp32 product within the rounding of the output."""
+    torch.manual_seed(N)
+    most = 1500
+    A = torch.randn(most, K, device=cuda).to(TORCH_DT[in_dt])
+    W = (torch.randn(N, K, device=cuda) * K ** -0.5).to(TORCH_DT[in_dt])
+    bias = torch.randn(N, device=cuda)
+    R = torch.randn(most, N, device=cuda).to(TORCH_DT[in_dt])
+
+    def run(M):
+        out = torch.full((M + 1, N), 7.0, dtype=TORCH_DT[out_dt], device=cuda)
+        check(lib().crl_gemm(p(A), K, p(W), K, p(out), N, M, N, K, in_dt, out_dt, p(bias), 0, 1.0, 0.5, p(R), N, in_dt, 1.0, None, 0, stream()), "gemm")
+        torch.cuda.synchronize()
+        assert bool((out[M] == 7).all())
+        return out[:M]
+
+    full = run(most)
+    ref = (A.double() @ W.double().t() + bias.double()) * 0.5 + R.double()
+    eps = {_lib.F32: 2 ** -18, _lib.BF16: 2 ** -8, _lib.F16: 2 ** -11}[out_dt]
+    assert ((full.double() - ref).abs() <= eps * ref.abs() + 2e-5).all()
+    for M in (1, 31, 32, 33, 64, 65, 128, 129, 256, 257, 512, 513, 1024, 1025):
+        assert torch.equal(run(M), full[:M]), M
+
+
 @pytest.mark.parametrize("C_,in_dt", [(256, _lib.F32), (1024, _lib.BF16), (512, _lib.BF16), (8192, _lib.BF16), (768, _lib.F32), (1536, _lib.F32)])
 def test_layernorm(cuda, C_, in_dt):
     torch.manual_seed(C_)
