@@ -18,77 +18,115 @@
 namespace crl {
 
 // (fp32 rows: a lane's columns are two groups of four per vector, see norm_column; 16-bit rows: eight consecutive ones)
-template <int IN_DT, int VPL, bool FULL = false>
+// Bound by memory at many rows, by one wave's trips to it at few: everything a wave reads (RPW rows, then scale and offset, which the rows share) is
+// requested before the first reduction. 97344 rows of 512 bf16 41.7 -> 35.0 us (5.7 TB/s), 32768 of 768 fp32 27.8 -> 25.5, 96000 73.7 -> 69.4, against one
+// row per wave with scale and offset read behind the reductions; four rows per wave 39.3 for the first.
+// ONCE: the rows are read past the caches (see the launch).
+template <int IN_DT, int VPL, bool FULL = false, int RPW = 1, bool ONCE = false>
 __global__ void __launch_bounds__(256) layernorm_kernel(const LayerNormArgs a) {
   constexpr bool F32 = IN_DT == DT_F32;
   const int lane = threadIdx.x & 63;
-  const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (row >= a.rows) return;
+  const long row0 = ((long)blockIdx.x * 4 + (threadIdx.x >> 6)) * RPW;
+  if (row0 >= a.rows) return;
   const int C = FULL ? VPL * 512 : a.C;
   auto has = [&](int i, int h) { return FULL || norm_column(F32, i, h, lane) < C; };
-  float x[VPL][8];
-#pragma unroll
-  for (int i = 0; i < VPL; ++i) load_norm8<IN_DT>(a.x, (long)row * a.ldx, i, lane, C, x[i]);
-  float s = 0.f;
-#pragma unroll
-  for (int i = 0; i < VPL; ++i)
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-      if (has(i, h)) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) s += x[i][4 * h + e];
-      }
-  // (1 / C by the hardware reciprocal, exact for the power-of-two widths and within one unit in the last place otherwise:
-  // two IEEE divisions are 22 of a row's ~400 instructions)
-  const float inv_c = fast_rcp((float)C);
   const bool rms = a.rms != 0;
-  const float mean = rms ? 0.f : wave_sum(s) * inv_c;
   const float* const beta = rms ? nullptr : a.beta;
-  float q = 0.f;
+  float x[RPW][VPL][8], g[VPL][8], b[VPL][8];
+#pragma unroll
+  for (int r = 0; r < RPW; ++r) {
+    const long row = RPW > 1 && row0 + r >= a.rows ? a.rows - 1 : row0 + r;
+#pragma unroll
+    for (int i = 0; i < VPL; ++i) {
+      if constexpr (ONCE) {
+        static_assert(!F32, "16-bit rows");
+        if (has(i, 0)) {
+          const i32x4_t raw = __builtin_nontemporal_load(reinterpret_cast<const i32x4_t*>(reinterpret_cast<const uint16_t*>(a.x) + row * a.ldx + norm_column(false, i, 0, lane)));
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const uint16_t lo = (uint16_t)((uint32_t)raw[e] & 0xffff), hi = (uint16_t)((uint32_t)raw[e] >> 16);
+            x[r][i][2 * e] = IN_DT == DT_BF16 ? bf16_bits_to_f32(lo) : f16_bits_to_f32(lo);
+            x[r][i][2 * e + 1] = IN_DT == DT_BF16 ? bf16_bits_to_f32(hi) : f16_bits_to_f32(hi);
+          }
+        }
+      } else {
+        load_norm8<IN_DT>(a.x, row * a.ldx, i, lane, C, x[r][i]);
+      }
+    }
+  }
 #pragma unroll
   for (int i = 0; i < VPL; ++i)
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
-      if (has(i, h)) {
+    for (int h = 0; h < 2; ++h) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) { const float d = x[i][4 * h + e] - mean; q += d * d; }
-      }
-  const float rstd = rsqrtf(wave_sum(q) * inv_c + a.eps);
-  if (a.stats && lane == 0) *reinterpret_cast<float2*>(a.stats + 2 * (long)row) = make_float2(rstd, -mean * rstd);   // (x - mean) * rstd = x * s0 + s1
-  float am = 0.f;
-#pragma unroll
-  for (int i = 0; i < VPL; ++i) {
-    float y[8];
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
+      for (int e = 0; e < 4; ++e) g[i][4 * h + e] = b[i][4 * h + e] = 0.f;
       if (has(i, h)) {
         const int col = norm_column(F32, i, h, lane);
         const float4 gv = *reinterpret_cast<const float4*>(a.gamma + col);
-        const float g[4] = {gv.x, gv.y, gv.z, gv.w};
-        float bo[4] = {0.f, 0.f, 0.f, 0.f};
+        g[i][4 * h] = gv.x; g[i][4 * h + 1] = gv.y; g[i][4 * h + 2] = gv.z; g[i][4 * h + 3] = gv.w;
         if (beta) {
           const float4 bv = *reinterpret_cast<const float4*>(beta + col);
-          bo[0] = bv.x; bo[1] = bv.y; bo[2] = bv.z; bo[3] = bv.w;
-        }
-#pragma unroll
-        for (int e = 0; e < 4; ++e) y[4 * h + e] = (x[i][4 * h + e] - mean) * rstd * g[e] + bo[e];
-        if (a.amax) {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) am = fmaxf(am, fabsf(y[4 * h + e]));
-        }
-        if constexpr (F32) {
-          const long off = (long)row * a.ldo + col;
-          if (a.out) store4(a.out, off, y + 4 * h, a.out_dtype);
-          if (a.out_b) store4(a.out_b, off, y + 4 * h, a.out_b_dtype);
-          if (a.out_fp8) store4_fp8(a.out_fp8, off, y + 4 * h, a.fp8_scale);
+          b[i][4 * h] = bv.x; b[i][4 * h + 1] = bv.y; b[i][4 * h + 2] = bv.z; b[i][4 * h + 3] = bv.w;
         }
       }
-    if constexpr (!F32) {
-      if (has(i, 0)) {
-        const long off = (long)row * a.ldo + norm_column(false, i, 0, lane);
-        if (a.out) store8(a.out, off, y, a.out_dtype);
-        if (a.out_b) store8(a.out_b, off, y, a.out_b_dtype);
-        if (a.out_fp8) store8_fp8(a.out_fp8, off, y, a.fp8_scale);
+    }
+  if constexpr (RPW > 1) __builtin_amdgcn_sched_barrier(0);   // (no use of a loaded value, and so no wait, moves up between the loads)
+  // (1 / C by the hardware reciprocal, exact for the power-of-two widths and within one unit in the last place otherwise:
+  // two IEEE divisions are 22 of a row's ~400 instructions)
+  const float inv_c = fast_rcp((float)C);
+  float am = 0.f;
+#pragma unroll
+  for (int r = 0; r < RPW; ++r) {
+    const long row = row0 + r;
+    if (RPW > 1 && row >= a.rows) break;
+    float s = 0.f;
+#pragma unroll
+    for (int i = 0; i < VPL; ++i)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        if (has(i, h)) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) s += x[r][i][4 * h + e];
+        }
+    const float mean = rms ? 0.f : wave_sum(s) * inv_c;
+    float q = 0.f;
+#pragma unroll
+    for (int i = 0; i < VPL; ++i)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        if (has(i, h)) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) { const float d = x[r][i][4 * h + e] - mean; q += d * d; }
+        }
+    const float rstd = rsqrtf(wave_sum(q) * inv_c + a.eps);
+    if (a.stats && lane == 0) *reinterpret_cast<float2*>(a.stats + 2 * row) = make_float2(rstd, -mean * rstd);   // (x - mean) * rstd = x * s0 + s1
+#pragma unroll
+    for (int i = 0; i < VPL; ++i) {
+      float y[8];
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        if (has(i, h)) {
+          const int col = norm_column(F32, i, h, lane);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) y[4 * h + e] = (x[r][i][4 * h + e] - mean) * rstd * g[i][4 * h + e] + b[i][4 * h + e];
+          if (a.amax) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) am = fmaxf(am, fabsf(y[4 * h + e]));
+          }
+          if constexpr (F32) {
+            const long off = row * a.ldo + col;
+            if (a.out) store4(a.out, off, y + 4 * h, a.out_dtype);
+            if (a.out_b) store4(a.out_b, off, y + 4 * h, a.out_b_dtype);
+            if (a.out_fp8) store4_fp8(a.out_fp8, off, y + 4 * h, a.fp8_scale);
+          }
+        }
+      if constexpr (!F32) {
+        if (has(i, 0)) {
+          const long off = row * a.ldo + norm_column(false, i, 0, lane);
+          if (a.out) store8(a.out, off, y, a.out_dtype);
+          if (a.out_b) store8(a.out_b, off, y, a.out_b_dtype);
+          if (a.out_fp8) store8_fp8(a.out_fp8, off, y, a.fp8_scale);
+        }
       }
     }
   }
@@ -240,6 +278,15 @@ __global__ void __launch_bounds__(256) layernorm_wide_kernel(const LayerNormArgs
   }
 }
 
+template <int IN_DT, bool ONCE>
+static hipError_t launch_ln_two_rows(const LayerNormArgs& a, int vecs, hipStream_t st) {
+  const dim3 grid((a.rows + 7) / 8), block(256);
+  if (vecs <= 1) hipLaunchKernelGGL((layernorm_kernel<IN_DT, 1, false, 2, ONCE>), grid, block, 0, st, a);
+  else if (a.C == 1024) hipLaunchKernelGGL((layernorm_kernel<IN_DT, 2, true, 2, ONCE>), grid, block, 0, st, a);
+  else hipLaunchKernelGGL((layernorm_kernel<IN_DT, 2, false, 2, ONCE>), grid, block, 0, st, a);
+  return hipGetLastError();
+}
+
 template <int IN_DT>
 static hipError_t launch_ln_dt(const LayerNormArgs& a, hipStream_t st) {
   const dim3 grid((a.rows + 3) / 4), block(256);
@@ -255,6 +302,17 @@ static hipError_t launch_ln_dt(const LayerNormArgs& a, hipStream_t st) {
       else launch_ln_trunk<2>(a, 4, st);
       return hipGetLastError();
     }
+  }
+  // Two rows per wave from where that leaves enough waves in flight (10 layers of 512 channels: 16000 rows 1.224 -> 1.234 ms, 22400 1.81 -> 1.79; 1024
+  // channels, f16: 4096 rows 2.23 -> 2.22 ms, 16000 5.79 -> 5.70).
+  if (vecs <= 2 && a.rows > (vecs == 1 ? 80 : 16) * device_cus()) {
+    if constexpr (IN_DT != DT_F32) {
+      // Rows of more than 80 MB, with what the products around this launch read and write, are past what the 256 MB cache on the memory side holds from
+      // one launch to the next: with the non-temporal hint they leave it to the others (10 layers of 512 channels: 97344 rows 5.99 -> 5.91 ms, 128000
+      // 7.93 -> 7.69, 256000 15.7 -> 15.1; 64000 rows 4.06 -> 4.08).
+      if ((long)a.rows * a.C * 2 > 80L << 20) return launch_ln_two_rows<IN_DT, true>(a, vecs, st);
+    }
+    return launch_ln_two_rows<IN_DT, false>(a, vecs, st);
   }
   if (vecs <= 1) hipLaunchKernelGGL((layernorm_kernel<IN_DT, 1>), grid, block, 0, st, a);
   else if (a.C == 1024) hipLaunchKernelGGL((layernorm_kernel<IN_DT, 2, true>), grid, block, 0, st, a);   // (the trunk's width: no column guards)

@@ -864,6 +864,39 @@ def test_layernorm_trunk_width_workgroups_by_row_count(cuda):
         assert abs(amax - ref[:n].float().abs().max().item()) <= 2 ** -8 * amax, n
 
 
+@pytest.mark.parametrize("C_,in_dt,rms", [(512, _lib.BF16, False), (768, _lib.F32, False), (768, _lib.F32, True), (256, _lib.F32, False), (1024, _lib.F16, False), (520, _lib.F16, True),
+                                          (1024, _lib.F32, False), (1024, _lib.BF16, True)])
+def test_norm_rows_in_pairs_equal_one_row_per_wave(cuda, C_, in_dt, rms):
+    """Many rows are taken two to a wave, and past a size read with a hint: an odd count, rows with a stride, and the same bits as in calls of few rows; nothing
+    past the last row or the last column."""
+    torch.manual_seed(C_)
+    cus = torch.cuda.get_device_properties(cuda).multi_processor_count
+    big = (80 << 20) // (2 * C_) + 3 if in_dt != _lib.F32 else 80 * cus + 3
+    ld = C_ + 8
+    x = (torch.randn(big, ld, device=cuda) * 2 + 0.5).to(TORCH_DT[in_dt])
+    g, b = torch.randn(C_, device=cuda), torch.randn(C_, device=cuda)
+
+    def run(lo, n):
+        out, amax = torch.full((n + 1, ld), 7.0, dtype=torch.bfloat16, device=cuda), torch.zeros(1, device=cuda)
+        if rms:
+            check(lib().crl_rmsnorm(p(x[lo:]), ld, in_dt, p(g), p(out), _lib.BF16, None, 1.0, ld, n, C_, 1e-5, p(amax), stream()), "rms")
+        else:
+            check(lib().crl_layernorm(p(x[lo:]), ld, in_dt, p(g), p(b), p(out), _lib.BF16, None, 1.0, ld, n, C_, 1e-5, p(amax), stream()), "ln")
+        torch.cuda.synchronize()
+        assert bool((out[n] == 7).all()) and bool((out[:, C_:] == 7).all())
+        return out[:n, :C_], amax.item()
+
+    small = 4 * cus
+    few = torch.cat([run(lo, min(small, big - lo))[0] for lo in range(0, big, small)])
+    ref = (F.rms_norm(x[:64, :C_].float(), (C_,), g, 1e-5) if rms else F.layer_norm(x[:64, :C_].float(), (C_,), g, b, 1e-5))
+    assert torch.allclose(few[:64].float(), ref, rtol=2 ** -8, atol=2 ** -8)
+    for n in (16 * cus, 16 * cus + 1, 80 * cus, 80 * cus + 1, 80 * cus + 2, big - 3, big):
+        if n <= big:
+            out, amax = run(0, n)
+            assert torch.equal(out, few[:n]), n
+            assert abs(amax - few[:n].float().abs().max().item()) <= 2 ** -8 * amax, n
+
+
 @pytest.mark.parametrize("C_,in_dt", [(256, _lib.F32), (1024, _lib.BF16), (8192, _lib.BF16), (1536, _lib.F16)])
 def test_rmsnorm(cuda, C_, in_dt):
     """crl_rmsnorm against torch.nn.functional.rms_norm on the same (rounded) input."""
