@@ -169,7 +169,8 @@ hipError_t launch_decode_attention(const void* q, long ldq, const void* cache, i
 // and, where asked for, the embedding of the token, wte[tok] + pe[64 + k] (model_bis.py:224, 233-235 for the last position only).
 // Wave 0 draws: its lane l owns the contiguous classes [l*CH, l*CH+CH), so the CDF is a lane-level scan plus a short walk. The logits come
 // in and the probabilities go out over all four waves, class by class; read and written by the owning lanes, each access touching
-// 64 lines, the step took 15.9 us for 128 sequences and its embedding another 4.0; together they take 9.9 us now.
+// 64 lines, the step took 15.9 us for 128 sequences and its embedding another 4.0; together they took 9.8, and 9.0 with what the rules and the
+// embedding read requested beside the logits and the searches without the LDS crossbar.
 constexpr int SAMPLE_CH = 32;
 
 __device__ __forceinline__ float uniform01(uint64_t seed, uint64_t a, uint64_t b) {
@@ -204,18 +205,25 @@ __global__ void __launch_bounds__(256) sample_kernel(const SampleArgs a) {
     const int c = i * 256 + tid;
     v[i] = c < a.V ? x[c] * invT : -INFINITY;
   }
+  // What the rules and the embedding read besides the draw, requested with the logits: behind the draw each would be a trip to memory of its own.
+  int nz = 0;
+  long two_back = -1;
+  if (a.rules && tid == 0) {
+    nz = a.num_zeros[b];
+    if (k >= 2) two_back = a.seq[(long)b * a.ld_seq + k - 2];
+  }
+  float4 pe0 = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (a.emb_out && tid * 4 < a.emb_C) pe0 = *reinterpret_cast<const float4*>(a.pe + (long)(64 + k) * a.emb_C + tid * 4);
   float wmx = -INFINITY;
   int wi = 0x7fffffff;
 #pragma unroll
   for (int i = 0; i < VPT; ++i)
     if (v[i] > wmx) { wmx = v[i]; wi = i * 256 + tid; }
-  // arg-max with the lowest index among equals
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    const float om = __shfl_xor(wmx, o, 64);
-    const int oi = __shfl_xor(wi, o, 64);
-    if (om > wmx || (om == wmx && oi < wi)) { wmx = om; wi = oi; }
-  }
+  // arg-max with the lowest index among equals: the maximum, then the lowest of its lanes' indexes (as floats: they are below 2^24)
+  const float wave_mx = wave_max(wmx);
+  const float low = wave_max(wmx == wave_mx && wi != 0x7fffffff ? -(float)wi : -INFINITY);
+  wi = low == -INFINITY ? 0x7fffffff : (int)-low;
+  wmx = wave_mx;
   if (lane == 0) { s_max[wave] = wmx; s_idx[wave] = wi; }
   __syncthreads();
 #pragma unroll
@@ -265,17 +273,14 @@ __global__ void __launch_bounds__(256) sample_kernel(const SampleArgs a) {
           }
         }
       }
-      // rounding can leave no lane (target == total): fall back to the arg-max
-      int found = pick;
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) found = max(found, __shfl_xor(found, o, 64));
-      if (found >= 0) tok = found;
+      // the last lane that has one; rounding can leave none (target == total): fall back to the arg-max
+      const uint64_t have = __ballot(pick >= 0);
+      if (have) tok = __builtin_amdgcn_readlane(pick, 63 - __builtin_clzll(have));
     }
     if (lane == 0) {
       if (a.rules) {
-        int nz = a.num_zeros[b];
         if (nz == 5) { tok = a.end_think; nz = 6; }
-        if (k >= 2 && a.seq[(long)b * a.ld_seq + k - 2] == a.end_think) tok = a.end_tok;
+        if (k >= 2 && two_back == a.end_think) tok = a.end_tok;
         nz += (tok == a.end_variation) ? 1 : 0;
         a.num_zeros[b] = nz;
       }
@@ -292,7 +297,7 @@ __global__ void __launch_bounds__(256) sample_kernel(const SampleArgs a) {
     const float* wte = a.wte + id * a.emb_C;
     const float* pe = a.pe + (long)(64 + k) * a.emb_C;
     for (int c = tid * 4; c < a.emb_C; c += 1024) {
-      const float4 w = *reinterpret_cast<const float4*>(wte + c), p = *reinterpret_cast<const float4*>(pe + c);
+      const float4 w = *reinterpret_cast<const float4*>(wte + c), p = c == tid * 4 ? pe0 : *reinterpret_cast<const float4*>(pe + c);
       const float4 r = make_float4(w.x + p.x, w.y + p.y, w.z + p.z, w.w + p.w);
       const long o = (long)b * a.emb_C + c;
       if (a.emb_dtype == DT_F32) *reinterpret_cast<float4*>(reinterpret_cast<float*>(a.emb_out) + o) = r;
