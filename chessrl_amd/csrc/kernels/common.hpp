@@ -132,6 +132,13 @@ __device__ __forceinline__ float wave_max(float v) {
   v = fmaxf(v, dpp_move<DPP_MIRROR>(v));
   return max_xor32(max_xor16(v));
 }
+// The wave's largest value and the lowest index that holds it (0x7fffffff: none; others below 2^24, exact as floats).
+__device__ __forceinline__ void lowest_argmax(float& v, int& idx) {
+  const float m = wave_max(v);
+  const float low = wave_max(v == m && idx != 0x7fffffff ? -(float)idx : -INFINITY);
+  idx = low == -INFINITY ? 0x7fffffff : (int)-low;
+  v = m;
+}
 
 // amax is kept as the bit pattern of a non-negative float so integer max orders it.
 __device__ __forceinline__ void atomic_amax(float* slot, float v) {

@@ -219,11 +219,8 @@ __global__ void __launch_bounds__(256) sample_kernel(const SampleArgs a) {
 #pragma unroll
   for (int i = 0; i < VPT; ++i)
     if (v[i] > wmx) { wmx = v[i]; wi = i * 256 + tid; }
-  // arg-max with the lowest index among equals: the maximum, then the lowest of its lanes' indexes (as floats: they are below 2^24)
-  const float wave_mx = wave_max(wmx);
-  const float low = wave_max(wmx == wave_mx && wi != 0x7fffffff ? -(float)wi : -INFINITY);
-  wi = low == -INFINITY ? 0x7fffffff : (int)-low;
-  wmx = wave_mx;
+  // arg-max with the lowest index among equals
+  lowest_argmax(wmx, wi);
   if (lane == 0) { s_max[wave] = wmx; s_idx[wave] = wi; }
   __syncthreads();
 #pragma unroll

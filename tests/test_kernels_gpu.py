@@ -814,6 +814,33 @@ def test_masked_nll_mean_counts_rows_beyond_what_a_float_counts(cuda):
     assert out.item() == (torch.tensor(896.0) / torch.tensor(2.0 ** 24 + 2)).item()
 
 
+@pytest.mark.parametrize("V", [1, 2, 63, 64, 65, 255, 256, 257, 1858, 2048])
+def test_argmax_takes_the_lowest_of_equals(cuda, V):
+    """The arg-max of the masked softmax and of the sampling step: ties inside a lane's classes, across lanes and across waves, -inf beside one finite class, and
+    rows of the lowest finite value."""
+    g = torch.Generator().manual_seed(V)
+    x = torch.randn(40, V, generator=g)
+    for r in range(30):
+        for c in torch.randint(0, V, (3,), generator=g).tolist():
+            x[r, c] = 9.0
+    x[30:34] = torch.finfo(torch.float32).min
+    for r in range(34, 38):
+        c = int(torch.randint(0, V, (1,), generator=g))
+        x[r] = -float("inf")
+        x[r, c] = -3.0
+    x[38] = 0.0
+    x[39] = -0.0
+    want = torch.tensor([int((row == row.max()).nonzero()[0]) for row in x])
+    xd = x.to(cuda)
+    am, probs = torch.empty(40, dtype=torch.int32, device=cuda), torch.empty(40, V, device=cuda)
+    check(lib().crl_masked_softmax(p(xd), V, None, 0, p(probs), V, p(am), 40, V, 0.0, stream()), "softmax")
+    toks = torch.empty(40, dtype=torch.int64, device=cuda)
+    check(lib().crl_sample(p(xd), V, 40, V, 0.0, 0, 0, p(toks), None, stream()), "sample")
+    torch.cuda.synchronize()
+    assert torch.equal(am.cpu().long(), want) and torch.equal(toks.cpu(), want)
+    assert torch.equal(probs.cpu(), F.one_hot(want, V).float())
+
+
 def test_sample_distribution_and_argmax(cuda):
     """crl_sample draws from softmax(logits/T): empirical frequencies over 200k rows, arg-max for T=0."""
     V, B = 37, 200000
