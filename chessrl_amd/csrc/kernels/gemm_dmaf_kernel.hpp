@@ -340,10 +340,15 @@ __global__ void __launch_bounds__(DmafCfg::NT, 2) gemm_dmaf_kernel(const GemmArg
   auto res_load = [&](auto sc) {
     constexpr int st = decltype(sc)::value, tm = st % TM, half = st / TM;
     if constexpr (HAS_RES && st < NSTEP) {
-      // (the hint on fp32 rows of 768 columns, K = 768, back to back, with and without: 96000 rows 173 and 191 us, 32768 rows 70 and 60, which still fit
-      // the memory-side cache there; K = 3072: 447 and 452, 152 and 163)
+      // (fp32 rows go past the caches where the output does, by the launcher's rule; 768 columns, K = 768, back to back, with and without the
+      // hint: 96000 rows 173 and 191 us, 32768 rows, which the memory-side cache holds, 70 and 60)
+      if (OUT_DT != DT_F32 || a.stream_out != 0) {
 #pragma unroll
-      for (int it = 0; it < ITS; ++it) res[st & 1][it] = dmaf_get16_nt(rsrc_r, vres + half * 128 + (tm * 32 + it * (64 / EPR)) * res_step);
+        for (int it = 0; it < ITS; ++it) res[st & 1][it] = dmaf_get16_nt(rsrc_r, vres + half * 128 + (tm * 32 + it * (64 / EPR)) * res_step);
+      } else {
+#pragma unroll
+        for (int it = 0; it < ITS; ++it) res[st & 1][it] = dmaf_get16(rsrc_r, vres + half * 128 + (tm * 32 + it * (64 / EPR)) * res_step);
+      }
       if constexpr (EPI == DMAF_RESNORM)
         row_st[st & 1] = dmaf_get8(dmaf_rsrc(a.res_stats + 2 * (long)m0, (long)(a.M - m0) * 8), (wm * Cfg::WM + tm * 32 + (dmaf_here(lane) & 31)) * 8);
     }

@@ -400,6 +400,19 @@ def test_gemm_persistent_tiles_on_ragged_edges_equal_the_small_tile(cuda, tile, 
     assert (got._base[:, N:] == 0).all()
 
 
+@pytest.mark.parametrize("tile", [10, 11])
+@pytest.mark.parametrize("M", [16384, 16385, 38400, 38401])
+def test_gemm_fp32_residual_read_and_stored_past_the_caches_or_not(cuda, tile, M):
+    """fp32 sums with a residual on either side of the sizes (64 MB without, 150 MB with a residual: the last rows of each pair) from which output and
+    residual carry the non-temporal hint: the same bits as the 64x64 tile."""
+    torch.manual_seed(M)
+    N, K = 1024, 128
+    A, W = torch.randn(M, K, device=cuda).bfloat16(), (torch.randn(N, K, device=cuda) * K ** -0.5).bfloat16()
+    bias, res = torch.randn(N, device=cuda), torch.randn(M, N, device=cuda)
+    for kw in (dict(), dict(res=res)):
+        assert torch.equal(run_gemm(A, W, _lib.F32, tile=tile, bias=bias, **kw), run_gemm(A, W, _lib.F32, tile=1, bias=bias, **kw))
+
+
 @pytest.mark.parametrize("M,N,out_dt", [(8448, 4096, _lib.BF16), (16384, 4096, _lib.F16), (131328, 384, _lib.BF16), (131072, 4096, _lib.BF16)])
 def test_gemm_short_k_rows_resident_equals_tiled(cuda, M, N, out_dt):
     """K = 256 e4m3 elements into a large 16-bit output (the attention-bias generator's product): the kernel whose
