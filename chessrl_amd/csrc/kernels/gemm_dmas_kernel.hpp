@@ -396,6 +396,7 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_dmas_kernel(const SmallArgs s_in
     const int kp = wave / (Cfg::WGM * Cfg::WGN);
 #pragma unroll 1
     for (int slab = kp, i = 0; i < nbar; ++i, slab += Cfg::KP) {
+      __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): the last round's fragments are in registers, behind this barrier its stages are refilled
       dmas_barrier();
       if (slab >= nslab) continue;
       static_for<0, KSTEPS>([&](auto ksc) { read_step((slab & (NSTAGE - 1)) * STAGE, f0, ksc); });

@@ -208,6 +208,7 @@ __global__ void __launch_bounds__(1024) gemm_norm_kernel(const NormGemmKArgs s) 
     if (slab + 1 < end) { step(slab + 1, f0, f1); last_step(f1); }
     else if (slab < end) last_step(f0);
   }
+  __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0)
   dmaf_barrier();   // both operands are read: their space becomes the patches of the sums
   if (multiplies) {
     float* const patch = reinterpret_cast<float*>(smem) + wave * 1024;
