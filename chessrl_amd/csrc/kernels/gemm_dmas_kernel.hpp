@@ -45,7 +45,6 @@ struct DmasCfg {
   static __device__ __forceinline__ int patch_off(int nslab, int w) {
     return ((nslab + w * 4096 / STAGE) & (NSTAGE - 1)) * STAGE + w * 4096 % STAGE;
   }
-  static constexpr int PER = KP;   // slabs a barrier announces
   static_assert(KP == 1 || 4 * KP <= NSTAGE, "a round in work, three requested");
   static_assert(AHEAD * LOADS < 64 && AHEAD + 2 <= NSTAGE, "the counted waits fit the counter; a stage is read before it is refilled");
   static_assert(LDS_BYTES <= 160 * 1024, "LDS of a CU");
@@ -217,9 +216,9 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_dmas_kernel(const SmallArgs s_in
   const int tile_m = s.by_cols ? inner : outer, tile_n = s.by_cols ? outer : inner;
   const int m0 = tile_m * BM, n0 = tile_n * BN;
 
-  // Barrier i (0 .. nbar - 1) of the workgroup says that slab i (KP > 1: slabs KP i .. KP i + KP - 1) has landed, barrier nbar that sums, residual and bias
+  // Barrier i (0 .. nbar - 1) of the workgroup says that slabs KP i .. KP i + KP - 1 have landed, barrier nbar that sums, residual and bias
   // lie in LDS. Every wave passes all of them.
-  const int nbar = (nslab + Cfg::PER - 1) / Cfg::PER;
+  const int nbar = (nslab + Cfg::KP - 1) / Cfg::KP;
   if (wave == Cfg::NCOMP + Cfg::NLOAD) {
     if (small_tile_full(s, n0, BN)) {
       if (s.bias) {
