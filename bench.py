@@ -98,7 +98,7 @@ def gemm_probe(a, torch, _lib, dev):
 
 
 def latency_workload(a, torch, models, board, dev):
-    """Leaf-evaluation latency of the full-size bf16 model (BASELINE's MCTS mode): batches of 1, 8, 64 and 256 positions from
+    """Leaf-evaluation latency of the full-size bf16 model (leaves of a tree search): batches of 1, 8, 64 and 256 positions from
     one seeded stream, each with its legal-move mask applied before the softmax; per batch size p50/p99 of a synchronous
     evaluate call, and the kernel launches of one forward pass."""
     model = models.BT4Class(15, 1024, 1536, 32, fp8=False, act_dtype=a.act_dtype, seed=0)

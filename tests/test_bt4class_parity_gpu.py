@@ -63,7 +63,7 @@ def anchored_case(init, B, act):
 
 @pytest.mark.parametrize("act,init,B", [("bf16", "benchmark", 1024), ("bf16", "test", 256), ("f16", "benchmark", 256), ("f16", "test", 256)])
 def test_16bit_forward_against_torch_16bit_anchor(cuda, act, init, B):
-    """BASELINE's bf16 configuration (batch 1024, benchmark initialisation) and the non-degenerate test weights: the HIP
+    """The bf16 configuration (15 x 1024, batch 1024, benchmark initialisation) and the non-degenerate test weights: the HIP
     forward and torch's own 16-bit forward of the same oracle, both against the fp32 oracle.
 
     Bars, all relative to the anchor measured in the same test (nothing here is set to what the kernels happened to reach):
@@ -279,7 +279,7 @@ def test_fp8_operand_codes_match_emulation(cuda):
 
 @pytest.mark.parametrize("fp8", [True, False])
 def test_large_batch_sweep_at_its_own_size(cuda, fp8):
-    """BASELINE's rollout-scoring sweep: the full-size model (benchmark initialisation) on 8192 and 16384 positions, 30 %
+    """Rollout scoring: the full-size model (benchmark initialisation) on 8192 and 16384 positions, 30 %
     of them late-game (at most ten pieces, sparse legal masks), walked in micro-batches of 4096. The 8192-position call
     equals the first half of the 16384-position one bit for bit; rows [0, 256), [4096, 4352) (the start of the second
     micro-batch) and [12288, 12544) are bit-equal to 256-position calls; everything is finite; the masked softmax is
