@@ -229,8 +229,9 @@ def test_bt4class_batch_invariance(cuda, fp8):
 @pytest.mark.parametrize("act,fp8", [("bf16", False), ("f16", False), ("bf16", True)])
 def test_bt4class_bias_generator_norms_inside_their_products(cuda, act, fp8):
     """Full width, the only one whose second bias-generator norm (over a position's 32 rows of 256) runs inside the product behind it: on 32 rows and one
-    tile up to 2 and 4 positions, on 64 rows and slices of N beyond, as a launch of its own from one position per compute unit on; the first norm on 32 rows up
-    to 64 positions. Odd positions leave a row block half empty. Same bits on all of them."""
+    tile up to 4 positions, on 64 rows and slices of N beyond, as a launch of its own beyond one position per compute unit; the first norm on 32 rows up
+    to 64 positions. Odd positions leave a row block half empty. Same bits on all of them, and, with 16-bit operands, as with both norms as launches of their
+    own, which is how a calibrating pass runs them: the last layer's residual sum behind either."""
     m = models.BT4Class(2, 1024, 1536, 32, fp8=fp8, act_dtype=act)
     m.load_state_dict(om.test_init_(om.BT4ClassOracle(policy_leela, 2, 1024, 1536, 32), seed=6).state_dict())
     cus = torch.cuda.get_device_properties(cuda).multi_processor_count
@@ -243,6 +244,13 @@ def test_bt4class_bias_generator_norms_inside_their_products(cuda, act, fp8):
         p2, w2 = m(x[47 - B % 47:47 - B % 47 + B].contiguous())
         lo = 47 - B % 47
         assert torch.equal(p2, pol[lo:lo + B]) and torch.equal(w2, wdl[lo:lo + B]), B
+    if not fp8:
+        for B in (1, 3, 4, 5, 33, 64, 65, 130, cus, cus + 1):
+            xb, dt = x[:B].contiguous(), torch.bfloat16 if act == "bf16" else torch.float16
+            m.calibrate(xb)
+            separate = m._engine.read_tensor("t", (B * 64, 1024), dt)
+            m(xb)
+            assert separate.float().abs().max() > 0 and torch.equal(m._engine.read_tensor("t", (B * 64, 1024), dt), separate), B
 
 
 @pytest.mark.parametrize("act", ["bf16", "f16"])
