@@ -100,7 +100,7 @@ def gemm_probe(a, torch, _lib, dev):
 def latency_workload(a, torch, models, board, dev):
     """Leaf-evaluation latency of the full-size bf16 model (leaves of a tree search): batches of 1, 8, 64 and 256 positions from
     one seeded stream, each with its legal-move mask applied before the softmax; per batch size p50/p99 of a synchronous
-    evaluate call, and the kernel launches of one forward pass."""
+    evaluate call, and the steps of one forward pass."""
     model = models.BT4Class(15, 1024, 1536, 32, fp8=False, act_dtype=a.act_dtype, seed=0)
     r = board.random_positions(3, 256, masks_leela=True)
     planes, masks = torch.from_numpy(r["planes"]).to(dev), torch.from_numpy(r["masks_leela"]).to(dev)
@@ -119,9 +119,10 @@ def latency_workload(a, torch, models, board, dev):
         model._engine.forward(lp)
         prof = model._engine.get_profile()
         model._engine.set_profiling(False)
-        # (the per-family counters do not see the two launches outside them: the side-to-move extraction and the masked softmax)
+        # (what the per-family counters count: a norm inside a product's launch is a step of its own, both passes of a long-K product are one;
+        # they do not see the side-to-move extraction and the masked softmax)
         per_batch["b%d" % nb] = {"p50_ms": round(ts[len(ts) // 2], 3), "p99_ms": round(ts[min(len(ts) - 1, int(len(ts) * 0.99))], 3),
-                                 "samples": len(ts), "launches_per_forward": sum(v["launches"] for v in prof.values()) + 2}
+                                 "samples": len(ts), "steps_per_forward": sum(v["launches"] for v in prof.values()) + 2}
     # for comparison: the e4m3 model of the headline workload in the same leaf-evaluation mode
     f8 = models.BT4Class(15, 1024, 1536, 32, fp8=True, act_dtype=a.act_dtype, seed=0)
     f8.calibrate(torch.from_numpy(board.random_positions(2, 512)["planes"]).to(dev))

@@ -738,7 +738,7 @@ hipError_t launch_gemm(GemmArgs a, int in_dt, int out_dt, int tile, hipStream_t 
   // caches so it does not push the operand tiles out (measured +6..10 % on the 0.5-1.6 GB outputs of a 4096-position batch).
   // fp32 sums with a residual are the next product's residual: up to 150 MB the memory-side cache still has them then, if neither side goes past it (calls of the
   // 6-layer model of 768 channels: 192 positions 1423 -> 1381 us, 400 2820 -> 2765, 100 sequences of 256 tokens 7.07 -> 6.94 ms; 800 and 1200 positions,
-  // 160 and 240 MB, keep the hint, without which a product of 96000 rows takes 191 us instead of 173).
+  // 160 and 240 MB, keep the hint, without which a product of 96000 rows takes 191 us instead of 173; set on this one width, and only time depends on it).
   const long keep = a.res && out_dt == DT_F32 ? 150L << 20 : 64L << 20;
   a.stream_out = (long)a.M * a.N * dtype_size(out_dt) > keep ? 1 : 0;
   if (tile == 14) { a.c_blocked = 1; tile = 13; }

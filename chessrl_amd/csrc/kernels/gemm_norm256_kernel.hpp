@@ -5,9 +5,10 @@
 // its 32 or 64 rows itself, keeps them as the MFMA operand in registers and walks a slice of N in steps of 64 columns, whose weights four waves
 // bring into a ring of three LDS stages; the first stage, on which a call of one position waits, is requested by all eight waves,
 // behind the rows, gains and offsets of the norm and ahead of its arithmetic.
-// Bound by the load latencies in a row (rows, then weights) on one position: 3.8 and 4.6 us where the two launches took 5.8 and 8.6 of a pass. On many
+// The 256 columns and the 32 rows of a position are the generator's sizes at 1024 channels and 32 heads; other sizes take two launches.
+// Bound by the load latencies in a row (rows, then weights) on one position: 4.0 and 4.6 us where the two kernels took 6.3 and 8.3, and a launch more. On many
 // rows by the weights' way into LDS: 64 KB in flight per CU and some 0.95 us a step of 64 x 64 outputs, of which the 16 MFMAs in one chain are 0.4
-// (250 bf16 positions: 32 us a launch, 35.5 before; results stored 8 bytes per lane and row, or finished behind the MFMAs instead of in the shadow of the
+// (256 bf16 positions: 31.6 us a launch, 33.9 before; results stored 8 bytes per lane and row, or finished behind the MFMAs instead of in the shadow of the
 // next tile's: 54 and 40 us). 32 rows a workgroup while every tile of 32 x 64 has a CU: that form has one stage and no loop.
 // The norms' arithmetic is that of layernorm_kernel and layernorm_wide_kernel, the products add K in the order of the tiled kernels: bit-equal to
 // the launches this replaces.

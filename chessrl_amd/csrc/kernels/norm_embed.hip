@@ -309,7 +309,7 @@ static hipError_t launch_ln_dt(const LayerNormArgs& a, hipStream_t st) {
     if constexpr (IN_DT != DT_F32) {
       // Rows of more than 80 MB, with what the products around this launch read and write, are past what the 256 MB cache on the memory side holds from
       // one launch to the next: with the non-temporal hint they leave it to the others (10 layers of 512 channels: 97344 rows 5.99 -> 5.91 ms, 128000
-      // 7.93 -> 7.69, 256000 15.7 -> 15.1; 64000 rows 4.06 -> 4.08).
+      // 7.93 -> 7.69, 256000 15.7 -> 15.1; 64000 rows 4.06 -> 4.08; set on this one model, and only time depends on it).
       if ((long)a.rows * a.C * 2 > 80L << 20) return launch_ln_two_rows<IN_DT, true>(a, vecs, st);
     }
     return launch_ln_two_rows<IN_DT, false>(a, vecs, st);

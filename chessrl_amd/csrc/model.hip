@@ -197,7 +197,8 @@ int Model::make_ffn(Layer& ly, const std::vector<float>& w1, const std::vector<f
 // meet themselves there again: every line is gone by the time it is asked for. The layers that go beyond the share below are read with the non-temporal
 // hint, which leaves the others where they are. One bf16 position of the 15 x 1024 model, layers kept: all 789 us, 11 759, 9 (208 MB with what is
 // not a layer's) 737, 7 749, 5 763, none 795; with the share below 792 -> 740, 4 positions 867 -> 827, 8 1062 -> 1013. Larger batches replace the
-// cache's contents themselves, and the kernels of their products share weight rows between many tiles.
+// cache's contents themselves, and the kernels of their products share weight rows between many tiles. (The share was found on this one model and counts
+// its weights as if no other model took turns with it; only the time of a call depends on the hint.)
 void Model::mark_streamed() {
   constexpr size_t KEEP = 200u << 20;
   auto bytes = [](const Lin& l) -> size_t { return (size_t)l.N * l.K * (l.w8 ? 1 : dtype_size(l.dt)); };
@@ -721,9 +722,10 @@ int Model::forward_chunk(const float* planes, const uint8_t* ids, const uint8_t*
       const int sc = cfg.smolgen_compress, sh = cfg.smolgen_hidden, sg = cfg.smolgen_gen;
       GOpt o; o.act = ACT_SWISH;
       RUN(gemm(ly.sm_hidden, ws.comp, 64 * sc, ad, ws.sh1, sh, ad, mb, o, st));
-      // Either norm runs inside the product behind it where the shapes are the kernel's (bit-equal; not while maxima are collected): the hidden layer's
-      // always (one launch of 15 layers: 1 position 2.0 us less, 64 3.1, 1000 6), the other on up to a position per compute unit (1 position 4.0 us
-      // less, 33 5.9, 64 3.6, 250 3.9; of 16-bit values 180 -1.2, 300 +4.9, 400 +9: whole rounds of large tiles do better there; of e4m3 ones 256 3.0,
+      // Either norm runs inside the product behind it where the shapes are the kernel's (bit-equal; not while maxima are collected). Kernel time of the
+      // bf16 pass, one launch against two: the hidden layer's always (1 position 4.0 and 6.3 us, 64 4.8 and 8.9, 256 7.2 and 14.3, 1000 15.5 and 24.2, 2048
+      // 26.0 and 31.0, 4096, a full micro-batch, 50.9 and 50.0 with a launch more), the other on up to a position per compute unit (1 position 4.6 and 8.3, 8
+      // 6.1 and 10.3, 64 13.5 and 16.9, 256 31.6 and 33.9; 300 +4.9, 400 +9 us a layer: whole rounds of large tiles do better there; of e4m3 values 256 -3.0,
       // beyond those the product that writes the blocked layout).
       const int gen_dt = f8 ? DT_FP8 : ad;
       if (!calibrate && sh == 256 && H * sg % 64 == 0 && mb <= 65536) {

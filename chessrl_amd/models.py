@@ -470,8 +470,8 @@ class _ModelBase:
 
 class GraphedEvaluator:
     """forward + legal-masked softmax for one fixed batch size, recorded once into a HIP graph and
-    replayed per call. The ~200 kernel launches of a forward pass dominate the latency of small
-    batches (MCTS leaf evaluation); a replay issues them as one graph launch. The library calls
+    replayed per call: the 160 kernels of a call (15 layers of BT4-class) are issued as one graph
+    launch, for hosts that cannot keep up with them one by one. The library calls
     record no memset nodes (flags and scratch are cleared by kernels)."""
 
     def __init__(self, model, batch, T=1.0, device="cuda"):
