@@ -4,24 +4,28 @@
 namespace crl {
 
 template <typename S>
-static hipError_t launch_small(const GemmArgs& a, int in_dt, int out_dt, hipStream_t st) {
+static hipError_t launch_small(const GemmArgs& a, int in_dt, int out_dt, hipStream_t st, SmallTile t) {
+#define SMALL(IN, OUT) launch_dmas<S, IN, OUT>(a, st, 1, t.bm, t.bn)
   if (in_dt == DT_FP8) {
     switch (out_dt) {
-      case DT_BF16: return launch_dmas<S, DT_FP8, DT_BF16>(a, st);
-      case DT_F16: return launch_dmas<S, DT_FP8, DT_F16>(a, st);
-      case DT_FP8: return launch_dmas<S, DT_FP8, DT_FP8>(a, st);
+      case DT_BF16: return SMALL(DT_FP8, DT_BF16);
+      case DT_F16: return SMALL(DT_FP8, DT_F16);
+      case DT_FP8: return SMALL(DT_FP8, DT_FP8);
     }
   }
-  if (in_dt == DT_BF16 && out_dt == DT_BF16) return launch_dmas<S, DT_BF16, DT_BF16>(a, st);
-  if (in_dt == DT_F16 && out_dt == DT_F16) return launch_dmas<S, DT_F16, DT_F16>(a, st);
-  if (in_dt == DT_BF16 && out_dt == DT_F32) return launch_dmas<S, DT_BF16, DT_F32>(a, st);
+  if (in_dt == DT_BF16 && out_dt == DT_BF16) return SMALL(DT_BF16, DT_BF16);
+  if (in_dt == DT_F16 && out_dt == DT_F16) return SMALL(DT_F16, DT_F16);
+  if (in_dt == DT_BF16 && out_dt == DT_F32) return SMALL(DT_BF16, DT_F32);
+#undef SMALL
   return hipErrorInvalidValue;
 }
 
-// tile_size: 64 (eight stages) or 32 (sixteen); the operand types are those of gemm_dmam_has. With k_parallel set the 32x32 tile spreads K over four waves.
+// tile_size: 64 (eight stages) or 32 (sixteen, and tiles of fewer rows or columns where there are CUs for them); the operand types are those of gemm_dmam_has. With k_parallel set the 32x32 tile spreads K over four waves.
 hipError_t launch_gemm_dmas(const GemmArgs& a, int in_dt, int out_dt, hipStream_t st, int tile_size) {
-  if (tile_size == 64) return launch_small<DmasCfg<64>>(a, in_dt, out_dt, st);
-  return a.k_parallel ? launch_small<DmasCfg<32, 4>>(a, in_dt, out_dt, st) : launch_small<DmasCfg<32>>(a, in_dt, out_dt, st);
+  if (tile_size == 64) return launch_small<DmasCfg<64>>(a, in_dt, out_dt, st, {64, 64});
+  const SmallTile t = small_tile(a.M, a.N, device_cus());
+  if (a.k_parallel) return launch_small<DmasCfg<32, 4>>(a, in_dt, out_dt, st, t);
+  return t.bm + t.bn <= 40 ? launch_small<DmasCfg<32, 1, 14>>(a, in_dt, out_dt, st, t) : launch_small<DmasCfg<32>>(a, in_dt, out_dt, st, t);
 }
 
 // K in 4 n equal shares (SLICED), 16-bit operands: the raw fp32 sums of share y in rows y M .. of C.

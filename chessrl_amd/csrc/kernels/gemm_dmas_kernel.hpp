@@ -21,18 +21,19 @@
 namespace crl {
 
 // BT = 64: eight stages of 16 KB, four computing waves of 32x32; BT = 32: sixteen stages of 8 KB, one. Eight loading waves either
-// way, which keep AHEAD slabs requested (at the CU's load rate a slab of 8 KB takes 128 cycles, and memory some 1000; twelve of them delay the first: GPT one position 217 -> 228 us), and one
-// wave that fetches what the epilogue needs.
+// way, which keep AHEAD slabs requested (at the CU's load rate a slab of 8 KB takes 128 cycles, and memory some 1000; twelve waves delay the first slab: GPT one position 217 -> 228 us), and one
+// wave that fetches what the epilogue needs. Fourteen slabs ahead where a slab has at most 40 rows: as many bytes as six of 64 rows. (Fourteen of those are
+// 112 KB that every CU asks for before it waits for its first slab, which then comes at 4400 cycles instead of 2500: one position 684 -> 711 us.)
 // KP > 1 (token steps, whose sums may be added in another order): KP computing waves per 32x32 take the slabs in turn, a round of KP slabs to a barrier and
 // three rounds requested ahead. With a barrier to each slab every wave waited for the one that had it: 128 rows, N = 768, K = 768 4.8 -> 4.1 us,
 // K = 3072 11.9 -> 9.4 (a token step of 128 sequences 311 -> 291).
-template <int BT, int KP_ = 1>
+template <int BT, int KP_ = 1, int AHEAD_ = (KP_ > 1 ? 3 * KP_ : 6)>
 struct DmasCfg {
   static_assert(BT == 64 || BT == 32, "two tile sizes");
   static_assert(KP_ == 1 || (BT == 32 && KP_ <= 4), "patches of the K groups lie in stages nothing is loaded into any more");
   static constexpr int BM = BT, BN = BT, WGM = BT / 32, WGN = BT / 32;
   static constexpr int KP = KP_, NCOMP = WGM * WGN * KP, NLOAD = 8, NT = 64 * (NCOMP + NLOAD + 1);
-  static constexpr int ROWB = 128, NSTAGE = 512 / BT, AHEAD = KP > 1 ? 3 * KP : 6;
+  static constexpr int ROWB = 128, NSTAGE = 512 / BT, AHEAD = AHEAD_;
   static constexpr int LOADS = 2 * BT / (8 * NLOAD);           // load instructions (8 rows each) of a wave per stage
   static constexpr int STAGE = BN * ROWB;                      // bytes of one operand's rows in one stage
   static constexpr int PART_BYTES = NSTAGE * STAGE;            // 64 KB: the weight rows of all stages, then the activation rows
@@ -60,6 +61,7 @@ struct SmallArgs {
   int inner; uint32_t m_inner; // tiles along the direction that is walked first, and the magic of dividing by them
   int by_cols;                 // 1: that direction is down a column of tiles
   int per_xcd;                 // workgroups per XCD
+  int bm, bn;                  // rows and columns of C a workgroup makes: BT, or fewer in multiples of eight
 };
 
 __device__ __forceinline__ void dmas_barrier() { asm volatile("s_barrier" ::: "memory"); }
@@ -214,26 +216,28 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_dmas_kernel(const SmallArgs s_in
   if (pid < (s.per_xcd << 3)) pid = (pid & 7) * s.per_xcd + (pid >> 3);
   const int outer = dmaf_div(pid, s.m_inner), inner = pid - outer * s.inner;
   const int tile_m = s.by_cols ? inner : outer, tile_n = s.by_cols ? outer : inner;
-  const int m0 = tile_m * BM, n0 = tile_n * BN;
+  const int bm = BM == 32 ? s.bm : BM, bn = BM == 32 ? s.bn : BN;
+  const int m0 = tile_m * bm, n0 = tile_n * bn;
 
   // Barrier i (0 .. nbar - 1) of the workgroup says that slabs KP i .. KP i + KP - 1 have landed, barrier nbar that sums, residual and bias
   // lie in LDS. Every wave passes all of them.
   const int nbar = (nslab + Cfg::KP - 1) / Cfg::KP;
   if (wave == Cfg::NCOMP + Cfg::NLOAD) {
-    if (small_tile_full(s, n0, BN)) {
+    if (small_tile_full(s, n0, bn)) {
       if (s.bias) {
         int n = n0 + lane;
         n = n < s.N ? n : s.N - 1;
         __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(s.bias + n), (__attribute__((address_space(3))) void*)(smem + Cfg::BIAS_OFF), 4, 0, 0);
       }
       if (s.res) {
-        // 16 bytes per lane: 64 / lpr rows per instruction (a row past the end reads the last one; nothing of it is stored)
+        // 16 bytes per lane: 64 / lpr rows per instruction (a row past the end reads the last one, a column past the tile the first ones; nothing of either is stored)
         const int rowb = s.res_dtype == DT_F32 ? BN * 4 : BN * 2, lpr = rowb >> 4;
         const int sh = 31 - __builtin_clz(lpr);
-        const char* const base = reinterpret_cast<const char*>(s.res) + ((long)n0 << (s.res_dtype == DT_F32 ? 2 : 1)) + ((lane & (lpr - 1)) << 4);
+        const int chunk = (lane & (lpr - 1)) << 4;
+        const char* const base = reinterpret_cast<const char*>(s.res) + ((long)n0 << (s.res_dtype == DT_F32 ? 2 : 1)) + (chunk < bn << (s.res_dtype == DT_F32 ? 2 : 1) ? chunk : 0);
         const long ldr_b = (long)s.ldr << (s.res_dtype == DT_F32 ? 2 : 1);
 #pragma unroll 1
-        for (int i = 0; i < BM * lpr / 64; ++i) {
+        for (int i = 0; i < (bm * lpr + 63) / 64; ++i) {
           int m = m0 + i * (64 >> sh) + (lane >> sh);
           m = m < s.M ? m : s.M - 1;
           if (__builtin_expect(s.res_rows > 0, 0)) m = m % s.res_rows;
@@ -256,7 +260,9 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_dmas_kernel(const SmallArgs s_in
     const bool loads_a = lw >= Cfg::NLOAD / 2;
     const int rbase = (lw & (Cfg::NLOAD / 2 - 1)) * (8 * LOADS);
     const int ld = loads_a ? s.lda_b : s.ldw_b;
-    const int rows_left = loads_a ? s.M - m0 : s.N - n0;
+    int rows_left = loads_a ? s.M - m0 : s.N - n0;
+    if constexpr (BM == 32) rows_left = min(rows_left, loads_a ? bm : bn);
+    const bool idle = BM == 32 && rbase >= (loads_a ? bm : bn);   // (a narrower tile has fewer groups of eight rows)
     uint32_t voff[LOADS];
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) {
@@ -269,6 +275,7 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_dmas_kernel(const SmallArgs s_in
     const __amdgpu_buffer_rsrc_t rsrc_mine = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(origin), 0, (rows_left < BM ? rows_left : BM) * ld, 0x00020000);
     const uint32_t lds_load0 = (loads_a ? Cfg::PART_BYTES : 0) + rbase * Cfg::ROWB;   // stage 0
     auto issue_slab = [&](int slab) {
+      if (idle) return;
       uint8_t* dst = smem + lds_load0 + (slab & (NSTAGE - 1)) * STAGE;
       static_for<0, LOADS>([&](auto ic) {
         constexpr int i = decltype(ic)::value;
@@ -344,10 +351,11 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_dmas_kernel(const SmallArgs s_in
 #pragma unroll
       for (int e = 0; e < EV; ++e) acc[e] = p == 0 ? part[e] : acc[e] + part[e];
     }
-    if (__builtin_expect(small_tile_full(s, n0, BN), 1))
-      small_full<OUT_DT, EV>(s, acc, m0 + er, n0 + ec, n0 < s.nsplit, reinterpret_cast<const float*>(smem + Cfg::BIAS_OFF) + ec,
+    const int m = BM == 32 && (er >= bm || ec >= bn) ? s.M : m0 + er;   // (M: nothing is stored)
+    if (__builtin_expect(small_tile_full(s, n0, bn), 1))
+      small_full<OUT_DT, EV>(s, acc, m, n0 + ec, n0 < s.nsplit, reinterpret_cast<const float*>(smem + Cfg::BIAS_OFF) + ec,
                              smem + Cfg::RES_OFF + (er * BN + ec) * (s.res_dtype == DT_F32 ? 4 : 2));
-    else small_edge<OUT_DT>(s, acc, EV, m0 + er, n0 + ec);
+    else small_edge<OUT_DT>(s, acc, EV, m, n0 + ec);
     return;
   }
 
@@ -436,12 +444,29 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_dmas_kernel(const SmallArgs s_in
   dmas_barrier();
 }
 
+// Rows and columns of C per workgroup of the 32x32 form: of the tiles that leave every one a CU, the one whose workgroup reads the fewest rows of both
+// operands. A CU gets 30 bytes a cycle from memory (some 64 KB in flight at 2000 cycles and more), less than half of what it gets from L2: the walk of 32 + 32
+// rows over weights that come from memory takes 310 cycles a slab where the MFMAs take 208. The same 64 rows by 1024 columns on 256 workgroups of 16x16 instead of
+// 64 of 32x32 read half as much each. Inside a pass of one position (bf16, weights past the caches), start to end of the launch: K = 1024 4.1 -> 3.4 us,
+// K = 1536 5.6 -> 4.2, FFN-1 (16x24) 4.0 -> 3.4; where the memory-side cache has the weights 3.0 and 3.1, 3.7 and 3.75. Whole calls: 684 -> 670 us; token steps of 128 sequences
+// 292 -> 288. MFMA lanes past the tile multiply whatever lies in LDS there; nothing of theirs is stored.
+struct SmallTile { int bm, bn; };
+inline SmallTile small_tile(int M, int N, int cus) {
+  SmallTile best{32, 32};
+  for (int bm = 8; bm <= 32; bm += 8)
+    for (int bn = 8; bn <= 32; bn += 8) {
+      if ((long)((M + bm - 1) / bm) * ((N + bn - 1) / bn) > cus) continue;
+      if (bm + bn < best.bm + best.bn || (bm + bn == best.bm + best.bn && bm * bn > best.bm * best.bn)) best = {bm, bn};
+    }
+  return best;
+}
+
 template <typename Cfg, int IN_DT, int OUT_DT, int ONCE = 0, int SLICED = 0>
-static hipError_t launch_dmas(const GemmArgs& a, hipStream_t st, int shares = 1) {
+static hipError_t launch_dmas(const GemmArgs& a, hipStream_t st, int shares = 1, int bm = Cfg::BM, int bn = Cfg::BN) {
   static_assert(!SLICED || (Cfg::KP == 1 && OUT_DT == DT_F32), "a share's sums as they are");
   if constexpr (Cfg::KP == 1 && !ONCE && !SLICED) {
     // (up to 512 rows: the weight rows that more tiles share do better kept in L2; 8 positions 1062 -> 1013 us, 12 the same, 16 1222 -> 1262)
-    if (a.w_once && a.M <= 512) return launch_dmas<Cfg, IN_DT, OUT_DT, 1>(a, st);
+    if (a.w_once && a.M <= 512) return launch_dmas<Cfg, IN_DT, OUT_DT, 1>(a, st, 1, bm, bn);
   }
   static std::atomic<bool> attr_set[16] = {};
   constexpr int ESZ = IN_DT == DT_FP8 ? 1 : 2;
@@ -456,8 +481,8 @@ static hipError_t launch_dmas(const GemmArgs& a, hipStream_t st, int shares = 1)
     if (e != hipSuccess) return e;
     if (dev >= 0 && dev < 16) attr_set[dev] = true;
   }
-  const int tiles_n = (a.N + Cfg::BN - 1) / Cfg::BN;
-  const int tiles = ((a.M + Cfg::BM - 1) / Cfg::BM) * tiles_n;
+  const int tiles_n = (a.N + bn - 1) / bn;
+  const int tiles = ((a.M + bm - 1) / bm) * tiles_n;
   if (tiles >= 65536) return hipErrorInvalidValue;
   SmallArgs s{};
   s.A = a.A; s.W = a.W; s.C = a.C; s.C2 = a.C2; s.bias = a.bias; s.res = a.res; s.amax = a.amax;
@@ -469,10 +494,10 @@ static hipError_t launch_dmas(const GemmArgs& a, hipStream_t st, int shares = 1)
   // of 2, 4 and 8 positions: 850 -> 835, 912 -> 868, 1083 -> 1065 us). Two rows of tiles gain nothing, and the K-shared form of 128 rows, 768
   // columns, K = 3072 loses 0.5 us a launch: rows first there.
   const int tiles_m = tiles / tiles_n, per = std::max(tiles >> 3, 1);
-  const int by_rows = (per + tiles_n - 1) / tiles_n + std::min(per, tiles_n), by_cols = (per + tiles_m - 1) / tiles_m + std::min(per, tiles_m);
+  const int by_rows = (per + tiles_n - 1) / tiles_n * bm + std::min(per, tiles_n) * bn, by_cols = (per + tiles_m - 1) / tiles_m * bn + std::min(per, tiles_m) * bm;
   s.by_cols = Cfg::KP == 1 && tiles_m >= 4 && by_cols < by_rows;
   s.inner = s.by_cols ? tiles_m : tiles_n;
-  s.m_inner = dmaf_magic(s.inner); s.per_xcd = tiles >> 3;
+  s.m_inner = dmaf_magic(s.inner); s.per_xcd = tiles >> 3; s.bm = bm; s.bn = bn;
   hipLaunchKernelGGL(kern, dim3(tiles, shares), dim3(Cfg::NT), Cfg::LDS_BYTES, st, s);
   return hipGetLastError();
 }

@@ -364,6 +364,30 @@ def test_gemm_mid_tile_direct_to_lds_equals_register_staged(cuda, M, N, K, dt):
     assert torch.allclose(out.float(), ref, rtol=2 ** -7, atol=2 ** -7 * ref.abs().max().item()), (out.float() - ref).abs().max()
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 3, 128), (1, 8, 2048), (1, 256, 2048), (1, 1929, 768), (8, 520, 64), (9, 776, 1024), (17, 1000, 768), (25, 1544, 1536), (33, 904, 192),
+                                   (64, 768, 3072), (64, 1024, 1024), (64, 1536, 1024), (63, 1535, 256), (128, 768, 768), (100, 1232, 1024)])
+@pytest.mark.parametrize("dt,out,res,act", [("bf16", _lib.BF16, torch.bfloat16, 0), ("bf16", _lib.F32, torch.float32, 0), ("bf16", _lib.BF16, None, 2), ("f16", _lib.F16, torch.float16, 1),
+                                            ("fp8", _lib.BF16, torch.bfloat16, 0), ("fp8", _lib.FP8, None, 2)])
+def test_gemm_small_tiles_of_fewer_rows_or_columns_equal_the_register_staged(cuda, M, N, K, dt, out, res, act):
+    """Tiles of 8 to 32 rows by 8 to 32 columns, whole and ragged: the same K order as every tiled kernel, so the same bits, and nothing behind row M or column N."""
+    torch.manual_seed(M * 5 + N)
+    if dt == "fp8":
+        K = (K + 127) // 128 * 128   # whole slabs
+        A, W = torch.randn(M, K, device=cuda).to(torch.float8_e4m3fn), torch.randn(N, K, device=cuda).to(torch.float8_e4m3fn)
+    else:
+        t16 = torch.bfloat16 if dt == "bf16" else torch.float16
+        A, W = torch.randn(M, K, device=cuda).to(t16), (torch.randn(N, K, device=cuda) / K ** 0.5).to(t16)
+    for ldc in (N, (N + 7) // 8 * 8 + 8):
+        kw = dict(bias=torch.randn(N, device=cuda), act=act, ldc=ldc, descale=0.75 if dt != "fp8" else 0.75 / K ** 0.5)
+        if res is not None:
+            kw["res"] = torch.randn(M, ldc, device=cuda).to(res)[:, :N]
+            kw["alpha"] = 0.625
+        small, ref = run_gemm(A, W, out, tile=16, **kw), run_gemm(A, W, out, tile=1, **kw)
+        assert torch.equal(small, ref)
+        behind = small.as_strided((M, ldc - N), (ldc, 1), N)
+        assert not behind.any()
+
+
 @pytest.mark.parametrize("M,N", [(1, 8192), (250, 8192), (1279, 8192), (1281, 8192), (2048, 6144), (2048, 6160), (4100, 8192), (3000, 12301)])
 @pytest.mark.parametrize("dt", ["bf16", "f16", "fp8"])
 def test_gemm_short_k_either_side_of_the_tile_rule(cuda, M, N, dt):
