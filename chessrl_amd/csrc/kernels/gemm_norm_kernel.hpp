@@ -1,11 +1,14 @@
 // C[M,N] = act(descale * norm(X)[M,K] · W[N,K]^T + bias): a LayerNorm (or RMSNorm) of fp32 rows of K <= 1024 columns and the product that
-// reads it as one launch, for products so small that every tile of 32 x 32 or 32 x 64 has a CU of its own (GPT on one to a few
+// reads it as one launch, for products so small that every tile of 16 or 32 rows has a CU of its own (GPT on one to a few
 // positions, the token steps of generation). There a norm is a launch of 4 us around a handful of rows. Here every workgroup normalises
-// its 32 rows itself: sixteen waves take two rows each, requested before anything is waited for, the workgroup's weight rows
-// follow straight to LDS, and the normalised rows go to LDS as the operand. With both operands whole in LDS (32 K + BN K elements, at most
+// its rows itself: sixteen waves take one or two rows each, requested before anything is waited for, the workgroup's weight rows
+// follow straight to LDS, and the normalised rows go to LDS as the operand. With both operands whole in LDS (at most
 // 150 KB) there is no ring; one barrier stands between gain and offset and their use, one between the operands and the product.
-// Bound by the CU's load rate at first (200 KB at 64 bytes a clock: 3500 of 11000 cycles), then by the norm's own vector instructions, which
-// every tile column repeats. One counted wait behind the last request lets the statistics run under the weight loads; the normalised rows wait for
+// Bound by the norm's own vector instructions, which every tile column repeats (four waves share a SIMD: 70 of them for a row's statistics are 1300 cycles), by the CU's
+// load rate before them (every wave's requests are issued after 2700 of 10400 cycles) and by the chain of a tile's MFMAs behind (3000). Hence 16 rows where the columns
+// then still fit: one position, K = 768, N = 2304 and 3072: 32x32 tiles 11100 cycles, 16x40 and 16x48 10400 and 10800; the last layer's one row, 32x32 10800, 16x16
+// 9600; vocabulary 10800 -> 9000 (whole call 186.0 -> 182.3 us).
+// One counted wait behind the last request lets the statistics run under the weight loads; the normalised rows wait for
 // them all the same, because the compiler drains every load into LDS in front of the first write to it. Measured in place: K = 768, N = 2304, 128 rows 8.4 us (12.4 for the norm riding on the K-sliced product before it and the
 // product), 64 rows 7.3 us (8.5 for two launches). The same for the 16-bit rows of 1024 columns of the BT4-class trunk took 9.4 us against 8.7
 // for two launches and is not here.
@@ -20,16 +23,27 @@ namespace crl {
 struct NormGemmKArgs {
   NormGemmArgs a;
   int nslab, tiles_m;
-  uint32_t m_tm;
+  uint32_t m_tm, m_bn2;        // magics of tiles_m and bn / 2
   int per_xcd;
+  int bn, nb;                  // columns of a tile, a multiple of eight, and its blocks of 32
+  int w_div, w_mod, loads;     // 16 / (bn / 8) and 16 % (bn / 8); weight requests of a wave
 };
 
-template <int IN_DT, int BN, int KP>
+template <int N>
+__device__ __forceinline__ void norm_wait(int loads) {   // all requests but the last `loads` (uniform, at most N) are there
+  if constexpr (N > 0) {
+    if (loads == N) wait_vmcnt_lgkm0<N>();
+    else norm_wait<N - 1>(loads);
+  } else {
+    wait_vmcnt_lgkm0<0>();
+  }
+}
+
+template <int IN_DT, int BM, int KP>
 __global__ void __launch_bounds__(1024) gemm_norm_kernel(const NormGemmKArgs s) {
-  constexpr int ESZ = IN_DT == DT_FP8 ? 1 : 2, ROWB = 128, BM = 32, NB = BN / 32;
+  constexpr int ESZ = IN_DT == DT_FP8 ? 1 : 2, ROWB = 128, RW = BM / 16;   // rows of X that a wave normalises
   constexpr int KSTEPS = ROWB / (IN_DT == DT_FP8 ? 64 : 32);
-  constexpr int EV = BM * BN / 1024;                // consecutive columns of an epilogue thread: 1 or 2
-  static_assert(NB * KP <= 16, "waves that multiply");
+  const int bn = s.bn;
   extern __shared__ __align__(16) uint8_t smem[];
   const NormGemmArgs& a = s.a;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -38,15 +52,15 @@ __global__ void __launch_bounds__(1024) gemm_norm_kernel(const NormGemmKArgs s) 
   int pid = blockIdx.x;
   if (pid < (s.per_xcd << 3)) pid = (pid & 7) * s.per_xcd + (pid >> 3);
   const int tile_n = dmaf_div(pid, s.m_tm), tile_m = pid - tile_n * s.tiles_m;
-  const int m0 = tile_m * BM, n0 = tile_n * BN;
-  uint8_t* const lds_w = smem;                                   // [slab][BN rows][128 bytes]
-  uint8_t* const lds_a = smem + nslab * BN * ROWB;               // [slab][32 rows][128 bytes]
+  const int m0 = tile_m * BM, n0 = tile_n * bn;
+  uint8_t* const lds_w = smem;                                   // [slab][bn rows][128 bytes]
+  uint8_t* const lds_a = smem + nslab * bn * ROWB;               // [slab][BM rows][128 bytes]
 
   float* const lds_g = reinterpret_cast<float*>(lds_a + nslab * BM * ROWB);   // [K] gain, then [K] offset
 
-  // ---- rows of X: wave w takes rows 2 w and 2 w + 1. A lane's 16 columns are those of layernorm_kernel (norm_columns).
+  // ---- rows of X: wave w takes rows RW w and on. A lane's 16 columns are those of layernorm_kernel (norm_columns).
   const int C = a.K;
-  float x[2][2][8];
+  float x[RW][2][8];
   auto has = [&](int i, int h) { return (2 * i + h) * 256 < C; };   // (whole groups of 256 columns: the same for all lanes)
   // Gain and offset first.
   // 256 columns per wave-instruction, waves 0-3 and 4-7
@@ -59,14 +73,15 @@ __global__ void __launch_bounds__(1024) gemm_norm_kernel(const NormGemmKArgs s) 
     else if (!src) *reinterpret_cast<f32x4_t*>(lds_g + 1024 + (wave & 3) * 256 + lane * 4) = f32x4_t{0.f, 0.f, 0.f, 0.f};
   }
 #pragma unroll
-  for (int r = 0; r < 2; ++r) {
-    int m = m0 + wave * 2 + r;
+  for (int r = 0; r < RW; ++r) {
+    int m = m0 + wave * RW + r;
     m = m < a.M ? m : a.M - 1;
 #pragma unroll
     for (int i = 0; i < 2; ++i) load_norm8<DT_F32>(a.x, (long)m * a.ldx, i, lane, C, x[r][i]);
   }
-  // the bias of this thread's columns
-  const int er = tid / (BN / EV), ec = (tid % (BN / EV)) * EV;
+  // the bias of this thread's columns: two consecutive ones of row er (threads past the tile have nothing to store)
+  constexpr int EV = 2;
+  const int er = dmaf_div(tid, s.m_bn2), ec = (tid - er * (bn >> 1)) * 2;
   float bias[EV];
 #pragma unroll
   for (int e = 0; e < EV; ++e) {
@@ -75,32 +90,34 @@ __global__ void __launch_bounds__(1024) gemm_norm_kernel(const NormGemmKArgs s) 
   }
   __builtin_amdgcn_sched_barrier(0);
   // ---- weight rows: 8 rows of 128 bytes per instruction, the swizzle applied on the global side
-  constexpr int GR = BN / 8;                                     // row groups of a slab, and weight requests of a wave
   {
-    const int grp = wave % GR, s0 = wave / GR, l8 = lane >> 3;
-    const int ldb = (int)a.ldw * ESZ, left = a.N - n0;
-    int r = grp * 8 + l8;
-    r = r < left ? r : left - 1;
-    const int voff = r * ldb + (((lane & 7) ^ l8 ^ (grp & 7)) << 4);
-    const __amdgpu_buffer_rsrc_t rs = dmaf_rsrc(reinterpret_cast<const uint8_t*>(a.W) + (long)n0 * ldb, (long)(left < BN ? left : BN) * ldb);
-    // (always the same number, those past K out of bounds and into a spare kilobyte: the wait for what was requested before counts past them)
+    const int rg = bn >> 3, ldb = (int)a.ldw * ESZ, left = a.N - n0 < bn ? a.N - n0 : bn, l8 = lane >> 3;   // (row groups of a slab)
+    int sl = 0, grp = wave;
+    while (grp >= rg) { grp -= rg; ++sl; }
+    const __amdgpu_buffer_rsrc_t rs = dmaf_rsrc(reinterpret_cast<const uint8_t*>(a.W) + (long)n0 * ldb, (long)left * ldb);
+    // (every wave asks as often, past K out of bounds and into a spare kilobyte: the wait for what was requested before counts past them)
     const __amdgpu_buffer_rsrc_t none = dmaf_rsrc(a.W, 0);
-#pragma unroll
-    for (int j = 0; j < GR; ++j) {
-      const int sl = s0 + j * (16 / GR);
-      dmaf_load16(sl < nslab ? rs : none, sl < nslab ? lds_w + (sl * BN + grp * 8) * ROWB : reinterpret_cast<uint8_t*>(lds_g) + 8192, voff, sl * ROWB);
+#pragma unroll 1
+    for (int j = 0; j < s.loads; ++j) {
+      int r = grp * 8 + l8;
+      r = r < left ? r : left - 1;
+      const int voff = r * ldb + (((lane & 7) ^ l8 ^ (grp & 7)) << 4);
+      dmaf_load16(sl < nslab ? rs : none, sl < nslab ? lds_w + (sl * bn + grp * 8) * ROWB : reinterpret_cast<uint8_t*>(lds_g) + 8192, voff, sl * ROWB);
+      sl += s.w_div;
+      grp += s.w_mod;
+      if (grp >= rg) { grp -= rg; ++sl; }
     }
   }
   __builtin_amdgcn_sched_barrier(0);
-  // Everything requested before the GR weight rows is there: this wave's rows and bias, and its share of gain and offset (the zeros in the place of
+  // Everything requested before the weight rows is there: this wave's rows and bias, and its share of gain and offset (the zeros in the place of
   // an offset are a write to LDS), which the barrier behind the statistics then hands to every wave; the barrier itself waits for nothing.
-  wait_vmcnt_lgkm0<GR>();
+  norm_wait<9>(s.loads);
   __builtin_amdgcn_sched_barrier(0);
   // ---- the norm
   const float inv_c = fast_rcp((float)C);
-  float mean[2], rstd[2];
+  float mean[RW], rstd[RW];
 #pragma unroll
-  for (int r = 0; r < 2; ++r) {
+  for (int r = 0; r < RW; ++r) {
     float sum = 0.f;
 #pragma unroll
     for (int i = 0; i < 2; ++i)
@@ -126,8 +143,8 @@ __global__ void __launch_bounds__(1024) gemm_norm_kernel(const NormGemmKArgs s) 
   dmaf_barrier();
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int r = 0; r < 2; ++r) {
-    const int row = wave * 2 + r;
+  for (int r = 0; r < RW; ++r) {
+    const int row = wave * RW + r;
     // A lane's place in the operand: 16-byte chunk of the column's 128-byte slab row; further groups of columns lie whole slabs behind.
     constexpr int GB = 4 * ESZ;       // bytes of the lane's consecutive columns
     const int lb = lane * GB;
@@ -159,11 +176,12 @@ __global__ void __launch_bounds__(1024) gemm_norm_kernel(const NormGemmKArgs s) 
 
 
   // ---- the product
-  const int nb = wave % NB, kp = wave / NB;
+  // (rows of a block past the tile are those of the next slab or part: only sums that are not stored read them)
+  const int kp = wave / s.nb, nb = wave - kp * s.nb;
   f32x16_t acc;
 #pragma unroll
   for (int r = 0; r < 16; ++r) acc[r] = 0.f;
-  const bool multiplies = wave < NB * KP && n0 + nb * 32 < a.N;
+  const bool multiplies = wave < s.nb * KP && n0 + nb * 32 < a.N;
   const int lr = lane & 31, g = lane >> 5;
   if (multiplies) {
     const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t*)smem);
@@ -173,13 +191,13 @@ __global__ void __launch_bounds__(1024) gemm_norm_kernel(const NormGemmKArgs s) 
     for (int k = 0; k < 4; ++k) {
       const int kc = IN_DT == DT_FP8 ? ((k & 1) | ((k >> 1) << 2)) : 2 * k;
       wb[k] = lds0 + (nb * 32 + lr) * ROWB + ((kc ^ LW) << 4);
-      xb[k] = lds0 + nslab * BN * ROWB + lr * ROWB + ((kc ^ LX) << 4);
+      xb[k] = lds0 + nslab * bn * ROWB + lr * ROWB + ((kc ^ LX) << 4);
     }
     struct Frags { Frag<IN_DT> w[KSTEPS], x[KSTEPS]; };
     auto piece = [](uint32_t at) -> i32x4_t { return *reinterpret_cast<const __attribute__((address_space(3))) i32x4_t*>(at); };
     auto read_step = [&](int slab, Frags& f, auto ksc) {
       constexpr int ks = decltype(ksc)::value;
-      const uint32_t wo = slab * BN * ROWB, xo = slab * BM * ROWB;
+      const uint32_t wo = slab * bn * ROWB, xo = slab * BM * ROWB;
       if constexpr (IN_DT == DT_FP8) {
         f.w[ks].lo = piece(wb[2 * ks] + wo); f.w[ks].hi = piece(wb[2 * ks + 1] + wo);
         f.x[ks].lo = piece(xb[2 * ks] + xo); f.x[ks].hi = piece(xb[2 * ks + 1] + xo);
@@ -219,13 +237,13 @@ __global__ void __launch_bounds__(1024) gemm_norm_kernel(const NormGemmKArgs s) 
   __syncthreads();
   // ---- epilogue: row er, columns ec .. ec + EV - 1
   const int m = m0 + er, n = n0 + ec;
-  if (m >= a.M || n >= a.N) return;
+  if (er >= BM || m >= a.M || n >= a.N) return;
   float v[EV];
 #pragma unroll
   for (int e = 0; e < EV; ++e) v[e] = 0.f;
 #pragma unroll
   for (int p = 0; p < KP; ++p) {
-    const float* patch = reinterpret_cast<const float*>(smem) + (p * NB + (ec >> 5)) * 1024 + er * 32 + ((((ec & 31) >> 2) ^ (er & 7)) << 2) + (ec & 3);
+    const float* patch = reinterpret_cast<const float*>(smem) + (p * s.nb + (ec >> 5)) * 1024 + er * 32 + ((((ec & 31) >> 2) ^ (er & 7)) << 2) + (ec & 3);
 #pragma unroll
     for (int e = 0; e < EV; ++e) v[e] = p == 0 ? patch[e] : v[e] + patch[e];
   }
@@ -247,7 +265,7 @@ __global__ void __launch_bounds__(1024) gemm_norm_kernel(const NormGemmKArgs s) 
   const bool first = n < a.nsplit;
   void* const out = first ? a.out : a.out2;
   const long o = first ? (long)m * a.ldo + n : (long)m * a.ldo2 + (n - a.nsplit);
-  if constexpr (EV == 2) {
+  {
     if (a.vec_ok && n + EV <= a.N) {
       if (a.out_dtype == DT_F32) *reinterpret_cast<float2*>(reinterpret_cast<float*>(out) + o) = make_float2(v[0], v[1]);
       else if (a.out_dtype == DT_FP8) *reinterpret_cast<uint16_t*>(reinterpret_cast<uint8_t*>(out) + o) = (uint16_t)pack_fp8x4(v[0], v[1], v[0], v[1]);

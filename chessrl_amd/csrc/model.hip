@@ -531,7 +531,7 @@ int Model::lnorm(const void* x, long ldx, int in_dt, const float* g, const float
 
 // (fp32 rows only)
 bool Model::norm_gemm_can(int M, const Lin& L, int in_dt, int x_dt) const {
-  return x_dt == DT_F32 && gemm_norm_width(M, L.N, L.K, in_dt, device_cus()) != 0;
+  return x_dt == DT_F32 && gemm_norm_tile(M, L.N, L.K, in_dt, device_cus()).bn != 0;
 }
 
 int Model::norm_gemm(const void* x, long ldx, const float* g, const float* b, const Lin& L, int in_dt, void* C, long ldc, int out_dt, int M, const GOpt& o,
@@ -547,7 +547,7 @@ int Model::norm_gemm(const void* x, long ldx, const float* g, const float* b, co
   const int fam = in_dt == DT_FP8 ? 0 : 5;
   if (profiling) { prof_flops[fam] += 2.0 * M * (double)(L.N - L.pad_N) * (L.K - L.pad_K); ++prof_n[2]; }
   prof_begin(fam, st);
-  const hipError_t e = launch_gemm_norm(a, in_dt, gemm_norm_width(M, L.N, L.K, in_dt, device_cus()), o.k_parallel, st);
+  const hipError_t e = launch_gemm_norm(a, in_dt, gemm_norm_tile(M, L.N, L.K, in_dt, device_cus()), o.k_parallel, st);
   prof_end(st);
   HIPCHK(e);
   return CRL_OK;

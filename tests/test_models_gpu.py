@@ -865,6 +865,20 @@ def test_gpt_norm_inside_the_product_is_bit_equal(cuda, kw, n_head, n_embd):
         assert torch.equal(m.forward((x[:B].contiguous(), idx[:B].contiguous()))[0], tokens[:B]), B
 
 
+@pytest.mark.parametrize("kw", [{}, {"fp8": True}])
+@pytest.mark.parametrize("n_head,n_embd", [(8, 256), (12, 768), (16, 1024)])
+def test_gpt_norm_inside_the_product_on_tiles_of_16_and_32_rows(cuda, kw, n_head, n_embd):
+    """The last layer's one row per position goes through tiles of 16 or 32 rows, whose columns get fewer as the rows do; bit-equal to the two launches of a large batch."""
+    planes, _ = positions(300, seed=4)
+    m = models.GPT(models.GPTConfig(block_size=128, vocab_size=1929, n_layer=2, n_head=n_head, n_embd=n_embd), **kw)
+    x = planes.to(cuda)
+    if kw.get("fp8"):
+        m.calibrate(x)
+    base = m.forward((x, None))[0]
+    for B in (4, 15, 16, 17, 31, 32, 47, 64, 65, 97, 128, 129, 160, 161):
+        assert torch.equal(m.forward((x[:B].contiguous(), None))[0], base[:B]), B
+
+
 @pytest.mark.parametrize("kw", [{}, {"norm_rms": True}, {"act_dtype": "f16"}, {"fp8": True}])
 @pytest.mark.parametrize("n_head,n_embd", [(8, 256), (12, 768), (16, 1024)])
 def test_gpt_norm_inside_the_product_takes_every_gain_and_offset(cuda, kw, n_head, n_embd):
