@@ -379,9 +379,9 @@ hipError_t launch_convert(const float* src, void* dst, long n, int dt, float sca
 hipError_t launch_widen(const void* src, int dt, float* dst, long n, hipStream_t st);
 hipError_t launch_kv_store(const void* qkv, void* cache, int B, int T, int Tmax, int C, hipStream_t st);
 // dyn_k (optional, device): the kernels take the token index k from it instead of from their arguments, so one captured
-// graph serves every step: position = 64 + k, keys = 65 + k.
+// graph serves every step: position = 64 + k, keys = 65 + k. past: read the cache with the non-temporal hint.
 hipError_t launch_decode_attention(const void* q, long ldq, const void* cache, int Tmax, int C, int n, const int* dyn_k, void* out, long ldo,
-                                   int B, int H, int head_dim, int in_dtype, float scale, hipStream_t st);
+                                   int B, int H, int head_dim, int in_dtype, float scale, bool past, hipStream_t st);
 // staging [B, 2C] -> row (pos or 64 + *dyn_k) of every sequence's [Tmax, 2C] cache
 hipError_t launch_kv_append(const void* staging, void* cache, int B, int Tmax, int C, int pos, const int* dyn_k, hipStream_t st);
 hipError_t launch_add_int(int* p, int v, hipStream_t st);

@@ -1012,6 +1012,15 @@ int Model::generate(const float* planes, int B, int steps, float temperature, ui
   RUN(forward_chunk(planes, nullptr, nullptr, gen_tok, 1, B, gen_logits, nullptr, nullptr, false, st));
   kv_capture = false;
   const float attn_scale = 1.0f / std::sqrt((float)hs);
+  // Keys and values that a step reads beyond what the memory-side cache keeps from one step to the next are read past it, the later layers' first: it then keeps
+  // the weights, which every product of a step waits for. 128 sequences (88 MB of weights, 63 MB of keys and values a layer on average), whole rollout: no layer read
+  // past it 54.3 ms, those beyond 260 MB 53.2, 200 52.6, 150 51.3, 100 51.4, all 52.1 (before the values were requested ahead: 260 and all); 64 sequences 41.3, 150 MB 39.7, all 39.9;
+  // 16 and fewer stay inside (all past it: +1.2 %).
+  constexpr size_t KEEP = 150u << 20;
+  size_t weights = (size_t)lm_head.N * lm_head.K * 2;
+  for (const Layer& y : layers)
+    for (const Lin* w : {&y.qkv, &y.proj, &y.ff1, &y.ff2}) weights += (size_t)w->N * w->K * 2;
+  auto past = [&](int l, int n) { return weights + (size_t)(l + 1) * B * n * 2 * C * 2 > KEEP; };
   // One token step: sample token k from gen_logits, then (unless it is the last) run it through the trunk at position
   // 64 + k against the cache and leave the next logits in gen_logits. With `dyn` the kernels read k from device memory
   // and the step ends by advancing it, so the same launches serve every k (the body of the replayed graph).
@@ -1050,7 +1059,7 @@ int Model::generate(const float* planes, int B, int steps, float temperature, ui
         }
         if (dyn) STEP_HIP(launch_kv_append(gen_kv_stage, kv_layers[l], B, kv_Tmax, C, 0, dyn, s));
       }
-      STEP_HIP(launch_decode_attention(ws.qkv, C, kv_layers[l], kv_Tmax, C, pos + 1, dyn, ws.ao, C, B, H, hs, ad, attn_scale, s));
+      STEP_HIP(launch_decode_attention(ws.qkv, C, kv_layers[l], kv_Tmax, C, pos + 1, dyn, ws.ao, C, B, H, hs, ad, attn_scale, past(l, dyn ? Tmax : pos + 1), s));
       bool normed2 = false;
       { GOpt o; o.k_parallel = true; o.res = ws.x; o.ldr = C; o.res_dt = xdt;
         if (!fused) { o.ln_g = ly.ln2_g; o.ln_b = ly.ln2_b; o.ln_out = ws.h; o.ln_dt = ad; o.ln_folded = &normed2; }

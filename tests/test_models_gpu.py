@@ -914,6 +914,32 @@ def test_generate_rows_do_not_depend_on_the_batch(cuda, kw):
         assert torch.equal(s, seq[:B]) and torch.equal(o, out[:B]), B
 
 
+def test_generate_rows_read_past_the_memory_side_cache_or_not(cuda):
+    """Six layers of 160 sequences hold more keys and values than are kept in the memory-side cache; the same rows in a small batch do not. Same bits."""
+    planes, _ = positions(160, seed=9)
+    m = models.GPT(models.GPTConfig(block_size=256, vocab_size=1929, n_layer=6, n_head=12, n_embd=768))
+    x = planes.to(cuda)
+    for graph in (False, True):
+        m._engine.set_decode_graph(graph)
+        seq, out = m._engine.generate(x, 8, T=0.0, rules=False, want_step_out=True, out_logits=True)
+        s, o = m._engine.generate(x[:5].contiguous(), 8, T=0.0, rules=False, want_step_out=True, out_logits=True)
+        assert torch.equal(s, seq[:5]) and torch.equal(o, out[:5])
+
+
+@pytest.mark.parametrize("n_head,n_embd,act", [(8, 256, "bf16"), (4, 256, "bf16"), (4, 256, "f16")])
+def test_generate_beyond_the_tokens_requested_at_once(cuda, n_head, n_embd, act):
+    """Cached attention over up to 364 tokens, heads of 32 and 64: the first 256 are requested at once, the others in a loop. Step logits against the uncached
+    forward's, up to summation order (bound as in the cached-against-recomputed test above)."""
+    B, steps = 2, 300
+    planes, _ = positions(B, seed=14)
+    m = models.GPT(models.GPTConfig(block_size=384, vocab_size=1929, n_layer=2, n_head=n_head, n_embd=n_embd), act_dtype=act)
+    x = planes.to(cuda)
+    seq, log = m._engine.generate(x, steps, T=0.0, rules=False, want_step_out=True, out_logits=True)
+    full = m._engine.forward_tokens(x, seq[:, :steps].contiguous(), last=False, every=True)[1]
+    for part in (slice(0, 192), slice(192, 200), slice(200, 300)):
+        assert rel_rms(log[:, part].cpu(), full[:, 64:64 + steps][:, part].cpu()) < 3e-3
+
+
 @pytest.mark.parametrize("kw", [{}, {"act_dtype": "f16"}, {"fp8": True}, {"stream_f32": False}])
 @pytest.mark.parametrize("B,t", [(1, 0), (3, 1), (255, 0), (256, 0), (250, 3), (130, 66)])
 def test_gpt_last_token_row(cuda, kw, B, t):
