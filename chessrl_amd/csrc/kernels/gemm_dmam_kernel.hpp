@@ -31,9 +31,31 @@ struct DmamCfg {
 // operation, i.e. for the slabs that are meant to stay in flight).
 __device__ __forceinline__ void dmam_barrier() { asm volatile("s_barrier" ::: "memory"); }
 
+// The order of the tiles: columns in groups of up to gw, inside a group row by row.
+struct DmamWalk {
+  int gw, lastw, per_group, ngroups;        // columns of a group, of the last one; tiles of a group
+  uint32_t m_group, m_gw, m_lastw;          // magics
+  __device__ __forceinline__ void pos(int t, int& tm, int& tn) const {
+    const int g = dmaf_div(t, m_group), r = t - g * per_group;
+    const bool last = g + 1 == ngroups;
+    tm = dmaf_div(r, last ? m_lastw : m_gw);
+    tn = g * gw + r - tm * (last ? lastw : gw);
+  }
+};
+inline DmamWalk dmam_walk(int tiles_m, int tiles_n) {
+  DmamWalk w{};
+  w.ngroups = (tiles_n + 5) / 6;
+  w.gw = (tiles_n + w.ngroups - 1) / w.ngroups;
+  w.ngroups = (tiles_n + w.gw - 1) / w.gw;
+  w.lastw = tiles_n - (w.ngroups - 1) * w.gw;
+  w.per_group = tiles_m * w.gw;
+  w.m_group = dmaf_magic(w.per_group); w.m_gw = dmaf_magic(w.gw); w.m_lastw = dmaf_magic(w.lastw);
+  return w;
+}
+
 // EPI, ACT: as in gemm_dmaf_kernel.hpp.
 template <int IN_DT, int OUT_DT, int EPI, int ACT = ACT_NONE>
-__global__ void __launch_bounds__(DmamCfg::NT) gemm_dmam_kernel(const GemmArgs a, const int tiles, const int tiles_n, const uint32_t m_tn) {
+__global__ void __launch_bounds__(DmamCfg::NT) gemm_dmam_kernel(const GemmArgs a, const int tiles, const DmamWalk walk) {
   typedef DmamCfg Cfg;
   constexpr bool PERSIST = EPI >= DMAF_PLAIN;
   constexpr bool HAS_RES = EPI == DMAF_RES16 || EPI == DMAF_RESNORM || EPI == DMAF_RES32;
@@ -69,7 +91,9 @@ __global__ void __launch_bounds__(DmamCfg::NT) gemm_dmam_kernel(const GemmArgs a
     __amdgpu_buffer_rsrc_t rsrc;
     int l_tile = tile, l_slab = 0, l_stage = 0;
     auto stream_tile = [&]() {
-      const int tm = dmaf_div(l_tile, m_tn), m0 = tm * BM, n0 = (l_tile - tm * tiles_n) * BN;
+      int tm, tn;
+      walk.pos(l_tile, tm, tn);
+      const int m0 = tm * BM, n0 = tn * BN;
       const int left = loads_a ? a.M - m0 : a.N - n0;
 #pragma unroll
       for (int i = 0; i < Cfg::LOADS; ++i) {
@@ -164,7 +188,9 @@ __global__ void __launch_bounds__(DmamCfg::NT) gemm_dmam_kernel(const GemmArgs a
   u32x2_t row_st[EPI == DMAF_RESNORM ? TM : 1];
 
   for (;;) {
-    const int tm0 = dmaf_div(tile, m_tn), m0 = tm0 * BM, n0 = (tile - tm0 * tiles_n) * BN;
+    int tm0, tn0;
+    walk.pos(tile, tm0, tn0);
+    const int m0 = tm0 * BM, n0 = tn0 * BN;
     const bool wave_active = (m0 + wm * Cfg::WM < a.M) && (n0 + wn * Cfg::WN < a.N);
     const int rows = a.M - m0 < BM ? a.M - m0 : BM;
     {
@@ -395,11 +421,11 @@ static hipError_t launch_dmam(const GemmArgs& a, int cus, hipStream_t st) {
     if (e != hipSuccess) return e;
     if (dev >= 0 && dev < 16) attr_set[dev] = true;
   }
-  const int tiles_n = (a.N + DmamCfg::BN - 1) / DmamCfg::BN, tiles = ((a.M + DmamCfg::BM - 1) / DmamCfg::BM) * tiles_n;
+  const int tiles_n = (a.N + DmamCfg::BN - 1) / DmamCfg::BN, tiles_m = (a.M + DmamCfg::BM - 1) / DmamCfg::BM, tiles = tiles_m * tiles_n;
   if (tiles >= 65536) return hipErrorInvalidValue;
   const int slots = cus >= 8 ? cus & ~7 : 256;
   const int grid = EPI >= DMAF_PLAIN && tiles > slots ? slots : tiles;
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(DmamCfg::NT), DmamCfg::LDS_BYTES, st, a, tiles, tiles_n, dmaf_magic(tiles_n));
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(DmamCfg::NT), DmamCfg::LDS_BYTES, st, a, tiles, dmam_walk(tiles_m, tiles_n));
   return hipGetLastError();
 }
 
