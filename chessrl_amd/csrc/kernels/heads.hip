@@ -449,6 +449,22 @@ hipError_t launch_convert(const float* src, void* dst, long n, int dt, float sca
   return hipGetLastError();
 }
 
+// out[n, k] = sum over f of w2[n, f] w1[f, k], in double precision: two linear layers with nothing between them as one, when weights are packed.
+__global__ void __launch_bounds__(256) fold_linears_kernel(const float* w2, const float* w1, float* out, int N, int F, int K) {
+  const int k = blockIdx.x * 256 + threadIdx.x, n = blockIdx.y;
+  if (k >= K) return;
+  double s = 0;
+#pragma unroll 8
+  for (int f = 0; f < F; ++f) s += (double)w2[(long)n * F + f] * (double)w1[(long)f * K + k];
+  out[(long)n * K + k] = (float)s;
+}
+hipError_t launch_fold_linears(const float* w2, const float* w1, float* out, int N, int F, int K, hipStream_t st) {
+  if (N <= 0 || K <= 0) return hipSuccess;
+  if (N > 65535) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(fold_linears_kernel, dim3((K + 255) / 256, N), dim3(256), 0, st, w2, w1, out, N, F, K);
+  return hipGetLastError();
+}
+
 __global__ void widen_kernel(const void* src, int dt, float* dst, long n) {
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;

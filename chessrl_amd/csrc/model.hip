@@ -193,6 +193,33 @@ int Model::make_ffn(Layer& ly, const std::vector<float>& w1, const std::vector<f
   return make_lin(ly.ff2, pad_to(w2, C, F, C, FP), &b2, C, FP, ad, cfg.fp8 != 0);
 }
 
+int Model::fold_ffn(Layer& ly, const std::vector<float>& w1, const std::vector<float>& b1, const std::vector<float>& w2, const std::vector<float>& b2) {
+  const int C = cfg.d_model, F = cfg.d_ff;
+  std::vector<float> b(C);
+  for (int n = 0; n < C; ++n) {
+    double s = b2[n];
+    for (int f = 0; f < F; ++f) s += (double)w2[(size_t)n * F + f] * b1[f];
+    b[n] = (float)s;
+  }
+  Lin& L = ly.ff;
+  L.N = L.K = C; L.dt = cfg.act_dtype;
+  float* tmp = nullptr;   // W1, W2, their product
+  const size_t cf = (size_t)C * F, cc = (size_t)C * C;
+  HIPCHK(hipMalloc((void**)&tmp, (2 * cf + cc) * sizeof(float)));
+  hipError_t e = hipMemcpy(tmp, w1.data(), cf * sizeof(float), hipMemcpyHostToDevice);
+  if (e == hipSuccess) e = hipMemcpy(tmp + cf, w2.data(), cf * sizeof(float), hipMemcpyHostToDevice);
+  if (e == hipSuccess) e = launch_fold_linears(tmp + cf, tmp, tmp + 2 * cf, C, F, C, nullptr);
+  if (e == hipSuccess) {
+    const int rc = dev_alloc(&L.w, cc * dtype_size(L.dt), false);
+    if (rc) { (void)hipFree(tmp); return rc; }
+    e = launch_convert(tmp + 2 * cf, L.w, (long)cc, L.dt, 1.f, nullptr);
+    if (e == hipSuccess) e = hipDeviceSynchronize();
+  }
+  (void)hipFree(tmp);
+  HIPCHK(e);
+  return upload(b, DT_F32, 1.f, (void**)&L.b);
+}
+
 // Weights that a pass reads beyond what the 256 MB memory-side cache keeps from one pass to the next. Read in turn, 311 MB of them (BT4-class, bf16) never
 // meet themselves there again: every line is gone by the time it is asked for. The layers that go beyond the share below are read with the non-temporal
 // hint, which leaves the others where they are. One bf16 position of the 15 x 1024 model, layers kept: all 789 us, 11 759, 9 (208 MB with what is
@@ -202,7 +229,11 @@ int Model::make_ffn(Layer& ly, const std::vector<float>& w1, const std::vector<f
 void Model::mark_streamed() {
   constexpr size_t KEEP = 200u << 20;
   auto bytes = [](const Lin& l) -> size_t { return (size_t)l.N * l.K * (l.w8 ? 1 : dtype_size(l.dt)); };
-  auto each = [](Layer& y, auto f) { for (Lin* l : {&y.qkv, &y.proj, &y.ff1, &y.ff2, &y.sm_hidden}) f(*l); };
+  auto each = [this](Layer& y, auto f) {
+    for (Lin* l : {&y.qkv, &y.proj, &y.sm_hidden}) f(*l);
+    if (folds_ffn()) f(y.ff);
+    else for (Lin* l : {&y.ff1, &y.ff2}) f(*l);
+  };
   size_t sum = 0;
   for (const Lin* l : {&lm_head, &pol_tok, &pol_qk, &pol_head, &val1, &val2, &val3, &sm_weight_gen}) sum += bytes(*l);
   for (Layer& y : layers) sum += bytes(y.sm_gen);   // (their kernel has no such reads)
@@ -298,6 +329,7 @@ int Model::finalize() {
       LIN(ly.qkv, wq, &bq, nq, C, ad, f8);
       LIN(ly.proj, w(p + "attention.out_proj.weight"), &w(p + "attention.out_proj.bias"), C, C, ad, f8);
       rc = make_ffn(ly, w(p + "ff1.weight"), w(p + "ff1.bias"), w(p + "ff2.weight"), w(p + "ff2.bias")); if (rc) return rc;
+      if (folds_ffn()) { rc = fold_ffn(ly, w(p + "ff1.weight"), w(p + "ff1.bias"), w(p + "ff2.weight"), w(p + "ff2.bias")); if (rc) return rc; }
       UP(w(p + "norm1.weight"), DT_F32, ly.ln1_g); UP(w(p + "norm1.bias"), DT_F32, ly.ln1_b);
       UP(w(p + "norm2.weight"), DT_F32, ly.ln2_g); UP(w(p + "norm2.bias"), DT_F32, ly.ln2_b);
       if (cfg.arch == CRL_ARCH_BT4) {
@@ -797,7 +829,10 @@ int Model::forward_chunk(const float* planes, const uint8_t* ids, const uint8_t*
       RUN(lnorm(ws.t, C, xdt, ly.ln1_g, ly.ln1_b, fold ? nullptr : ws.h, xdt, f8 ? ws.h8 : nullptr, f8 ? act_scale(l, 2) : 1.f, C, M, C, am(l, 2), st,
                 fold ? ws.st1 : nullptr, (sf32p && !f8) ? ws.h16 : nullptr, ad));
       const void* h_in = f8 ? (const void*)ws.h8 : (const void*)h_op;
-      if (cfg.arch == CRL_ARCH_BT4) {
+      if (folds_ffn() && !calibrate) {   // (the hidden tensor's maximum is one of the table's)
+        GOpt o; o.act = ACT_GELU; o.res = ws.h; o.ldr = C; o.res_dt = xdt;
+        RUN(gemm(ly.ff, h_in, C, ao_dt, ws.t, C, xdt, M, o, st));
+      } else if (cfg.arch == CRL_ARCH_BT4) {
         // y = ff2(ff1(h)) with no activation in between; t = gelu(y) + h (new_paradigm/value.py:65-70)
         { GOpt o; o.a_scale = f8 ? act_scale(l, 2) : 1.f; o.out_scale = f8 ? act_scale(l, 3) : 1.f; o.amax = am(l, 3);
           RUN(gemm(ly.ff1, h_in, C, ao_dt, f8 ? (void*)ws.f8 : (void*)ws.f, F, ao_dt, M, o, st)); }

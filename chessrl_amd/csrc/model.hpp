@@ -37,6 +37,7 @@ struct Lin {
 
 struct Layer {
   Lin qkv, proj, ff1, ff2, sm_hidden, sm_gen;
+  Lin ff;   // ff1 and ff2 as one layer (Model::folds_ffn)
   float *ln1_g = nullptr, *ln1_b = nullptr, *ln2_g = nullptr, *ln2_b = nullptr;
   float *sm_ln1_g = nullptr, *sm_ln1_b = nullptr, *sm_ln2_g = nullptr, *sm_ln2_b = nullptr;
   void* pos = nullptr;
@@ -73,6 +74,10 @@ struct Model {
     const int q = cfg.fp8 ? 128 : 64, padded = (cfg.d_ff + q - 1) / q * q;
     return (padded - cfg.d_ff) * 16 <= cfg.d_ff ? padded : cfg.d_ff;
   }
+  // BT4's FFN has nothing between its two linear layers (new_paradigm/value.py:65-70): in 16 bits it runs as the one layer W2 W1 with bias W2 b1 + b2, wherever
+  // that is the smaller product. Its rounding is that of one weight where there were two weights and the hidden tensor. 31744 rows, 512 columns, 736 hidden: two products of
+  // 30 and 32 us, one of 20; in e4m3 the layers stay apart, each with its own scales.
+  bool folds_ffn() const { return cfg.arch == CRL_ARCH_BT4 && !cfg.fp8 && cfg.d_model < 2 * cfg.d_ff; }
   // q and k columns of the concatenated q|k|v weight paired head by head (BT4-class with 64-byte head rows)
   bool qk_paired() const { return cfg.arch == CRL_ARCH_BT4CLASS && cfg.d_model / cfg.n_head == 32; }
   crl_model_config cfg;
@@ -153,6 +158,7 @@ struct Model {
   int dev_alloc(void** p, size_t bytes, bool ws);
   int upload(const std::vector<float>& v, int dt, float scale, void** out);
   int make_lin(Lin& L, const std::vector<float>& W, const std::vector<float>* bias, int N, int K, int dt16, bool fp8, float amax_all = -1.f);
+  int fold_ffn(Layer& ly, const std::vector<float>& w1, const std::vector<float>& b1, const std::vector<float>& w2, const std::vector<float>& b2);
   int make_ffn(Layer& ly, const std::vector<float>& w1, const std::vector<float>& b1, const std::vector<float>& w2, const std::vector<float>& b2);
   int ensure_ws(int mb);
   int forward_chunk(const float* planes, const uint8_t* ids, const uint8_t* flags, const int64_t* idx, int t, int mb, float* policy,

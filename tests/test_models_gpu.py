@@ -145,6 +145,35 @@ def test_padded_ffn_equals_the_model_with_the_zeros_in_its_weights(cuda, arch, f
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("Cm,Fm,H", [(256, 368, 4), (256, 128, 4), (256, 136, 8), (512, 736, 8)])
+@pytest.mark.parametrize("act", ["bf16", "f16"])
+def test_bt4_ffn_as_one_layer(cuda, Cm, Fm, H, act):
+    """BT4's two FFN layers run as one where the hidden width is more than half the model's (else as two). Layers that nearly cancel (W2 W1 far smaller than |W2| |W1|, b1 and b2 of
+    the size of the sums) against fp32: one rounding of a weight to 8 or 11 bits, bound as for the other 16-bit BT4 tests. Calibration still sees the hidden tensor."""
+    oracle = om.test_init_(om.BT4Oracle(2, Cm, Fm, H), seed=3)
+    sd, g = oracle.state_dict(), torch.Generator().manual_seed(2)
+    for k in sd:
+        if "ff1.bias" in k or "ff2.bias" in k:
+            sd[k] = torch.randn(sd[k].shape, generator=g)
+        if "ff1.weight" in k:
+            sd[k][Fm // 2:Fm // 2 * 2] = sd[k][:Fm // 2]
+            w2 = k.replace("ff1", "ff2")
+            sd[w2][:, Fm // 2:Fm // 2 * 2] = -0.9 * sd[w2][:, :Fm // 2]
+    oracle.load_state_dict(sd)
+    planes, mask = positions(70, seed=2)
+    rpol, rwdl = oracle.forward_pv(planes)
+    m = models.BT4(2, Cm, Fm, H, act_dtype=act)
+    m.load_state_dict(sd)
+    x = planes.to(cuda)
+    pol, wdl = m._engine.forward(x)
+    assert rel_rms(pol.cpu(), rpol) < (2e-2 if act == "bf16" else 4e-3)
+    assert (wdl.cpu() - rwdl).abs().max() <= (1e-2 if act == "bf16" else 2e-3)
+    one = m._engine.forward(x[:1].contiguous())
+    assert torch.equal(one[0], pol[:1]) and torch.equal(one[1], wdl[:1])
+    m._engine.calibrate(x)
+    assert bool((torch.as_tensor(m._engine.get_amax())[:, :4] > 0).all())
+
+
 def test_bt4_fp32_stream(cuda):
     """BT4 with the residual stream kept in fp32 (16-bit GEMM operands): closer to the oracle than the 16-bit stream."""
     oracle = om.test_init_(om.BT4Oracle(10, 512, 736, 8), seed=1)
