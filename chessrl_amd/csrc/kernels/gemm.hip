@@ -613,8 +613,8 @@ static hipError_t launch_in_out(const GemmArgs& a, int tile, hipStream_t st) {
   // that is what it is for: M = 131072, N = 4096 takes 280 us through the 256x256 tile, 310 us here row-major and 191 us
   // here in blocks, so nothing picks it for a row-major output unasked.
   if (a.c_blocked || tile == 13) return launch_gemm_shortk(a, IN_DT, OUT_DT, st);
-  // Token steps of generation, a tile of 32x32 per CU at most: the ring kernel with four waves on a tile's K (M=128, N=768, on average over K=768 and
-  // K=3072: 8.5 us, against 12.2 and 13.9 us for the two passes of the sliced form with the next norm on the second).
+  // Token steps of generation, a tile of 32x32 per CU at most: the ring kernel (M=128, N=768, on average over K=768 and K=3072: 3.7 us, against 12.2 and 13.9 us for the two
+  // passes of the sliced form with the next norm on the second).
   if (tile == 0 && a.k_parallel && !a.ln_out && !a.res_stats && ((long)a.K * (IN_DT == DT_FP8 ? 1 : 2)) % 128 == 0 && gemm_dmam_has(IN_DT, OUT_DT) &&
       (long)((a.M + 31) / 32) * ((a.N + 31) / 32) <= device_cus())
     return launch_gemm_dmas(a, IN_DT, OUT_DT, st, 32);

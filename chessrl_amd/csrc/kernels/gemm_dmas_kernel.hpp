@@ -5,34 +5,37 @@
 //  * Loading and computing waves are different waves. A load instruction of 64 x 16 bytes holds its wave for 100 to 150
 //    cycles, and a CU moves 64 bytes per clock into LDS at most: eight waves that do nothing else reach that (146 GB/s; one
 //    wave pulls 23), the computing ones start on the first slab while the later ones are still being requested.
-//  * The fragments of slab s + 1 are read from LDS between the MFMAs of slab s: a 32x32 wave tile is one chain of dependent
-//    MFMAs (52 cycles each), and a wave issues in order.
+//  * The fragments of slab s + 1 are read from LDS between the MFMAs of slab s, which are one chain, and a wave issues in order.
 //  * The epilogue belongs to the loading waves: 512 threads need a third of the time one wave needs for a tile of 1024 elements,
 //    which is a chain of some 300 instructions there. Residual and bias are brought into LDS meanwhile by a wave of their own.
 //  * Everything the kernel needs to know travels in 128 bytes of arguments, requested at once (they are read from memory, cold,
 //    before the first address can be formed).
-// Measured back to back on M = 64, N = 1024 (bf16, residual and bias): 6.2 -> 4.25 us at K = 1024 against two waves that load and
-// compute in turn, 4.9 us at K = 1536, 3.2 at K = 256; with N = 3072 and weights from HBM 7.6 -> 5.75 us. What is left at K = 1024 are some 1400 cycles
-// until the first slab is there, 3500 of MFMA chain and 1200 of epilogue around a launch of 1.6 us.
+// Measured inside passes of one position (bf16, start to end of a launch, of which its first slab takes 1900 to 2800 cycles and its epilogue 1000): M = 64, N = 1024, K = 1024 2.5 us
+// where the memory-side cache has the weights and 2.9 past it (3.0 and 4.1 on 32x32 tiles with 32x32x16 MFMAs), K = 1536 3.0 and 3.3 (3.7 and 5.6), N = 768, K = 3072 4.1 (5.7);
+// M = 128, N = 768, K = 3072 4.8 (7.3 with four waves on K). One position of 15 layers 685 -> 643 us, of GPT 182 -> 171; token steps of 128 sequences 51.1 -> 48.5 ms a rollout.
 // Same K order and same arithmetic per element as the other tiled kernels: bit-equal results.
 #pragma once
 #include "gemm_dmaf_kernel.hpp"
 
 namespace crl {
 
-// BT = 64: eight stages of 16 KB, four computing waves of 32x32; BT = 32: sixteen stages of 8 KB, one. Eight loading waves either
-// way, which keep AHEAD slabs requested (at the CU's load rate a slab of 8 KB takes 128 cycles, and memory some 1000; twelve waves delay the first slab: GPT one position 217 -> 228 us), and one
-// wave that fetches what the epilogue needs. Fourteen slabs ahead where a slab has at most 40 rows: as many bytes as six of 64 rows. (Fourteen of those are
-// 112 KB that every CU asks for before it waits for its first slab, which then comes at 4400 cycles instead of 2500: one position 684 -> 711 us.)
-// KP > 1 (token steps, whose sums may be added in another order): KP computing waves per 32x32 take the slabs in turn, a round of KP slabs to a barrier and
-// three rounds requested ahead. With a barrier to each slab every wave waited for the one that had it: 128 rows, N = 768, K = 768 4.8 -> 4.1 us,
-// K = 3072 11.9 -> 9.4 (a token step of 128 sequences 311 -> 291).
-template <int BT, int KP_ = 1, int AHEAD_ = (KP_ > 1 ? 3 * KP_ : 6)>
+// BT = 64: eight stages of 16 KB, four computing waves of 32x32; BT = 32: sixteen stages of 8 KB. Eight loading waves either way (twelve delay the first slab: GPT one position
+// 217 -> 228 us), which keep AHEAD stages requested, and one wave that fetches what the epilogue needs. AHEAD is some 64 KB, all that a CU has in flight: the first slab is
+// announced when AHEAD have been asked for, and 14 stages of 64 rows put that at 4400 cycles instead of 2500 (one position 684 -> 711 us), of 32 rows
+// (PAIRS) K = 1536 past the caches at 3900 instead of 2560.
+// QUADS (BT = 32, 16-bit operands): four computing waves, a quarter of the tile each, with 16x16x32 MFMAs. Those add K exactly as two 32x32x16 do (checked on sums of
+// normal, wide-ranged and all-positive values: the same bits), but follow each other in at most 32 cycles where two of the other take 97: a slab 136 cycles with its barrier
+// instead of 208. (e4m3 has no such pair: 16x16x128 differs from two 32x32x64 in one sum of eight.)
+// PAIRS (tiles of at most 16 x 16): a stage holds two slabs, the second in rows 16 to 31 of either operand: a barrier for two slabs, 105 cycles each.
+template <int BT, int QUADS_ = 0, int AHEAD_ = 6, int PAIRS_ = 0>
 struct DmasCfg {
   static_assert(BT == 64 || BT == 32, "two tile sizes");
-  static_assert(KP_ == 1 || (BT == 32 && KP_ <= 4), "patches of the K groups lie in stages nothing is loaded into any more");
-  static constexpr int BM = BT, BN = BT, WGM = BT / 32, WGN = BT / 32;
-  static constexpr int KP = KP_, NCOMP = WGM * WGN * KP, NLOAD = 8, NT = 64 * (NCOMP + NLOAD + 1);
+  static constexpr bool QUADS = QUADS_ != 0;
+  static_assert(!QUADS || BT == 32, "quarters of 16x16");
+  static constexpr bool PAIRS = PAIRS_ != 0;
+  static_assert(!PAIRS || QUADS, "one quarter");
+  static constexpr int BM = BT, BN = BT, WGM = QUADS ? 2 : BT / 32, WGN = QUADS ? 2 : BT / 32, WT = QUADS ? 16 : 32;   // rows and columns of a computing wave
+  static constexpr int NCOMP = WGM * WGN, NLOAD = 8, NT = 64 * (NCOMP + NLOAD + 1);
   static constexpr int ROWB = 128, NSTAGE = 512 / BT, AHEAD = AHEAD_;
   static constexpr int LOADS = 2 * BT / (8 * NLOAD);           // load instructions (8 rows each) of a wave per stage
   static constexpr int STAGE = BN * ROWB;                      // bytes of one operand's rows in one stage
@@ -41,12 +44,11 @@ struct DmasCfg {
   static constexpr int BIAS_OFF = RES_OFF + BM * BN * 4;
   static constexpr int LDS_BYTES = BIAS_OFF + 64 * 4;
   static constexpr int EV = BM * BN / (64 * NLOAD);            // elements of an epilogue thread: 2 or 8 consecutive columns of one row
-  // The sums of computing wave w on their way to the epilogue: a 32x32 patch in the weight rows of the stage(s) behind the last
+  // The sums of 32x32 block w on their way to the epilogue: a patch in the weight rows of the stage(s) behind the last
   // slab's, which held slab nslab - NSTAGE and which nothing is loaded into any more.
   static __device__ __forceinline__ int patch_off(int nslab, int w) {
     return ((nslab + w * 4096 / STAGE) & (NSTAGE - 1)) * STAGE + w * 4096 % STAGE;
   }
-  static_assert(KP == 1 || 4 * KP <= NSTAGE, "a round in work, three requested");
   static_assert(AHEAD * LOADS < 64 && AHEAD + 2 <= NSTAGE, "the counted waits fit the counter; a stage is read before it is refilled");
   static_assert(LDS_BYTES <= 160 * 1024, "LDS of a CU");
 };
@@ -209,7 +211,7 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_dmas_kernel(const SmallArgs s_in
   // (all arguments in registers at this point: left alone, the compiler asks for them in four batches, one wait after the other)
   asm volatile("" ::"s"(s.A), "s"(s.W), "s"(s.C), "s"(s.bias), "s"(s.res), "s"(s.amax), "s"(s.lda_b), "s"(s.ldr), "s"(s.nsplit), "s"(s.vec_ok), "s"(s.per_xcd));
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int nslab = s.nslab;
+  const int nslab = Cfg::PAIRS ? (s.nslab + 1) >> 1 : s.nslab;   // stages to fill
 
   // Workgroup b runs on XCD b & 7, which owns a contiguous range of the tile order (rows or columns first, see the launch).
   int pid = blockIdx.x;
@@ -219,9 +221,8 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_dmas_kernel(const SmallArgs s_in
   const int bm = BM == 32 ? s.bm : BM, bn = BM == 32 ? s.bn : BN;
   const int m0 = tile_m * bm, n0 = tile_n * bn;
 
-  // Barrier i (0 .. nbar - 1) of the workgroup says that slabs KP i .. KP i + KP - 1 have landed, barrier nbar that sums, residual and bias
+  // Barrier i (0 .. nslab - 1) of the workgroup says that slab i has landed, barrier nslab that sums, residual and bias
   // lie in LDS. Every wave passes all of them.
-  const int nbar = (nslab + Cfg::KP - 1) / Cfg::KP;
   if (wave == Cfg::NCOMP + Cfg::NLOAD) {
     if (small_tile_full(s, n0, bn)) {
       if (s.bias) {
@@ -247,7 +248,7 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_dmas_kernel(const SmallArgs s_in
       }
     }
 #pragma unroll 1
-    for (int i = 0; i < nbar; ++i) dmas_barrier();
+    for (int i = 0; i < nslab; ++i) dmas_barrier();
     wait_vmcnt<0>();
     dmas_barrier();
     return;
@@ -262,24 +263,24 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_dmas_kernel(const SmallArgs s_in
     const int ld = loads_a ? s.lda_b : s.ldw_b;
     int rows_left = loads_a ? s.M - m0 : s.N - n0;
     if constexpr (BM == 32) rows_left = min(rows_left, loads_a ? bm : bn);
-    const bool idle = BM == 32 && rbase >= (loads_a ? bm : bn);   // (a narrower tile has fewer groups of eight rows)
+    const bool idle = BM == 32 && (Cfg::PAIRS ? rbase & 15 : rbase) >= (loads_a ? bm : bn);   // (a narrower tile has fewer groups of eight rows)
     uint32_t voff[LOADS];
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) {
-      int r = rbase + 8 * i + (lane >> 3);
+      int r = (Cfg::PAIRS ? rbase & 15 : rbase + 8 * i) + (lane >> 3);
       r = r < rows_left ? r : rows_left - 1;
-      voff[i] = (uint32_t)r * (uint32_t)ld + (((lane & 7) ^ (lane >> 3) ^ ((rbase / 8 + i) & 7)) << 4);
+      voff[i] = (uint32_t)r * (uint32_t)ld + (Cfg::PAIRS ? (rbase >> 4) * Cfg::ROWB : 0) + (((lane & 7) ^ (lane >> 3) ^ ((rbase / 8 + i) & 7)) << 4);
     }
-    // (the rows of a tile span less than 2 GB: the launcher checks)
+    // (the rows of a tile span less than 2 GB: the launcher checks; they end with K, which the second slab of a last pair may lie behind)
     const uint8_t* origin = reinterpret_cast<const uint8_t*>(loads_a ? s.A : s.W) + (long)(loads_a ? m0 : n0) * ld + (SLICED ? (long)((blockIdx.y >> 2) * 4 * nslab + (blockIdx.y & 3)) * Cfg::ROWB : 0);
-    const __amdgpu_buffer_rsrc_t rsrc_mine = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(origin), 0, (rows_left < BM ? rows_left : BM) * ld, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rsrc_mine = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(origin), 0, SLICED ? (rows_left < BM ? rows_left : BM) * ld : ((rows_left < BM ? rows_left : BM) - 1) * ld + s.nslab * Cfg::ROWB, 0x00020000);
     const uint32_t lds_load0 = (loads_a ? Cfg::PART_BYTES : 0) + rbase * Cfg::ROWB;   // stage 0
     auto issue_slab = [&](int slab) {
       if (idle) return;
       uint8_t* dst = smem + lds_load0 + (slab & (NSTAGE - 1)) * STAGE;
       static_for<0, LOADS>([&](auto ic) {
         constexpr int i = decltype(ic)::value;
-        constexpr int STEP = SLICED ? 4 * Cfg::ROWB : Cfg::ROWB;
+        constexpr int STEP = SLICED ? 4 * Cfg::ROWB : Cfg::PAIRS ? 2 * Cfg::ROWB : Cfg::ROWB;
         if (ONCE && !loads_a) dmaf_load16_nt(rsrc_mine, dst + i * 1024, (int)voff[i], slab * STEP);
         else dmaf_load16(rsrc_mine, dst + i * 1024, (int)voff[i], slab * STEP);
       });
@@ -287,30 +288,7 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_dmas_kernel(const SmallArgs s_in
 #pragma unroll
     for (int s0 = 0; s0 < AHEAD; ++s0)
       if (s0 < nslab) issue_slab(s0);
-    if constexpr (Cfg::KP > 1) {
-      constexpr int KP = Cfg::KP;
-      int r = 0;
-#pragma unroll 1
-      for (; r + 3 < nbar; ++r) {
-        wait_vmcnt<2 * KP * LOADS>();
-        dmas_barrier();
-        // (into the stages of round r - 1, which the computing waves had in registers before they came here)
-#pragma unroll
-        for (int i = 0; i < KP; ++i)
-          if ((r + 3) * KP + i < nslab) issue_slab((r + 3) * KP + i);
-      }
-      // The last three rounds, or all there are; where the last one is short its slabs are waited for with the round before.
-      const bool full = nslab % KP == 0;
-      static_for<0, 3>([&](auto ic) {
-        constexpr int left = 3 - decltype(ic)::value;
-        if (nbar - r >= left) {
-          if (full) wait_vmcnt<(left - 1) * KP * LOADS>();
-          else wait_vmcnt<(left > 2 ? left - 2 : 0) * KP * LOADS>();
-          dmas_barrier();
-          ++r;
-        }
-      });
-    } else {
+    {
       int slab = 0;
 #pragma unroll 1
       for (; slab + AHEAD < nslab; ++slab) {
@@ -335,21 +313,15 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_dmas_kernel(const SmallArgs s_in
     const int et = tid - 64 * Cfg::NCOMP, er = et / TPR, ec = (et % TPR) * EV;
     const int pr = er & 31, pc = ec & 31;
     float acc[EV];
+    const float* const patch = reinterpret_cast<const float*>(smem + Cfg::patch_off(nslab, (er >> 5) + (ec >> 5) * (BM / 32))) + pr * 32;
+    if constexpr (EV == 8) {
+      const f32x4_t lo = *reinterpret_cast<const f32x4_t*>(patch + (((pc >> 2) ^ (pr & 7)) << 2));
+      const f32x4_t hi = *reinterpret_cast<const f32x4_t*>(patch + ((((pc >> 2) + 1) ^ (pr & 7)) << 2));
 #pragma unroll
-    for (int p = 0; p < Cfg::KP; ++p) {
-      const float* patch = reinterpret_cast<const float*>(smem + Cfg::patch_off(nslab, (er >> 5) + (ec >> 5) * Cfg::WGM + p * Cfg::WGM * Cfg::WGN));
-      float part[EV];
-      if constexpr (EV == 8) {
-        const f32x4_t lo = *reinterpret_cast<const f32x4_t*>(patch + pr * 32 + (((pc >> 2) ^ (pr & 7)) << 2));
-        const f32x4_t hi = *reinterpret_cast<const f32x4_t*>(patch + pr * 32 + ((((pc >> 2) + 1) ^ (pr & 7)) << 2));
-#pragma unroll
-        for (int e = 0; e < 4; ++e) { part[e] = lo[e]; part[4 + e] = hi[e]; }
-      } else {
-        const float2 p2 = *reinterpret_cast<const float2*>(patch + pr * 32 + (((pc >> 2) ^ (pr & 7)) << 2) + (pc & 3));
-        part[0] = p2.x; part[1] = p2.y;
-      }
-#pragma unroll
-      for (int e = 0; e < EV; ++e) acc[e] = p == 0 ? part[e] : acc[e] + part[e];
+      for (int e = 0; e < 4; ++e) { acc[e] = lo[e]; acc[4 + e] = hi[e]; }
+    } else {
+      const float2 p2 = *reinterpret_cast<const float2*>(patch + (((pc >> 2) ^ (pr & 7)) << 2) + (pc & 3));
+      acc[0] = p2.x; acc[1] = p2.y;
     }
     const int m = BM == 32 && (er >= bm || ec >= bn) ? s.M : m0 + er;   // (M: nothing is stored)
     if (__builtin_expect(small_tile_full(s, n0, bn), 1))
@@ -359,28 +331,32 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_dmas_kernel(const SmallArgs s_in
     return;
   }
 
-  const int wm = wave % Cfg::WGM, wn = wave / Cfg::WGM % Cfg::WGN;
-  if (m0 + wm * 32 >= s.M || n0 + wn * 32 >= s.N) {
-    for (int i = 0; i <= nbar; ++i) dmas_barrier();
+  const int wm = wave % Cfg::WGM, wn = wave / Cfg::WGM;
+  constexpr int WT = Cfg::WT;
+  if (m0 + wm * WT >= s.M || n0 + wn * WT >= s.N || (BM == 32 && (wm * WT >= bm || wn * WT >= bn))) {
+    for (int i = 0; i <= nslab; ++i) dmas_barrier();
     return;
   }
-  // Fragment addresses, as in gemm_dmaf_kernel.hpp: chunk Kc ^ L with L = (2g or g) ^ swizzle(row) per lane and a
-  // compile-time Kc that takes four values.
-  const int lr = lane & 31, g = lane >> 5;
-  const int LW = (IN_DT == DT_FP8 ? 2 * g : g) ^ lds_swizzle(wn * 32 + lr);
-  const int LX = (IN_DT == DT_FP8 ? 2 * g : g) ^ lds_swizzle(wm * 32 + lr);
+  // Fragment addresses, as in gemm_dmaf_kernel.hpp: lane group g (of 64 / WT) holds chunks (16 bytes of a row's 128; e4m3: pairs of them) g and on, one step of K behind
+  // the other; chunk Kc ^ L with L per lane and a compile-time Kc that takes four values, two in quarters.
+  constexpr int STEPS = Cfg::PAIRS ? 4 : Cfg::QUADS ? 2 : KSTEPS;   // of a stage
+  const int lr = lane & (WT - 1), g = lane / WT;
+  const int LW = (IN_DT == DT_FP8 ? 2 * g : g) ^ lds_swizzle(wn * WT + lr);
+  const int LX = (IN_DT == DT_FP8 ? 2 * g : g) ^ lds_swizzle(wm * WT + lr);
   const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t*)smem);
-  uint32_t wb0[4], xb0[4];
+  constexpr int NB = Cfg::QUADS && !Cfg::PAIRS ? 2 : 4;
+  uint32_t wb0[NB], xb0[NB];
 #pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const int kc = IN_DT == DT_FP8 ? ((k & 1) | ((k >> 1) << 2)) : 2 * k;
-    wb0[k] = lds0 + (wn * 32 + lr) * Cfg::ROWB + ((kc ^ LW) << 4);
-    xb0[k] = lds0 + Cfg::PART_BYTES + (wm * 32 + lr) * Cfg::ROWB + ((kc ^ LX) << 4);
+  for (int k = 0; k < NB; ++k) {
+    // (pairs: steps 2 and 3 are those of rows 16 further, whose swizzle has bit 1 flipped)
+    const int kc = Cfg::PAIRS ? (4 * (k & 1)) ^ (k & 2) : Cfg::QUADS ? 4 * k : IN_DT == DT_FP8 ? ((k & 1) | ((k >> 1) << 2)) : 2 * k;
+    const int second = Cfg::PAIRS && k >= 2 ? 16 * Cfg::ROWB : 0;
+    wb0[k] = lds0 + (wn * WT + lr) * Cfg::ROWB + second + ((kc ^ LW) << 4);
+    xb0[k] = lds0 + Cfg::PART_BYTES + (wm * WT + lr) * Cfg::ROWB + second + ((kc ^ LX) << 4);
   }
-  f32x16_t acc;
-#pragma unroll
-  for (int r = 0; r < 16; ++r) acc[r] = 0.f;
-  struct Frags { Frag<IN_DT> w[KSTEPS], x[KSTEPS]; };
+  typedef std::conditional_t<Cfg::QUADS, f32x4_t, f32x16_t> Acc;
+  Acc acc{};
+  struct Frags { Frag<IN_DT> w[STEPS], x[STEPS]; };
   auto read_step = [&](uint32_t soff, Frags& f, auto ksc) {
     constexpr int ks = decltype(ksc)::value;
     auto piece = [&](uint32_t base) -> i32x4_t { return *reinterpret_cast<const __attribute__((address_space(3))) i32x4_t*>(base + soff); };
@@ -393,63 +369,59 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_dmas_kernel(const SmallArgs s_in
       f.x[ks].lo = piece(xb0[ks]);
     }
   };
+  auto mul_step = [&](const Frags& f, auto ksc) {
+    constexpr int ks = decltype(ksc)::value;
+    if constexpr (Cfg::QUADS) acc = mfma_quad<IN_DT>(f.w[ks], f.x[ks], acc);
+    else acc = mfma_frag<IN_DT>(f.w[ks], f.x[ks], acc);
+  };
   __builtin_amdgcn_s_setprio(2);
   Frags f0, f1;
-  auto last_step = [&](Frags& cur) {
-    static_for<0, KSTEPS>([&](auto ksc) { constexpr int ks = decltype(ksc)::value; acc = mfma_frag<IN_DT>(cur.w[ks], cur.x[ks], acc); });
+  auto last_step = [&](Frags& cur) {   // (the last pair may be a single slab)
+    static_for<0, Cfg::PAIRS ? 2 : STEPS>([&](auto ksc) { mul_step(cur, ksc); });
+    if (Cfg::PAIRS && (s.nslab & 1) == 0) static_for<2, STEPS>([&](auto ksc) { mul_step(cur, ksc); });
   };
-  if constexpr (Cfg::KP > 1) {
-    // This wave's slabs are kp, kp + KP, ...: one of every round.
-    const int kp = wave / (Cfg::WGM * Cfg::WGN);
-#pragma unroll 1
-    for (int slab = kp, i = 0; i < nbar; ++i, slab += Cfg::KP) {
-      __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): the last round's fragments are in registers, behind this barrier its stages are refilled
-      dmas_barrier();
-      if (slab >= nslab) continue;
-      static_for<0, KSTEPS>([&](auto ksc) { read_step((slab & (NSTAGE - 1)) * STAGE, f0, ksc); });
-      last_step(f0);
-    }
-  } else {
-    dmas_barrier();
-    static_for<0, KSTEPS>([&](auto ksc) { read_step(0, f0, ksc); });
-    auto step = [&](int slab, Frags& cur, Frags& nxt) {
-      dmas_barrier();    // slab + 1 has landed
-      const uint32_t soff = ((slab + 1) & (NSTAGE - 1)) * STAGE;
-      static_for<0, KSTEPS>([&](auto ksc) {
-        constexpr int ks = decltype(ksc)::value;
-        acc = mfma_frag<IN_DT>(cur.w[ks], cur.x[ks], acc);
-        __builtin_amdgcn_sched_barrier(0);
-        read_step(soff, nxt, ksc);
-        __builtin_amdgcn_sched_barrier(0);
-      });
-    };
-    int slab = 0;
-    for (; slab + 2 < nslab; slab += 2) {
-      step(slab, f0, f1);
-      step(slab + 1, f1, f0);
-    }
-    if (slab + 1 < nslab) {
-      step(slab, f0, f1);
-      last_step(f1);
-    } else {
-      last_step(f0);
-    }
+  dmas_barrier();
+  static_for<0, STEPS>([&](auto ksc) { read_step(0, f0, ksc); });
+  auto step = [&](int slab, Frags& cur, Frags& nxt) {
+    dmas_barrier();    // slab + 1 has landed
+    const uint32_t soff = ((slab + 1) & (NSTAGE - 1)) * STAGE;
+    static_for<0, STEPS>([&](auto ksc) {
+      mul_step(cur, ksc);
+      __builtin_amdgcn_sched_barrier(0);
+      read_step(soff, nxt, ksc);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  };
+  int slab = 0;
+  for (; slab + 2 < nslab; slab += 2) {
+    step(slab, f0, f1);
+    step(slab + 1, f1, f0);
   }
-  // The sums go to this wave's patch, rows of 32 floats in 16-byte chunks swizzled by row: acc[4 rq + e] is column 8 rq + 4 g + e of row lr.
-  float* const patch = reinterpret_cast<float*>(smem + Cfg::patch_off(nslab, wave));
+  if (slab + 1 < nslab) {
+    step(slab, f0, f1);
+    last_step(f1);
+  } else {
+    last_step(f0);
+  }
+  // The sums go to a 32x32 block's patch, rows of 32 floats in 16-byte chunks swizzled by row: acc[4 rq + e] is column 8 rq + 4 g + e of row lr (in quarters: column 4 g + e).
+  if constexpr (Cfg::QUADS) {
+    const int row = wm * WT + lr;
+    float* const patch = reinterpret_cast<float*>(smem + Cfg::patch_off(nslab, 0));
+    *reinterpret_cast<f32x4_t*>(patch + row * 32 + (((4 * wn + g) ^ (row & 7)) << 2)) = acc;
+  } else {
+    float* const patch = reinterpret_cast<float*>(smem + Cfg::patch_off(nslab, wave));
 #pragma unroll
-  for (int rq = 0; rq < 4; ++rq)
-    *reinterpret_cast<f32x4_t*>(patch + lr * 32 + (((2 * rq + g) ^ (lr & 7)) << 2)) = f32x4_t{acc[4 * rq], acc[4 * rq + 1], acc[4 * rq + 2], acc[4 * rq + 3]};
+    for (int rq = 0; rq < 4; ++rq)
+      *reinterpret_cast<f32x4_t*>(patch + lr * 32 + (((2 * rq + g) ^ (lr & 7)) << 2)) = f32x4_t{acc[4 * rq], acc[4 * rq + 1], acc[4 * rq + 2], acc[4 * rq + 3]};
+  }
   __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): the patch is written
   dmas_barrier();
 }
 
 // Rows and columns of C per workgroup of the 32x32 form: of the tiles that leave every one a CU, the one whose workgroup reads the fewest rows of both
 // operands. A CU gets 30 bytes a cycle from memory (some 64 KB in flight at 2000 cycles and more), less than half of what it gets from L2: the walk of 32 + 32
-// rows over weights that come from memory takes 310 cycles a slab where the MFMAs take 208. The same 64 rows by 1024 columns on 256 workgroups of 16x16 instead of
-// 64 of 32x32 read half as much each. Inside a pass of one position (bf16, weights past the caches), start to end of the launch: K = 1024 4.1 -> 3.4 us,
-// K = 1536 5.6 -> 4.2, FFN-1 (16x24) 4.0 -> 3.4; where the memory-side cache has the weights 3.0 and 3.1, 3.7 and 3.75. Whole calls: 684 -> 670 us; token steps of 128 sequences
-// 292 -> 288. MFMA lanes past the tile multiply whatever lies in LDS there; nothing of theirs is stored.
+// rows over weights that come from memory takes 310 cycles a slab. The same 64 rows by 1024 columns on 256 workgroups of 16x16 instead of
+// 64 of 32x32 read half as much each. MFMA lanes past the tile multiply whatever lies in LDS there; nothing of theirs is stored.
 struct SmallTile { int bm, bn; };
 inline SmallTile small_tile(int M, int N, int cus) {
   SmallTile best{32, 32};
@@ -463,8 +435,8 @@ inline SmallTile small_tile(int M, int N, int cus) {
 
 template <typename Cfg, int IN_DT, int OUT_DT, int ONCE = 0, int SLICED = 0>
 static hipError_t launch_dmas(const GemmArgs& a, hipStream_t st, int shares = 1, int bm = Cfg::BM, int bn = Cfg::BN) {
-  static_assert(!SLICED || (Cfg::KP == 1 && OUT_DT == DT_F32), "a share's sums as they are");
-  if constexpr (Cfg::KP == 1 && !ONCE && !SLICED) {
+  static_assert(!SLICED || OUT_DT == DT_F32, "a share's sums as they are");
+  if constexpr (!ONCE && !SLICED) {
     // (up to 512 rows: the weight rows that more tiles share do better kept in L2; 8 positions 1062 -> 1013 us, 12 the same, 16 1222 -> 1262)
     if (a.w_once && a.M <= 512) return launch_dmas<Cfg, IN_DT, OUT_DT, 1>(a, st, 1, bm, bn);
   }
@@ -495,7 +467,7 @@ static hipError_t launch_dmas(const GemmArgs& a, hipStream_t st, int shares = 1,
   // columns, K = 3072 loses 0.5 us a launch: rows first there.
   const int tiles_m = tiles / tiles_n, per = std::max(tiles >> 3, 1);
   const int by_rows = (per + tiles_n - 1) / tiles_n * bm + std::min(per, tiles_n) * bn, by_cols = (per + tiles_m - 1) / tiles_m * bn + std::min(per, tiles_m) * bm;
-  s.by_cols = Cfg::KP == 1 && tiles_m >= 4 && by_cols < by_rows;
+  s.by_cols = tiles_m >= 4 && by_cols < by_rows;
   s.inner = s.by_cols ? tiles_m : tiles_n;
   s.m_inner = dmaf_magic(s.inner); s.per_xcd = tiles >> 3; s.bm = bm; s.bn = bn;
   hipLaunchKernelGGL(kern, dim3(tiles, shares), dim3(Cfg::NT), Cfg::LDS_BYTES, st, s);

@@ -58,6 +58,14 @@ __device__ __forceinline__ f32x16_t mfma_frag(const Frag<IN_DT>& w, const Frag<I
   }
 }
 
+// 16x16 of sums over a step of K twice as long (16-bit operands): lane l holds 8 elements of row l % 16 from 8 (l / 16) on, and sums 4 (l / 16) .. + 3 of column l % 16.
+template <int IN_DT>
+__device__ __forceinline__ f32x4_t mfma_quad(const Frag<IN_DT>& w, const Frag<IN_DT>& x, f32x4_t acc) {
+  static_assert(IN_DT == DT_BF16 || IN_DT == DT_F16, "16-bit operands");
+  if constexpr (IN_DT == DT_BF16) return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, w.lo), __builtin_bit_cast(bf16x8_t, x.lo), acc, 0, 0, 0);
+  else return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, w.lo), __builtin_bit_cast(f16x8_t, x.lo), acc, 0, 0, 0);
+}
+
 template <int OUT_DT>
 __device__ __forceinline__ void store1(void* base, long off, float v) {
   if constexpr (OUT_DT == DT_F32) reinterpret_cast<float*>(base)[off] = v;
