@@ -212,7 +212,7 @@ hipError_t launch_gemm_norm256(const Norm256Args& a, hipStream_t st);
 int device_cus();   // compute units of the current device (gemm.hip)
 struct NormTile { int bm, bn; };
 NormTile gemm_norm_tile(int M, int N, int K, int in_dt, int cus);
-hipError_t launch_gemm_norm(NormGemmArgs a, int in_dt, NormTile t, bool k_parallel, hipStream_t st);
+hipError_t launch_gemm_norm(NormGemmArgs a, int in_dt, NormTile t, hipStream_t st);
 
 struct LayerNormArgs {
   const void* x;        // [rows, C]

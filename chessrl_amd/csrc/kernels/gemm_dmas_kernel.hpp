@@ -255,8 +255,7 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_dmas_kernel(const SmallArgs s_in
   }
   if (wave >= Cfg::NCOMP) {
     // Loading waves: the first half fills the weight rows of a stage, the second half the activation rows, 8 LOADS consecutive
-    // rows each: 8 rows per wave-instruction, eight 16-byte chunks per row, the swizzle applied on the global side
-    // (row r = rbase + 8 i + lane / 8 has swizzle lds_swizzle(r) = (lane / 8) ^ ((rbase / 8 + i) & 7)).
+    // rows each: 8 rows per wave-instruction, eight 16-byte chunks per row, the swizzle applied on the global side.
     const int lw = wave - Cfg::NCOMP;
     const bool loads_a = lw >= Cfg::NLOAD / 2;
     const int rbase = (lw & (Cfg::NLOAD / 2 - 1)) * (8 * LOADS);
@@ -269,7 +268,7 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_dmas_kernel(const SmallArgs s_in
     for (int i = 0; i < LOADS; ++i) {
       int r = (Cfg::PAIRS ? rbase & 15 : rbase + 8 * i) + (lane >> 3);
       r = r < rows_left ? r : rows_left - 1;
-      voff[i] = (uint32_t)r * (uint32_t)ld + (Cfg::PAIRS ? (rbase >> 4) * Cfg::ROWB : 0) + (((lane & 7) ^ (lane >> 3) ^ ((rbase / 8 + i) & 7)) << 4);
+      voff[i] = (uint32_t)r * (uint32_t)ld + (Cfg::PAIRS ? (rbase >> 4) * Cfg::ROWB : 0) + (((lane & 7) ^ lds_swizzle16(rbase + 8 * i + (lane >> 3))) << 4);
     }
     // (the rows of a tile span less than 2 GB: the launcher checks; they end with K, which the second slab of a last pair may lie behind)
     const uint8_t* origin = reinterpret_cast<const uint8_t*>(loads_a ? s.A : s.W) + (long)(loads_a ? m0 : n0) * ld + (SLICED ? (long)((blockIdx.y >> 2) * 4 * nslab + (blockIdx.y & 3)) * Cfg::ROWB : 0);
@@ -341,8 +340,8 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_dmas_kernel(const SmallArgs s_in
   // the other; chunk Kc ^ L with L per lane and a compile-time Kc that takes four values, two in quarters.
   constexpr int STEPS = Cfg::PAIRS ? 4 : Cfg::QUADS ? 2 : KSTEPS;   // of a stage
   const int lr = lane & (WT - 1), g = lane / WT;
-  const int LW = (IN_DT == DT_FP8 ? 2 * g : g) ^ lds_swizzle(wn * WT + lr);
-  const int LX = (IN_DT == DT_FP8 ? 2 * g : g) ^ lds_swizzle(wm * WT + lr);
+  const int LW = (IN_DT == DT_FP8 ? 2 * g : g) ^ lds_swizzle16(wn * WT + lr);
+  const int LX = (IN_DT == DT_FP8 ? 2 * g : g) ^ lds_swizzle16(wm * WT + lr);
   const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t*)smem);
   constexpr int NB = Cfg::QUADS && !Cfg::PAIRS ? 2 : 4;
   uint32_t wb0[NB], xb0[NB];

@@ -5,13 +5,13 @@ namespace crl {
 
 constexpr int NORM_SPARE = 9216, NORM_LDS = 160 * 1024;   // gain and offset, the spare kilobyte
 
-template <int IN_DT, int BM, int KP>
+template <int IN_DT, int BM>
 static hipError_t launch_norm(const NormGemmArgs& a, int bn, hipStream_t st) {
   static std::atomic<bool> attr_set[16] = {};
   constexpr int ESZ = IN_DT == DT_FP8 ? 1 : 2;
   int dev = 0;
   (void)hipGetDevice(&dev);
-  auto kern = gemm_norm_kernel<IN_DT, BM, KP>;
+  auto kern = gemm_norm_kernel<IN_DT, BM>;
   if (dev < 0 || dev >= 16 || !attr_set[dev]) {
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, NORM_LDS);
     if (e != hipSuccess) return e;
@@ -25,10 +25,12 @@ static hipError_t launch_norm(const NormGemmArgs& a, int bn, hipStream_t st) {
   const int tiles = k.tiles_m * ((a.N + bn - 1) / bn), rg = bn / 8;
   if (tiles >= 65536) return hipErrorInvalidValue;
   k.per_xcd = tiles >> 3;
-  k.bn = bn; k.nb = (bn + 31) / 32; k.m_bn2 = dmaf_magic(bn / 2);
+  k.bn = bn; k.m_bn2 = dmaf_magic(bn / 2);
   k.w_div = 16 / rg; k.w_mod = 16 % rg; k.loads = (rg * k.nslab + 15) / 16;
-  if (k.loads > 9 || k.nb * KP > 16 || BM * bn > 2048) return hipErrorInvalidValue;
-  const int lds = std::max((BM + bn) * a.K * ESZ + NORM_SPARE, k.nb * KP * 4096);   // operands, gain and offset, the spare kilobyte; the patches of the sums
+  if (k.loads > 9 || BM * bn > 2048) return hipErrorInvalidValue;
+  // operands, gain and offset, the spare kilobyte; the patches of the sums; what is read ahead of the last slab of W
+  const int lds = std::max({(BM + bn) * a.K * ESZ + NORM_SPARE, (bn + 31) / 32 * 4096, (k.nslab + 3) * bn * 128 + 4096});
+  if (lds > NORM_LDS) return hipErrorInvalidValue;
   hipLaunchKernelGGL(kern, dim3(tiles), dim3(1024), lds, st, k);
   return hipGetLastError();
 }
@@ -39,7 +41,7 @@ static hipError_t launch_norm(const NormGemmArgs& a, int bn, hipStream_t st) {
 NormTile gemm_norm_tile(int M, int N, int K, int in_dt, int cus) {
   const long kb = (long)K * (in_dt == DT_FP8 ? 1 : 2);
   if (M <= 0 || N <= 0 || kb % 128 || K > 1024 || K % 256) return {0, 0};
-  auto fits = [&](int bm, int bn) { return (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn) <= cus && (bm + bn) * kb + NORM_SPARE <= NORM_LDS && bn * kb <= 9 * 16 * 1024; };
+  auto fits = [&](int bm, int bn) { return (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn) <= cus && (bm + bn) * kb + NORM_SPARE <= NORM_LDS && bn * kb <= 9 * 16 * 1024 && (kb / 128 + 3) * bn * 128 + 4096 <= NORM_LDS; };
   if (!fits(32, 64) && !fits(32, 32)) return {0, 0};
   for (int bm = 16; bm <= 32; bm += 16)
     for (int bn = 8; bn <= (bm == 16 ? 96 : 64); bn += 8)
@@ -47,7 +49,7 @@ NormTile gemm_norm_tile(int M, int N, int K, int in_dt, int cus) {
   return {0, 0};
 }
 
-hipError_t launch_gemm_norm(NormGemmArgs a, int in_dt, NormTile t, bool k_parallel, hipStream_t st) {
+hipError_t launch_gemm_norm(NormGemmArgs a, int in_dt, NormTile t, hipStream_t st) {
   const int esz = in_dt == DT_FP8 ? 1 : 2, osz = a.out_dtype == DT_F32 ? 4 : a.out_dtype == DT_FP8 ? 1 : 2;
   auto al16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
   if (gemm_norm_tile(a.M, a.N, a.K, in_dt, 1 << 16).bn == 0 || (t.bm != 16 && t.bm != 32) || t.bn < 8 || t.bn % 8 || a.ldx % 4 || !al16(a.x) || !al16(a.gamma) || (a.beta && !al16(a.beta)) ||
@@ -58,7 +60,7 @@ hipError_t launch_gemm_norm(NormGemmArgs a, int in_dt, NormTile t, bool k_parall
   if (a.rms) a.beta = nullptr;
   // groups of four columns: aligned, and on one side of the split
   a.vec_ok = al16(a.out) && al16(a.out2) && (a.ldo * osz) % 16 == 0 && (a.ldo2 * osz) % 16 == 0 && (a.nsplit == a.N || a.nsplit % 4 == 0);
-#define NORM(DT) (t.bm == 16 ? (k_parallel ? launch_norm<DT, 16, 4>(a, t.bn, st) : launch_norm<DT, 16, 1>(a, t.bn, st)) : (k_parallel ? launch_norm<DT, 32, 4>(a, t.bn, st) : launch_norm<DT, 32, 1>(a, t.bn, st)))
+#define NORM(DT) (t.bm == 16 ? launch_norm<DT, 16>(a, t.bn, st) : launch_norm<DT, 32>(a, t.bn, st))
   switch (in_dt) {
     case DT_BF16: return NORM(DT_BF16);
     case DT_F16: return NORM(DT_F16);

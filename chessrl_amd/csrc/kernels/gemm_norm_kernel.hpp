@@ -5,15 +5,15 @@
 // follow straight to LDS, and the normalised rows go to LDS as the operand. With both operands whole in LDS (at most
 // 150 KB) there is no ring; one barrier stands between gain and offset and their use, one between the operands and the product.
 // Bound by the norm's own vector instructions, which every tile column repeats (four waves share a SIMD: 70 of them for a row's statistics are 1300 cycles), by the CU's
-// load rate before them (every wave's requests are issued after 2700 of 10400 cycles) and by the chain of a tile's MFMAs behind (3000). Hence 16 rows where the columns
-// then still fit: one position, K = 768, N = 2304 and 3072: 32x32 tiles 11100 cycles, 16x40 and 16x48 10400 and 10800; the last layer's one row, 32x32 10800, 16x16
-// 9600; vocabulary 10800 -> 9000 (whole call 186.0 -> 182.3 us).
+// load rate before them (every wave's requests are issued after 2600 of 9000 cycles) and by the chain of a tile's MFMAs behind (1600). Hence 16 rows where the columns
+// then still fit: one position, K = 768, N = 2304 and 3072: 32x32 tiles 11100 cycles, 16x40 and 16x48 10400 and 10800, with 16x16x32 MFMAs 9000 and 9400; the last layer's one row
+// 10800, 9600 and 8000; vocabulary 10800, 9000, 7500 (whole call 186.0 -> 182.3 us, 171.0 -> 163.7).
 // One counted wait behind the last request lets the statistics run under the weight loads; the normalised rows wait for
 // them all the same, because the compiler drains every load into LDS in front of the first write to it. Measured in place: K = 768, N = 2304, 128 rows 8.4 us (12.4 for the norm riding on the K-sliced product before it and the
 // product), 64 rows 7.3 us (8.5 for two launches). The same for the 16-bit rows of 1024 columns of the BT4-class trunk took 9.4 us against 8.7
 // for two launches and is not here.
-// The norm's arithmetic is that of layernorm_kernel row by row and the product adds K in the order of the other tiled kernels (KP = 1): bit-equal to
-// the two launches. KP = 4 (token steps, which may add in another order): four waves share a tile's K and their sums are added in order.
+// The norm's arithmetic is that of layernorm_kernel row by row and the product adds K in the order of the other tiled kernels: bit-equal to
+// the two launches.
 #pragma once
 #include "gemm_dmaf_kernel.hpp"
 #include "norm_rows.hpp"
@@ -25,7 +25,7 @@ struct NormGemmKArgs {
   int nslab, tiles_m;
   uint32_t m_tm, m_bn2;        // magics of tiles_m and bn / 2
   int per_xcd;
-  int bn, nb;                  // columns of a tile, a multiple of eight, and its blocks of 32
+  int bn;                      // columns of a tile, a multiple of eight
   int w_div, w_mod, loads;     // 16 / (bn / 8) and 16 % (bn / 8); weight requests of a wave
 };
 
@@ -39,7 +39,7 @@ __device__ __forceinline__ void norm_wait(int loads) {   // all requests but the
   }
 }
 
-template <int IN_DT, int BM, int KP>
+template <int IN_DT, int BM>
 __global__ void __launch_bounds__(1024) gemm_norm_kernel(const NormGemmKArgs s) {
   constexpr int ESZ = IN_DT == DT_FP8 ? 1 : 2, ROWB = 128, RW = BM / 16;   // rows of X that a wave normalises
   constexpr int KSTEPS = ROWB / (IN_DT == DT_FP8 ? 64 : 32);
@@ -101,7 +101,7 @@ __global__ void __launch_bounds__(1024) gemm_norm_kernel(const NormGemmKArgs s) 
     for (int j = 0; j < s.loads; ++j) {
       int r = grp * 8 + l8;
       r = r < left ? r : left - 1;
-      const int voff = r * ldb + (((lane & 7) ^ l8 ^ (grp & 7)) << 4);
+      const int voff = r * ldb + (((lane & 7) ^ lds_swizzle16(grp * 8 + l8)) << 4);
       dmaf_load16(sl < nslab ? rs : none, sl < nslab ? lds_w + (sl * bn + grp * 8) * ROWB : reinterpret_cast<uint8_t*>(lds_g) + 8192, voff, sl * ROWB);
       sl += s.w_div;
       grp += s.w_mod;
@@ -148,7 +148,7 @@ __global__ void __launch_bounds__(1024) gemm_norm_kernel(const NormGemmKArgs s) 
     // A lane's place in the operand: 16-byte chunk of the column's 128-byte slab row; further groups of columns lie whole slabs behind.
     constexpr int GB = 4 * ESZ;       // bytes of the lane's consecutive columns
     const int lb = lane * GB;
-    uint8_t* const dst = lds_a + ((lb >> 7) * BM + row) * ROWB + ((((lb & 127) >> 4) ^ lds_swizzle(row)) << 4) + (lb & 15);
+    uint8_t* const dst = lds_a + ((lb >> 7) * BM + row) * ROWB + ((((lb & 127) >> 4) ^ lds_swizzle16(row)) << 4) + (lb & 15);
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -175,77 +175,89 @@ __global__ void __launch_bounds__(1024) gemm_norm_kernel(const NormGemmKArgs s) 
   dmaf_barrier();      // the operands are there
 
 
-  // ---- the product
-  // (rows of a block past the tile are those of the next slab or part: only sums that are not stored read them)
-  const int kp = wave / s.nb, nb = wave - kp * s.nb;
-  f32x16_t acc;
-#pragma unroll
-  for (int r = 0; r < 16; ++r) acc[r] = 0.f;
-  const bool multiplies = wave < s.nb * KP && n0 + nb * 32 < a.N;
-  const int lr = lane & 31, g = lane >> 5;
+  // ---- the product: a wave per block of WT x WT. 16-bit operands: 16x16x32 MFMAs (the same bits as 32x32x16 and a shorter chain, see gemm_dmas_kernel.hpp).
+  // What a wave issues between two MFMAs of its chain counts: two blocks to a wave, whose fragments of X they share, with offsets worked out read by read took 2600 cycles
+  // for K = 768, a block to a wave with offsets that run on 1500, 32x32x16 3000.
+  // (rows of a block past the tile, and slabs read ahead past the last, are what lies behind: only sums that are not stored read them)
+  constexpr bool QUADS = IN_DT != DT_FP8;
+  constexpr int WT = QUADS ? 16 : 32, WROWS = (BM + WT - 1) / WT, STEPS = QUADS ? 2 : KSTEPS, NB = QUADS ? 2 : 4;
+  const int wm = wave % WROWS, nb = wave / WROWS;
+  typedef std::conditional_t<QUADS, f32x4_t, f32x16_t> Acc;
+  Acc acc{};
+  const bool multiplies = nb * WT < bn && n0 + nb * WT < a.N;
+  const int lr = lane & (WT - 1), g = lane / WT;
   if (multiplies) {
     const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t*)smem);
-    const int LW = (IN_DT == DT_FP8 ? 2 * g : g) ^ lds_swizzle(nb * 32 + lr), LX = (IN_DT == DT_FP8 ? 2 * g : g) ^ lds_swizzle(lr);
-    uint32_t wb[4], xb[4];
+    uint32_t wb[NB], xb[NB];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const int kc = IN_DT == DT_FP8 ? ((k & 1) | ((k >> 1) << 2)) : 2 * k;
-      wb[k] = lds0 + (nb * 32 + lr) * ROWB + ((kc ^ LW) << 4);
-      xb[k] = lds0 + nslab * bn * ROWB + lr * ROWB + ((kc ^ LX) << 4);
+    for (int k = 0; k < NB; ++k) {
+      const int kc = QUADS ? 4 * k : (k & 1) | ((k >> 1) << 2), c = (QUADS ? g : 2 * g) ^ kc;
+      wb[k] = lds0 + (nb * WT + lr) * ROWB + ((c ^ lds_swizzle16(nb * WT + lr)) << 4);
+      xb[k] = lds0 + nslab * bn * ROWB + (wm * WT + lr) * ROWB + ((c ^ lds_swizzle16(wm * WT + lr)) << 4);
     }
-    struct Frags { Frag<IN_DT> w[KSTEPS], x[KSTEPS]; };
+    struct Frags { Frag<IN_DT> w[STEPS], x[STEPS]; };
     auto piece = [](uint32_t at) -> i32x4_t { return *reinterpret_cast<const __attribute__((address_space(3))) i32x4_t*>(at); };
-    auto read_step = [&](int slab, Frags& f, auto ksc) {
-      constexpr int ks = decltype(ksc)::value;
-      const uint32_t wo = slab * bn * ROWB, xo = slab * BM * ROWB;
-      if constexpr (IN_DT == DT_FP8) {
-        f.w[ks].lo = piece(wb[2 * ks] + wo); f.w[ks].hi = piece(wb[2 * ks + 1] + wo);
-        f.x[ks].lo = piece(xb[2 * ks] + xo); f.x[ks].hi = piece(xb[2 * ks + 1] + xo);
-      } else {
-        f.w[ks].lo = piece(wb[ks] + wo);
-        f.x[ks].lo = piece(xb[ks] + xo);
+    constexpr int SETS = BM == 16 && QUADS ? 4 : 2;   // slabs whose fragments are in registers or on their way; K is whole 256s, i.e. a multiple of them
+    // (fragments of the slab the addresses stand at, and `ahead` slabs on for X; the addresses of W move on by a slab, those of X by a round of SETS)
+    const uint32_t w_step = bn * ROWB;
+    auto read_slab = [&](Frags& f, auto ahead) {
+      constexpr int off = decltype(ahead)::value * BM * ROWB;
+#pragma unroll
+      for (int ks = 0; ks < STEPS; ++ks) {
+        if constexpr (IN_DT == DT_FP8) {
+          f.w[ks].lo = piece(wb[2 * ks]); f.w[ks].hi = piece(wb[2 * ks + 1]);
+          f.x[ks].lo = piece(xb[2 * ks] + off); f.x[ks].hi = piece(xb[2 * ks + 1] + off);
+        } else {
+          f.w[ks].lo = piece(wb[ks]);
+          f.x[ks].lo = piece(xb[ks] + off);
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < NB; ++k) wb[k] += w_step;
+    };
+    auto mul_slab = [&](const Frags& f) {
+#pragma unroll
+      for (int ks = 0; ks < STEPS; ++ks) {
+        if constexpr (QUADS) acc = mfma_quad<IN_DT>(f.w[ks], f.x[ks], acc);
+        else acc = mfma_frag<IN_DT>(f.w[ks], f.x[ks], acc);
       }
     };
-    int slab = nslab * kp / KP;
-    const int end = nslab * (kp + 1) / KP;
-    Frags f0, f1;
-    static_for<0, KSTEPS>([&](auto ksc) { read_step(slab < end ? slab : 0, f0, ksc); });
-    auto step = [&](int next, Frags& cur, Frags& nxt) {
-      static_for<0, KSTEPS>([&](auto ksc) {
-        constexpr int ks = decltype(ksc)::value;
-        acc = mfma_frag<IN_DT>(cur.w[ks], cur.x[ks], acc);
+    Frags f[SETS];
+    static_for<0, SETS - 1>([&](auto jc) { read_slab(f[decltype(jc)::value], jc); });
+    for (int slab = 0; slab < nslab; slab += SETS) {
+      static_for<0, SETS>([&](auto jc) {
+        constexpr int j = decltype(jc)::value;
+        read_slab(f[(j + SETS - 1) % SETS], std::integral_constant<int, j + SETS - 1>{});
         __builtin_amdgcn_sched_barrier(0);
-        read_step(next, nxt, ksc);
+        mul_slab(f[j]);
         __builtin_amdgcn_sched_barrier(0);
       });
-    };
-    auto last_step = [&](Frags& cur) {
-      static_for<0, KSTEPS>([&](auto ksc) { constexpr int ks = decltype(ksc)::value; acc = mfma_frag<IN_DT>(cur.w[ks], cur.x[ks], acc); });
-    };
-    for (; slab + 2 < end; slab += 2) { step(slab + 1, f0, f1); step(slab + 2, f1, f0); }
-    if (slab + 1 < end) { step(slab + 1, f0, f1); last_step(f1); }
-    else if (slab < end) last_step(f0);
+#pragma unroll
+      for (int k = 0; k < NB; ++k) xb[k] += SETS * BM * ROWB;
+    }
   }
   __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0)
-  dmaf_barrier();   // both operands are read: their space becomes the patches of the sums
+  dmaf_barrier();   // both operands are read: their space becomes the patches of the sums, one per 32 columns
   if (multiplies) {
-    float* const patch = reinterpret_cast<float*>(smem) + wave * 1024;
+    if constexpr (QUADS) {
+      const int row = wm * WT + lr;
+      *reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(smem) + (nb >> 1) * 1024 + row * 32 + (((4 * (nb & 1) + g) ^ (row & 7)) << 2)) = acc;
+    } else {
+      float* const patch = reinterpret_cast<float*>(smem) + nb * 1024;
 #pragma unroll
-    for (int rq = 0; rq < 4; ++rq)
-      *reinterpret_cast<f32x4_t*>(patch + lr * 32 + (((2 * rq + g) ^ (lr & 7)) << 2)) = f32x4_t{acc[4 * rq], acc[4 * rq + 1], acc[4 * rq + 2], acc[4 * rq + 3]};
+      for (int rq = 0; rq < 4; ++rq)
+        *reinterpret_cast<f32x4_t*>(patch + lr * 32 + (((2 * rq + g) ^ (lr & 7)) << 2)) = f32x4_t{acc[4 * rq], acc[4 * rq + 1], acc[4 * rq + 2], acc[4 * rq + 3]};
+    }
   }
   __syncthreads();
   // ---- epilogue: row er, columns ec .. ec + EV - 1
   const int m = m0 + er, n = n0 + ec;
   if (er >= BM || m >= a.M || n >= a.N) return;
   float v[EV];
+  {
+    const float* patch = reinterpret_cast<const float*>(smem) + (ec >> 5) * 1024 + er * 32 + ((((ec & 31) >> 2) ^ (er & 7)) << 2) + (ec & 3);
 #pragma unroll
-  for (int e = 0; e < EV; ++e) v[e] = 0.f;
-#pragma unroll
-  for (int p = 0; p < KP; ++p) {
-    const float* patch = reinterpret_cast<const float*>(smem) + (p * s.nb + (ec >> 5)) * 1024 + er * 32 + ((((ec & 31) >> 2) ^ (er & 7)) << 2) + (ec & 3);
-#pragma unroll
-    for (int e = 0; e < EV; ++e) v[e] = p == 0 ? patch[e] : v[e] + patch[e];
+    for (int e = 0; e < EV; ++e) v[e] = patch[e];
   }
   const bool fused_mish = a.out_dtype == DT_FP8 && a.act == ACT_MISH;   // as in gemm_epilogue
 #pragma unroll

@@ -9,6 +9,9 @@
 namespace crl {
 
 __device__ __forceinline__ int lds_swizzle(int row) { return (row ^ (row >> 3)) & 7; }
+// The same for rows that are read 16 at a time, four chunks of each (16x16x32 MFMAs): with lds_swizzle every such read meets a bank twice (eight waves reading: 2104 cycles
+// where linear addresses take 1080); rows 8 to 15 flipped in bit 2 as well, it and the reads of 32 rows take 1084 and 1088.
+__device__ __forceinline__ int lds_swizzle16(int row) { return (row ^ (row >> 3) ^ ((row >> 1) & 4)) & 7; }
 
 // Compile-time loop: f is called with std::integral_constant<int, I> for I in [0, N), so
 // register arrays indexed by I never need dynamic indexing whatever the body size.

@@ -579,7 +579,7 @@ int Model::norm_gemm(const void* x, long ldx, const float* g, const float* b, co
   const int fam = in_dt == DT_FP8 ? 0 : 5;
   if (profiling) { prof_flops[fam] += 2.0 * M * (double)(L.N - L.pad_N) * (L.K - L.pad_K); ++prof_n[2]; }
   prof_begin(fam, st);
-  const hipError_t e = launch_gemm_norm(a, in_dt, gemm_norm_tile(M, L.N, L.K, in_dt, device_cus()), o.k_parallel, st);
+  const hipError_t e = launch_gemm_norm(a, in_dt, gemm_norm_tile(M, L.N, L.K, in_dt, device_cus()), st);
   prof_end(st);
   HIPCHK(e);
   return CRL_OK;
