@@ -105,15 +105,13 @@ __global__ void __launch_bounds__(SPLIT ? 128 : 64 * AttnWaves<MODE>::N, (SPLIT 
   constexpr int DT_TILES = HS / 32;
   constexpr int NW = SPLIT ? 1 : AttnWaves<MODE>::N;   // units of the workgroup
   __shared__ __align__(16) uint16_t s_vt[NW][HS * VT_STRIDE];
-  __shared__ float s_sp[MODE == ATTN_RELSHIFT ? 64 * SP_STRIDE : 1];
-  __shared__ __align__(16) float s_uv[MODE == ATTN_RELSHIFT ? 2 : 1][MODE == ATTN_RELSHIFT ? 2 * HS : 1];
   // Output tile of the workgroup's NW heads (head size 32): 64 rows of NW * HS elements, 16 bytes of padding
   // per row. A wave's own output is 64 row pieces of 32 (e4m3) or 64 bytes, which it would have to store 16 bytes per
   // lane and row, a quarter or an eighth of a line at a time; gathered here, the workgroup stores whole lines (measured
   // on 4096 positions x 32 heads in e4m3: the stores were 9 % of the kernel's bytes and 21 % of its time).
   static_assert(!LAST || (MODE == ATTN_CAUSAL && !COOP), "one-row form");
   static_assert(!SPLIT || (!COOP && !LAST), "one query tile per wave");
-  static_assert(SPLIT || MODE != ATTN_RELSHIFT, "the relative mode has one form");
+  static_assert(MODE != ATTN_RELSHIFT, "the relative mode has a kernel of its own");
   constexpr int NIT = LAST || SPLIT ? 1 : 2;   // query tiles of a wave
   static_assert(!COOP || (HS == 32 && (NW == 4 || NW == 8 || NW == 16)), "the output tile is laid out for head size 32");
   constexpr int OSZ = OUT_FP8 ? 1 : 2;
@@ -198,7 +196,7 @@ __global__ void __launch_bounds__(SPLIT ? 128 : 64 * AttnWaves<MODE>::N, (SPLIT 
       *reinterpret_cast<uint2*>(vt2 + (8 * dc + 2 * e2) * VT_STRIDE + 4 * jq) = lo;
       *reinterpret_cast<uint2*>(vt2 + (8 * dc + 2 * e2 + 1) * VT_STRIDE + 4 * jq) = hi;
     }
-  } else if constexpr (MODE != ATTN_RELSHIFT) {
+  } else {
     v_load();
     v_write();
   }
@@ -249,69 +247,7 @@ __global__ void __launch_bounds__(SPLIT ? 128 : 64 * AttnWaves<MODE>::N, (SPLIT 
 #pragma unroll
       for (int r = 0; r < 16; ++r) s[jt][it][r] = 0.f;
 
-  if constexpr (MODE == ATTN_RELSHIFT) {
-    // content = (q+u)·k, position = (q+v)·p, both with the bias folded into the query. Everything the wave reads is requested up front (left alone, the
-    // compiler asks for the positional table and the biases step by step, a memory round trip each), V last, which is wanted last. With the shift's
-    // reads in one go too, and a wave per query tile, a layer of 496 positions of 8 heads takes 41 us instead of 51 and one of 1488 126 instead of 150 (bytes:
-    // 26 and 77 us); held to three waves per SIMD (158 registers instead of 192) the same.
-    const uint16_t* pp = reinterpret_cast<const uint16_t*>(a.pos) + h * HS;
-    const long ldp = (long)a.H * HS;
-    hvec pf[2][KS];
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) pf[t][ks] = *reinterpret_cast<const hvec*>(pp + (long)(32 * t + lr) * ldp + 16 * ks + 8 * g);
-    const float ul = a.u_bias[h * HS + lane % HS], vl = a.v_bias[h * HS + lane % HS];
-    v_load();
-    __builtin_amdgcn_sched_barrier(0);
-    float* const uv = s_uv[wave];   // u, then v (a wave's own copy)
-    if (lane < HS) { uv[lane] = ul; uv[HS + lane] = vl; }
-    wave_fence();
-    f32x16_t sp[2];
-#pragma unroll
-    for (int jt = 0; jt < 2; ++jt)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) sp[jt][r] = 0.f;
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      float ub[8], vb[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) { ub[e] = uv[16 * ks + 8 * g + e]; vb[e] = uv[HS + 16 * ks + 8 * g + e]; }
-      const hvec qu = add_bias_h<H16>(qf[0][ks], ub);
-      const hvec qv = add_bias_h<H16>(qf[0][ks], vb);
-#pragma unroll
-      for (int jt = 0; jt < 2; ++jt) {
-        s[jt][0] = H16::mfma(kf[jt][ks], qu, s[jt][0]);
-        sp[jt] = H16::mfma(pf[jt][ks], qv, sp[jt]);
-      }
-    }
-    v_write();
-    // Shifted read-back (new_paradigm/attn.py:525-533): with T=64,
-    //   out[i][j] = P[i][63-i+j] (j<=i), 0 (j==i+1), P[i+1][j-i-2] (j>i+1).
-    const int i = 32 * it0 + lr;
-#pragma unroll
-    for (int jt = 0; jt < 2; ++jt)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) s_sp[i * SP_STRIDE + 32 * jt + 8 * (r >> 2) + 4 * g + (r & 3)] = sp[jt][r];
-    __syncthreads();   // (row 32 of the shift is the other wave's, as is half of V^T)
-    // (both cases at one address but for a constant; the element between them is zero; all reads ahead of their use)
-    const float* const back = s_sp + i * (SP_STRIDE - 1) + 63 + 4 * g;
-#pragma unroll
-    for (int jt = 0; jt < 2; ++jt)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int j0 = 32 * jt + 8 * (r >> 2) + (r & 3);
-        sp[jt][r] = back[j0 + (j0 + 4 * g > i ? SP_STRIDE - 65 : 0)];
-      }
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int jt = 0; jt < 2; ++jt)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const float pv = 32 * jt + 8 * (r >> 2) + 4 * g + (r & 3) == i + 1 ? 0.f : sp[jt][r];
-        s[jt][0][r] = (s[jt][0][r] + pv) * a.scale;
-      }
-  } else {
+  {
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
@@ -345,7 +281,7 @@ __global__ void __launch_bounds__(SPLIT ? 128 : 64 * AttnWaves<MODE>::N, (SPLIT 
   float inv_l[NIT];
   auto softmax = [&](int it, auto tc) {
     constexpr int TILE = decltype(tc)::value;
-    constexpr bool SCALED = MODE == ATTN_BIAS || MODE == ATTN_RELSHIFT;   // (the scores are finished)
+    constexpr bool SCALED = MODE == ATTN_BIAS;   // (the scores are finished)
     constexpr int JT = MODE == ATTN_CAUSAL ? TILE + 1 : 2;
     float mx = -INFINITY;
 #pragma unroll
@@ -389,7 +325,7 @@ __global__ void __launch_bounds__(SPLIT ? 128 : 64 * AttnWaves<MODE>::N, (SPLIT 
   }
 
   // ---- O^T = V^T · P^T ------------------------------------------------------------------
-  if constexpr (VPAIR || (SPLIT && MODE != ATTN_RELSHIFT)) {
+  if constexpr (VPAIR || SPLIT) {
     __syncthreads();   // (the other wave of the pair wrote half of this head's V^T)
   } else {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -491,6 +427,265 @@ __global__ void __launch_bounds__(SPLIT ? 128 : 64 * AttnWaves<MODE>::N, (SPLIT 
     am = wave_max(am);
     if (lane == 0) atomic_amax(a.amax, am);
   }
+}
+
+// Relative-position attention of 64 tokens (new_paradigm/attn.py:507-533): two waves per unit, one per query tile; a workgroup keeps one head and walks positions.
+// content = (q+u)·k, position = (q+v)·p, both with the bias folded into the query, the second shifted (pad and reshape) through LDS.
+// With a workgroup per unit and operands read as the MFMAs hold them (a lane per row: 64 lanes of a load on 32 rows, which holds it for 190 cycles, and stores of 32 bytes a row)
+// a unit took 11300 cycles, 2300 of them to issue the loads, 1900 the stores. Here queries and keys go straight to LDS and results leave through it, whole rows at a time, the
+// keys once for both waves; the next position's are requested behind the shift, its values once V is transposed, and the positional table's fragments
+// stay in registers. 496 positions of 8 heads of 64 40.1 -> 34.4 us (bytes: 26), 1521 122.9 -> 89.7 (81). Registers alone, without LDS: 40.8 and 113.4.
+// Requests past the last position go through empty descriptors and move nothing. 50 KB of LDS: three workgroups a CU.
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ void attn_load_lds(__amdgpu_buffer_rsrc_t r, uint8_t* dst, int off) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, off, 0, 0, 0);
+}
+template <int HS, int OUT_FP8, int IN_DT>
+__global__ void __launch_bounds__(128, 2) relshift_kernel(const AttnArgs a, const int slices) {
+  typedef Half16<IN_DT> H16;
+  typedef typename H16::vec hvec;
+  constexpr int KS = HS / 16, DT_TILES = HS / 32;
+  constexpr int ROWB = HS * 2, CPR = ROWB / 16, QK_LOADS = 2 * 64 * ROWB / 1024 / 2;   // bytes and 16-byte chunks of a row, requests of a wave for q and k
+  constexpr int ORB = HS * (OUT_FP8 ? 1 : 2), OCH = ORB / 16, NST = 32 * ORB / 1024;    // an output row's bytes and chunks; stores of a wave's tile
+  __shared__ __align__(16) uint8_t s_qk[2][64 * ROWB];
+  __shared__ __align__(16) uint8_t s_out[2][32 * ORB];
+  __shared__ __align__(16) uint16_t s_vt[HS * VT_STRIDE];
+  __shared__ float s_sp[64 * SP_STRIDE];
+  __shared__ __align__(16) float s_uv[2][2 * HS];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int lr = lane & 31, g = lane >> 5;
+  // (workgroup indices go round the eight XCDs: renumbered so that the heads of a position sit together)
+  int bid = blockIdx.x;
+  {
+    const int per = gridDim.x >> 3;
+    if (bid < (per << 3)) bid = (bid & 7) * per + (bid >> 3);
+  }
+  const int h = bid % a.H, b0 = bid / a.H;
+  const int i = 32 * wave + lr;   // this lane's query
+
+  hvec pf[2][KS];
+  {
+    const uint16_t* pp = reinterpret_cast<const uint16_t*>(a.pos) + h * HS;
+    const long ldp = (long)a.H * HS;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) pf[t][ks] = *reinterpret_cast<const hvec*>(pp + (long)(32 * t + lr) * ldp + 16 * ks + 8 * g);
+  }
+  float* const uv = s_uv[wave];   // u, then v (a wave's own copy)
+  if (lane < HS) { uv[lane] = a.u_bias[h * HS + lane]; uv[HS + lane] = a.v_bias[h * HS + lane]; }
+
+  // ---- requests: offsets inside a position's 64 rows, the same for every position
+  const int ldq2 = (int)a.ldq * 2, ldk2 = (int)a.ldk * 2, ldv2 = (int)a.ldv * 2;
+  auto rows = [&](const void* base, int b, int ld2) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(reinterpret_cast<const char*>(base)) + (long)b * 64 * ld2 + h * (HS * 2), 0, b < a.B ? 63 * ld2 + HS * 2 : 0, 0x00020000);
+  };
+  // Queries and keys straight into LDS, whole rows at a time (64 lanes of 32 rows, as the MFMAs want them, hold a load for 190 cycles and a store for more: 2300 and 1900 of a
+  // unit's 11300): wave 0 the queries, wave 1 the keys, 16-byte chunks swizzled by row on the global side.
+  auto swz = [](int row) { return CPR == 8 ? (row ^ (row >> 3)) & 7 : (row >> 1) & 3; };
+  const int ldw2 = wave ? ldk2 : ldq2;
+  int wo[QK_LOADS];
+#pragma unroll
+  for (int j = 0; j < QK_LOADS; ++j) {
+    const int row = j * (64 / CPR) + lane / CPR;
+    wo[j] = row * ldw2 + (((lane % CPR) ^ swz(row)) << 4);
+  }
+  auto qk_load = [&](int b) {
+    const __amdgpu_buffer_rsrc_t r = rows(wave ? a.k : a.q, b, ldw2);
+#pragma unroll
+    for (int j = 0; j < QK_LOADS; ++j) attn_load_lds(r, s_qk[wave] + j * 1024, wo[j]);
+  };
+  auto frag = [&](const uint8_t* rows_, int row, int ks) -> hvec {
+    return *reinterpret_cast<const hvec*>(rows_ + row * ROWB + (((2 * ks + g) ^ swz(row)) << 4));
+  };
+  // V rows of this wave, half of the unit's: four of one 16-byte chunk a lane (head size 32: half the lanes)
+  constexpr int DC = HS / 8, PASSES = (16 * DC) / 64;
+  static_assert(PASSES == 1 || PASSES == 2, "head sizes 32 and 64");
+  const bool v_mine = PASSES == 2 || !g;
+  const int v_id = PASSES == 2 ? wave * 64 + lane : 32 * wave + lr, jq = v_id / DC, dc = v_id - jq * DC;
+  const int vo = 4 * jq * ldv2 + 16 * dc;
+  u32x4_t vrow[4];
+  auto v_load = [&](int b) {
+    const __amdgpu_buffer_rsrc_t rv = rows(a.v, b, ldv2);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) vrow[t] = __builtin_amdgcn_raw_buffer_load_b128(rv, vo + t * ldv2, 0, 0);
+  };
+  auto barrier = [&]() {   // (a bare one: a __syncthreads may wait for what is meant to stay in flight)
+    __builtin_amdgcn_s_waitcnt(0xC07F);
+    asm volatile("s_barrier" ::: "memory");
+  };
+
+  v_load(b0);
+  qk_load(b0);
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
+  float am = 0.f;
+#pragma unroll 1
+  for (int b = b0; b < a.B; b += slices) {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(0x0F70 | NST);   // everything but the last position's stores: this one's queries or keys are there
+    barrier();                                  // and the other wave's part; it is also through with the last position's shift and values
+    __builtin_amdgcn_sched_barrier(0);
+    f32x16_t s[2], sp[2];
+#pragma unroll
+    for (int jt = 0; jt < 2; ++jt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[jt][r] = sp[jt][r] = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      float ub[8], vb[8];
+      const hvec qf = frag(s_qk[0], i, ks);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) { ub[e] = uv[16 * ks + 8 * g + e]; vb[e] = uv[HS + 16 * ks + 8 * g + e]; }
+      const hvec qu = add_bias_h<H16>(qf, ub);
+      const hvec qv = add_bias_h<H16>(qf, vb);
+#pragma unroll
+      for (int jt = 0; jt < 2; ++jt) {
+        s[jt] = H16::mfma(frag(s_qk[1], 32 * jt + lr, ks), qu, s[jt]);
+        sp[jt] = H16::mfma(pf[jt][ks], qv, sp[jt]);
+      }
+    }
+    if (v_mine) {
+#pragma unroll
+      for (int e2 = 0; e2 < 4; ++e2) {
+        // d = 8dc + 2e2 (low halves) and d+1 (high halves)
+        const uint32_t w0 = vrow[0][e2], w1 = vrow[1][e2], w2 = vrow[2][e2], w3 = vrow[3][e2];
+        *reinterpret_cast<uint2*>(s_vt + (8 * dc + 2 * e2) * VT_STRIDE + 4 * jq) = make_uint2((w0 & 0xffffu) | (w1 << 16), (w2 & 0xffffu) | (w3 << 16));
+        *reinterpret_cast<uint2*>(s_vt + (8 * dc + 2 * e2 + 1) * VT_STRIDE + 4 * jq) = make_uint2((w0 >> 16) | (w1 & 0xffff0000u), (w2 >> 16) | (w3 & 0xffff0000u));
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    v_load(b + slices);
+    __builtin_amdgcn_sched_barrier(0);
+    // Shifted read-back (new_paradigm/attn.py:525-533): with T=64,
+    //   out[i][j] = P[i][63-i+j] (j<=i), 0 (j==i+1), P[i+1][j-i-2] (j>i+1).
+#pragma unroll
+    for (int jt = 0; jt < 2; ++jt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s_sp[i * SP_STRIDE + 32 * jt + 8 * (r >> 2) + 4 * g + (r & 3)] = sp[jt][r];
+    barrier();   // (row 32 of the shift is the other wave's, as is half of V^T; both have read their queries and keys)
+    __builtin_amdgcn_sched_barrier(0);
+    qk_load(b + slices);
+    __builtin_amdgcn_sched_barrier(0);
+    // (both cases at one address but for a constant; the element between them is zero; all reads ahead of their use)
+    const float* const back = s_sp + i * (SP_STRIDE - 1) + 63 + 4 * g;
+#pragma unroll
+    for (int jt = 0; jt < 2; ++jt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int j0 = 32 * jt + 8 * (r >> 2) + (r & 3);
+        sp[jt][r] = back[j0 + (j0 + 4 * g > i ? SP_STRIDE - 65 : 0)];
+      }
+    __builtin_amdgcn_sched_barrier(0);
+    float mx = -INFINITY;
+#pragma unroll
+    for (int jt = 0; jt < 2; ++jt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const float pv = 32 * jt + 8 * (r >> 2) + 4 * g + (r & 3) == i + 1 ? 0.f : sp[jt][r];
+        s[jt][r] = (s[jt][r] + pv) * a.scale;
+        mx = fmaxf(mx, s[jt][r]);
+      }
+    // softmax over keys (registers + lane^32)
+    mx = max_xor32(mx);
+    float sum = 0.f;
+#pragma unroll
+    for (int jt = 0; jt < 2; ++jt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const float p = __expf(s[jt][r] - mx);
+        s[jt][r] = p;
+        sum += p;
+      }
+    sum = add_xor32(sum);
+    const float inv_l = 1.0f / sum;
+
+    // O^T = V^T · P^T
+    f32x16_t o[DT_TILES];
+#pragma unroll
+    for (int dt = 0; dt < DT_TILES; ++dt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o[dt][r] = 0.f;
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) {
+      hvec p8;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) p8[e] = (typename H16::elem)s[kb >> 1][8 * (kb & 1) + e];
+#pragma unroll
+      for (int dt = 0; dt < DT_TILES; ++dt) {
+        const uint16_t* vrow_t = s_vt + (32 * dt + lr) * VT_STRIDE + 16 * kb + 4 * g;
+        const uint2 lo = *reinterpret_cast<const uint2*>(vrow_t);
+        const uint2 hi = *reinterpret_cast<const uint2*>(vrow_t + 8);
+        const uint4 packed = make_uint4(lo.x, lo.y, hi.x, hi.y);
+        o[dt] = H16::mfma(__builtin_bit_cast(hvec, packed), p8, o[dt]);
+      }
+    }
+    // normalise and store, as in attention_kernel
+#pragma unroll
+    for (int dt = 0; dt < DT_TILES; ++dt)
+#pragma unroll
+      for (int rp = 0; rp < 2; ++rp) {
+        uint32_t pk[2][2];
+#pragma unroll
+        for (int q2 = 0; q2 < 2; ++q2) {
+          const int rq = 2 * rp + q2;
+          float v[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            v[e] = o[dt][4 * rq + e] * inv_l;
+            am = fmaxf(am, fabsf(v[e]));
+          }
+          if constexpr (OUT_FP8) {
+            pk[q2][0] = pack_fp8x4(v[0] * a.out_scale, v[1] * a.out_scale, v[2] * a.out_scale, v[3] * a.out_scale);
+            pk[q2][1] = 0;
+          } else {
+            pk[q2][0] = H16::pack2(v[0], v[1]);
+            pk[q2][1] = H16::pack2(v[2], v[3]);
+          }
+        }
+        lanes_swap32(pk[0][0], pk[1][0]);
+        // through the wave's own patch, so that a store writes whole rows; chunks swizzled by row
+        const int piece = 4 * dt + 2 * rp + g, chunk = OUT_FP8 ? piece >> 1 : piece;
+        uint8_t* const d = s_out[wave] + lr * ORB + ((chunk ^ (lr & (OCH - 1))) << 4);
+        if constexpr (OUT_FP8) {
+          *reinterpret_cast<uint2*>(d + 8 * (piece & 1)) = make_uint2(pk[0][0], pk[1][0]);
+        } else {
+          lanes_swap32(pk[0][1], pk[1][1]);
+          *reinterpret_cast<uint4*>(d) = make_uint4(pk[0][0], pk[0][1], pk[1][0], pk[1][1]);
+        }
+      }
+    wave_fence();
+    {
+      uint8_t* const ob = reinterpret_cast<uint8_t*>(a.out) + ((long)b * 64 + 32 * wave) * a.ldo * (OUT_FP8 ? 1 : 2) + h * ORB;
+#pragma unroll
+      for (int j = 0; j < NST; ++j) {
+        const int row = j * (64 / OCH) + lane / OCH, c = lane % OCH;
+        *reinterpret_cast<uint4*>(ob + row * (a.ldo * (OUT_FP8 ? 1 : 2)) + c * 16) = *reinterpret_cast<const uint4*>(s_out[wave] + row * ORB + ((c ^ (row & (OCH - 1))) << 4));
+      }
+    }
+  }
+  if (a.amax) {
+    am = wave_max(am);
+    if (lane == 0) atomic_amax(a.amax, am);
+  }
+}
+
+template <int HS, int IN_DT>
+static hipError_t launch_relshift_dt(const AttnArgs& a, hipStream_t st) {
+  // Three workgroups fit a CU: the positions of a head in as many slices as that gives, evened out.
+  const int cus = device_cus() > 0 ? device_cus() : 256, most = std::max(3 * cus / a.H, 1), each = (a.B + most - 1) / most, slices = (a.B + each - 1) / each;
+  const dim3 grid(slices * a.H), block(128);
+  if (a.out_dtype == DT_FP8) hipLaunchKernelGGL((relshift_kernel<HS, 1, IN_DT>), grid, block, 0, st, a, slices);
+  else if (a.out_dtype == IN_DT) hipLaunchKernelGGL((relshift_kernel<HS, 0, IN_DT>), grid, block, 0, st, a, slices);
+  else return hipErrorInvalidValue;
+  return hipGetLastError();
+}
+template <int HS>
+static hipError_t launch_relshift(const AttnArgs& a, hipStream_t st) {
+  if (a.qk_hstride || a.ldq >= 1L << 24 || a.ldk >= 1L << 24 || a.ldv >= 1L << 24) return hipErrorInvalidValue;
+  if (a.in_dtype == DT_F16) return launch_relshift_dt<HS, DT_F16>(a, st);
+  if (a.in_dtype == DT_BF16) return launch_relshift_dt<HS, DT_BF16>(a, st);
+  return hipErrorInvalidValue;
 }
 
 // Causal attention over T > 64 tokens per position (the board tokens followed by move tokens,
@@ -921,15 +1116,14 @@ static hipError_t launch_attn_dt(const AttnArgs& a, hipStream_t st) {
   // softmax and output bounds a call that does not fill the chip, and this halves all of it but the loads: 15 layers of 32 heads of 32, one
   // position 6.8 -> 4.2 us a launch, 8 positions 7.2 -> 4.5, 33 9.0 -> 7.9, 64 the same, 250 +10 %; 6 layers of 12 heads of 64, one position 6.9 -> 4.8 us,
   // 16 7.2 -> 5.0, 32 -0.6 us, 64 +0.4, 256 +9. Beyond the lines the second reading of the keys costs more than the shorter chain gives.
-  // The relative mode has no other form.
-  if (MODE == ATTN_RELSHIFT || (!a.last_row && 2L * a.B * a.H <= (HS == 32 ? 9L : 4L) * device_cus())) {
+  if (!a.last_row && 2L * a.B * a.H <= (HS == 32 ? 9L : 4L) * device_cus()) {
     const dim3 units(a.B * a.H), two(128);
     if (a.out_dtype == DT_FP8) hipLaunchKernelGGL((attention_kernel<HS, MODE, 1, IN_DT, 0, 0, 1>), units, two, 0, st, a);
     else if (a.out_dtype == IN_DT) hipLaunchKernelGGL((attention_kernel<HS, MODE, 0, IN_DT, 0, 0, 1>), units, two, 0, st, a);
     else return hipErrorInvalidValue;
     return hipGetLastError();
   }
-  if constexpr (HS == 32 && MODE != ATTN_RELSHIFT && (NW == 4 || NW == 8 || NW == 16)) {
+  if constexpr (HS == 32 && (NW == 4 || NW == 8 || NW == 16)) {
     // Whole workgroups only: H a multiple of 4 puts four heads of one position in every workgroup and leaves none partly
     // filled; 16-byte stores need rows and base aligned to that.
     const int osz = a.out_dtype == DT_FP8 ? 1 : 2;
@@ -948,11 +1142,9 @@ static hipError_t launch_attn_dt(const AttnArgs& a, hipStream_t st) {
       return hipGetLastError();
     }
   }
-  if constexpr (MODE != ATTN_RELSHIFT) {
-    if (a.out_dtype == DT_FP8) hipLaunchKernelGGL((attention_kernel<HS, MODE, 1, IN_DT>), grid, block, 0, st, a);
-    else if (a.out_dtype == IN_DT) hipLaunchKernelGGL((attention_kernel<HS, MODE, 0, IN_DT>), grid, block, 0, st, a);
-    else return hipErrorInvalidValue;
-  }
+  if (a.out_dtype == DT_FP8) hipLaunchKernelGGL((attention_kernel<HS, MODE, 1, IN_DT>), grid, block, 0, st, a);
+  else if (a.out_dtype == IN_DT) hipLaunchKernelGGL((attention_kernel<HS, MODE, 0, IN_DT>), grid, block, 0, st, a);
+  else return hipErrorInvalidValue;
   return hipGetLastError();
 }
 
@@ -969,7 +1161,7 @@ static hipError_t launch_attn_hs(const AttnArgs& a, hipStream_t st) {
     case ATTN_PLAIN: return launch_attn_mode<HS, ATTN_PLAIN>(a, st);
     case ATTN_CAUSAL: return launch_attn_mode<HS, ATTN_CAUSAL>(a, st);
     case ATTN_BIAS: return launch_attn_mode<HS, ATTN_BIAS>(a, st);
-    case ATTN_RELSHIFT: return launch_attn_mode<HS, ATTN_RELSHIFT>(a, st);
+    case ATTN_RELSHIFT: return launch_relshift<HS>(a, st);
   }
   return hipErrorInvalidValue;
 }

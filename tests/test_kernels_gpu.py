@@ -726,6 +726,23 @@ def test_attention_relshift_sizes_and_types(cuda, B, H, hs, dtype):
     assert ((o8.view(torch.float8_e4m3fn).float() / so - ref).abs() <= bound).all()
 
 
+@pytest.mark.parametrize("B,H", [(800, 1), (130, 8), (197, 8), (290, 8), (259, 3)])
+@pytest.mark.parametrize("hs,dtype,out_dt", [(64, torch.bfloat16, None), (32, torch.float16, None), (64, torch.float16, _lib.FP8), (32, torch.bfloat16, _lib.FP8)])
+def test_attention_relshift_workgroups_that_walk_positions(cuda, B, H, hs, dtype, out_dt):
+    """Beyond three workgroups per compute unit a workgroup takes several positions of its head, the last one fewer: the same bits as positions by the few, which get a
+    workgroup each."""
+    qkv, Cm = make_qkv(B, H, hs, cuda, 23 + B, dtype)
+    pos = torch.randn(64, Cm, device=cuda).to(dtype)
+    u, vb = torch.randn(Cm, device=cuda) * 0.3, torch.randn(Cm, device=cuda) * 0.3
+    kw = dict(pos=pos, u=u, v=vb) if out_dt is None else dict(pos=pos, u=u, v=vb, out_dt=out_dt, out_scale=30.0)
+    run = lambda n, x: run_attn(x, n, H, hs, _lib.ATTN_RELSHIFT, 1 / math.sqrt(Cm), **kw)
+    whole = run(B, qkv)
+    for b in range(0, B, 90):
+        n = min(90, B - b)
+        few = run(n, qkv[b * 64:(b + n) * 64].contiguous())
+        assert torch.equal(whole[b * 64:(b + n) * 64], few), b
+
+
 @pytest.mark.parametrize("T", [1.0, 0.5, 0.0])
 def test_masked_softmax(cuda, T):
     torch.manual_seed(3)
