@@ -186,7 +186,9 @@ struct GemmArgs {
 
 // LayerNorm (or RMSNorm) of X's rows and the product with W behind it, one launch (gemm_norm_kernel.hpp).
 struct NormGemmArgs {
-  const float* x; long ldx;                    // [M, K] rows to normalise
+  const void* x; long ldx; int x_dtype;        // [M, K] rows to normalise: fp32, or of the operands' 16-bit type with K in whole 512s
+  void* norm_out; long ld_norm;                // 16-bit rows: the normalised rows are also written here (null: nowhere)
+  int w_once;                                  // GemmArgs::w_once
   const float* gamma; const float* beta;       // [K]; beta may be null
   float eps; int rms;
   float x_scale;                               // e4m3 operands: the normalised values are multiplied by this before the conversion

@@ -5,13 +5,13 @@ namespace crl {
 
 constexpr int NORM_SPARE = 9216, NORM_LDS = 160 * 1024;   // gain and offset, the spare kilobyte
 
-template <int IN_DT, int BM>
+template <int IN_DT, int BM, bool X16>
 static hipError_t launch_norm(const NormGemmArgs& a, int bn, hipStream_t st) {
   static std::atomic<bool> attr_set[16] = {};
   constexpr int ESZ = IN_DT == DT_FP8 ? 1 : 2;
   int dev = 0;
   (void)hipGetDevice(&dev);
-  auto kern = gemm_norm_kernel<IN_DT, BM>;
+  auto kern = gemm_norm_kernel<IN_DT, BM, X16>;
   if (dev < 0 || dev >= 16 || !attr_set[dev]) {
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, NORM_LDS);
     if (e != hipSuccess) return e;
@@ -60,11 +60,13 @@ hipError_t launch_gemm_norm(NormGemmArgs a, int in_dt, NormTile t, hipStream_t s
   if (a.rms) a.beta = nullptr;
   // groups of four columns: aligned, and on one side of the split
   a.vec_ok = al16(a.out) && al16(a.out2) && (a.ldo * osz) % 16 == 0 && (a.ldo2 * osz) % 16 == 0 && (a.nsplit == a.N || a.nsplit % 4 == 0);
-#define NORM(DT) (t.bm == 16 ? launch_norm<DT, 16>(a, t.bn, st) : launch_norm<DT, 32>(a, t.bn, st))
+  if (a.x_dtype != DT_F32 && (a.x_dtype != in_dt || in_dt == DT_FP8 || a.K % 512 || a.ldx % 8 || !al16(a.x) || (a.norm_out && (a.ld_norm % 8 || !al16(a.norm_out))))) return hipErrorInvalidValue;
+  if (a.x_dtype == DT_F32 && a.norm_out) return hipErrorInvalidValue;
+#define NORM(DT, X) (t.bm == 16 ? launch_norm<DT, 16, X>(a, t.bn, st) : launch_norm<DT, 32, X>(a, t.bn, st))
   switch (in_dt) {
-    case DT_BF16: return NORM(DT_BF16);
-    case DT_F16: return NORM(DT_F16);
-    case DT_FP8: return NORM(DT_FP8);
+    case DT_BF16: return a.x_dtype == DT_F32 ? NORM(DT_BF16, false) : NORM(DT_BF16, true);
+    case DT_F16: return a.x_dtype == DT_F32 ? NORM(DT_F16, false) : NORM(DT_F16, true);
+    case DT_FP8: return NORM(DT_FP8, false);
   }
 #undef NORM
   return hipErrorInvalidValue;

@@ -10,8 +10,10 @@
 // 10800, 9600 and 8000; vocabulary 10800, 9000, 7500 (whole call 186.0 -> 182.3 us, 171.0 -> 163.7).
 // One counted wait behind the last request lets the statistics run under the weight loads; the normalised rows wait for
 // them all the same, because the compiler drains every load into LDS in front of the first write to it. Measured in place: K = 768, N = 2304, 128 rows 8.4 us (12.4 for the norm riding on the K-sliced product before it and the
-// product), 64 rows 7.3 us (8.5 for two launches). The same for the 16-bit rows of 1024 columns of the BT4-class trunk took 9.4 us against 8.7
-// for two launches and is not here.
+// product), 64 rows 7.3 us (8.5 for two launches). 16-bit rows of 1024 columns (BT4-class, one position: the
+// tile's rows are 16) 5.7 us for N = 3584 and 4.8 for N = 1536 against 7.6 and 6.5 for two launches with the gap between them. Taken back: the weights requested behind a barrier, so
+// that no wave's rows queue behind another's weights, LDS writes that do not wait for the weights, 16-bit rows straight to LDS (each wave then waits for all the others first): one
+// position 621 -> 637 us for the call.
 // The norm's arithmetic is that of layernorm_kernel row by row and the product adds K in the order of the other tiled kernels: bit-equal to
 // the two launches.
 #pragma once
@@ -39,7 +41,8 @@ __device__ __forceinline__ void norm_wait(int loads) {   // all requests but the
   }
 }
 
-template <int IN_DT, int BM>
+// X16: the rows are of the operands' 16-bit type, whole groups of 512 columns, and the normalised ones are also left in memory (by the first tile column).
+template <int IN_DT, int BM, bool X16>
 __global__ void __launch_bounds__(1024) gemm_norm_kernel(const NormGemmKArgs s) {
   constexpr int ESZ = IN_DT == DT_FP8 ? 1 : 2, ROWB = 128, RW = BM / 16;   // rows of X that a wave normalises
   constexpr int KSTEPS = ROWB / (IN_DT == DT_FP8 ? 64 : 32);
@@ -61,7 +64,8 @@ __global__ void __launch_bounds__(1024) gemm_norm_kernel(const NormGemmKArgs s) 
   // ---- rows of X: wave w takes rows RW w and on. A lane's 16 columns are those of layernorm_kernel (norm_columns).
   const int C = a.K;
   float x[RW][2][8];
-  auto has = [&](int i, int h) { return (2 * i + h) * 256 < C; };   // (whole groups of 256 columns: the same for all lanes)
+  i32x4_t raw[RW][2];
+  auto has = [&](int i, int h) { return (X16 ? i * 512 : (2 * i + h) * 256) < C; };   // (whole groups of columns: the same for all lanes)
   // Gain and offset first.
   // 256 columns per wave-instruction, waves 0-3 and 4-7
   if (wave < 8) {
@@ -77,7 +81,13 @@ __global__ void __launch_bounds__(1024) gemm_norm_kernel(const NormGemmKArgs s) 
     int m = m0 + wave * RW + r;
     m = m < a.M ? m : a.M - 1;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) load_norm8<DT_F32>(a.x, (long)m * a.ldx, i, lane, C, x[r][i]);
+    for (int i = 0; i < 2; ++i) {
+      if constexpr (X16) {
+        if (has(i, 0)) raw[r][i] = *reinterpret_cast<const i32x4_t*>(reinterpret_cast<const uint16_t*>(a.x) + (long)m * a.ldx + norm_column(false, i, 0, lane));
+      } else {
+        load_norm8<DT_F32>(a.x, (long)m * a.ldx, i, lane, C, x[r][i]);
+      }
+    }
   }
   // the bias of this thread's columns: two consecutive ones of row er (threads past the tile have nothing to store)
   constexpr int EV = 2;
@@ -97,16 +107,22 @@ __global__ void __launch_bounds__(1024) gemm_norm_kernel(const NormGemmKArgs s) 
     const __amdgpu_buffer_rsrc_t rs = dmaf_rsrc(reinterpret_cast<const uint8_t*>(a.W) + (long)n0 * ldb, (long)left * ldb);
     // (every wave asks as often, past K out of bounds and into a spare kilobyte: the wait for what was requested before counts past them)
     const __amdgpu_buffer_rsrc_t none = dmaf_rsrc(a.W, 0);
+    auto request = [&](auto once) {
 #pragma unroll 1
-    for (int j = 0; j < s.loads; ++j) {
-      int r = grp * 8 + l8;
-      r = r < left ? r : left - 1;
-      const int voff = r * ldb + (((lane & 7) ^ lds_swizzle16(grp * 8 + l8)) << 4);
-      dmaf_load16(sl < nslab ? rs : none, sl < nslab ? lds_w + (sl * bn + grp * 8) * ROWB : reinterpret_cast<uint8_t*>(lds_g) + 8192, voff, sl * ROWB);
-      sl += s.w_div;
-      grp += s.w_mod;
-      if (grp >= rg) { grp -= rg; ++sl; }
-    }
+      for (int j = 0; j < s.loads; ++j) {
+        int r = grp * 8 + l8;
+        r = r < left ? r : left - 1;
+        const int voff = r * ldb + (((lane & 7) ^ lds_swizzle16(grp * 8 + l8)) << 4);
+        uint8_t* const dst = sl < nslab ? lds_w + (sl * bn + grp * 8) * ROWB : reinterpret_cast<uint8_t*>(lds_g) + 8192;
+        if constexpr (decltype(once)::value) dmaf_load16_nt(sl < nslab ? rs : none, dst, voff, sl * ROWB);
+        else dmaf_load16(sl < nslab ? rs : none, dst, voff, sl * ROWB);
+        sl += s.w_div;
+        grp += s.w_mod;
+        if (grp >= rg) { grp -= rg; ++sl; }
+      }
+    };
+    if (a.w_once) request(std::true_type{});
+    else request(std::false_type{});
   }
   __builtin_amdgcn_sched_barrier(0);
   // Everything requested before the weight rows is there: this wave's rows and bias, and its share of gain and offset (the zeros in the place of
@@ -115,6 +131,18 @@ __global__ void __launch_bounds__(1024) gemm_norm_kernel(const NormGemmKArgs s) 
   __builtin_amdgcn_sched_barrier(0);
   // ---- the norm
   const float inv_c = fast_rcp((float)C);
+  if constexpr (X16) {
+#pragma unroll
+    for (int r = 0; r < RW; ++r)
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const uint32_t w = (uint32_t)raw[r][i][e];
+          x[r][i][2 * e] = IN_DT == DT_F16 ? f16_bits_to_f32((uint16_t)(w & 0xffff)) : bf16_bits_to_f32((uint16_t)(w & 0xffff));
+          x[r][i][2 * e + 1] = IN_DT == DT_F16 ? f16_bits_to_f32((uint16_t)(w >> 16)) : bf16_bits_to_f32((uint16_t)(w >> 16));
+        }
+  }
   float mean[RW], rstd[RW];
 #pragma unroll
   for (int r = 0; r < RW; ++r) {
@@ -146,7 +174,7 @@ __global__ void __launch_bounds__(1024) gemm_norm_kernel(const NormGemmKArgs s) 
   for (int r = 0; r < RW; ++r) {
     const int row = wave * RW + r;
     // A lane's place in the operand: 16-byte chunk of the column's 128-byte slab row; further groups of columns lie whole slabs behind.
-    constexpr int GB = 4 * ESZ;       // bytes of the lane's consecutive columns
+    constexpr int GB = (X16 ? 8 : 4) * ESZ;       // bytes of the lane's consecutive columns
     const int lb = lane * GB;
     uint8_t* const dst = lds_a + ((lb >> 7) * BM + row) * ROWB + ((((lb & 127) >> 4) ^ lds_swizzle16(row)) << 4) + (lb & 15);
 #pragma unroll
@@ -154,7 +182,7 @@ __global__ void __launch_bounds__(1024) gemm_norm_kernel(const NormGemmKArgs s) 
 #pragma unroll
       for (int h = 0; h < 2; ++h)
         if (has(i, h)) {
-          const int col = norm_column(true, i, h, lane);
+          const int col = norm_column(!X16, i, h, lane);
           const f32x4_t gv = *reinterpret_cast<const f32x4_t*>(lds_g + col), bv = *reinterpret_cast<const f32x4_t*>(lds_g + 1024 + col);
           float y[4];
 #pragma unroll
@@ -163,8 +191,14 @@ __global__ void __launch_bounds__(1024) gemm_norm_kernel(const NormGemmKArgs s) 
 #pragma unroll
             for (int e = 0; e < 4; ++e) asm volatile("" : "+v"(y[e]));
           }
-          uint8_t* const d = dst + (2 * i + h) * 64 * GB / 128 * (BM * ROWB);
-          if constexpr (IN_DT == DT_FP8) *reinterpret_cast<uint32_t*>(d) = pack_fp8x4(y[0] * a.x_scale, y[1] * a.x_scale, y[2] * a.x_scale, y[3] * a.x_scale);
+          uint8_t* const d = X16 ? dst + i * 64 * GB / 128 * (BM * ROWB) + 8 * h : dst + (2 * i + h) * 64 * GB / 128 * (BM * ROWB);
+          if constexpr (X16) {
+            uint2 w;
+            if constexpr (IN_DT == DT_BF16) w = make_uint2(pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3]));
+            else w = make_uint2((uint32_t)f32_to_f16_bits(y[0]) | ((uint32_t)f32_to_f16_bits(y[1]) << 16), (uint32_t)f32_to_f16_bits(y[2]) | ((uint32_t)f32_to_f16_bits(y[3]) << 16));
+            raw[r][i][2 * h] = (int)w.x; raw[r][i][2 * h + 1] = (int)w.y;
+            if (h == 1) *reinterpret_cast<i32x4_t*>(d - 8) = raw[r][i];
+          } else if constexpr (IN_DT == DT_FP8) *reinterpret_cast<uint32_t*>(d) = pack_fp8x4(y[0] * a.x_scale, y[1] * a.x_scale, y[2] * a.x_scale, y[3] * a.x_scale);
           else if constexpr (IN_DT == DT_BF16) *reinterpret_cast<uint2*>(d) = make_uint2(pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3]));
           else
             *reinterpret_cast<uint2*>(d) = make_uint2((uint32_t)f32_to_f16_bits(y[0]) | ((uint32_t)f32_to_f16_bits(y[1]) << 16),
@@ -173,6 +207,15 @@ __global__ void __launch_bounds__(1024) gemm_norm_kernel(const NormGemmKArgs s) 
   }
   wait_vmcnt_lgkm0<0>();
   dmaf_barrier();      // the operands are there
+  if constexpr (X16) {
+    if (a.norm_out && tile_n == 0)
+#pragma unroll
+      for (int r = 0; r < RW; ++r)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+          if (has(i, 0) && m0 + wave * RW + r < a.M)
+            *reinterpret_cast<i32x4_t*>(reinterpret_cast<uint16_t*>(a.norm_out) + (long)(m0 + wave * RW + r) * a.ld_norm + norm_column(false, i, 0, lane)) = raw[r][i];
+  }
 
 
   // ---- the product: a wave per block of WT x WT. 16-bit operands: 16x16x32 MFMAs (the same bits as 32x32x16 and a shorter chain, see gemm_dmas_kernel.hpp).

@@ -502,6 +502,8 @@ struct GOpt {
   const float* ln_g = nullptr; const float* ln_b = nullptr; void* ln_out = nullptr; int ln_dt = DT_BF16; bool* ln_folded = nullptr;
   // The residual is LayerNorm(res), normalised in the epilogue from these row statistics, gain and offset.
   const float* res_stats = nullptr; const float* res_g = nullptr; const float* res_b = nullptr;
+  // norm_gemm: type of the rows to normalise; where the normalised ones go besides (16-bit rows).
+  int norm_x_dt = DT_F32; void* norm_out = nullptr;
   // Ask for the blocked output layout (GemmArgs::c_blocked) where the GEMM has a kernel for it; *c_blocked says whether it was used.
   bool* c_blocked = nullptr;
 };
@@ -561,16 +563,20 @@ int Model::lnorm(const void* x, long ldx, int in_dt, const float* g, const float
   return CRL_OK;
 }
 
-// (fp32 rows only)
+// (fp32 rows only; 16-bit ones: norm16_gemm_can)
 bool Model::norm_gemm_can(int M, const Lin& L, int in_dt, int x_dt) const {
   return x_dt == DT_F32 && gemm_norm_tile(M, L.N, L.K, in_dt, device_cus()).bn != 0;
+}
+
+bool Model::norm16_gemm_can(int M, const Lin& L) const {
+  return L.K % 512 == 0 && gemm_norm_tile(M, L.N, L.K, cfg.act_dtype, device_cus()).bn != 0;
 }
 
 int Model::norm_gemm(const void* x, long ldx, const float* g, const float* b, const Lin& L, int in_dt, void* C, long ldc, int out_dt, int M, const GOpt& o,
                      hipStream_t st) {
   NormGemmArgs a;
   std::memset(&a, 0, sizeof(a));
-  a.x = reinterpret_cast<const float*>(x); a.ldx = ldx; a.gamma = g; a.beta = b; a.eps = cfg.eps; a.rms = cfg.norm_rms; a.x_scale = o.a_scale;
+  a.x = x; a.ldx = ldx; a.x_dtype = o.norm_x_dt; a.norm_out = o.norm_out; a.ld_norm = L.K; a.w_once = L.once ? 1 : 0; a.gamma = g; a.beta = b; a.eps = cfg.eps; a.rms = cfg.norm_rms; a.x_scale = o.a_scale;
   a.W = in_dt == DT_FP8 ? L.w8 : L.w; a.ldw = L.K; a.bias = L.b;
   if (!a.W) { set_error("norm_gemm: weight copy for the requested element type is missing"); return CRL_ERR_STATE; }
   a.out = C; a.ldo = ldc; a.out2 = o.C2; a.ldo2 = o.ldc2; a.nsplit = o.nsplit;
@@ -716,6 +722,10 @@ int Model::forward_chunk(const float* planes, const uint8_t* ids, const uint8_t*
   const bool one_row = gpt && policy && !all_logits && !calibrate && L > 0;
   // GPT64, few rows: a norm runs inside the product behind it (norm_gemm; bit-equal to the two launches). Not while maxima are collected.
   auto fuses = [&](int rows, const Lin& lin, int dt) { return gpt && !calibrate && !win && norm_gemm_can(rows, lin, dt, xdt); };
+  // The post-LN trunks in 16 bits, few rows: the same; the normalised rows, the residual of a product further on, are left behind by the launch.
+  // Whole calls, two launches -> one: BT4-class bf16, 1 and 2 positions 659 -> 621 us and 714 -> 709 (no tile from 3 on: 763), BT4 bf16, 1, 3 and 5 positions
+  // 300 -> 268 us, 298 -> 271 and 297 -> 277 (no tile from 6 on). Not where the rows are also wanted in e4m3 or in fp32.
+  auto fuses16 = [&](const Lin& lin) { return !gpt && !f8 && !sf32p && !calibrate && !win && norm16_gemm_can(M, lin); };
   for (int l = l0; l < l1; ++l) {
     const Layer& ly = layers[l];
     const bool last = l + 1 == l1;
@@ -736,7 +746,10 @@ int Model::forward_chunk(const float* planes, const uint8_t* ids, const uint8_t*
       GOpt o; o.a_scale = a_sc;
       if (cfg.arch == CRL_ARCH_BT4CLASS) { o.C2 = ws.comp; o.ldc2 = cfg.smolgen_compress; o.nsplit = 3 * C; }
       // (the third of the product that makes unread queries costs more than a second launch from about 16384 rows on)
-      if (fused_qkv) {
+      if (!gpt && l > l0 && fuses16(ly.qkv)) {   // x = LN2(t) of the layer before
+        o.norm_x_dt = ad; o.norm_out = ws.x;
+        RUN(norm_gemm(ws.t, C, layers[l - 1].ln2_g, layers[l - 1].ln2_b, ly.qkv, ad, ws.qkv, 3 * C, ad, M, o, st));
+      } else if (fused_qkv) {
         RUN(norm_gemm(ws.x, C, ly.ln1_g, ly.ln1_b, ly.qkv, a_dt, ws.qkv, 3 * C, ad, M, o, st));
       } else if (tail && M >= 16384) {
         char* const qkv_last = reinterpret_cast<char*>(ws.qkv) + (size_t)(T - 1) * 3 * C * dtype_size(ad);
@@ -826,8 +839,10 @@ int Model::forward_chunk(const float* planes, const uint8_t* ids, const uint8_t*
       { GOpt o; o.res = ws.x; o.ldr = C; o.res_dt = xdt; o.alpha = alpha; o.a_scale = f8 ? act_scale(l, 1) : 1.f;
         if (fold && l > l0) { o.res = ws.t; o.res_stats = ws.st2; o.res_g = layers[l - 1].ln2_g; o.res_b = layers[l - 1].ln2_b; }
         RUN(gemm(ly.proj, ao_in, C, ao_dt, ws.t, C, xdt, M, o, st)); }
-      RUN(lnorm(ws.t, C, xdt, ly.ln1_g, ly.ln1_b, fold ? nullptr : ws.h, xdt, f8 ? ws.h8 : nullptr, f8 ? act_scale(l, 2) : 1.f, C, M, C, am(l, 2), st,
-                fold ? ws.st1 : nullptr, (sf32p && !f8) ? ws.h16 : nullptr, ad));
+      const bool norm_inside = cfg.arch == CRL_ARCH_BT4CLASS && fuses16(ly.ff1);
+      if (!norm_inside)
+        RUN(lnorm(ws.t, C, xdt, ly.ln1_g, ly.ln1_b, fold ? nullptr : ws.h, xdt, f8 ? ws.h8 : nullptr, f8 ? act_scale(l, 2) : 1.f, C, M, C, am(l, 2), st,
+                  fold ? ws.st1 : nullptr, (sf32p && !f8) ? ws.h16 : nullptr, ad));
       const void* h_in = f8 ? (const void*)ws.h8 : (const void*)h_op;
       if (folds_ffn() && !calibrate) {   // (the hidden tensor's maximum is one of the table's)
         GOpt o; o.act = ACT_GELU; o.res = ws.h; o.ldr = C; o.res_dt = xdt;
@@ -840,13 +855,19 @@ int Model::forward_chunk(const float* planes, const uint8_t* ids, const uint8_t*
           RUN(gemm(ly.ff2, f8 ? (const void*)ws.f8 : (const void*)ws.f, F, ao_dt, ws.t, C, xdt, M, o, st)); }
       } else {
         { GOpt o; o.act = ACT_MISH; o.a_scale = f8 ? act_scale(l, 2) : 1.f; o.out_scale = f8 ? act_scale(l, 3) : 1.f; o.amax = am(l, 3);
-          RUN(gemm(ly.ff1, h_in, C, ao_dt, f8 ? (void*)ws.f8 : (void*)ws.f, F, ao_dt, M, o, st)); }
+          if (norm_inside) {
+            o.norm_x_dt = ad; o.norm_out = ws.h;
+            RUN(norm_gemm(ws.t, C, ly.ln1_g, ly.ln1_b, ly.ff1, ad, ws.f, F, ad, M, o, st));
+          } else {
+            RUN(gemm(ly.ff1, h_in, C, ao_dt, f8 ? (void*)ws.f8 : (void*)ws.f, F, ao_dt, M, o, st));
+          } }
         { GOpt o; o.res = ws.h; o.ldr = C; o.res_dt = xdt; o.alpha = alpha; o.a_scale = f8 ? act_scale(l, 3) : 1.f;
           if (fold) { o.res = ws.t; o.res_stats = ws.st1; o.res_g = ly.ln1_g; o.res_b = ly.ln1_b; }
           RUN(gemm(ly.ff2, f8 ? (const void*)ws.f8 : (const void*)ws.f, F, ao_dt, ws.t, C, xdt, M, o, st)); }
       }
       // x = LN2(t); the last layer's output feeds only the heads (as an e4m3 copy alone when they run in e4m3).
       const bool x8_out = f8 && (!last || f8h);
+      if (!last && fuses16(layers[l + 1].qkv)) continue;
       RUN(lnorm(ws.t, C, xdt, ly.ln2_g, ly.ln2_b, ((fold && !last) || (last && f8h)) ? nullptr : ws.x, last ? hd : xdt, x8_out ? ws.x8 : nullptr,
                 x8_out ? act_scale(l + 1, 0) : 1.f, C, M, C, (last && !cal_heads) ? nullptr : am(l + 1, 0), st, (fold && !last) ? ws.st2 : nullptr,
                 (sf32p && !f8 && !last) ? ws.x16 : nullptr, ad));

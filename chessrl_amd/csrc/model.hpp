@@ -169,6 +169,7 @@ struct Model {
             bool trunk = true);
   // Norm of x's rows (fp32) and the product behind it in one launch; in_dt is the product's operand type. norm_gemm_can: the call is small enough.
   bool norm_gemm_can(int M, const Lin& L, int in_dt, int x_dt) const;
+  bool norm16_gemm_can(int M, const Lin& L) const;   // the same for rows of the operands' 16-bit type
   int norm_gemm(const void* x, long ldx, const float* g, const float* b, const Lin& L, int in_dt, void* C, long ldc, int out_dt, int M, const GOpt& o, hipStream_t st);
   // One of the bias generator's norms (grouped: over a position's 32 rows of 256) and the product behind it in one launch.
   int norm256(const void* x, long ldx, int grouped, const float* g, const float* b, const Lin& L, int in_dt, float x_scale, void* C, long ldc, int M, hipStream_t st);

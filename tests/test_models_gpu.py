@@ -930,6 +930,40 @@ def test_gpt_norm_inside_the_product_takes_every_gain_and_offset(cuda, kw, n_hea
         assert torch.equal(m.forward((x[:B].contiguous(), None))[0], base[:B]), B
 
 
+@pytest.mark.parametrize("act", ["bf16", "f16"])
+@pytest.mark.parametrize("make", ["bt4class", "bt4class_rms", "bt4", "bt4_1024"])
+def test_post_norm_trunks_norm_inside_the_product_is_bit_equal(cuda, make, act):
+    """The 16-bit rows of the post-LN trunks are normalised inside the product of small calls, in tiles of 16 and 32 rows, and left behind for the residual; gains and offsets that
+    differ from column to column. Bit-equal to the two launches of a large batch; an fp32 stream never goes this way."""
+    planes, _ = positions(40, seed=5)
+    if make.startswith("bt4class"):
+        m = models.BT4Class(3, 1024, 1536, 32, act_dtype=act, norm_rms=make.endswith("rms"))
+    else:
+        C = 1024 if make.endswith("1024") else 512
+        m = models.BT4(3, C, 736, C // 64, act_dtype=act)
+    sd, g = m.state_dict(), torch.Generator().manual_seed(7)
+    for k in sd:
+        if "ln" in k or "norm" in k:
+            sd[k] = 0.3 * torch.randn(sd[k].shape, generator=g) + (1.0 if k.endswith("weight") else 0.0)
+    m.load_state_dict(sd)
+    x = planes.to(cuda)
+    base = m._engine.forward(x)
+    for B in (1, 2, 3, 4, 5, 6, 9):
+        got = m._engine.forward(x[:B].contiguous())
+        assert torch.isfinite(got[0]).all() and torch.equal(got[0], base[0][:B]) and torch.equal(got[1], base[1][:B]), B
+
+
+@pytest.mark.parametrize("n_head,n_embd", [(8, 512), (16, 1024)])
+def test_gpt_16bit_stream_does_not_take_the_norm_of_fp32_rows(cuda, n_head, n_embd):
+    """Token steps and calls of one position with the residual stream in 16 bits, at widths that the kernel has 16-bit rows for: the separate norm, as in a large batch."""
+    planes, _ = positions(40, seed=6)
+    m = models.GPT(models.GPTConfig(block_size=128, vocab_size=1929, n_layer=2, n_head=n_head, n_embd=n_embd), stream_f32=False)
+    x = planes.to(cuda)
+    base = m.forward((x, None))[0]
+    for B in (1, 3):
+        assert torch.equal(m.forward((x[:B].contiguous(), None))[0], base[:B]), B
+
+
 @pytest.mark.parametrize("kw", [{}, {"norm_rms": True}])
 def test_generate_rows_do_not_depend_on_the_batch(cuda, kw):
     """Token steps of 1 to 160 sequences: norms inside the products, K of the residual products over four waves. Same sums for
