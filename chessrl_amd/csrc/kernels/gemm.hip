@@ -661,7 +661,13 @@ static hipError_t launch_in_out(const GemmArgs& a, int tile, hipStream_t st) {
       } else if (slabs && gemm_dmam_has(IN_DT, OUT_DT) && mid < 65536) {
         const long kb = (long)a.K * (IN_DT == DT_FP8 ? 1 : 2);
         const double ratio = kb <= 512 ? (a.N * kb > (3L << 20) ? 3.0 : big <= 2 * cus ? 4.2 : 3.3) : IN_DT == DT_FP8 ? 3.3 : 2.55;
-        tile = ratio * (double)((big + cus - 1) / cus) <= (double)((mid + cus - 1) / cus) ? 3 : 11;
+        const double big_rounds = ratio * (double)((big + cus - 1) / cus), mid_rounds = (double)((mid + cus - 1) / cus);
+        tile = big_rounds <= mid_rounds ? 3 : 11;
+        // 128x192 (tile 17, where it serves the call): a round of 1.25 of the 128x128 tile's (K=1024: 13 us). It fills the gap where N cuts into a last round of few small tiles, or
+        // one round of large ones that leaves CUs idle. Whole calls without and with it: BT4-class bf16 at 44, 64, 90, 180, 250 and 450 positions 1833 -> 1749 us, 1990 -> 1964,
+        // 2715 -> 2619, 4397 -> 4316, 5619 -> 5566 (f16), 8939 -> 8805; GPT at 32 and 128 454 -> 423 and 1018 -> 987. At 1.2, 200 positions lose 0.8 %, at 1.3 the gains at 160 and 250 go.
+        const long wide = (long)((a.M + 127) / 128) * ((a.N + 191) / 192);
+        if (1.25 * (double)((wide + cus - 1) / cus) < std::min(mid_rounds, big_rounds) && gemm_dmam_wide_can(a, IN_DT, OUT_DT)) tile = 17;
       }
     } else if (tile == 1 && ring_ok) {   // (token steps)
       tile = (long)((a.M + 31) / 32) * ((a.N + 31) / 32) <= device_cus() ? 16 : small <= device_cus() ? 15 : 11;
@@ -691,6 +697,7 @@ static hipError_t launch_in_out(const GemmArgs& a, int tile, hipStream_t st) {
   // with loading and multiplying waves (gemm_dmam_kernel.hpp, tile 11; bit-equal; M=4096, bf16: N=1024, K=1024 16.5 -> 13.9 us,
   // N=1536 27.9 -> 20.9).
   if (tile == 15 || tile == 16) return slabs && !a.res_stats && gemm_dmam_has(IN_DT, OUT_DT) ? launch_gemm_dmas(a, IN_DT, OUT_DT, st, tile == 16 ? 32 : 64) : hipErrorInvalidValue;
+  if (tile == 17) return slabs ? launch_gemm_dmam_wide(a, IN_DT, OUT_DT, device_cus(), st) : hipErrorInvalidValue;
   if (tile == 11 && !slabs) tile = 12;
   if (tile == 2 || tile == 11) {
     const long mid_tiles = (long)((a.M + 127) / 128) * ((a.N + 127) / 128);

@@ -2,13 +2,15 @@
 // whose 256x256 tiles would leave CUs idle (a batch of 16 to 64 positions).
 // Four waves load and eight multiply. A load instruction holds its wave for 100 cycles and more; eight waves that loaded and
 // multiplied in turn took 1.3 times the sum of both (M = 4096, N = 1024, K = 1024, one tile per CU: 16.0 us, of which
-// 3.4 are loads and 3.5 MFMAs). The loading waves keep three of the four 32 KB stages of the ring requested; slab s is announced by a workgroup barrier, at
+// 3.4 are loads and 3.5 MFMAs). The loading waves keep all but one of the ring's four stages of 32 KB (three of 40) requested; slab s is announced by a workgroup barrier, at
 // which the multiplying waves are through with slab s - 1, so its stage is the next to be filled. They read the fragments
 // of a slab from LDS between the MFMAs of the one before.
 // Workgroups are persistent, one per CU, where the epilogue below serves the call: the loading waves run on into the next tile while the
 // multiplying ones finish theirs, each for itself, in the accumulator layout and through 2 KB of LDS of its own outside the ring (as in
 // gemm_dmaf_kernel.hpp). Residuals are requested half way through a tile's walk over K.
 // Measured (bf16, M = 4096): N = 1024, K = 1024 with residual 16.5 -> 13.9 us, K = 1536 21.3 -> 18.1, N = 1536 with mish 27.9 -> 20.9 (register-staged before);
+// 128x192 tiles (twelve multiplying waves, three stages of 40 KB) do the work of 1.5 tiles in 1.25 of their time: M = 4096, N = 1536, K = 1024 one round instead of two, 20.9 -> 19 us,
+// M = 2816 19.5 -> 14.
 // e4m3, M = 2112: N = 3104 16.4 -> 11.8. A slab takes 680 cycles where its MFMAs take 512; weights that come from memory add 3000 cycles to a tile.
 // Same K order and same arithmetic per element as the other tiled kernels: bit-equal results.
 #pragma once
@@ -16,16 +18,19 @@
 
 namespace crl {
 
-struct DmamCfg {
-  static constexpr int BM = 128, BN = 128, WGM = 2, WGN = 4, NCOMP = 8, NLOAD = 4, NT = 64 * (NCOMP + NLOAD);
+template <int BN_>
+struct DmamCfgN {
+  static constexpr int BM = 128, BN = BN_, WGM = 2, WGN = BN / 32, NCOMP = WGM * WGN, NLOAD = 4, NT = 64 * (NCOMP + NLOAD);
   static constexpr int WM = BM / WGM, WN = BN / WGN, TM = WM / 32;       // 64x32 per wave
-  static constexpr int ROWB = 128, NSTAGE = 4, AHEAD = 3, LOADS = 8;     // load instructions of a loading wave per slab
+  static constexpr int ROWB = 128, NSTAGE = BN == 128 ? 4 : 3, AHEAD = NSTAGE - 1;
+  static constexpr int LOADS = (BM + BN) / 32;                           // load instructions of a loading wave per slab
   static constexpr int STAGE = (BM + BN) * ROWB;                         // weight rows, then activation rows
   static constexpr int PATCH_OFF = NSTAGE * STAGE, PATCH = 2048;         // a wave's patch: 32 rows of 64 bytes
   static constexpr int COLS_OFF = PATCH_OFF + NCOMP * PATCH;             // per-column constants: [wave][bias, gain, offset][64] (a load lands 64)
   static constexpr int LDS_BYTES = COLS_OFF + NCOMP * 3 * 64 * 4;
-  static_assert(LDS_BYTES <= 160 * 1024 && AHEAD * LOADS < 64 && AHEAD < NSTAGE, "LDS of a CU; the counted waits; the ring");
+  static_assert(LDS_BYTES <= 160 * 1024 && AHEAD * LOADS < 64 && AHEAD < NSTAGE && NT <= 1024, "LDS of a CU; the counted waits; the ring; a workgroup");
 };
+typedef DmamCfgN<128> DmamCfg;
 
 // A bare barrier: the waits it needs are written out in front of it (a __syncthreads waits for every outstanding memory
 // operation, i.e. for the slabs that are meant to stay in flight).
@@ -54,9 +59,9 @@ inline DmamWalk dmam_walk(int tiles_m, int tiles_n) {
 }
 
 // EPI, ACT: as in gemm_dmaf_kernel.hpp.
-template <int IN_DT, int OUT_DT, int EPI, int ACT = ACT_NONE>
-__global__ void __launch_bounds__(DmamCfg::NT) gemm_dmam_kernel(const GemmArgs a, const int tiles, const DmamWalk walk) {
-  typedef DmamCfg Cfg;
+template <int IN_DT, int OUT_DT, int EPI, int ACT = ACT_NONE, int TILE_N = 128>
+__global__ void __launch_bounds__(DmamCfgN<TILE_N>::NT) gemm_dmam_kernel(const GemmArgs a, const int tiles, const DmamWalk walk) {
+  typedef DmamCfgN<TILE_N> Cfg;
   constexpr bool PERSIST = EPI >= DMAF_PLAIN;
   constexpr bool HAS_RES = EPI == DMAF_RES16 || EPI == DMAF_RESNORM || EPI == DMAF_RES32;
   constexpr int ESZ = IN_DT == DT_FP8 ? 1 : 2, OSZ = OUT_DT == DT_F32 ? 4 : OUT_DT == DT_FP8 ? 1 : 2, RSZ = EPI == DMAF_RES32 ? 4 : 2;
@@ -81,42 +86,45 @@ __global__ void __launch_bounds__(DmamCfg::NT) gemm_dmam_kernel(const GemmArgs a
   }
 
   if (wave >= Cfg::NCOMP) {
-    // ---- loading waves: two for the weight rows of a slab, two for its activation rows, 64 rows each: 8 rows per
+    // ---- loading waves, a quarter of a slab's weight rows and of its activation rows each: 8 rows per
     // wave-instruction, eight 16-byte chunks per row, the swizzle applied on the global side. They announce slab s (barrier s) and then request
     // slab s + AHEAD, whose stage is the one slab s - 1 has left. Past the last slab the requests are out of bounds: they keep the counts.
     const int lw = wave - Cfg::NCOMP, l8 = lane >> 3;
-    const bool loads_a = lw >= 2;
-    const int ld = (int)(loads_a ? a.lda : a.ldw) * ESZ, rbase = (lw & 1) * 64;
+    constexpr int LW = Cfg::BN / 32, LA = Cfg::BM / 32;   // load instructions: of weight rows, of activation rows
     uint32_t voff[Cfg::LOADS];
-    __amdgpu_buffer_rsrc_t rsrc;
+    __amdgpu_buffer_rsrc_t rw, ra;
     int l_tile = tile, l_slab = 0, l_stage = 0;
     auto stream_tile = [&]() {
       int tm, tn;
       walk.pos(l_tile, tm, tn);
       const int m0 = tm * BM, n0 = tn * BN;
-      const int left = loads_a ? a.M - m0 : a.N - n0;
+      const int left_w = a.N - n0 < BN ? a.N - n0 : BN, left_a = a.M - m0 < BM ? a.M - m0 : BM;
+      const int ldw = (int)a.ldw * ESZ, lda = (int)a.lda * ESZ;
 #pragma unroll
       for (int i = 0; i < Cfg::LOADS; ++i) {
-        int r = rbase + 8 * i + l8;
+        const int q = i < LW ? lw * LW + i : lw * LA + i - LW, left = i < LW ? left_w : left_a;
+        int r = q * 8 + l8;
         r = r < left ? r : left - 1;
-        voff[i] = (uint32_t)r * (uint32_t)ld + (((lane & 7) ^ l8 ^ i) << 4);
+        voff[i] = (uint32_t)r * (uint32_t)(i < LW ? ldw : lda) + (((lane & 7) ^ l8 ^ (q & 7)) << 4);
       }
-      rsrc = dmaf_rsrc(reinterpret_cast<const uint8_t*>(loads_a ? a.A : a.W) + (long)(loads_a ? m0 : n0) * ld, (long)(left < BM ? left : BM) * ld);
+      rw = dmaf_rsrc(reinterpret_cast<const uint8_t*>(a.W) + (long)n0 * ldw, (long)left_w * ldw);
+      ra = dmaf_rsrc(reinterpret_cast<const uint8_t*>(a.A) + (long)m0 * lda, (long)left_a * lda);
     };
     auto request = [&]() {
       if (l_slab == nslab) {
         l_slab = 0;
         l_tile += step;
         if (l_tile < hi) stream_tile();
-        else rsrc = dmaf_rsrc(a.A, 0);
+        else rw = ra = dmaf_rsrc(a.A, 0);
       }
-      uint8_t* dst = smem + l_stage * Cfg::STAGE + ((loads_a ? BN : 0) + rbase) * Cfg::ROWB;
+      uint8_t* const dst = smem + l_stage * Cfg::STAGE;
       static_for<0, Cfg::LOADS>([&](auto ic) {
         constexpr int i = decltype(ic)::value;
-        dmaf_load16(rsrc, dst + i * 1024, (int)voff[i], l_slab * Cfg::ROWB);
+        if constexpr (i < LW) dmaf_load16(rw, dst + (lw * LW + i) * 1024, (int)voff[i], l_slab * Cfg::ROWB);
+        else dmaf_load16(ra, dst + BN * Cfg::ROWB + (lw * LA + i - LW) * 1024, (int)voff[i], l_slab * Cfg::ROWB);
       });
       ++l_slab;
-      l_stage = (l_stage + 1) & (Cfg::NSTAGE - 1);
+      l_stage = l_stage + 1 == Cfg::NSTAGE ? 0 : l_stage + 1;
     };
     stream_tile();
 #pragma unroll
@@ -136,7 +144,7 @@ __global__ void __launch_bounds__(DmamCfg::NT) gemm_dmam_kernel(const GemmArgs a
   // ---- multiplying waves
   const int wm = wave % Cfg::WGM, wn = wave / Cfg::WGM, lr = lane & 31, g = lane >> 5;
   // Fragment addresses, as in gemm_dmaf_kernel.hpp: chunk Kc ^ L with L = (2g or g) ^ swizzle(row) per lane and a compile-time Kc that
-  // takes four values; rows of 64 per loading wave, so the swizzle is that of the row inside its 64.
+  // takes four values; the swizzle has the period of 64 rows.
   const int wrow = wn * Cfg::WN + lr;
   const int LW = (IN_DT == DT_FP8 ? 2 * g : g) ^ lds_swizzle(wrow & 63), LX = (IN_DT == DT_FP8 ? 2 * g : g) ^ lds_swizzle(lr);
   const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t*)smem);
@@ -230,7 +238,7 @@ __global__ void __launch_bounds__(DmamCfg::NT) gemm_dmam_kernel(const GemmArgs a
       __builtin_amdgcn_s_waitcnt(0xC07F);
       dmam_barrier();
       const uint32_t soff = r_stage * Cfg::STAGE;
-      r_stage = (r_stage + 1) & (Cfg::NSTAGE - 1);
+      r_stage = r_stage + 1 == Cfg::NSTAGE ? 0 : r_stage + 1;
       return soff;
     };
     {
@@ -408,24 +416,25 @@ __global__ void __launch_bounds__(DmamCfg::NT) gemm_dmam_kernel(const GemmArgs a
   }
 }
 
-template <int IN_DT, int OUT_DT, int EPI, int ACT = ACT_NONE>
+template <int IN_DT, int OUT_DT, int EPI, int ACT = ACT_NONE, int TILE_N = 128>
 static hipError_t launch_dmam(const GemmArgs& a, int cus, hipStream_t st) {
   static std::atomic<bool> attr_set[16] = {};
+  typedef DmamCfgN<TILE_N> Cfg;
   constexpr int ESZ = IN_DT == DT_FP8 ? 1 : 2;
-  if ((a.K * ESZ) % DmamCfg::ROWB != 0 || a.K <= 0 || (long)a.lda * ESZ * 128 >= (1L << 31) || (long)a.ldw * ESZ * 128 >= (1L << 31)) return hipErrorInvalidValue;
+  if ((a.K * ESZ) % Cfg::ROWB != 0 || a.K <= 0 || (long)a.lda * ESZ * 128 >= (1L << 31) || (long)a.ldw * ESZ * TILE_N >= (1L << 31)) return hipErrorInvalidValue;
   int dev = 0;
   (void)hipGetDevice(&dev);
-  auto kern = gemm_dmam_kernel<IN_DT, OUT_DT, EPI, ACT>;
+  auto kern = gemm_dmam_kernel<IN_DT, OUT_DT, EPI, ACT, TILE_N>;
   if (dev < 0 || dev >= 16 || !attr_set[dev]) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, DmamCfg::LDS_BYTES);
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::LDS_BYTES);
     if (e != hipSuccess) return e;
     if (dev >= 0 && dev < 16) attr_set[dev] = true;
   }
-  const int tiles_n = (a.N + DmamCfg::BN - 1) / DmamCfg::BN, tiles_m = (a.M + DmamCfg::BM - 1) / DmamCfg::BM, tiles = tiles_m * tiles_n;
+  const int tiles_n = (a.N + Cfg::BN - 1) / Cfg::BN, tiles_m = (a.M + Cfg::BM - 1) / Cfg::BM, tiles = tiles_m * tiles_n;
   if (tiles >= 65536) return hipErrorInvalidValue;
   const int slots = cus >= 8 ? cus & ~7 : 256;
   const int grid = EPI >= DMAF_PLAIN && tiles > slots ? slots : tiles;
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(DmamCfg::NT), DmamCfg::LDS_BYTES, st, a, tiles, dmam_walk(tiles_m, tiles_n));
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(Cfg::NT), Cfg::LDS_BYTES, st, a, tiles, dmam_walk(tiles_m, tiles_n));
   return hipGetLastError();
 }
 

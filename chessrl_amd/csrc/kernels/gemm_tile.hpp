@@ -536,6 +536,9 @@ hipError_t launch_gemm_dmaf(const GemmArgs& a, int in_dt, int out_dt, int cus, h
 // gemm_dmam.hip: the 128x128 tile with loading and multiplying waves (K in whole 128-byte slabs), on `cus` compute units.
 bool gemm_dmam_has(int in_dt, int out_dt);
 hipError_t launch_gemm_dmam(const GemmArgs& a, int in_dt, int out_dt, int cus, hipStream_t st);
+// 128x192 tiles of the same kernel, for the calls that gemm_dmam_wide_can names.
+bool gemm_dmam_wide_can(const GemmArgs& a, int in_dt, int out_dt);
+hipError_t launch_gemm_dmam_wide(const GemmArgs& a, int in_dt, int out_dt, int cus, hipStream_t st);
 // gemm_dmas.hip: the 64x64 and 32x32 tiles of products that leave every tile a CU (the operand types of gemm_dmam_has).
 hipError_t launch_gemm_dmas(const GemmArgs& a, int in_dt, int out_dt, hipStream_t st, int tile_size);
 hipError_t launch_gemm_dmas_sliced(const GemmArgs& a, int in_dt, hipStream_t st, int tile_size, int shares);

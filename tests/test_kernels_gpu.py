@@ -264,6 +264,21 @@ def test_gemm_guardless_epilogue_instances_equal_general_kernel(cuda, M, N, K):
             assert torch.equal(run_gemm(A, W, kw["out_dt"], tile=11, **args), run_gemm(A, W, kw["out_dt"], tile=12, **args)), (M, N, K, sorted(args))
 
 
+@pytest.mark.parametrize("dt,act", [(_lib.BF16, 0), (_lib.BF16, 1), (_lib.BF16, 2), (_lib.F16, 0), (_lib.F16, 2)])
+@pytest.mark.parametrize("M,N,K", [(2817, 1536, 1024), (4096, 1536, 192), (2700, 1544, 256), (5500, 1536, 128), (2049, 2312, 768)])
+def test_gemm_tiles_of_192_columns_equal_those_of_128(cuda, M, N, K, dt, act):
+    """Sizes at which the automatic choice takes 128x192 tiles (fewer rounds over 256 CUs): one round and two, ragged last rows and columns, K of two slabs and more. Bit-equal to 128x128, whose
+    sums are checked against fp32 (one rounding of the output)."""
+    g = torch.Generator(device=cuda).manual_seed(M + N + K)
+    A = torch.randn(M, K, device=cuda, generator=g).to(TORCH_DT[dt])
+    W = (torch.randn(N, K, device=cuda, generator=g) * 0.05).to(TORCH_DT[dt])
+    bias = torch.randn(N, device=cuda, generator=g)
+    out = run_gemm(A, W, dt, bias=bias, act=act)
+    assert torch.equal(out, run_gemm(A, W, dt, bias=bias, act=act, tile=11))
+    ref = ref_act(A.float() @ W.float().t() + bias, act)
+    assert torch.allclose(out.float(), ref, rtol=2.0 ** (-8 if dt == _lib.BF16 else -11) + 1e-4, atol=1e-3 * math.sqrt(K / 64))
+
+
 @pytest.mark.parametrize("M,nsplit,extra,K", [(16384, 3072, 32, 1024), (12288, 3072, 16, 1536), (1024, 512, 32, 256), (16640, 3072, 32, 1024), (16384, 3072, 40, 1024)])
 def test_gemm_split_output_last_tile_column_carries_the_columns_behind_it(cuda, M, nsplit, extra, K):
     """crl_gemm_split: columns [0, nsplit) into C, the rest into C2. The columns behind a split at a multiple of 256 are a last,
