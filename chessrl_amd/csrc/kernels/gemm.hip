@@ -666,8 +666,10 @@ static hipError_t launch_in_out(const GemmArgs& a, int tile, hipStream_t st) {
         // 128x192 (tile 17, where it serves the call): a round of 1.25 of the 128x128 tile's (K=1024: 13 us). It fills the gap where N cuts into a last round of few small tiles, or
         // one round of large ones that leaves CUs idle. Whole calls without and with it: BT4-class bf16 at 44, 64, 90, 180, 250 and 450 positions 1833 -> 1749 us, 1990 -> 1964,
         // 2715 -> 2619, 4397 -> 4316, 5619 -> 5566 (f16), 8939 -> 8805; GPT at 32 and 128 454 -> 423 and 1018 -> 987. At 1.2, 200 positions lose 0.8 %, at 1.3 the gains at 160 and 250 go.
+        // e4m3, 1.42: 44, 64, 112 and 250 positions 1351 -> 1298 us, 1502 -> 1463, 2178 -> 2127, 3844 -> 3788, none slower up to 1000; at 1.35 200 and 350 lose 1.7 and 3.3 %, at 1.5 the gains
+        // at 112 and 250 go.
         const long wide = (long)((a.M + 127) / 128) * ((a.N + 191) / 192);
-        if (1.25 * (double)((wide + cus - 1) / cus) < std::min(mid_rounds, big_rounds) && gemm_dmam_wide_can(a, IN_DT, OUT_DT)) tile = 17;
+        if ((IN_DT == DT_FP8 ? 1.42 : 1.25) * (double)((wide + cus - 1) / cus) < std::min(mid_rounds, big_rounds) && gemm_dmam_wide_can(a, IN_DT, OUT_DT)) tile = 17;
       }
     } else if (tile == 1 && ring_ok) {   // (token steps)
       tile = (long)((a.M + 31) / 32) * ((a.N + 31) / 32) <= device_cus() ? 16 : small <= device_cus() ? 15 : 11;

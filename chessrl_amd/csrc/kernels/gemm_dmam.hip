@@ -10,17 +10,20 @@ bool gemm_dmam_has(int in_dt, int out_dt) {
   return in_dt == out_dt && (in_dt == DT_BF16 || in_dt == DT_F16);
 }
 
-// Tiles of 128x192: 16-bit operands and outputs, no residual (its registers spill beside twelve multiplying waves: BT4-class at 150 positions 3661 -> 3903 us with it).
+// Tiles of 128x192: outputs of the operands' type, or bf16 of e4m3 operands, without a residual (its registers spill beside twelve multiplying waves: BT4-class bf16 at 150 positions
+// 3661 -> 3903 us with it).
 bool gemm_dmam_wide_can(const GemmArgs& a, int in_dt, int out_dt) {
-  if ((in_dt != DT_BF16 && in_dt != DT_F16) || a.res_stats || (long)((a.M + 127) / 128) * ((a.N + 191) / 192) >= 65536) return false;
-  return in_dt == out_dt && dmaf_epilogue(a, in_dt, out_dt, 192) == DMAF_PLAIN && (a.act == ACT_NONE || a.act == ACT_MISH || (a.act == ACT_GELU && in_dt == DT_BF16));
+  if (a.res_stats || (long)((a.M + 127) / 128) * ((a.N + 191) / 192) >= 65536 || dmaf_epilogue(a, in_dt, out_dt, 192) != DMAF_PLAIN) return false;
+  if (in_dt == DT_FP8) return (out_dt == DT_FP8 && a.act == ACT_MISH) || (out_dt == DT_BF16 && a.act == ACT_NONE);
+  return in_dt == out_dt && (in_dt == DT_BF16 || in_dt == DT_F16) && (a.act == ACT_NONE || a.act == ACT_MISH || (a.act == ACT_GELU && in_dt == DT_BF16));
 }
 
 hipError_t launch_gemm_dmam_wide(const GemmArgs& a, int in_dt, int out_dt, int cus, hipStream_t st) {
   if (!gemm_dmam_wide_can(a, in_dt, out_dt)) return hipErrorInvalidValue;
-#define WIDE(DT, ACT) launch_dmam<DT, DT, DMAF_PLAIN, ACT, 192>(a, cus, st)
-  if (in_dt == DT_F16) return a.act == ACT_MISH ? WIDE(DT_F16, ACT_MISH) : WIDE(DT_F16, ACT_NONE);
-  return a.act == ACT_GELU ? WIDE(DT_BF16, ACT_GELU) : a.act == ACT_MISH ? WIDE(DT_BF16, ACT_MISH) : WIDE(DT_BF16, ACT_NONE);
+#define WIDE(IN, OUT, ACT) launch_dmam<IN, OUT, DMAF_PLAIN, ACT, 192>(a, cus, st)
+  if (in_dt == DT_FP8) return out_dt == DT_FP8 ? WIDE(DT_FP8, DT_FP8, ACT_MISH) : WIDE(DT_FP8, DT_BF16, ACT_NONE);
+  if (in_dt == DT_F16) return a.act == ACT_MISH ? WIDE(DT_F16, DT_F16, ACT_MISH) : WIDE(DT_F16, DT_F16, ACT_NONE);
+  return a.act == ACT_GELU ? WIDE(DT_BF16, DT_BF16, ACT_GELU) : a.act == ACT_MISH ? WIDE(DT_BF16, DT_BF16, ACT_MISH) : WIDE(DT_BF16, DT_BF16, ACT_NONE);
 #undef WIDE
 }
 

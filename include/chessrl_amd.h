@@ -122,7 +122,7 @@ int crl_random_positions(uint64_t seed, int n, int max_plies, double late_fracti
  * 15 and 16 = the 64x64 tile on an eight-stage and the 32x32 tile on a sixteen-stage ring of direct-to-LDS loads (same sums
  * and bits as 1; whole slabs; e4m3 operands with a 16-bit or e4m3 output, bf16/f16 operands with an output of their own
  * type, bf16 operands with an fp32 output; else CRL_ERR_ARG). Where those apply, tile 0 runs 16 while every 32x32 tile has a CU
- * of its own, 15 while every 64x64 tile has, and beyond that 11, 3 or (16-bit operands and output, no residual)
+ * of its own, 15 while every 64x64 tile has, and beyond that 11, 3 or (no residual; an output of the operands' type, or bf16 of e4m3 ones)
  * 128x192 tiles of the kernel of 11, whichever takes fewer rounds of its tiles over the CUs at the measured time of a round; elsewhere 3 from 160 tiles of 256x256 on, 2 from 256 of 128x128 on, else 1.
  * 13 and 14 name the kernel for K = 256 e4m3 elements whose workgroups keep 256 rows of A in registers and walk N (the
  * attention-bias generator's product): a bare scaled product (no bias, activation, residual or amax; alpha = 1) into a

@@ -279,6 +279,23 @@ def test_gemm_tiles_of_192_columns_equal_those_of_128(cuda, M, N, K, dt, act):
     assert torch.allclose(out.float(), ref, rtol=2.0 ** (-8 if dt == _lib.BF16 else -11) + 1e-4, atol=1e-3 * math.sqrt(K / 64))
 
 
+@pytest.mark.parametrize("out_dt,act", [(_lib.FP8, 2), (_lib.BF16, 0)])
+@pytest.mark.parametrize("M,N,K", [(2817, 1536, 1024), (4096, 1536, 256), (2700, 1552, 384), (5600, 1536, 512)])
+def test_gemm_e4m3_tiles_of_192_columns_equal_those_of_128(cuda, M, N, K, out_dt, act):
+    """The same for e4m3 operands (e4m3 output with mish and a scale, bf16 output)."""
+    g = torch.Generator(device=cuda).manual_seed(M + N + K)
+    A = torch.randn(M, K, device=cuda, generator=g).to(torch.float8_e4m3fn)
+    W = torch.randn(N, K, device=cuda, generator=g).to(torch.float8_e4m3fn)
+    bias = torch.randn(N, device=cuda, generator=g)
+    kw = dict(bias=bias, act=act, descale=0.05, out_scale=4.0 if out_dt == _lib.FP8 else 1.0)
+    out = run_gemm(A, W, out_dt, **kw)
+    assert torch.equal(out, run_gemm(A, W, out_dt, tile=11, **kw))
+    ref = ref_act((A.float() @ W.float().t()) * 0.05 + bias, act)
+    got = out.view(torch.float8_e4m3fn).float() / 4.0 if out_dt == _lib.FP8 else out.float()
+    sel = ref.abs() < 100   # (e4m3 ends at 448, here 112)
+    assert torch.allclose(got[sel], ref[sel], rtol=2.0 ** (-4 if out_dt == _lib.FP8 else -8) + 1e-4, atol=2e-3 * math.sqrt(K / 64))
+
+
 @pytest.mark.parametrize("M,nsplit,extra,K", [(16384, 3072, 32, 1024), (12288, 3072, 16, 1536), (1024, 512, 32, 256), (16640, 3072, 32, 1024), (16384, 3072, 40, 1024)])
 def test_gemm_split_output_last_tile_column_carries_the_columns_behind_it(cuda, M, nsplit, extra, K):
     """crl_gemm_split: columns [0, nsplit) into C, the rest into C2. The columns behind a split at a multiple of 256 are a last,
