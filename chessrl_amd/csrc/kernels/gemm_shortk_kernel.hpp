@@ -3,7 +3,7 @@
 // general kernels is all prologue and epilogue (of the 11 us a 256x256 tile lives, 4 are its main loop), and no
 // workgroup can overlap them with another's: the product ran at half the rate its 1 GB of output can be written at.
 //
-// Here a workgroup of eight waves owns 256 rows of A for the whole launch and walks N in steps of 128 columns:
+// Here a workgroup of eight waves owns 256 rows of A for the whole launch and walks N, or a slice of it, in steps of 128 columns:
 //  * its A operand fragments are loaded once, straight from global memory into registers (64 per lane: the whole K of
 //    the wave's 64 rows), and never pass through LDS;
 //  * the 128 weight rows of a step (32 KB, both slabs) arrive by direct-to-LDS loads in a two-stage ring, requested
@@ -36,7 +36,7 @@ struct ShortKCfg {
 };
 
 template <int OUT_DT>
-__global__ void __launch_bounds__(ShortKCfg::NT, 2) gemm_shortk_kernel(const GemmArgs a) {
+__global__ void __launch_bounds__(ShortKCfg::NT, 2) gemm_shortk_kernel(const GemmArgs a, const int groups, const int steps) {
   typedef ShortKCfg Cfg;
   constexpr int TM = Cfg::TM, TN = Cfg::TN, KSTEPS = Cfg::KSTEPS, LOADS = Cfg::LOADS;
   extern __shared__ __align__(16) uint8_t smem[];
@@ -44,8 +44,8 @@ __global__ void __launch_bounds__(ShortKCfg::NT, 2) gemm_shortk_kernel(const Gem
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave % Cfg::WGM, wn = wave / Cfg::WGM;
   const int lr = lane & 31, g = lane >> 5;
-  const int m0 = blockIdx.x * Cfg::BM;
-  const int nsteps = a.N / Cfg::BN;
+  const int slice = (int)blockIdx.x / groups, m0 = ((int)blockIdx.x - slice * groups) * Cfg::BM;
+  const int first = slice * steps, last = first + steps < a.N / Cfg::BN ? first + steps : a.N / Cfg::BN;   // this workgroup's steps of N
 
   // Weight loads: wave-instruction q = 4 wave + i of a stage's 32 covers rows 8 (q & 15) .. +8 of slab q >> 4, eight
   // 16-byte chunks per row, the swizzle applied on the global side.
@@ -61,14 +61,14 @@ __global__ void __launch_bounds__(ShortKCfg::NT, 2) gemm_shortk_kernel(const Gem
   const __amdgpu_buffer_rsrc_t rsrc_none = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.W), 0, 0, 0x00020000);
   const int step_bytes = Cfg::BN * (int)a.ldw;
   auto issue_step = [&](int step) {
-    const __amdgpu_buffer_rsrc_t r = step < nsteps ? rsrc_w : rsrc_none;
+    const __amdgpu_buffer_rsrc_t r = step < last ? rsrc_w : rsrc_none;
     uint8_t* dst = smem + (step & 1) * Cfg::STAGE_BYTES + wave * LOADS * 1024;
     static_for<0, LOADS>([&](auto ic) {
       constexpr int i = decltype(ic)::value;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)(dst + i * 1024), 16, (int)voff[i], step * step_bytes, 0, 0);
     });
   };
-  issue_step(0);
+  issue_step(first);
 
   // The wave's A fragments: rows m0 + 64 wm + 32 tm + lr, bytes [64 ks + 32 g, +32) of each. Rows past M repeat the last one.
   Frag<DT_FP8> xf[TM][KSTEPS];
@@ -185,13 +185,13 @@ __global__ void __launch_bounds__(ShortKCfg::NT, 2) gemm_shortk_kernel(const Gem
   // front of the barrier has to be for everything (loads and stores retire in no fixed order with respect to each
   // other, so no count separates this step's weights from the stores before them); placed like this it finds the
   // stores a whole MFMA phase old and the weights an epilogue and an MFMA phase old.
-  for (int step = 0; step <= nsteps; ++step) {
+  for (int step = first; step <= last; ++step) {
     wait_vmcnt<0>();
     dmam_barrier();
     // Every wave has read the other stage for the last time before it reached this barrier.
     issue_step(step + 1);
-    if (step > 0) epilogue(step - 1);
-    if (step == nsteps) break;
+    if (step > first) epilogue(step - 1);
+    if (step == last) break;
     const uint32_t stage_off = (step & 1) * Cfg::STAGE_BYTES;
     static_for<0, KSTEPS>([&](auto ksc) {
       constexpr int ks = decltype(ksc)::value;
@@ -221,7 +221,16 @@ static hipError_t launch_shortk(const GemmArgs& a, hipStream_t st) {
     if (e != hipSuccess) return e;
     attr_set[dev] = true;
   }
-  hipLaunchKernelGGL(kern, dim3((a.M + ShortKCfg::BM - 1) / ShortKCfg::BM), dim3(ShortKCfg::NT), ShortKCfg::LDS_BYTES, st, a);
+  // Slices of N: one workgroup fits a CU, so the call takes rounds of workgroups, each its slice's steps long and some three steps more for launch, rows and first weights (one to six:
+  // the same times). Below 256 blocks of rows a workgroup per block leaves CUs without work. Whole BT4-class e4m3 calls, all of N -> slices: 264 positions (33 blocks) 4862 -> 4177 us,
+  // 400 6351 -> 5712, 600 8460 -> 7984, 1000 (125 blocks) 12052 -> 11807; from 1504 on one slice, 17587 and 17572.
+  const long groups = (a.M + ShortKCfg::BM - 1) / ShortKCfg::BM, nsteps = a.N / ShortKCfg::BN, cus = device_cus() > 0 ? device_cus() : 256;
+  long steps = nsteps, best = -1;
+  for (long s = nsteps; s > 0; --s) {
+    const long units = groups * ((nsteps + s - 1) / s), cost = (units + cus - 1) / cus * (s + 3);
+    if (best < 0 || cost < best) { best = cost; steps = s; }
+  }
+  hipLaunchKernelGGL(kern, dim3((uint32_t)(groups * ((nsteps + steps - 1) / steps))), dim3(ShortKCfg::NT), ShortKCfg::LDS_BYTES, st, a, (int)groups, (int)steps);
   return hipGetLastError();
 }
 

@@ -490,6 +490,12 @@ def test_gemm_short_k_rows_resident_equals_tiled(cuda, M, N, out_dt):
     assert torch.allclose(rows[sample].float(), exact, rtol=2 ** -7, atol=2 ** -7 * exact.abs().max().item())
 
 
+@pytest.mark.parametrize("M,N,dt", [(8448, 4224, 2), (9216, 4096, 1), (22016, 1664, 1), (33024, 4096, 2)])
+def test_gemm_short_k_in_slices_of_n(cuda, M, N, dt):
+    """Fewer blocks of 256 rows than CUs: several workgroups share a block's columns, the last with fewer steps than the others (33, 32 and 13 steps over 33 to 129 blocks)."""
+    test_gemm_short_k_rows_resident_equals_tiled(cuda, M, N, dt)
+
+
 def test_gemm_short_k_rows_resident_rejects_what_it_cannot_do(cuda):
     """Tile 13 is a bare scaled product for K = 256, whole blocks of 256 rows and outputs beyond 64 MB: anything else
     is refused (CRL_ERR_ARG), never computed by another kernel behind the caller's back."""
