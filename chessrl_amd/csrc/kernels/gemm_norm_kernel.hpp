@@ -1,5 +1,5 @@
-// C[M,N] = act(descale * norm(X)[M,K] · W[N,K]^T + bias): a LayerNorm (or RMSNorm) of fp32 rows of K <= 1024 columns and the product that
-// reads it as one launch, for products so small that every tile of 16 or 32 rows has a CU of its own (GPT on one to a few
+// C[M,N] = act(descale * norm(X)[M,K] · W[N,K]^T + bias): a LayerNorm (or RMSNorm) of fp32 or 16-bit rows of K <= 1024 columns and the product that
+// reads it as one launch, for products so small that every tile of 16 or 32 rows has a CU of its own (GPT and the post-norm trunks on one to a few
 // positions, the token steps of generation). There a norm is a launch of 4 us around a handful of rows. Here every workgroup normalises
 // its rows itself: sixteen waves take one or two rows each, requested before anything is waited for, the workgroup's weight rows
 // follow straight to LDS, and the normalised rows go to LDS as the operand. With both operands whole in LDS (at most
@@ -10,8 +10,8 @@
 // 10800, 9600 and 8000; vocabulary 10800, 9000, 7500 (whole call 186.0 -> 182.3 us, 171.0 -> 163.7).
 // One counted wait behind the last request lets the statistics run under the weight loads; the normalised rows wait for
 // them all the same, because the compiler drains every load into LDS in front of the first write to it. Measured in place: K = 768, N = 2304, 128 rows 8.4 us (12.4 for the norm riding on the K-sliced product before it and the
-// product), 64 rows 7.3 us (8.5 for two launches). 16-bit rows of 1024 columns (BT4-class, one position: the
-// tile's rows are 16) 5.7 us for N = 3584 and 4.8 for N = 1536 against 7.6 and 6.5 for two launches with the gap between them. Taken back: the weights requested behind a barrier, so
+// product), 64 rows 7.3 us (8.5 for two launches). 16-bit rows of 1024 columns (BT4-class, one position, tiles
+// of 16 rows, N = 3104 and 1536) 7.3 us on average inside the call, two launches 8.2 and the gap of 1.2 between them (whole call 659 -> 621). Taken back: the weights requested behind a barrier, so
 // that no wave's rows queue behind another's weights, LDS writes that do not wait for the weights, 16-bit rows straight to LDS (each wave then waits for all the others first): one
 // position 621 -> 637 us for the call.
 // The norm's arithmetic is that of layernorm_kernel row by row and the product adds K in the order of the other tiled kernels: bit-equal to
