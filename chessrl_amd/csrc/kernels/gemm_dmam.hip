@@ -11,9 +11,9 @@ bool gemm_dmam_has(int in_dt, int out_dt) {
 }
 
 // Tiles of 128x192: outputs of the operands' type, or bf16 of e4m3 operands, without a residual (its registers spill beside twelve multiplying waves: BT4-class bf16 at 150 positions
-// 3661 -> 3903 us with it).
+// 3661 -> 3903 us with it), rows of W no further apart than 192 of them can be addressed (128x128 tiles reach half as far again: they serve what lies between).
 bool gemm_dmam_wide_can(const GemmArgs& a, int in_dt, int out_dt) {
-  if (a.res_stats || (long)((a.M + 127) / 128) * ((a.N + 191) / 192) >= 65536 || dmaf_epilogue(a, in_dt, out_dt, 192) != DMAF_PLAIN) return false;
+  if (a.res_stats || !dmam_reaches(a, in_dt == DT_FP8 ? 1 : 2, 192) || (long)((a.M + 127) / 128) * ((a.N + 191) / 192) >= 65536 || dmaf_epilogue(a, in_dt, out_dt, 192) != DMAF_PLAIN) return false;
   if (in_dt == DT_FP8) return (out_dt == DT_FP8 && a.act == ACT_MISH) || (out_dt == DT_BF16 && a.act == ACT_NONE);
   return in_dt == out_dt && (in_dt == DT_BF16 || in_dt == DT_F16) && (a.act == ACT_NONE || a.act == ACT_MISH || (a.act == ACT_GELU && in_dt == DT_BF16));
 }

@@ -416,12 +416,17 @@ __global__ void __launch_bounds__(DmamCfgN<TILE_N>::NT) gemm_dmam_kernel(const G
   }
 }
 
+// The rows of a tile's operands lie within the 31-bit offsets of a buffer descriptor.
+inline bool dmam_reaches(const GemmArgs& a, int esz, int tile_n) {
+  return (long)a.lda * esz * DmamCfg::BM < (1L << 31) && (long)a.ldw * esz * tile_n < (1L << 31);
+}
+
 template <int IN_DT, int OUT_DT, int EPI, int ACT = ACT_NONE, int TILE_N = 128>
 static hipError_t launch_dmam(const GemmArgs& a, int cus, hipStream_t st) {
   static std::atomic<bool> attr_set[16] = {};
   typedef DmamCfgN<TILE_N> Cfg;
   constexpr int ESZ = IN_DT == DT_FP8 ? 1 : 2;
-  if ((a.K * ESZ) % Cfg::ROWB != 0 || a.K <= 0 || (long)a.lda * ESZ * 128 >= (1L << 31) || (long)a.ldw * ESZ * TILE_N >= (1L << 31)) return hipErrorInvalidValue;
+  if ((a.K * ESZ) % Cfg::ROWB != 0 || a.K <= 0 || !dmam_reaches(a, ESZ, TILE_N)) return hipErrorInvalidValue;
   int dev = 0;
   (void)hipGetDevice(&dev);
   auto kern = gemm_dmam_kernel<IN_DT, OUT_DT, EPI, ACT, TILE_N>;

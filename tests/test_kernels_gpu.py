@@ -296,6 +296,22 @@ def test_gemm_e4m3_tiles_of_192_columns_equal_those_of_128(cuda, M, N, K, out_dt
     assert torch.allclose(got[sel], ref[sel], rtol=2.0 ** (-4 if out_dt == _lib.FP8 else -8) + 1e-4, atol=2e-3 * math.sqrt(K / 64))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float8_e4m3fn])
+def test_gemm_weight_rows_too_far_apart_for_tiles_of_192_columns(cuda, dtype):
+    """A size for which the automatic choice takes 128x192 tiles, with rows of W so far apart that 128 but not 192 of them lie within 2 GB: 128x128 tiles serve it, with their bits."""
+    esz = 1 if dtype == torch.float8_e4m3fn else 2
+    M, N, K, ldw = 32768, 192, 256, (12 << 20) // esz
+    torch.manual_seed(6)
+    A = torch.randn(M, K, device=cuda).to(dtype)
+    near = (torch.randn(N, K, device=cuda) * (1.0 if esz == 1 else 0.05)).to(dtype)
+    W = torch.empty(N * ldw * esz, dtype=torch.uint8, device=cuda).view(dtype).view(N, ldw)[:, :K]
+    W.copy_(near)
+    out = run_gemm(A, W, _lib.BF16, descale=0.05)
+    assert torch.equal(out, run_gemm(A, near, _lib.BF16, descale=0.05, tile=11))
+    ref = (A.float() @ near.float().t()) * 0.05
+    assert torch.allclose(out.float(), ref, rtol=2.0 ** -8 + 1e-4, atol=2e-3 * math.sqrt(K / 64))
+
+
 @pytest.mark.parametrize("M,nsplit,extra,K", [(16384, 3072, 32, 1024), (12288, 3072, 16, 1536), (1024, 512, 32, 256), (16640, 3072, 32, 1024), (16384, 3072, 40, 1024)])
 def test_gemm_split_output_last_tile_column_carries_the_columns_behind_it(cuda, M, nsplit, extra, K):
     """crl_gemm_split: columns [0, nsplit) into C, the rest into C2. The columns behind a split at a multiple of 256 are a last,
