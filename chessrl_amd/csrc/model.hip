@@ -1068,15 +1068,22 @@ int Model::generate(const float* planes, int B, int steps, float temperature, ui
   RUN(forward_chunk(planes, nullptr, nullptr, gen_tok, 1, B, gen_logits, nullptr, nullptr, false, st));
   kv_capture = false;
   const float attn_scale = 1.0f / std::sqrt((float)hs);
-  // Keys and values that a step reads beyond what the memory-side cache keeps from one step to the next are read past it, the later layers' first: it then keeps
-  // the weights, which every product of a step waits for. 128 sequences (88 MB of weights, 63 MB of keys and values a layer on average), whole rollout: no layer read
-  // past it 54.3 ms, those beyond 260 MB 53.2, 200 52.6, 150 51.3, 100 51.4, all 52.1 (before the values were requested ahead: 260 and all); 64 sequences 41.3, 150 MB 39.7, all 39.9;
-  // 16 and fewer stay inside (all past it: +1.2 %).
-  constexpr size_t KEEP = 150u << 20;
+  // Weights, keys and values are read once a step. What of them the memory-side cache cannot keep from one step to the next is read past it, the later layers' keys and values:
+  // it then keeps the weights, which every product of a step waits for. Three lines, whole rollouts of 191 tokens in ms (plain launches; replayed), no layer read past it -> as below:
+  // Weights and all rows up to 200 MB stay inside: 6 layers of 768 (88 MB of weights, 0.47 MB a sequence and layer on average), 16 sequences 30.9, 24 32.4, 28 32.3 either way; with layers
+  // beyond 150 MB read past it 24 take 32.6 (replayed 36.1 -> 36.4). Beyond, the layers past 150 MB of weights and rows: 40 sequences 34.4 -> 33.8 (37.7 -> 37.6), 48 36.5 -> 36.1, 64
+  // 39.8 -> 37.9 (42.3 -> 40.9), 96 47.5 -> 44.4 (49.9 -> 47.6), 128 52.2 -> 48.8 (55.4 -> 52.0); 200 MB in place of 150 128 49.2, every layer 49.0, only what is beyond 256 MB 50.3. Up to 32 MB
+  // of rows stay inside whatever the weights take: 12 layers of 1024 (306 MB of weights), all past it: 1 to 3 sequences 61.4 -> 62.7, 62.0 -> 63.3, 62.9 -> 63.6, 4 64.3 -> 63.9 (68.5 -> 69.3), 6 66.2 ->
+  // 64.2; 18 of 768 (258 MB): 2 85.4 -> 86.4, 4 89.4 -> 87.0.
+  constexpr size_t FIT = 200u << 20, KEEP = 150u << 20, FEW = 32u << 20;
   size_t weights = (size_t)lm_head.N * lm_head.K * 2;
   for (const Layer& y : layers)
     for (const Lin* w : {&y.qkv, &y.proj, &y.ff1, &y.ff2}) weights += (size_t)w->N * w->K * 2;
-  auto past = [&](int l, int n) { return weights + (size_t)(l + 1) * B * n * 2 * C * 2 > KEEP; };
+  auto past = [&](int l, int n) {
+    const size_t rows = (size_t)B * n * 2 * C * 2, all = L * rows;
+    return all > FEW && weights + all > FIT && weights + (l + 1) * rows > KEEP;
+  };
+  const int mean_n = (66 + Tmax) / 2;   // of a replayed step, whose launches serve every length
   // One token step: sample token k from gen_logits, then (unless it is the last) run it through the trunk at position
   // 64 + k against the cache and leave the next logits in gen_logits. With `dyn` the kernels read k from device memory
   // and the step ends by advancing it, so the same launches serve every k (the body of the replayed graph).
@@ -1115,7 +1122,7 @@ int Model::generate(const float* planes, int B, int steps, float temperature, ui
         }
         if (dyn) STEP_HIP(launch_kv_append(gen_kv_stage, kv_layers[l], B, kv_Tmax, C, 0, dyn, s));
       }
-      STEP_HIP(launch_decode_attention(ws.qkv, C, kv_layers[l], kv_Tmax, C, pos + 1, dyn, ws.ao, C, B, H, hs, ad, attn_scale, past(l, dyn ? Tmax : pos + 1), s));
+      STEP_HIP(launch_decode_attention(ws.qkv, C, kv_layers[l], kv_Tmax, C, pos + 1, dyn, ws.ao, C, B, H, hs, ad, attn_scale, past(l, dyn ? mean_n : pos + 1), s));
       bool normed2 = false;
       { GOpt o; o.k_parallel = true; o.res = ws.x; o.ldr = C; o.res_dt = xdt;
         if (!fused) { o.ln_g = ly.ln2_g; o.ln_b = ly.ln2_b; o.ln_out = ws.h; o.ln_dt = ad; o.ln_folded = &normed2; }

@@ -264,7 +264,7 @@ int crl_model_forward_tokens(crl_model* m, const float* planes, const int64_t* i
  * the kernels then read the token index from a device counter) and replays it; results are bit-identical, the call
  * returns after the stream has drained, and the stream must not itself be under capture. It is off by default: a
  * token step is bound by its kernels' run time on the device, not by the host's launches (measured at 128 sequences:
- * 60.8 ms plain, 64.4 ms replayed, where storing keys and values and advancing the counter are launches of their own), so
+ * 48.7 ms plain, 52.1 ms replayed, where storing keys and values and advancing the counter are launches of their own), so
  * the option is for hosts that cannot keep up. The profiling mode always launches plainly. */
 int crl_model_generate(crl_model* m, const float* planes, int B, int steps, float temperature, uint64_t seed, int rules,
                        int64_t* sequences, float* step_out, int out_logits, void* stream);
