@@ -436,11 +436,12 @@ __global__ void __launch_bounds__(SPLIT ? 128 : 64 * AttnWaves<MODE>::N, (SPLIT 
 // keys once for both waves; the next position's are requested behind the shift, its values once V is transposed, and the positional table's fragments
 // stay in registers. 496 positions of 8 heads of 64 40.1 -> 34.4 us (bytes: 26), 1521 122.9 -> 89.7 (81). Registers alone, without LDS: 40.8 and 113.4.
 // Requests past the last position go through empty descriptors and move nothing. 50 KB of LDS: three workgroups a CU.
+// FAR: rows further apart than the 31-bit offsets inside a position reach (2^24 elements), or in descending order: 64-bit addresses; past the last position the last one is read again.
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ void attn_load_lds(__amdgpu_buffer_rsrc_t r, uint8_t* dst, int off) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, off, 0, 0, 0);
 }
-template <int HS, int OUT_FP8, int IN_DT>
+template <int HS, int OUT_FP8, int IN_DT, bool FAR>
 __global__ void __launch_bounds__(128, 2) relshift_kernel(const AttnArgs a, const int slices) {
   typedef Half16<IN_DT> H16;
   typedef typename H16::vec hvec;
@@ -476,24 +477,33 @@ __global__ void __launch_bounds__(128, 2) relshift_kernel(const AttnArgs a, cons
   if (lane < HS) { uv[lane] = a.u_bias[h * HS + lane]; uv[HS + lane] = a.v_bias[h * HS + lane]; }
 
   // ---- requests: offsets inside a position's 64 rows, the same for every position
-  const int ldq2 = (int)a.ldq * 2, ldk2 = (int)a.ldk * 2, ldv2 = (int)a.ldv * 2;
-  auto rows = [&](const void* base, int b, int ld2) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(reinterpret_cast<const char*>(base)) + (long)b * 64 * ld2 + h * (HS * 2), 0, b < a.B ? 63 * ld2 + HS * 2 : 0, 0x00020000);
+  typedef std::conditional_t<FAR, long, int> Off;
+  const Off ldq2 = (Off)a.ldq * 2, ldk2 = (Off)a.ldk * 2, ldv2 = (Off)a.ldv * 2;
+  auto unit = [&](const void* base, int b, Off ld2) { return reinterpret_cast<const char*>(base) + (long)b * 64 * ld2 + h * (HS * 2); };
+  auto rows = [&](const void* base, int b, Off ld2) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(unit(base, b, ld2)), 0, b < a.B ? 63 * (int)ld2 + HS * 2 : 0, 0x00020000);
   };
   // Queries and keys straight into LDS, whole rows at a time (64 lanes of 32 rows, as the MFMAs want them, hold a load for 190 cycles and a store for more: 2300 and 1900 of a
   // unit's 11300): wave 0 the queries, wave 1 the keys, 16-byte chunks swizzled by row on the global side.
   auto swz = [](int row) { return CPR == 8 ? (row ^ (row >> 3)) & 7 : (row >> 1) & 3; };
-  const int ldw2 = wave ? ldk2 : ldq2;
-  int wo[QK_LOADS];
+  const Off ldw2 = wave ? ldk2 : ldq2;
+  Off wo[QK_LOADS];
 #pragma unroll
   for (int j = 0; j < QK_LOADS; ++j) {
     const int row = j * (64 / CPR) + lane / CPR;
     wo[j] = row * ldw2 + (((lane % CPR) ^ swz(row)) << 4);
   }
   auto qk_load = [&](int b) {
-    const __amdgpu_buffer_rsrc_t r = rows(wave ? a.k : a.q, b, ldw2);
+    if constexpr (FAR) {
+      const char* const p = unit(wave ? a.k : a.q, b < a.B ? b : a.B - 1, ldw2);
 #pragma unroll
-    for (int j = 0; j < QK_LOADS; ++j) attn_load_lds(r, s_qk[wave] + j * 1024, wo[j]);
+      for (int j = 0; j < QK_LOADS; ++j)
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(p + wo[j]), (__attribute__((address_space(3))) void*)(s_qk[wave] + j * 1024), 16, 0, 0);
+    } else {
+      const __amdgpu_buffer_rsrc_t r = rows(wave ? a.k : a.q, b, ldw2);
+#pragma unroll
+      for (int j = 0; j < QK_LOADS; ++j) attn_load_lds(r, s_qk[wave] + j * 1024, wo[j]);
+    }
   };
   auto frag = [&](const uint8_t* rows_, int row, int ks) -> hvec {
     return *reinterpret_cast<const hvec*>(rows_ + row * ROWB + (((2 * ks + g) ^ swz(row)) << 4));
@@ -503,12 +513,18 @@ __global__ void __launch_bounds__(128, 2) relshift_kernel(const AttnArgs a, cons
   static_assert(PASSES == 1 || PASSES == 2, "head sizes 32 and 64");
   const bool v_mine = PASSES == 2 || !g;
   const int v_id = PASSES == 2 ? wave * 64 + lane : 32 * wave + lr, jq = v_id / DC, dc = v_id - jq * DC;
-  const int vo = 4 * jq * ldv2 + 16 * dc;
+  const Off vo = 4 * jq * ldv2 + 16 * dc;
   u32x4_t vrow[4];
   auto v_load = [&](int b) {
-    const __amdgpu_buffer_rsrc_t rv = rows(a.v, b, ldv2);
+    if constexpr (FAR) {
+      const char* const p = unit(a.v, b < a.B ? b : a.B - 1, ldv2) + vo;
 #pragma unroll
-    for (int t = 0; t < 4; ++t) vrow[t] = __builtin_amdgcn_raw_buffer_load_b128(rv, vo + t * ldv2, 0, 0);
+      for (int t = 0; t < 4; ++t) vrow[t] = *reinterpret_cast<const u32x4_t*>(p + t * ldv2);
+    } else {
+      const __amdgpu_buffer_rsrc_t rv = rows(a.v, b, ldv2);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) vrow[t] = __builtin_amdgcn_raw_buffer_load_b128(rv, vo + t * ldv2, 0, 0);
+    }
   };
   auto barrier = [&]() {   // (a bare one: a __syncthreads may wait for what is meant to stay in flight)
     __builtin_amdgcn_s_waitcnt(0xC07F);
@@ -670,21 +686,23 @@ __global__ void __launch_bounds__(128, 2) relshift_kernel(const AttnArgs a, cons
   }
 }
 
-template <int HS, int IN_DT>
+template <int HS, int IN_DT, bool FAR>
 static hipError_t launch_relshift_dt(const AttnArgs& a, hipStream_t st) {
   // Three workgroups fit a CU: the positions of a head in as many slices as that gives, evened out.
   const int cus = device_cus() > 0 ? device_cus() : 256, most = std::max(3 * cus / a.H, 1), each = (a.B + most - 1) / most, slices = (a.B + each - 1) / each;
   const dim3 grid(slices * a.H), block(128);
-  if (a.out_dtype == DT_FP8) hipLaunchKernelGGL((relshift_kernel<HS, 1, IN_DT>), grid, block, 0, st, a, slices);
-  else if (a.out_dtype == IN_DT) hipLaunchKernelGGL((relshift_kernel<HS, 0, IN_DT>), grid, block, 0, st, a, slices);
+  if (a.out_dtype == DT_FP8) hipLaunchKernelGGL((relshift_kernel<HS, 1, IN_DT, FAR>), grid, block, 0, st, a, slices);
+  else if (a.out_dtype == IN_DT) hipLaunchKernelGGL((relshift_kernel<HS, 0, IN_DT, FAR>), grid, block, 0, st, a, slices);
   else return hipErrorInvalidValue;
   return hipGetLastError();
 }
 template <int HS>
 static hipError_t launch_relshift(const AttnArgs& a, hipStream_t st) {
-  if (a.qk_hstride || a.ldq >= 1L << 24 || a.ldk >= 1L << 24 || a.ldv >= 1L << 24) return hipErrorInvalidValue;
-  if (a.in_dtype == DT_F16) return launch_relshift_dt<HS, DT_F16>(a, st);
-  if (a.in_dtype == DT_BF16) return launch_relshift_dt<HS, DT_BF16>(a, st);
+  if (a.qk_hstride) return hipErrorInvalidValue;
+  auto near = [](long ld) { return ld >= 0 && ld < 1L << 24; };
+  const bool far = !near(a.ldq) || !near(a.ldk) || !near(a.ldv);
+  if (a.in_dtype == DT_F16) return far ? launch_relshift_dt<HS, DT_F16, true>(a, st) : launch_relshift_dt<HS, DT_F16, false>(a, st);
+  if (a.in_dtype == DT_BF16) return far ? launch_relshift_dt<HS, DT_BF16, true>(a, st) : launch_relshift_dt<HS, DT_BF16, false>(a, st);
   return hipErrorInvalidValue;
 }
 

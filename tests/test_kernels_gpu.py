@@ -797,6 +797,40 @@ def test_attention_relshift_workgroups_that_walk_positions(cuda, B, H, hs, dtype
         assert torch.equal(whole[b * 64:(b + n) * 64], few), b
 
 
+@pytest.mark.parametrize("B,H,hs,dtype,out_dt", [(1, 2, 64, torch.bfloat16, None), (3, 512, 32, torch.float16, None), (2, 400, 64, torch.bfloat16, _lib.FP8), (1, 3, 32, torch.bfloat16, None)])
+@pytest.mark.parametrize("far", ["qkv", "q", "v", "descending"])
+def test_attention_relshift_rows_further_apart_than_offsets_of_31_bits(cuda, B, H, hs, dtype, out_dt, far):
+    """Row strides of 2^24 elements and more, of all three inputs or of one, and rows in descending order (negative strides): the bits of rows that lie close. 512 heads of three positions
+    and 400 of two: workgroups that walk positions (768 fit 256 CUs)."""
+    Cm = H * hs
+    torch.manual_seed(B + H)
+    q, k, v, pos = (torch.randn(n * 64, Cm, device=cuda).to(dtype) for n in (B, B, B, 1))
+    u, vb = torch.randn(Cm, device=cuda) * 0.3, torch.randn(Cm, device=cuda) * 0.3
+    odt = (_lib.F16 if dtype == torch.float16 else _lib.BF16) if out_dt is None else out_dt
+
+    def run(rows):
+        out = torch.zeros(B * 64, Cm, dtype=dtype if out_dt is None else torch.uint8, device=cuda)
+        args = [x for t, ld, at in rows for x in (C.c_void_p(t.data_ptr() + at), ld)]
+        check(lib().crl_attention(*args, _lib.F16 if dtype == torch.float16 else _lib.BF16, p(out), Cm, odt, 30.0, B, H, hs, _lib.ATTN_RELSHIFT, 1 / math.sqrt(Cm), None, p(pos), p(u), p(vb),
+                                  None, stream()), "attn")
+        torch.cuda.synchronize()
+        return out
+
+    def spread(x, ld):
+        wide = torch.empty((B * 64, ld), dtype=dtype, device=cuda)
+        wide[:, :Cm] = x
+        return wide, ld, 0
+
+    rows = [(x, Cm, 0) for x in (q, k, v)]
+    ref = run(rows)
+    for i, name in enumerate("qkv"):
+        if far == "descending":
+            rows[i] = (rows[i][0].flip(0).contiguous(), -Cm, (B * 64 - 1) * Cm * 2)
+        elif name in far:
+            rows[i] = spread(rows[i][0], (1 << 24) + 8 * i)
+    assert torch.equal(run(rows), ref)
+
+
 @pytest.mark.parametrize("T", [1.0, 0.5, 0.0])
 def test_masked_softmax(cuda, T):
     torch.manual_seed(3)
