@@ -438,6 +438,7 @@ __global__ void __launch_bounds__(SPLIT ? 128 : 64 * AttnWaves<MODE>::N, (SPLIT 
 // Requests past the last position go through empty descriptors and move nothing. 50 KB of LDS: three workgroups a CU.
 // FAR: rows further apart than the 31-bit offsets inside a position reach (2^24 elements), or in descending order: 64-bit addresses; past the last position the last one is read again.
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4_any_t __attribute__((ext_vector_type(4), aligned(1)));   // output rows start wherever the caller's pointer and stride (a multiple of four elements) put them
 __device__ __forceinline__ void attn_load_lds(__amdgpu_buffer_rsrc_t r, uint8_t* dst, int off) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, off, 0, 0, 0);
 }
@@ -676,7 +677,7 @@ __global__ void __launch_bounds__(128, 2) relshift_kernel(const AttnArgs a, cons
 #pragma unroll
       for (int j = 0; j < NST; ++j) {
         const int row = j * (64 / OCH) + lane / OCH, c = lane % OCH;
-        *reinterpret_cast<uint4*>(ob + row * (a.ldo * (OUT_FP8 ? 1 : 2)) + c * 16) = *reinterpret_cast<const uint4*>(s_out[wave] + row * ORB + ((c ^ (row & (OCH - 1))) << 4));
+        *reinterpret_cast<u32x4_any_t*>(ob + row * (a.ldo * (OUT_FP8 ? 1 : 2)) + c * 16) = *reinterpret_cast<const u32x4_t*>(s_out[wave] + row * ORB + ((c ^ (row & (OCH - 1))) << 4));
       }
     }
   }

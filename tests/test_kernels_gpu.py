@@ -831,6 +831,29 @@ def test_attention_relshift_rows_further_apart_than_offsets_of_31_bits(cuda, B, 
     assert torch.equal(run(rows), ref)
 
 
+@pytest.mark.parametrize("hs", [32, 64])
+@pytest.mark.parametrize("fp8,gap,start", [(True, 16, 16), (True, 8, 8), (True, 4, 4), (True, 8, 0), (False, 4, 4), (False, 8, 8), (False, 4, 0)])
+def test_attention_relshift_output_rows_off_16_bytes(cuda, hs, fp8, gap, start):
+    """Output rows that start 4, 8 or 16 bytes off a multiple of 16, by the stride (`gap` elements behind a row) or by the pointer (`start` elements): the same bits, and nothing written in
+    front of the first row or between rows."""
+    B, H = 3, 3
+    qkv, Cm = make_qkv(B, H, hs, cuda, 9 + gap, torch.bfloat16)
+    pos = torch.randn(64, Cm, device=cuda).bfloat16()
+    u, vb = torch.randn(Cm, device=cuda) * 0.3, torch.randn(Cm, device=cuda) * 0.3
+    odt, esz = (_lib.FP8, 1) if fp8 else (_lib.BF16, 2)
+    ref = run_attn(qkv, B, H, hs, _lib.ATTN_RELSHIFT, 1 / math.sqrt(Cm), pos=pos, u=u, v=vb, out_dt=odt, out_scale=30.0)
+    ldo = Cm + gap
+    buf = torch.full((start + B * 64 * ldo + 16,), 0x55 if fp8 else 0x5555, dtype=torch.uint8 if fp8 else torch.int16, device=cuda)
+    base = qkv.data_ptr()
+    check(lib().crl_attention(C.c_void_p(base), 3 * Cm, C.c_void_p(base + 2 * Cm), 3 * Cm, C.c_void_p(base + 4 * Cm), 3 * Cm, _lib.BF16, C.c_void_p(buf.data_ptr() + start * esz), ldo, odt, 30.0,
+                              B, H, hs, _lib.ATTN_RELSHIFT, 1 / math.sqrt(Cm), None, p(pos), p(u), p(vb), None, stream()), "attn")
+    torch.cuda.synchronize()
+    rows = buf[start:start + B * 64 * ldo].view(B * 64, ldo)
+    assert torch.equal(rows[:, :Cm], ref if fp8 else ref.view(torch.int16))
+    mark = 0x55 if fp8 else 0x5555
+    assert (rows[:, Cm:] == mark).all() and (buf[:start] == mark).all() and (buf[start + B * 64 * ldo:] == mark).all()
+
+
 @pytest.mark.parametrize("T", [1.0, 0.5, 0.0])
 def test_masked_softmax(cuda, T):
     torch.manual_seed(3)
