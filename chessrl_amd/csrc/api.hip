@@ -235,7 +235,7 @@ int crl_gemm(const void* A, int64_t lda, const void* W, int64_t ldw, void* C, in
              float out_scale, float* amax, int tile, void* stream) {
   if (!A || !W || !C || M < 0 || N < 0 || K <= 0) return arg_fail("crl_gemm: bad arguments");
   if (in_dtype != DT_BF16 && in_dtype != DT_F16 && in_dtype != DT_FP8) return arg_fail("crl_gemm: in_dtype must be bf16, f16 or fp8");
-  if (out_dtype < 0 || out_dtype > 3 || tile < 0 || tile > 16 || tile == 6 || tile == 8) return arg_fail("crl_gemm: bad out_dtype or tile");
+  if (out_dtype < 0 || out_dtype > 3 || tile < 0 || tile > 17 || tile == 6 || tile == 8) return arg_fail("crl_gemm: bad out_dtype or tile");
   GemmArgs g;
   std::memset(&g, 0, sizeof(g));
   g.A = A; g.lda = lda; g.W = W; g.ldw = ldw; g.C = C; g.ldc = ldc; g.M = M; g.N = N; g.K = K; g.nsplit = N;
@@ -252,7 +252,7 @@ int crl_gemm_split(const void* A, int64_t lda, const void* W, int64_t ldw, void*
   if (!A || !W || !C || !C2 || M < 0 || N < 0 || K <= 0) return arg_fail("crl_gemm_split: bad arguments");
   if (nsplit <= 0 || nsplit >= N || nsplit % 8 != 0) return arg_fail("crl_gemm_split: nsplit must be a multiple of 8 inside (0, N)");
   if (in_dtype != DT_BF16 && in_dtype != DT_F16 && in_dtype != DT_FP8) return arg_fail("crl_gemm_split: in_dtype must be bf16, f16 or fp8");
-  if (out_dtype < 0 || out_dtype > 3 || (tile != 0 && tile != 3 && tile != 7 && tile != 10)) return arg_fail("crl_gemm_split: bad out_dtype or tile");
+  if (out_dtype < 0 || out_dtype > 3 || (tile != 0 && tile != 3 && tile != 7 && tile != 10 && tile != 17)) return arg_fail("crl_gemm_split: bad out_dtype or tile");
   GemmArgs g;
   std::memset(&g, 0, sizeof(g));
   g.A = A; g.lda = lda; g.W = W; g.ldw = ldw; g.C = C; g.ldc = ldc; g.C2 = C2; g.ldc2 = ldc2; g.M = M; g.N = N; g.K = K; g.nsplit = nsplit;

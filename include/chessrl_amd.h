@@ -122,8 +122,11 @@ int crl_random_positions(uint64_t seed, int n, int max_plies, double late_fracti
  * 15 and 16 = the 64x64 tile on an eight-stage and the 32x32 tile on a sixteen-stage ring of direct-to-LDS loads (same sums
  * and bits as 1; whole slabs; e4m3 operands with a 16-bit or e4m3 output, bf16/f16 operands with an output of their own
  * type, bf16 operands with an fp32 output; else CRL_ERR_ARG). Where those apply, tile 0 runs 16 while every 32x32 tile has a CU
- * of its own, 15 while every 64x64 tile has, and beyond that 11, 3 or (no residual; an output of the operands' type, or bf16 of e4m3 ones)
- * 128x192 tiles of the kernel of 11, whichever takes fewer rounds of its tiles over the CUs at the measured time of a round; elsewhere 3 from 160 tiles of 256x256 on, 2 from 256 of 128x128 on, else 1.
+ * of its own, 15 while every 64x64 tile has, and beyond that 11, 3 or 17, whichever takes fewer rounds of its tiles over the CUs at the measured time of
+ * a round; elsewhere 3 from 160 tiles of 256x256 on, 2 from 256 of 128x128 on, else 1. 17 = the kernel of 11 with 128x192 tiles (same sums and bits): no
+ * residual or amax, alpha = 1, K of two whole slabs at least, 16-byte aligned rows of C in whole groups of 8 columns (16 in e4m3), and one of: bf16 or f16
+ * operands with an output of their type and no activation or mish (bf16: or gelu), e4m3 operands with a bf16 output and no activation or an e4m3 output
+ * with mish; 192 rows of W within 2 GB. Anything else is CRL_ERR_ARG.
  * 13 and 14 name the kernel for K = 256 e4m3 elements whose workgroups keep 256 rows of A in registers and walk N (the
  * attention-bias generator's product): a bare scaled product (no bias, activation, residual or amax; alpha = 1) into a
  * bf16/f16 output of more than 64 MB, M a multiple of 256, N of 128; anything else is CRL_ERR_ARG. 13 writes C row-major
@@ -138,8 +141,8 @@ int crl_gemm(const void* A, int64_t lda, const void* W, int64_t ldw, void* C, in
  * ldc2, column n at n - nsplit), both of out_dtype; epilogue descale * acc + bias. This is how the BT4-class layer runs the
  * q, k, v projections and the 32-column compression of the attention-bias generator as one product over one
  * concatenated weight (the reference's layers call one nn.Linear per projection, new_paradigm/attn.py:501-503; the
- * generator follows lc0's smolgen, which the reference does not contain). tile: 0 = automatic, or 3, 7, 10 as in crl_gemm
- * (same sums and result bits in every case). */
+ * generator follows lc0's smolgen, which the reference does not contain). tile: 0 = automatic, or 3, 7, 10, 17 as in crl_gemm
+ * (same sums and result bits in every case; 17: nsplit a multiple of 192). */
 int crl_gemm_split(const void* A, int64_t lda, const void* W, int64_t ldw, void* C, int64_t ldc, void* C2, int64_t ldc2, int nsplit,
                    int M, int N, int K, int in_dtype, int out_dtype, const float* bias, float descale, int tile, void* stream);
 /* No counterpart in the reference: crl_gemm with tile = 4 (K cut into slices, a second kernel adds them) for callers that

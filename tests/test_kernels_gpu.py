@@ -267,16 +267,71 @@ def test_gemm_guardless_epilogue_instances_equal_general_kernel(cuda, M, N, K):
 @pytest.mark.parametrize("dt,act", [(_lib.BF16, 0), (_lib.BF16, 1), (_lib.BF16, 2), (_lib.F16, 0), (_lib.F16, 2)])
 @pytest.mark.parametrize("M,N,K", [(2817, 1536, 1024), (4096, 1536, 192), (2700, 1544, 256), (5500, 1536, 128), (2049, 2312, 768)])
 def test_gemm_tiles_of_192_columns_equal_those_of_128(cuda, M, N, K, dt, act):
-    """Sizes at which the automatic choice takes 128x192 tiles (fewer rounds over 256 CUs): one round and two, ragged last rows and columns, K of two slabs and more. Bit-equal to 128x128, whose
-    sums are checked against fp32 (one rounding of the output)."""
+    """128x192 tiles (17), at sizes for which the automatic choice takes them on 256 CUs: one round and two, ragged last rows and columns, K of two slabs and more. Bit-equal to 128x128, whose
+    sums are checked against fp32 (one rounding of the output), and to the automatic choice."""
     g = torch.Generator(device=cuda).manual_seed(M + N + K)
     A = torch.randn(M, K, device=cuda, generator=g).to(TORCH_DT[dt])
     W = (torch.randn(N, K, device=cuda, generator=g) * 0.05).to(TORCH_DT[dt])
     bias = torch.randn(N, device=cuda, generator=g)
-    out = run_gemm(A, W, dt, bias=bias, act=act)
-    assert torch.equal(out, run_gemm(A, W, dt, bias=bias, act=act, tile=11))
+    out = run_gemm(A, W, dt, bias=bias, act=act, tile=17)
+    assert torch.equal(out, run_gemm(A, W, dt, bias=bias, act=act, tile=11)) and torch.equal(out, run_gemm(A, W, dt, bias=bias, act=act))
     ref = ref_act(A.float() @ W.float().t() + bias, act)
     assert torch.allclose(out.float(), ref, rtol=2.0 ** (-8 if dt == _lib.BF16 else -11) + 1e-4, atol=1e-3 * math.sqrt(K / 64))
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 8, 128), (129, 192, 128), (127, 200, 320), (300, 376, 1024), (70, 1000, 192)])
+def test_gemm_tiles_of_192_columns_at_few_tiles(cuda, M, N, K):
+    """128x192 tiles asked for by name where nothing would choose them: fewer tiles than XCDs, one row, waves without columns. Nothing is written behind row M or column N."""
+    torch.manual_seed(M + N)
+    A, W = torch.randn(M, K, device=cuda).bfloat16(), (torch.randn(N, K, device=cuda) * 0.05).bfloat16()
+    bias = torch.randn(N, device=cuda)
+    out = torch.full((M + 3, N + 8), 7.0, dtype=torch.bfloat16, device=cuda)
+    check(lib().crl_gemm(p(A), K, p(W), K, p(out), N + 8, M, N, K, _lib.BF16, _lib.BF16, p(bias), 2, 1.0, 1.0, None, 0, _lib.BF16, 1.0, None, 17, stream()), "gemm")
+    torch.cuda.synchronize()
+    assert torch.equal(out[:M, :N], run_gemm(A, W, _lib.BF16, bias=bias, act=2, tile=11))
+    assert bool((out[M:] == 7).all()) and bool((out[:, N:] == 7).all())
+
+
+@pytest.mark.parametrize("M,nsplit,extra,K,dt", [(1600, 3072, 32, 1024, "bf16"), (2624, 3072, 32, 1024, "f16"), (1600, 3072, 32, 1024, "fp8"), (5700, 3072, 32, 256, "fp8"), (300, 192, 192, 256, "bf16"), (129, 576, 40, 384, "f16")])
+def test_gemm_split_on_a_boundary_of_192_columns(cuda, M, nsplit, extra, K, dt):
+    """Columns split over two outputs on a boundary of the 128x192 tile (q|k|v and the compression columns of 25, 41 and 89 positions take it): bit-equal to the general 256x256 kernel and to
+    the automatic choice, nothing written behind the rows of either output. A split off the boundary is refused by name and served by the automatic choice."""
+    torch.manual_seed(M + nsplit)
+    N = nsplit + extra
+    td = {"bf16": torch.bfloat16, "f16": torch.float16, "fp8": torch.float8_e4m3fn}[dt]
+    ind, odt = {"bf16": (_lib.BF16, _lib.BF16), "f16": (_lib.F16, _lib.F16), "fp8": (_lib.FP8, _lib.BF16)}[dt]
+    A, W = torch.randn(M, K, device=cuda).to(td), (torch.randn(N, K, device=cuda) * (1.0 if dt == "fp8" else 0.05)).to(td)
+    bias = torch.randn(N, device=cuda)
+
+    def run(tile, split=nsplit):
+        C1, C2 = (torch.full((M + 1, w), 7.0, dtype=TORCH_DT[odt], device=cuda) for w in (split, N - split + 8))
+        rc = lib().crl_gemm_split(p(A), K, p(W), K, p(C1), split, p(C2), N - split + 8, split, M, N, K, ind, odt, p(bias), 0.05, tile, stream())
+        torch.cuda.synchronize()
+        if rc == 0:
+            assert bool((C1[M] == 7).all()) and bool((C2[M] == 7).all()) and bool((C2[:, N - split:] == 7).all())
+        return rc, torch.cat([C1[:M], C2[:M, :N - split]], 1)
+
+    wide, general, auto = run(17), run(7), run(0)
+    assert wide[0] == general[0] == auto[0] == 0
+    assert torch.equal(wide[1], general[1]) and torch.equal(wide[1], auto[1])
+    assert run(17, nsplit - 8)[0] == -1
+    off = run(0, nsplit - 8)
+    assert off[0] == 0 and torch.equal(off[1], general[1])
+
+
+def test_gemm_tiles_of_192_columns_reject_what_they_cannot_do(cuda):
+    """Tile 17 outside its types, activations and layouts is CRL_ERR_ARG, never another kernel behind the caller's back."""
+    A, W = (torch.zeros(256, 256, device=cuda).bfloat16() for _ in range(2))
+    out, amax = torch.zeros(256, 256, device=cuda), torch.zeros(1, device=cuda)
+
+    def call(N=256, K=256, ldc=256, in_dt=_lib.BF16, odt=_lib.BF16, act=0, alpha=1.0, res=None, am=None, at=0, ldw=256):
+        return lib().crl_gemm(p(A), 256, p(W), ldw, C.c_void_p(out.data_ptr() + at), ldc, 64, N, K, in_dt, odt, None, act, 1.0, alpha, p(res), 256, _lib.BF16, 1.0, p(am), 17, stream())
+
+    assert call() == 0
+    for kw in (dict(odt=_lib.F32), dict(act=3), dict(in_dt=_lib.F16, odt=_lib.F16, act=1), dict(in_dt=_lib.FP8, odt=_lib.FP8, act=1), dict(in_dt=_lib.FP8, odt=_lib.F16), dict(K=64), dict(K=200),
+               dict(alpha=0.5), dict(res=A), dict(am=amax), dict(N=252), dict(ldc=260), dict(at=8), dict(ldw=6 << 20)):
+        assert call(**kw) == -1, kw
+    torch.cuda.synchronize()
 
 
 @pytest.mark.parametrize("out_dt,act", [(_lib.FP8, 2), (_lib.BF16, 0)])
@@ -288,8 +343,8 @@ def test_gemm_e4m3_tiles_of_192_columns_equal_those_of_128(cuda, M, N, K, out_dt
     W = torch.randn(N, K, device=cuda, generator=g).to(torch.float8_e4m3fn)
     bias = torch.randn(N, device=cuda, generator=g)
     kw = dict(bias=bias, act=act, descale=0.05, out_scale=4.0 if out_dt == _lib.FP8 else 1.0)
-    out = run_gemm(A, W, out_dt, **kw)
-    assert torch.equal(out, run_gemm(A, W, out_dt, tile=11, **kw))
+    out = run_gemm(A, W, out_dt, tile=17, **kw)
+    assert torch.equal(out, run_gemm(A, W, out_dt, tile=11, **kw)) and torch.equal(out, run_gemm(A, W, out_dt, **kw))
     ref = ref_act((A.float() @ W.float().t()) * 0.05 + bias, act)
     got = out.view(torch.float8_e4m3fn).float() / 4.0 if out_dt == _lib.FP8 else out.float()
     sel = ref.abs() < 100   # (e4m3 ends at 448, here 112)
