@@ -126,7 +126,8 @@ def test_bt4_torch(cuda, cfg, act="bf16"):
 
 @pytest.mark.parametrize("arch,fp8,Fm,FP", [("bt4", False, 248, 256), ("bt4", False, 1000, 1024), ("bt4class", True, 240, 256)])
 def test_padded_ffn_equals_the_model_with_the_zeros_in_its_weights(cuda, arch, fp8, Fm, FP):
-    """Hidden FFN tensors whose rows are filled up to whole slabs: bit-equal to the model that holds the zeros itself, and read back unpadded."""
+    """Hidden FFN tensors whose rows are filled up to whole slabs: bit-equal to the model that holds the zeros itself, and read back unpadded. (BT4 in 16 bits runs its two layers as one, whose
+    sums appended zeros leave alone; its padded layers run below.)"""
     L, Cm, H = 2, 256, 8
     oracle = om.test_init_(om.BT4Oracle(L, Cm, Fm, H) if arch == "bt4" else om.BT4ClassOracle(policy_leela, L, Cm, Fm, H), seed=5)
     planes = positions(70, seed=6, leela=arch == "bt4class")[0].to(cuda)
@@ -141,6 +142,31 @@ def test_padded_ffn_equals_the_model_with_the_zeros_in_its_weights(cuda, arch, f
         rows = [m.evaluate(planes[:n].contiguous()) for n in (1, 70)]
         hidden = m._engine.read_tensor("f8", (70 * 64, width))[:, :Fm] if fp8 else planes[0]
         out.append([t for r in rows for t in r] + [hidden])
+    for a, b in zip(*out):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("arch,Cm,Fm,FP", [("bt4class", 256, 248, 256), ("bt4class", 256, 1000, 1024), ("bt4", 512, 248, 256), ("bt4_calibrated", 256, 248, 256), ("bt4_calibrated", 256, 1000, 1024)])
+@pytest.mark.parametrize("act", ["bf16", "f16"])
+def test_padded_ffn_layers_in_16_bits(cuda, arch, Cm, Fm, FP, act):
+    """The same for the padded layers of 16-bit models that run them: BT4-class, BT4 whose hidden width is at most half the model's, and the calibration pass of any BT4, whose table of
+    maxima holds the hidden tensor's."""
+    L, H = 2, 8
+    oracle = om.BT4ClassOracle(policy_leela, L, Cm, Fm, H) if arch == "bt4class" else om.BT4Oracle(L, Cm, Fm, H)
+    sd = om.test_init_(oracle, seed=5).state_dict()
+    planes = positions(70, seed=6, leela=arch == "bt4class")[0].to(cuda)
+    zeros = torch.nn.functional.pad
+    pad = lambda k, v: zeros(v, (0, 0, 0, FP - Fm)) if "ff1.weight" in k else zeros(v, (0, FP - Fm)) if "ff1.bias" in k or "ff2.weight" in k else v
+    out = []
+    for width, state in ((Fm, sd), (FP, {k: pad(k, v) for k, v in sd.items()})):
+        m = (models.BT4Class if arch == "bt4class" else models.BT4)(L, Cm, width, H, act_dtype=act)
+        m.load_state_dict(state)
+        if arch == "bt4_calibrated":
+            m._engine.calibrate(planes)
+            out.append([torch.as_tensor(m._engine.get_amax())])
+            assert bool((out[-1][0][:, :4] > 0).all())
+        else:
+            out.append([t for n in (1, 70) for t in m.evaluate(planes[:n].contiguous())])
     for a, b in zip(*out):
         assert torch.equal(a, b)
 
@@ -966,8 +992,8 @@ def test_gpt_16bit_stream_does_not_take_the_norm_of_fp32_rows(cuda, n_head, n_em
 
 @pytest.mark.parametrize("kw", [{}, {"norm_rms": True}])
 def test_generate_rows_do_not_depend_on_the_batch(cuda, kw):
-    """Token steps of 1 to 160 sequences: norms inside the products, K of the residual products over four waves. Same sums for
-    every tile width, so a sequence's tokens and logits have the same bits in every such batch."""
+    """Token steps of 1 to 160 sequences: norms inside the products, residual products on tiles of 8 to 32 rows and columns. Same sums for
+    every tile, so a sequence's tokens and logits have the same bits in every such batch."""
     planes, _ = positions(160, seed=8)
     m = models.GPT(models.GPTConfig(block_size=256, vocab_size=1929, n_layer=2, n_head=12, n_embd=768), **kw)
     x = planes.to(cuda)
