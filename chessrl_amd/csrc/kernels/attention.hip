@@ -540,7 +540,7 @@ __global__ void __launch_bounds__(128, 2) relshift_kernel(const AttnArgs a, cons
 #pragma unroll 1
   for (int b = b0; b < a.B; b += slices) {
     __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_waitcnt(0x0F70 | NST);   // everything but the last position's stores: this one's queries or keys are there
+    __builtin_amdgcn_s_waitcnt(0x0F70 | NST);   // everything but the last position's stores, which follow this one's requests (loads and stores retire in order of issue): its queries or keys are there
     barrier();                                  // and the other wave's part; it is also through with the last position's shift and values
     __builtin_amdgcn_sched_barrier(0);
     f32x16_t s[2], sp[2];

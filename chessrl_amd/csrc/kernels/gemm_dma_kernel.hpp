@@ -43,6 +43,8 @@ template <int CHUNKS>
 __device__ __forceinline__ int dma_sw(int r) { return CHUNKS == 4 ? dma_swizzle(r) : lds_swizzle(r); }
 
 // s_waitcnt with only vmcnt constrained (gfx9 encoding: vmcnt[3:0] | expcnt[6:4] | lgkmcnt[11:8] | vmcnt_hi[15:14]).
+// vmcnt counts a wave's loads, into registers and into LDS, and its stores alike and goes down in the order they were issued, so a count tells that a load has landed whatever stores
+// have followed it. The compiler's own waits rest on the same: in front of the use of a load with two stores behind it gfx950 code waits for vmcnt(2).
 template <int N>
 __device__ __forceinline__ void wait_vmcnt() {
   __builtin_amdgcn_s_waitcnt((N & 0xF) | ((N >> 4) << 14) | (0x7 << 4) | (0xF << 8));

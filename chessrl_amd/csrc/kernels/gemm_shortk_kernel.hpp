@@ -182,9 +182,8 @@ __global__ void __launch_bounds__(ShortKCfg::NT, 2) gemm_shortk_kernel(const Gem
   };
 
   // The loop is rotated: iteration `step` writes out the result of step - 1 and then multiplies step. The wait in
-  // front of the barrier has to be for everything (loads and stores retire in no fixed order with respect to each
-  // other, so no count separates this step's weights from the stores before them); placed like this it finds the
-  // stores a whole MFMA phase old and the weights an epilogue and an MFMA phase old.
+  // front of the barrier is for everything, the stores behind this step's weights too (a count could leave them out,
+  // see wait_vmcnt); placed like this it finds the stores a whole MFMA phase old and the weights an epilogue and an MFMA phase old.
   for (int step = first; step <= last; ++step) {
     wait_vmcnt<0>();
     dmam_barrier();
