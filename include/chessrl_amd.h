@@ -170,7 +170,8 @@ int crl_rmsnorm(const void* x, int64_t ldx, int in_dtype, const float* gamma, vo
 /* Attention over 64 tokens per position, q/k/v of in_dtype (bf16 or f16) with head h at columns [h*head_dim, ...).
  * mode CAUSAL: model_bis.py:71; RELSHIFT: new_paradigm/attn.py:507-521 with pos = pos_proj(PE)
  * (in_dtype [64,H*head_dim]) and u_bias/v_bias fp32[H*head_dim]; BIAS: bias of in_dtype [B,H,64,64] in the
- * order crl_attn_bias_slot defines. out is of in_dtype or fp8 (value*out_scale) [B*64, ldo]. */
+ * order crl_attn_bias_slot defines. out is of in_dtype or fp8 (value*out_scale) [B*64, ldo]. q, k and v start at multiples
+ * of 16 bytes with row strides in multiples of 8 elements, ldo is a multiple of 4. */
 int crl_attention(const void* q, int64_t ldq, const void* k, int64_t ldk, const void* v, int64_t ldv, int in_dtype,
                   void* out, int64_t ldo, int out_dtype, float out_scale,
                   int B, int H, int head_dim, int mode, float scale,
@@ -313,7 +314,9 @@ int crl_model_search_1ply(crl_model* m, const char* const* fens, int n, int chun
 int crl_model_run_layers(crl_model* m, const float* x_in, int B, int first, int last, float* x_out, void* stream);
 int crl_model_read_tensor(crl_model* m, const char* name, void* out, int64_t bytes, void* stream);
 int crl_model_vocab(const crl_model* m);
-/* 2*MAC count of one position through this model (for roofline accounting). */
+/* 2*MAC count of one position through this model as its layers are defined (for roofline accounting). Work that a call does
+ * not execute is in it: BT4's two FFN layers count 4*64*d_model*d_ff per encoder layer also where 16-bit calls run them as one layer of
+ * 2*64*d_model^2 (d_model < 2*d_ff; crl_model_get_profile counts what is launched). */
 double crl_model_flops_per_position(const crl_model* m);
 /* Switch: bracket every kernel launch with HIP events on the call's stream; each forward then
  * ends with a stream synchronise and accumulates, per kernel family, the elapsed milliseconds,
