@@ -613,8 +613,8 @@ static hipError_t launch_in_out(const GemmArgs& a, int tile, hipStream_t st) {
   // that is what it is for: M = 131072, N = 4096 takes 280 us through the 256x256 tile, 310 us here row-major and 191 us
   // here in blocks, so nothing picks it for a row-major output unasked.
   if (a.c_blocked || tile == 13) return launch_gemm_shortk(a, IN_DT, OUT_DT, st);
-  // Token steps of generation, a tile of 32x32 per CU at most: the ring kernel (M=128, N=768, on average over K=768 and K=3072: 3.7 us, against 12.2 and 13.9 us for the two
-  // passes of the sliced form with the next norm on the second).
+  // Token steps of generation, a tile of 32x32 per CU at most: the ring kernel (M=128, N=768, kernel times by the profiler's trace: K=768 4.5 us, K=3072 6.9, against 10.3 and 12.8 for the two
+  // passes of the sliced form, without the launch gap between them).
   if (tile == 0 && a.k_parallel && !a.ln_out && !a.res_stats && ((long)a.K * (IN_DT == DT_FP8 ? 1 : 2)) % 128 == 0 && gemm_dmam_has(IN_DT, OUT_DT) &&
       (long)((a.M + 31) / 32) * ((a.N + 31) / 32) <= device_cus())
     return launch_gemm_dmas(a, IN_DT, OUT_DT, st, 32);
@@ -665,7 +665,7 @@ static hipError_t launch_in_out(const GemmArgs& a, int tile, hipStream_t st) {
         tile = big_rounds <= mid_rounds ? 3 : 11;
         // 128x192 (tile 17, where it serves the call): a round of 1.25 of the 128x128 tile's (K=1024: 13 us). It fills the gap where N cuts into a last round of few small tiles, or
         // one round of large ones that leaves CUs idle. Whole calls without and with it: BT4-class bf16 at 44, 64, 90, 180, 250 and 450 positions 1833 -> 1749 us, 1990 -> 1964,
-        // 2715 -> 2619, 4397 -> 4316, 5619 -> 5566 (f16), 8939 -> 8805; GPT at 32 and 128 454 -> 423 and 1018 -> 987. At 1.2, 200 positions lose 0.8 %, at 1.3 the gains at 160 and 250 go.
+        // 2715 -> 2619, 4397 -> 4316, 5619 -> 5566 (f16; about what two runs differ by), 8939 -> 8805; GPT at 32 and 128 454 -> 423 and 1018 -> 987. At 1.2, 200 positions lose 0.8 %, at 1.3 the gains at 160 and 250 go.
         // e4m3, 1.42: 44, 64, 112 and 250 positions 1351 -> 1298 us, 1502 -> 1463, 2178 -> 2127, 3844 -> 3788, none slower up to 1000; at 1.35 200 and 350 lose 1.7 and 3.3 %, at 1.5 the gains
         // at 112 and 250 go.
         const long wide = (long)((a.M + 127) / 128) * ((a.N + 191) / 192);

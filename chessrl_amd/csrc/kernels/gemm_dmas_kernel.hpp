@@ -8,9 +8,10 @@
 //  * The fragments of slab s + 1 are read from LDS between the MFMAs of slab s, which are one chain, and a wave issues in order.
 //  * The epilogue belongs to the loading waves: 512 threads need a third of the time one wave needs for a tile of 1024 elements,
 //    which is a chain of some 300 instructions there. Residual and bias are brought into LDS meanwhile by a wave of their own.
-//  * Everything the kernel needs to know travels in 128 bytes of arguments, requested at once (they are read from memory, cold,
+//  * Everything the kernel needs to know travels in 144 bytes of arguments, requested at once (they are read from memory, cold,
 //    before the first address can be formed).
-// Measured inside passes of one position (bf16, start to end of a launch, of which its first slab takes 1900 to 2800 cycles and its epilogue 1000): M = 64, N = 1024, K = 1024 2.5 us
+// Measured inside passes of one position (bf16, by the workgroups' own clock from their first to their last instruction, of which the first slab takes 1900 to 2800 cycles and the epilogue
+// 1000; launch and drain, which the profiler's trace counts too, come on top: 4.4 to 5.0 us a launch of one position there): M = 64, N = 1024, K = 1024 2.5 us
 // where the memory-side cache has the weights and 2.9 past it (3.0 and 4.1 on 32x32 tiles with 32x32x16 MFMAs), K = 1536 3.0 and 3.3 (3.7 and 5.6), N = 768, K = 3072 4.1 (5.7);
 // M = 128, N = 768, K = 3072 4.8 (7.3 with four waves on K). One position of 15 layers 685 -> 643 us, of GPT 182 -> 171; token steps of 128 sequences 51.1 -> 48.5 ms a rollout.
 // Same K order and same arithmetic per element as the other tiled kernels: bit-equal results.
@@ -462,8 +463,7 @@ static hipError_t launch_dmas(const GemmArgs& a, hipStream_t st, int shares = 1,
   s.act = a.act; s.res_dtype = a.res_dtype; s.res_rows = a.res_rows; s.vec_ok = a.vec_ok;
   s.descale = a.descale; s.alpha = a.alpha; s.out_scale = a.out_scale;
   // Rows or columns of tiles first, whichever lets an XCD read fewer rows of both operands: each XCD's L2 fetches its own copy (BT4-class bf16, whole calls
-  // of 2, 4 and 8 positions: 850 -> 835, 912 -> 868, 1083 -> 1065 us). Two rows of tiles gain nothing, and the K-shared form of 128 rows, 768
-  // columns, K = 3072 loses 0.5 us a launch: rows first there.
+  // of 2, 4 and 8 positions: 850 -> 835, 912 -> 868, 1083 -> 1065 us). Two rows of tiles gain nothing.
   const int tiles_m = tiles / tiles_n, per = std::max(tiles >> 3, 1);
   const int by_rows = (per + tiles_n - 1) / tiles_n * bm + std::min(per, tiles_n) * bn, by_cols = (per + tiles_m - 1) / tiles_m * bn + std::min(per, tiles_m) * bm;
   s.by_cols = tiles_m >= 4 && by_cols < by_rows;

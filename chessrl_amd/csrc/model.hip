@@ -497,7 +497,7 @@ struct GOpt {
   float out_scale = 1.f;
   float* amax = nullptr;
   void* C2 = nullptr; long ldc2 = 0; int nsplit = 0;
-  bool k_parallel = false;  // token steps of generation: few rows, so K is spread over more waves (different summation order)
+  bool k_parallel = false;  // token steps of generation: products that the small tiles do not take may cut K into slices or groups (different summation order)
   // LayerNorm that follows this GEMM, to be folded into it where the GEMM kernel can (*ln_folded says whether it did).
   const float* ln_g = nullptr; const float* ln_b = nullptr; void* ln_out = nullptr; int ln_dt = DT_BF16; bool* ln_folded = nullptr;
   // The residual is LayerNorm(res), normalised in the epilogue from these row statistics, gain and offset.

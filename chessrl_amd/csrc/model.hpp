@@ -75,8 +75,8 @@ struct Model {
     return (padded - cfg.d_ff) * 16 <= cfg.d_ff ? padded : cfg.d_ff;
   }
   // BT4's FFN has nothing between its two linear layers (new_paradigm/value.py:65-70): in 16 bits it runs as the one layer W2 W1 with bias W2 b1 + b2, wherever
-  // that is the smaller product. Its rounding is that of one weight where there were two weights and the hidden tensor. 31744 rows, 512 columns, 736 hidden: two products of
-  // 30 and 32 us, one of 20; in e4m3 the layers stay apart, each with its own scales.
+  // that is the smaller product. Its rounding is that of one weight where there were two weights and the hidden tensor. 31744 rows, 512 columns, 736 hidden, kernel times by the
+  // profiler's trace: two products of 40 and 39 us, one of 32; in e4m3 the layers stay apart, each with its own scales.
   bool folds_ffn() const { return cfg.arch == CRL_ARCH_BT4 && !cfg.fp8 && cfg.d_model < 2 * cfg.d_ff; }
   // q and k columns of the concatenated q|k|v weight paired head by head (BT4-class with 64-byte head rows)
   bool qk_paired() const { return cfg.arch == CRL_ARCH_BT4CLASS && cfg.d_model / cfg.n_head == 32; }

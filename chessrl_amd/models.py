@@ -470,7 +470,7 @@ class _ModelBase:
 
 class GraphedEvaluator:
     """forward + legal-masked softmax for one fixed batch size, recorded once into a HIP graph and
-    replayed per call: the 160 kernels of a call (15 layers of BT4-class) are issued as one graph
+    replayed per call: the 160 kernels of a call (15 layers of BT4-class; 131 at one position) are issued as one graph
     launch, for hosts that cannot keep up with them one by one. The library calls
     record no memset nodes (flags and scratch are cleared by kernels)."""
 
