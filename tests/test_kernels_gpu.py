@@ -491,6 +491,26 @@ def test_gemm_small_tiles_of_fewer_rows_or_columns_equal_the_register_staged(cud
         assert not behind.any()
 
 
+@pytest.mark.parametrize("M,N,K", [(16, 64, 768), (33, 904, 1088), (128, 768, 768)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_gemm_small_tiles_equal_the_register_staged_on_values_at_the_edges(cuda, M, N, K, dtype):
+    """The small tiles' 16x16x32 MFMAs against 32x32x16 ones where sums could part: subnormal operands, products below the normal range, exponents far apart, sums beyond the largest finite
+    value, terms that cancel, infinities and NaN. The same bits (NaN in the same places)."""
+    torch.manual_seed(M)
+    far = 14 if dtype == torch.float16 else 60
+    scales = {"subnormal": 2.0 ** (-16 if dtype == torch.float16 else -128), "tiny products": 2.0 ** -70, "huge": 2.0 ** (far + 2), "cancel": 1.0, "inf": 1.0}
+    for kind in ("subnormal", "tiny products", "apart", "huge", "cancel", "inf"):
+        draw = lambda n: (torch.randn(n, K, device=cuda) * (torch.exp2(torch.randint(-far, far, (n, K), device=cuda).float()) if kind == "apart" else scales[kind])).to(dtype)
+        A, W = draw(M), torch.randn(N, K, device=cuda).to(dtype) if kind == "subnormal" else draw(N)
+        if kind == "cancel":
+            A[:, K // 2:], W[:, K // 2:] = A[:, :K // 2].clone(), -W[:, :K // 2]
+        if kind == "inf":
+            A.view(-1)[::1977], A.view(-1)[5::2231] = float("inf"), float("nan")
+        out = _lib.F16 if dtype == torch.float16 else _lib.F32
+        small, ref = run_gemm(A, W, out, tile=16), run_gemm(A, W, out, tile=1)
+        assert torch.equal(small.isnan(), ref.isnan()) and torch.equal(small[~ref.isnan()], ref[~ref.isnan()]), kind
+
+
 @pytest.mark.parametrize("M,N", [(1, 8192), (250, 8192), (1279, 8192), (1281, 8192), (2048, 6144), (2048, 6160), (4100, 8192), (3000, 12301)])
 @pytest.mark.parametrize("dt", ["bf16", "f16", "fp8"])
 def test_gemm_short_k_either_side_of_the_tile_rule(cuda, M, N, dt):
